@@ -82,6 +82,79 @@ def test_ce_rows_kernel_vs_fp64(vocab):
     assert np.all(grad_bits[~valid] == 0)
 
 
+@pytest.mark.parametrize("vocab", [
+    3, 8, 2048, 2056, 4104, 6152, 8200, 10240,       # one wave a row, 4 to 20 vectors a thread
+    10248, 12296, 16392, 20480, 20488, 24585, 40960,  # two and four waves
+    40968, 81920, 81928, 98312, 163840, 163843,       # eight and sixteen waves
+    163848, 165000,                                   # too long for registers
+])
+def test_ce_rows_at_the_edges_of_the_row_shapes(vocab):
+    """The row kernel on both sides of every change of its threads and vectors a row: losses and
+    gradients against fp64, the loss-only pass bit for bit equal, -inf, NaN and +inf where only
+    some threads or batches see them, and nothing written past the rows. Bounds: a sum of
+    positive exponentials in fp32 is off by at most one rounding of 2^-24 per addition on the
+    longest chain: 20 vectors of 3 levels, 5 rescales and 10 merges on the vector path (38, and 3
+    an exponential), vocab / 1024 on an odd row's element path; lse moves by that plus its own
+    roundings, and a gradient is one bf16 rounding of a value that close."""
+    from torchure_amd import _native
+
+    lib, st = _native.lib(), _native.stream_handle(DEV)
+    g = torch.Generator(device=DEV).manual_seed(vocab)
+    rows = 13
+    buf = torch.zeros(rows * vocab + 16, dtype=torch.bfloat16, device=DEV)
+    buf[rows * vocab:] = 7.0
+    x = buf[: rows * vocab].view(rows, vocab)
+    x.copy_(torch.randn(rows, vocab, device=DEV, generator=g) * 3.0)
+    x[1, : vocab // 2] = float("-inf")       # whole threads' vectors
+    x[2, : max(1, vocab - 2)] = float("-inf")
+    x[3] = 3.390625e38                       # equal to the largest finite values
+    x[4] -= 300.0
+    x[5, vocab // 3] = float("nan")
+    x[6] = float("-inf")
+    x[6, vocab - 1] = float("nan")           # a NaN under a maximum of -inf elsewhere
+    x[7, vocab // 2] = float("inf")
+    labels = torch.randint(0, vocab, (rows,), device=DEV, generator=g)
+    labels[1:3] = vocab - 1
+    labels[8] = -100
+    xd = x.double()
+    loss_only, loss = torch.empty(rows, device=DEV), torch.empty(rows, device=DEV)
+    for fn, out in ((lib.tm_ce_rows_loss_bf16, loss_only), (lib.tm_ce_rows_bf16, loss)):
+        _native.check(fn(x.data_ptr(), vocab, labels.data_ptr(), rows, vocab, -100, out.data_ptr(), st), "rows")
+    assert torch.equal(loss_only.view(torch.int32), loss.view(torch.int32))
+    assert (buf[rows * vocab:] == 7.0).all()
+    fine = [r for r in range(rows) if r not in (5, 6, 7)]
+    lse = torch.logsumexp(xd, dim=1)
+    want = lse - xd.gather(1, labels.clamp_min(0)[:, None])[:, 0]
+    want[8] = 0.0
+    chain = 41 + (vocab // 1024 if vocab % 8 else 0)
+    tol = 2.0 ** -24 * (chain + 2 * lse.abs())
+    assert ((loss.double() - want).abs() <= tol)[fine].all(), (loss, want)
+    assert loss[5].isnan() and loss[6].isnan() and not loss[7].isfinite()
+    probs = torch.exp(xd - lse[:, None])
+    probs[torch.arange(rows), labels.clamp_min(0)] -= 1.0
+    probs[8] = 0.0
+    got = x.double()
+    # one rounding (2^-9 relative), the exponent's error at |lse|, and the p - 1 of a sure label
+    off = (got - probs).abs() - (2.0 ** -8 * probs.abs() + (4e-6 + 2.0 ** -22 * lse.abs()[:, None].clamp_max(512)))
+    assert (off <= 0)[fine].all(), off[fine].max()
+    assert got[5].isnan().all() and got[6].isnan().all()
+
+
+def test_ce_rows_beyond_one_launch_of_single_waves():
+    """More rows than one launch of 64-thread workgroups holds."""
+    from torchure_amd import _native
+
+    rows, v = 0xFFFFFFFF // 64 + 77, 2
+    x = torch.zeros(rows, v, dtype=torch.bfloat16, device=DEV)
+    x[:, 1] = (torch.arange(rows, device=DEV) % 5).to(torch.bfloat16)
+    labels = torch.zeros(rows, dtype=torch.int64, device=DEV)
+    loss = torch.empty(rows, device=DEV)
+    _native.check(_native.lib().tm_ce_rows_loss_bf16(x.data_ptr(), v, labels.data_ptr(), rows, v, -100,
+                                                     loss.data_ptr(), _native.stream_handle(DEV)), "rows")
+    want = torch.log1p(torch.exp(torch.arange(5, device=DEV).double()))[torch.arange(rows, device=DEV) % 5]
+    torch.testing.assert_close(loss.double(), want, rtol=1e-6, atol=1e-6)
+
+
 def test_ce_rows_beyond_one_launch():
     """More rows than one launch of 1024-thread blocks holds (2^32 work-items): the
     entry point splits them, and every row still matches an fp64 restatement (here in

@@ -5,11 +5,12 @@
 //   grad_logits = bf16(softmax - onehot) on valid rows (0 on ignored rows),
 //   grad_h = grad_logits @ W, grad_W += grad_logits^T @ h,
 // and scales both grads by grad_out / n_valid in backward (:94-127).
-// The GEMMs are plain library GEMMs (hipBLASLt). These kernels do the rest:
+// The GEMMs are in tm_ce_gemm.hip. These kernels do the rest:
 //   ce_rows_kernel        one workgroup per row: row max, sum of exp, target logit,
 //                         per-row loss, then softmax - onehot written back over the
 //                         logits as bf16 (RNE). A row of up to kRegCols vectors per
-//                         thread stays in registers (one HBM read, one write); longer
+//                         thread (1 to 16 waves by the vocabulary) stays in registers
+//                         (one HBM read, one write); longer
 //                         rows use an online (max, sum-of-exp) read, then a second
 //                         read for the write pass. exp is the hardware base-2 exp
 //                         (full-range exp2f wherever a result would be denormal), and
@@ -35,11 +36,11 @@
 
 namespace {
 
-constexpr int kRowThreadsRegs = 1024;   // 16 wave64 per row when the row stays in registers
+constexpr int kRowThreadsMax = 1024;    // 16 wave64 on a row of the largest vocabularies kept in registers
 constexpr int kRowThreadsStream = 256;  // threads per row on the streaming path (longer rows)
 constexpr int kStreamUnroll = 4;  // vectors per thread loaded together on the streaming path
-constexpr int kRegCols = 20;  // 8-element vectors per thread kept in registers (V <= 163,840)
-constexpr int kMaxWaves = (kRowThreadsRegs > kRowThreadsStream ? kRowThreadsRegs : kRowThreadsStream) / 64;
+constexpr int kRegCols = 20;  // most 8-element vectors per thread kept in registers (V <= 163,840)
+constexpr int kMaxWaves = kRowThreadsMax / 64;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -133,63 +134,66 @@ __device__ __forceinline__ void block_ms(float& m, float& s) {
   __syncthreads();
 }
 
-template <int kCeThreads>
-__device__ __forceinline__ float block_max(float m) {
-  constexpr int kCeWaves = kCeThreads / 64;
-  __shared__ float lm[kMaxWaves];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-  if ((threadIdx.x & 63) == 0) lm[threadIdx.x >> 6] = m;
-  __syncthreads();
-  m = lm[0];
-  for (int w = 1; w < kCeWaves; ++w) m = fmaxf(m, lm[w]);
-  __syncthreads();
-  return m;
+// (m, s) and (m2, s2) combined against the larger maximum (0 where both are -inf): unlike
+// ms_merge, a NaN sum under a maximum of -inf (a part of the row that is all NaN) is kept.
+__device__ __forceinline__ void ms_join(float& m, float& s, float m2, float s2) {
+  const float top = fmaxf(m, m2);
+  const float ref = top == -INFINITY ? 0.0f : top;
+  s = s * exp_shift(m, ref) + s2 * exp_shift(m2, ref);
+  m = top;
 }
 
-// Block-wide max of a and max of b in one reduction (b carries a negated minimum).
+// Block-wide (max, sum of exp) and maximum of b (a negated minimum) in one fixed-order
+// reduction; every thread receives the results.
 template <int kCeThreads>
-__device__ __forceinline__ void block_max2(float& a, float& b) {
+__device__ __forceinline__ void block_join(float& m, float& s, float& b) {
   constexpr int kCeWaves = kCeThreads / 64;
-  __shared__ float la[kMaxWaves], lb[kMaxWaves];
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
-    a = fmaxf(a, __shfl_xor(a, off, 64));
+    const float m2 = __shfl_xor(m, off, 64), s2 = __shfl_xor(s, off, 64);
+    ms_join(m, s, m2, s2);
     b = fmaxf(b, __shfl_xor(b, off, 64));
   }
-  if ((threadIdx.x & 63) == 0) {
-    la[threadIdx.x >> 6] = a;
-    lb[threadIdx.x >> 6] = b;
-  }
-  __syncthreads();
-  a = la[0];
-  b = lb[0];
-  for (int w = 1; w < kCeWaves; ++w) {
-    a = fmaxf(a, la[w]);
-    b = fmaxf(b, lb[w]);
-  }
-  __syncthreads();
-}
-
-template <int kCeThreads>
-__device__ __forceinline__ float block_sum_f(float s) {
-  constexpr int kCeWaves = kCeThreads / 64;
-  __shared__ float ls[kMaxWaves];
+  if constexpr (kCeWaves > 1) {
+    __shared__ float lm[kMaxWaves], ls[kMaxWaves], lb[kMaxWaves];
+    if ((threadIdx.x & 63) == 0) {
+      lm[threadIdx.x >> 6] = m;
+      ls[threadIdx.x >> 6] = s;
+      lb[threadIdx.x >> 6] = b;
+    }
+    __syncthreads();
+    // every wave reduces the waves' results itself, in lanes (a serial walk over 16 of them took
+    // a chain of 32 exponentials)
+    const int w = threadIdx.x & (kCeWaves - 1);
+    m = lm[w];
+    s = ls[w];
+    b = lb[w];
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  if ((threadIdx.x & 63) == 0) ls[threadIdx.x >> 6] = s;
-  __syncthreads();
-  s = ls[0];
-  for (int w = 1; w < kCeWaves; ++w) s += ls[w];
-  __syncthreads();
-  return s;
+    for (int off = kCeWaves / 2; off > 0; off >>= 1) {
+      const float m2 = __shfl_xor(m, off, 64), s2 = __shfl_xor(s, off, 64);
+      ms_join(m, s, m2, s2);
+      b = fmaxf(b, __shfl_xor(b, off, 64));
+    }
+  }
 }
 
 // logits: rows x vocab bf16 (row-major, row stride ld elements), overwritten with
 // grad_logits (kGrad; without it the logits are only read). labels: int64 per row.
 // row_loss: fp32 per row (0 for ignored rows).
-template <bool kInRegs, int kCeThreads, bool kGrad>
-__global__ __launch_bounds__(kCeThreads) void ce_rows_kernel(uint16_t* __restrict__ logits,
+//
+// kCols > 0: the row stays in registers, kCols vectors of 8 a thread (kCols * kCeThreads * 8 >=
+// vocab); kCols = 0: a row too long for them. Bound: HBM, at 4 bytes an element (2 without the
+// gradient), once enough rows are in flight. A workgroup goes through load, reduce, exponentials
+// and stores in series, so a CU needs other rows to load while one reduces: the fewest waves
+// whose registers hold the row (row_shape) leave room for 16 rows a CU up to a vocabulary of
+// 10,240, 4 at 32,768 and one from 81,921 up, where a row fills the register file. A fixed
+// 1024 threads of 20 vectors had one row a CU at every vocabulary, and reloaded the last vector
+// in place of the missing ones. Measured on MI355X, logits not in cache, fixed / this shape:
+//   8192 x 4096: 253 / 26 us (5.2 TB/s); 4096 x 32,768: 188 / 109 us; 4096 x 81,920: 304 / 249 us;
+//   8192 x 151,936: 965 / 965 us (5.2 TB/s), 1024 rows of it 143 / 131 us; loss only 475 / 364 us
+//   (6.8 TB/s: with 12 vectors held instead of the row, two rows a CU).
+template <int kCols, int kCeThreads, bool kGrad>
+__global__ __launch_bounds__(kCeThreads, kGrad ? 4 : 8) void ce_rows_kernel(uint16_t* __restrict__ logits,
                                                              int64_t ld,
                                                              const int64_t* __restrict__ labels,
                                                              int64_t vocab, int64_t ignore_index,
@@ -202,68 +206,90 @@ __global__ __launch_bounds__(kCeThreads) void ce_rows_kernel(uint16_t* __restric
   const bool vec = ((reinterpret_cast<uint64_t>(row) & 15u) == 0);
   const int64_t vend = vec ? nvec * 8 : 0;
 
-  u32x4 keep[kInRegs ? kRegCols : 1];
+  constexpr bool kInRegs = kCols > 0;
+  constexpr int kBatch = 4;                                       // vectors a thread takes together
+  constexpr int kHeld = kGrad ? kCols : (kCols < 12 ? kCols : 12);  // vectors a thread holds
+  u32x4 keep[kInRegs ? kHeld : 1];
   float lse;
   float row_min = -INFINITY;  // known only on the register path
   if constexpr (kInRegs) {
-    // The row stays in registers: max pass, then sum-of-exp pass, no second read.
-    float m = -INFINITY;
-    float nmin = -INFINITY;  // -(row minimum), reduced with the maximum
+    // Each thread keeps a running (max, sum of exp) over batches of kBatch vectors, so a batch
+    // is reduced while the later ones are still loading. With the gradient the whole row stays
+    // in registers, every load issued before any is used; the loss alone needs each batch once
+    // and holds three. Compile-time indices keep `keep` in VGPRs. A thread past the row's last
+    // vector loads that vector again, a real element of the row, which leaves the max and min as
+    // they are; the sum and the stores below skip those slots. The loss-only pass reads the row
+    // non-temporally (3-22% faster than temporal loads from 1024 to 8192 rows of the Qwen3
+    // vocabulary, same bits); the gradient pass, which rewrites the row, measured no better with
+    // them at 2048 rows and beyond.
+    float m = -INFINITY, s = 0.0f;
+    float nmin = -INFINITY;  // -(row minimum), for the gradient pass
     if (vec && nvec > 0) {
-      // Every load is issued before any is used (fully unrolled, compile-time indices, so
-      // `keep` stays in VGPRs): a load under a per-thread branch next to its use made each
-      // of them wait for the one before. A thread past the row's last vector loads that
-      // last vector again, a real element of the row, which leaves the max and min as they
-      // are; the sum and the stores below skip those slots. The loss-only pass reads the
-      // row non-temporally: 3-22% faster than temporal loads from 1024 to 8192 rows of the
-      // Qwen3 vocabulary (same bits); the gradient pass, which rewrites the row, measured
-      // no better with them at 2048 rows and beyond.
-#pragma unroll
-      for (int k = 0; k < kRegCols; ++k) {
+      auto load = [&](int k) {
         const int64_t v = threadIdx.x + static_cast<int64_t>(k) * kCeThreads;
         const u32x4* src = reinterpret_cast<const u32x4*>(row + (v < nvec ? v : nvec - 1) * 8);
-        keep[k] = kGrad ? *src : __builtin_nontemporal_load(src);
-      }
+        keep[k % kHeld] = kGrad ? *src : __builtin_nontemporal_load(src);
+      };
+#pragma unroll
+      for (int k = 0; k < kHeld; ++k) load(k);
       __builtin_amdgcn_sched_barrier(0);  // keep the scheduler from starting the max before the last load
 #pragma unroll
-      for (int k = 0; k < kRegCols; ++k) {
-        const u32x4 w = keep[k];
-        m = fmaxf(m, fmaxf(fmaxf(fmaxf(lo16(w.x), hi16(w.x)), fmaxf(lo16(w.y), hi16(w.y))),
-                           fmaxf(fmaxf(lo16(w.z), hi16(w.z)), fmaxf(lo16(w.w), hi16(w.w)))));
-        nmin = fmaxf(nmin, -fminf(fminf(fminf(lo16(w.x), hi16(w.x)), fminf(lo16(w.y), hi16(w.y))),
-                                  fminf(fminf(lo16(w.z), hi16(w.z)), fminf(lo16(w.w), hi16(w.w)))));
-      }
-    }
-    for (int64_t i = vend + threadIdx.x; i < vocab; i += kCeThreads) {
-      const float x = __uint_as_float(static_cast<uint32_t>(row[i]) << 16);
-      m = fmaxf(m, x);
-      nmin = fmaxf(nmin, -x);
-    }
-    block_max2<kCeThreads>(m, nmin);
-    row_min = -nmin;
-    const float cm = m * kLog2e;
-    // terms below 2^-126 (flushed by the bare exp) cannot move a sum that is >= 1
-    auto sum_exp = [&](auto fold) {
-      constexpr bool F = decltype(fold)::value;
-      float acc = 0.0f;
+      for (int k0 = 0; k0 < kCols; k0 += kBatch) {
+        float top = m;
 #pragma unroll
-      for (int k = 0; k < kRegCols; ++k) {
-        const int64_t v = threadIdx.x + static_cast<int64_t>(k) * kCeThreads;
-        if (v < nvec) {
-          const u32x4 w = keep[k];
-          acc += exp2_hw(tlog2<F>(lo16(w.x), m, cm)) + exp2_hw(tlog2<F>(hi16(w.x), m, cm)) +
-                 exp2_hw(tlog2<F>(lo16(w.y), m, cm)) + exp2_hw(tlog2<F>(hi16(w.y), m, cm)) +
-                 exp2_hw(tlog2<F>(lo16(w.z), m, cm)) + exp2_hw(tlog2<F>(hi16(w.z), m, cm)) +
-                 exp2_hw(tlog2<F>(lo16(w.w), m, cm)) + exp2_hw(tlog2<F>(hi16(w.w), m, cm));
+        for (int k = k0; k < k0 + kBatch; ++k) {
+          const u32x4 w = keep[k % kHeld];
+          top = fmaxf(top, fmaxf(fmaxf(fmaxf(lo16(w.x), hi16(w.x)), fmaxf(lo16(w.y), hi16(w.y))),
+                                 fmaxf(fmaxf(lo16(w.z), hi16(w.z)), fmaxf(lo16(w.w), hi16(w.w)))));
+          if (kGrad)
+            nmin = fmaxf(nmin, -fminf(fminf(fminf(lo16(w.x), hi16(w.x)), fminf(lo16(w.y), hi16(w.y))),
+                                      fminf(fminf(lo16(w.z), hi16(w.z)), fminf(lo16(w.w), hi16(w.w)))));
+        }
+        // the compiler must finish the minimum here and unpack the vectors again for each use: put
+        // off, or kept unpacked, the row's elements take twice the registers and spill
+        asm volatile("" : "+v"(nmin));
+        auto opaque = [&] {
+#pragma unroll
+          for (int k = k0; k < k0 + kBatch; ++k)
+            asm volatile("" : "+v"(keep[k % kHeld]));
+        };
+        opaque();
+        const float ref = top == -INFINITY ? 0.0f : top;
+        // terms below 2^-126 (flushed by the bare exp) cannot move a sum that is >= 1
+        s = s * exp2_hw(tlog2<false>(m, ref, 0.0f));
+        m = top;
+#pragma unroll
+        for (int k = k0; k < k0 + kBatch; ++k) {
+          if (threadIdx.x + static_cast<int64_t>(k) * kCeThreads < nvec) {
+            const u32x4 w = keep[k % kHeld];
+            auto e = [&](float x) { return exp2_hw(tlog2<false>(x, ref, 0.0f)); };
+            s += ((e(lo16(w.x)) + e(hi16(w.x))) + (e(lo16(w.y)) + e(hi16(w.y)))) +
+                 ((e(lo16(w.z)) + e(hi16(w.z))) + (e(lo16(w.w)) + e(hi16(w.w))));
+          }
+        }
+        opaque();
+        __builtin_amdgcn_sched_barrier(0);  // and one batch's exponentials at a time
+        if (!kGrad) {
+#pragma unroll
+          for (int k = k0 + kHeld; k < k0 + kHeld + kBatch && k < kCols; ++k) load(k);
         }
       }
-      return acc;
-    };
-    float s = 0.0f;
-    if (vec) s = fabsf(m) <= kFoldMax ? sum_exp(std::true_type{}) : sum_exp(std::false_type{});
-    for (int64_t i = vend + threadIdx.x; i < vocab; i += kCeThreads)
-      s += exp_shift(__uint_as_float(static_cast<uint32_t>(row[i]) << 16), m);
-    s = block_sum_f<kCeThreads>(s);
+    }
+    if (vend < vocab) {  // the last few elements, or a row that is not 16-byte aligned
+      float top = m;
+      for (int64_t i = vend + threadIdx.x; i < vocab; i += kCeThreads) {
+        const float x = __uint_as_float(static_cast<uint32_t>(row[i]) << 16);
+        top = fmaxf(top, x);
+        nmin = fmaxf(nmin, -x);
+      }
+      const float ref = top == -INFINITY ? 0.0f : top;
+      s = s * exp_shift(m, ref);
+      m = top;
+      for (int64_t i = vend + threadIdx.x; i < vocab; i += kCeThreads)
+        s += exp_shift(__uint_as_float(static_cast<uint32_t>(row[i]) << 16), ref);
+    }
+    block_join<kCeThreads>(m, s, nmin);
+    row_min = -nmin;
     lse = m + logf(s);
   } else {
     // Row too long for registers: one online (max, sum-of-exp) read, one write pass.
@@ -364,11 +390,13 @@ __global__ __launch_bounds__(kCeThreads) void ce_rows_kernel(uint16_t* __restric
     __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(row + b));
   };
   auto write_row = [&](auto fold_tag) {
-    if constexpr (kInRegs) {
+    if constexpr (kInRegs && kGrad) {
 #pragma unroll
-      for (int k = 0; k < kRegCols; ++k) {
+      for (int k = 0; k < kCols; ++k) {
         const int64_t v = threadIdx.x + static_cast<int64_t>(k) * kCeThreads;
-        if (v < nvec) put8(keep[k], v, fold_tag);
+        u32x4 w = keep[k];
+        asm volatile("" : "+v"(w));  // unpacked here, not before the branches
+        if (v < nvec) put8(w, v, fold_tag);
       }
     } else {
       int64_t v = threadIdx.x;
@@ -636,8 +664,57 @@ int ce_check_launch(const char* what) {
   return TM_OK;
 }
 
-// One block per row. The kernel (register or streaming path) depends only on the vocabulary,
-// so the loss-only pass runs the same arithmetic as the gradient pass and gives the same bits.
+// Threads a row and vectors a thread of the register path: the fewest waves whose threads hold
+// the row in at most kRegCols vectors each, then the smallest count compiled that covers it.
+// cols = 0: the row is too long for registers (streaming path).
+struct RowShape {
+  int threads, cols;
+};
+
+RowShape row_shape(int64_t vocab, bool aligned) {
+  const int64_t nvec = vocab >> 3;
+  // rows off 16 bytes go element by element (but for the aligned one in eight): as many threads
+  // as a row takes (87 us against 114 for 1024 rows of 32,001 with 256 threads a row)
+  for (int threads = aligned ? 64 : kRowThreadsMax; threads <= kRowThreadsMax; threads *= 2) {
+    if (nvec > static_cast<int64_t>(threads) * kRegCols) continue;
+    const int need = static_cast<int>((nvec + threads - 1) / threads);
+    const int least = threads == 64 ? 4 : 12;
+    return {threads, need <= least ? least : (need + 3) / 4 * 4};
+  }
+  return {kRowThreadsStream, 0};
+}
+
+struct RowArgs {
+  uint16_t* logits;
+  int64_t ld;
+  const int64_t* labels;
+  int64_t vocab, ignore_index;
+  float* row_loss;
+  uint32_t rows;
+  hipStream_t stream;
+};
+
+template <int kCols, int kThreads, bool kGrad>
+void row_launch(const RowArgs& a) {
+  hipLaunchKernelGGL((ce_rows_kernel<kCols, kThreads, kGrad>), dim3(a.rows), dim3(kThreads), 0, a.stream, a.logits,
+                     a.ld, a.labels, a.vocab, a.ignore_index, a.row_loss);
+}
+
+// More than one wave a row means more than kRegCols / 2 vectors a thread.
+template <int kThreads, bool kGrad>
+void row_launch_cols(int cols, const RowArgs& a) {
+  if constexpr (kThreads == 64) {
+    if (cols == 4) return row_launch<4, kThreads, kGrad>(a);
+    if (cols == 8) return row_launch<8, kThreads, kGrad>(a);
+  }
+  if (cols == 12) return row_launch<12, kThreads, kGrad>(a);
+  if (cols == 16) return row_launch<16, kThreads, kGrad>(a);
+  row_launch<20, kThreads, kGrad>(a);
+}
+
+// One block per row. The kernel (register or streaming path, and its shape) depends only on the
+// vocabulary, so the loss-only pass runs the same arithmetic as the gradient pass and gives the
+// same bits.
 template <bool kGrad>
 int ce_rows_launch(uint16_t* d_logits, int64_t ld, const int64_t* d_labels, int64_t rows, int64_t vocab,
                    int64_t ignore_index, float* d_row_loss, void* stream, const char* who) {
@@ -646,20 +723,20 @@ int ce_rows_launch(uint16_t* d_logits, int64_t ld, const int64_t* d_labels, int6
                    (long long)vocab, (long long)ld);
   if (rows == 0) return TM_OK;
   if (!d_logits || !d_labels || !d_row_loss) return ce_fail(TM_EINVAL, "%s: null pointer", who);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool regs = (vocab >> 3) <= static_cast<int64_t>(kRowThreadsRegs) * kRegCols;
+  const RowShape shape = row_shape(vocab, ld % 8 == 0 && (reinterpret_cast<uintptr_t>(d_logits) & 15u) == 0);
   // a launch holds fewer than 2^32 work-items: longer row lists (small vocabularies in one
   // chunk) go in several launches
-  const int64_t max_rows = 0xFFFFFFFFll / (regs ? kRowThreadsRegs : kRowThreadsStream);
+  const int64_t max_rows = 0xFFFFFFFFll / shape.threads;
   for (int64_t r0 = 0; r0 < rows; r0 += max_rows) {
-    const uint32_t nr = static_cast<uint32_t>(rows - r0 < max_rows ? rows - r0 : max_rows);
-    uint16_t* lg = d_logits + r0 * ld;
-    if (regs)
-      hipLaunchKernelGGL((ce_rows_kernel<true, kRowThreadsRegs, kGrad>), dim3(nr), dim3(kRowThreadsRegs), 0, s,
-                         lg, ld, d_labels + r0, vocab, ignore_index, d_row_loss + r0);
-    else
-      hipLaunchKernelGGL((ce_rows_kernel<false, kRowThreadsStream, kGrad>), dim3(nr), dim3(kRowThreadsStream),
-                         0, s, lg, ld, d_labels + r0, vocab, ignore_index, d_row_loss + r0);
+    const RowArgs a = {d_logits + r0 * ld, ld, d_labels + r0, vocab, ignore_index, d_row_loss + r0,
+                       static_cast<uint32_t>(rows - r0 < max_rows ? rows - r0 : max_rows),
+                       static_cast<hipStream_t>(stream)};
+    if (shape.cols == 0) row_launch<0, kRowThreadsStream, kGrad>(a);
+    else if (shape.threads == 64) row_launch_cols<64, kGrad>(shape.cols, a);
+    else if (shape.threads == 128) row_launch_cols<128, kGrad>(shape.cols, a);
+    else if (shape.threads == 256) row_launch_cols<256, kGrad>(shape.cols, a);
+    else if (shape.threads == 512) row_launch_cols<512, kGrad>(shape.cols, a);
+    else row_launch_cols<1024, kGrad>(shape.cols, a);
     if (int rc = ce_check_launch(who)) return rc;
   }
   return TM_OK;
