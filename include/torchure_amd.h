@@ -386,6 +386,34 @@ int tm_ce_logits_bf16(uint16_t* d_logits, const uint16_t* d_hidden, const uint16
 int tm_ce_grad_w_bf16(uint16_t* d_grad_w, const uint16_t* d_grad_logits, const uint16_t* d_hidden, int64_t rows,
                       int64_t vocab, int64_t dim, void* stream);
 
+/*
+ * The chunk's kernels on padded logits, so that any row count and vocabulary runs on the same
+ * MFMA kernels: a chunk's logits are pad_rows x ld, ld a multiple of 8 (of 64 for grad_h, or at
+ * least the vocabulary's next multiple of 64), of which rows x vocab are used.
+ *   tm_ce_logits_ld_bf16     tm_ce_logits_bf16 into rows ld >= vocab elements apart; with ld a
+ *                            multiple of 8, columns vocab .. (next multiple of 8) - 1 of a row are
+ *                            overwritten with unspecified values.
+ *   tm_ce_rows_padded_bf16   tm_ce_rows_bf16 on the first `rows` rows; the rest of the buffer,
+ *                            columns vocab .. ld - 1 and rows rows .. pad_rows - 1, becomes 0.
+ *   tm_ce_grad_h_ld_bf16     tm_ce_grad_h_bf16 for any rows and vocab and dim a multiple of 8;
+ *                            columns vocab .. (next multiple of 64) - 1 must be 0. d_ws holds
+ *                            tm_ce_grad_h_ld_workspace_bytes(rows, vocab, dim) bytes.
+ *   tm_ce_grad_w_ld_bf16     tm_ce_grad_w_bf16 for any rows and vocab: rows rows .. pad_rows - 1
+ *                            of d_grad_logits must be 0 (pad_rows a multiple of 64, less than 512
+ *                            past rows); d_hidden has `rows` rows.
+ * A padding zero times any finite value adds nothing; where the last weight or hidden row holds
+ * an infinity or a NaN, its own products already make the same outputs NaN.
+ */
+int tm_ce_logits_ld_bf16(uint16_t* d_logits, int64_t ld, const uint16_t* d_hidden, const uint16_t* d_weight,
+                         int64_t rows, int64_t vocab, int64_t dim, void* stream);
+int tm_ce_rows_padded_bf16(uint16_t* d_logits, int64_t ld, const int64_t* d_labels, int64_t rows, int64_t pad_rows,
+                           int64_t vocab, int64_t ignore_index, float* d_row_loss, void* stream);
+size_t tm_ce_grad_h_ld_workspace_bytes(int64_t rows, int64_t vocab, int64_t dim);
+int tm_ce_grad_h_ld_bf16(uint16_t* d_grad_h, const uint16_t* d_grad_logits, int64_t ld, const uint16_t* d_w,
+                         int64_t rows, int64_t vocab, int64_t dim, void* d_ws, size_t ws_bytes, void* stream);
+int tm_ce_grad_w_ld_bf16(uint16_t* d_grad_w, const uint16_t* d_grad_logits, int64_t ld, int64_t pad_rows,
+                         const uint16_t* d_hidden, int64_t rows, int64_t vocab, int64_t dim, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

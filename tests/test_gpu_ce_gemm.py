@@ -449,6 +449,102 @@ def test_grad_w_ring_kernel_equals_one_tile_kernel(rows, vocab, dim):
     assert torch.equal(ring, tile)
 
 
+@pytest.mark.parametrize("rows,vocab,dim", [
+    (1, 1, 64),            # one element of one tile; 63 rows and columns of padding
+    (63, 65, 64),          # one short of a K slice, one past
+    (65, 1001, 128),       # two row slices: the one-tile grad_W kernel, its last slice ragged
+    (129, 1003, 192),      # persistent kernels from here: 3 K slices for the logits (their minimum)
+    (255, 4095, 320),      # 5 K slices (odd: the ring's stages alternate between tiles)
+    (257, 4097, 320),      # one row and column past the tile
+    (300, 7169, 448),      # 7 K slices
+    (1000, 32001, 768),
+    (513, 640, 1216),      # 19 K slices
+    (384, 4160, 192),      # aligned rows and vocabulary, odd slices
+])
+def test_padded_chunk_kernels_on_ragged_shapes(rows, vocab, dim):
+    """The chunk's kernels on padded logits: the logits equal to tm_ce_logits_bf16 bit for bit, the
+    padding zero after the row kernel and the rows those of tm_ce_rows_bf16 on an aligned copy,
+    grad_h and grad_W within one bf16 ulp of the exact product plus 2^-20 of the absolute sum (as
+    the unpadded GEMMs). The rows after the hidden states and the weight hold NaN, which one load
+    past either would bring into every output; guards around the outputs stay as they were."""
+    from torchure_amd.loss.fused_linear_ce import padded_rows, padded_vocab
+
+    native, lib, stream = _lib()
+    g = torch.Generator(device=DEV).manual_seed(rows * 3 + vocab * 5 + dim)
+
+    def fenced(n, d, std):
+        t = torch.full((n + 160, d), float("nan"), dtype=torch.bfloat16, device=DEV)
+        t[:n] = (torch.randn(n, d, device=DEV, generator=g) * std).to(torch.bfloat16)
+        return t[:n]
+
+    def guarded(*shape):
+        n = shape[0] * shape[1]
+        buf = torch.full((n + 128,), -12345, dtype=torch.int16, device=DEV)
+        return buf, buf[64: 64 + n].view(torch.bfloat16).view(shape)
+
+    def intact(buf):
+        return bool((buf[:64] == -12345).all()) and bool((buf[-64:] == -12345).all())
+
+    h, w = fenced(rows, dim, 1.0), fenced(vocab, dim, 0.05)
+    pad, ld = padded_rows(rows), padded_vocab(vocab)
+    assert pad % 64 == 0 and ld % 64 == 0 and rows <= pad < rows + 256 and vocab <= ld < vocab + 64
+    buf, logits = guarded(pad, ld)
+    logits.fill_(float("nan"))
+    native.check(lib.tm_ce_logits_ld_bf16(logits.data_ptr(), ld, h.data_ptr(), w.data_ptr(), rows, vocab, dim, stream),
+                 "logits")
+    plain, _ = _logits(h, w)
+    assert torch.equal(logits[:rows, :vocab].view(torch.int16), plain.view(torch.int16))
+    assert bool(logits[rows:].isnan().all())
+    labels = torch.randint(0, vocab, (rows,), device=DEV, generator=g)
+    labels[::7] = -100
+    loss, want_loss = torch.empty(rows, device=DEV), torch.empty(rows, device=DEV)
+    aligned = torch.zeros(rows, ld, dtype=torch.bfloat16, device=DEV)
+    aligned[:, :vocab] = plain
+    native.check(lib.tm_ce_rows_padded_bf16(logits.data_ptr(), ld, labels.data_ptr(), rows, pad, vocab, -100,
+                                            loss.data_ptr(), stream), "rows")
+    native.check(lib.tm_ce_rows_bf16(aligned.data_ptr(), ld, labels.data_ptr(), rows, vocab, -100,
+                                     want_loss.data_ptr(), stream), "rows")
+    assert torch.equal(loss.view(torch.int32), want_loss.view(torch.int32))
+    assert torch.equal(logits[:rows, :vocab].view(torch.int16), aligned[:, :vocab].view(torch.int16))
+    assert bool((logits[rows:] == 0).all()) and bool((logits[:, vocab:] == 0).all()) and intact(buf)
+
+    a, wd, hd = logits[:rows, :vocab].double(), w.double(), h.double()
+
+    def check(out, want, absum):
+        d = (out.double() - want).abs()
+        assert bool((d <= _bf16_ulp(torch.maximum(out.double().abs(), want.abs())) + absum * 2.0 ** -20).all())
+
+    nbytes = lib.tm_ce_grad_h_ld_workspace_bytes(rows, vocab, dim)
+    ws = torch.full((nbytes,), 0x7F, dtype=torch.uint8, device=DEV)
+    buf, gh = guarded(rows, dim)
+    native.check(lib.tm_ce_grad_h_ld_bf16(gh.data_ptr(), logits.data_ptr(), ld, w.data_ptr(), rows, vocab, dim,
+                                          ws.data_ptr(), nbytes, stream), "grad_h")
+    check(gh, a @ wd, a.abs() @ wd.abs())
+    assert intact(buf)
+    buf, gw = guarded(vocab, dim)
+    native.check(lib.tm_ce_grad_w_ld_bf16(gw.data_ptr(), logits.data_ptr(), ld, pad, h.data_ptr(), rows, vocab, dim,
+                                          stream), "grad_w")
+    check(gw, a.t().contiguous() @ hd, a.abs().t().contiguous() @ hd.abs())
+    assert intact(buf)
+
+
+def test_padded_chunk_kernels_argument_checks():
+    """Strides, paddings and sizes that the padded kernels do not take are refused before a launch."""
+    native, lib, stream = _lib()
+    t = torch.empty(1 << 16, dtype=torch.bfloat16, device=DEV)
+    p = t.data_ptr()
+    assert lib.tm_ce_logits_ld_bf16(p, 63, p, p, 8, 64, 64, stream) < 0       # rows shorter than vocab
+    for ld, rows, pad in ((100, 8, 8), (64, 8, 7), (64, 0, 8)):
+        assert lib.tm_ce_rows_padded_bf16(p, ld, p, rows, pad, 60, -100, p, stream) < 0
+    assert lib.tm_ce_rows_padded_bf16(p + 2, 64, p, 8, 8, 60, -100, p, stream) < 0
+    for ld, rows, vocab, dim in ((64, 8, 65, 64), (100, 8, 100, 64), (64, 8, 64, 60), (64, 0, 64, 64)):
+        assert lib.tm_ce_grad_h_ld_bf16(p, p, ld, p, rows, vocab, dim, p, 1 << 30, stream) < 0
+    assert lib.tm_ce_grad_h_ld_bf16(p, p, 64, p, 8, 64, 64, p, 16, stream) < 0  # workspace too small
+    for ld, pad, rows, vocab, dim in ((64, 100, 100, 64, 64), (64, 64, 65, 64, 64), (64, 1024, 64, 64, 64),
+                                      (60, 64, 64, 60, 64), (64, 64, 64, 65, 64), (64, 64, 64, 64, 60)):
+        assert lib.tm_ce_grad_w_ld_bf16(p, p, ld, pad, p, rows, vocab, dim, stream) < 0
+
+
 def test_grad_w_gemm_argument_checks():
     """Row counts off a multiple of 64, vocab or dim off a multiple of 8 and misaligned pointers
     are refused before any launch."""

@@ -179,7 +179,8 @@ __device__ __forceinline__ void block_join(float& m, float& s, float& b) {
 
 // logits: rows x vocab bf16 (row-major, row stride ld elements), overwritten with
 // grad_logits (kGrad; without it the logits are only read). labels: int64 per row.
-// row_loss: fp32 per row (0 for ignored rows).
+// row_loss: fp32 per row (0 for ignored rows). Columns vocab .. width - 1, and rows from n_rows
+// on, are padding that the gradient pass sets to zero for the GEMMs (width = vocab: no padding).
 //
 // kCols > 0: the row stays in registers, kCols vectors of 8 a thread (kCols * kCeThreads * 8 >=
 // vocab); kCols = 0: a row too long for them. Bound: HBM, at 4 bytes an element (2 without the
@@ -197,9 +198,15 @@ __global__ __launch_bounds__(kCeThreads, kGrad ? 4 : 8) void ce_rows_kernel(uint
                                                              int64_t ld,
                                                              const int64_t* __restrict__ labels,
                                                              int64_t vocab, int64_t ignore_index,
-                                                             float* __restrict__ row_loss) {
+                                                             float* __restrict__ row_loss, int64_t n_rows,
+                                                             int64_t width) {
   const int64_t r = blockIdx.x;
   uint16_t* row = logits + r * ld;
+  if (kGrad && r >= n_rows) {  // a padding row, 16-byte aligned and whole vectors
+    for (int64_t v = threadIdx.x; v < width / 8; v += kCeThreads)
+      __builtin_nontemporal_store(u32x4{0u, 0u, 0u, 0u}, reinterpret_cast<u32x4*>(row + v * 8));
+    return;
+  }
   const int64_t label = labels[r];
   const bool valid = label != ignore_index;
   const int64_t nvec = vocab >> 3;  // full 8-element vectors (16 B)
@@ -417,6 +424,7 @@ __global__ __launch_bounds__(kCeThreads, kGrad ? 4 : 8) void ce_rows_kernel(uint
   }
   for (int64_t i = vend + threadIdx.x; i < vocab; i += kCeThreads)
     row[i] = static_cast<uint16_t>(rne16(g_of(__uint_as_float(static_cast<uint32_t>(row[i]) << 16), i)));
+  for (int64_t i = vocab + threadIdx.x; i < width; i += kCeThreads) row[i] = 0;
 }
 
 // (max, sum of exp(x - max)) with the full-precision expf, for fp32 outputs.
@@ -690,14 +698,15 @@ struct RowArgs {
   const int64_t* labels;
   int64_t vocab, ignore_index;
   float* row_loss;
-  uint32_t rows;
+  uint32_t blocks;
+  int64_t rows, width;
   hipStream_t stream;
 };
 
 template <int kCols, int kThreads, bool kGrad>
 void row_launch(const RowArgs& a) {
-  hipLaunchKernelGGL((ce_rows_kernel<kCols, kThreads, kGrad>), dim3(a.rows), dim3(kThreads), 0, a.stream, a.logits,
-                     a.ld, a.labels, a.vocab, a.ignore_index, a.row_loss);
+  hipLaunchKernelGGL((ce_rows_kernel<kCols, kThreads, kGrad>), dim3(a.blocks), dim3(kThreads), 0, a.stream, a.logits,
+                     a.ld, a.labels, a.vocab, a.ignore_index, a.row_loss, a.rows, a.width);
 }
 
 // More than one wave a row means more than kRegCols / 2 vectors a thread.
@@ -716,20 +725,21 @@ void row_launch_cols(int cols, const RowArgs& a) {
 // vocabulary, so the loss-only pass runs the same arithmetic as the gradient pass and gives the
 // same bits.
 template <bool kGrad>
-int ce_rows_launch(uint16_t* d_logits, int64_t ld, const int64_t* d_labels, int64_t rows, int64_t vocab,
-                   int64_t ignore_index, float* d_row_loss, void* stream, const char* who) {
+int ce_rows_launch(uint16_t* d_logits, int64_t ld, const int64_t* d_labels, int64_t rows, int64_t pad_rows,
+                   int64_t vocab, int64_t width, int64_t ignore_index, float* d_row_loss, void* stream,
+                   const char* who) {
   if (rows < 0 || vocab <= 0 || ld < vocab)
     return ce_fail(TM_EINVAL, "%s: bad sizes rows=%lld vocab=%lld ld=%lld", who, (long long)rows,
                    (long long)vocab, (long long)ld);
-  if (rows == 0) return TM_OK;
+  if (rows == 0) return TM_OK;  // pad_rows is 0 too, or the caller's check has refused it
   if (!d_logits || !d_labels || !d_row_loss) return ce_fail(TM_EINVAL, "%s: null pointer", who);
   const RowShape shape = row_shape(vocab, ld % 8 == 0 && (reinterpret_cast<uintptr_t>(d_logits) & 15u) == 0);
   // a launch holds fewer than 2^32 work-items: longer row lists (small vocabularies in one
   // chunk) go in several launches
   const int64_t max_rows = 0xFFFFFFFFll / shape.threads;
-  for (int64_t r0 = 0; r0 < rows; r0 += max_rows) {
+  for (int64_t r0 = 0; r0 < pad_rows; r0 += max_rows) {
     const RowArgs a = {d_logits + r0 * ld, ld, d_labels + r0, vocab, ignore_index, d_row_loss + r0,
-                       static_cast<uint32_t>(rows - r0 < max_rows ? rows - r0 : max_rows),
+                       static_cast<uint32_t>(pad_rows - r0 < max_rows ? pad_rows - r0 : max_rows), rows - r0, width,
                        static_cast<hipStream_t>(stream)};
     if (shape.cols == 0) row_launch<0, kRowThreadsStream, kGrad>(a);
     else if (shape.threads == 64) row_launch_cols<64, kGrad>(shape.cols, a);
@@ -826,14 +836,23 @@ extern "C" {
 
 int tm_ce_rows_bf16(uint16_t* d_logits, int64_t ld, const int64_t* d_labels, int64_t rows,
                     int64_t vocab, int64_t ignore_index, float* d_row_loss, void* stream) {
-  return ce_rows_launch<true>(d_logits, ld, d_labels, rows, vocab, ignore_index, d_row_loss, stream,
+  return ce_rows_launch<true>(d_logits, ld, d_labels, rows, rows, vocab, vocab, ignore_index, d_row_loss, stream,
                               "tm_ce_rows_bf16");
+}
+
+int tm_ce_rows_padded_bf16(uint16_t* d_logits, int64_t ld, const int64_t* d_labels, int64_t rows, int64_t pad_rows,
+                           int64_t vocab, int64_t ignore_index, float* d_row_loss, void* stream) {
+  if (rows < 1 || pad_rows < rows || ld % 8 || (reinterpret_cast<uintptr_t>(d_logits) & 15u))
+    return ce_fail(TM_EINVAL, "tm_ce_rows_padded_bf16: rows %lld of %lld, 16-byte aligned rows wanted (ld %lld)",
+                   (long long)rows, (long long)pad_rows, (long long)ld);
+  return ce_rows_launch<true>(d_logits, ld, d_labels, rows, pad_rows, vocab, ld, ignore_index, d_row_loss, stream,
+                              "tm_ce_rows_padded_bf16");
 }
 
 int tm_ce_rows_loss_bf16(const uint16_t* d_logits, int64_t ld, const int64_t* d_labels, int64_t rows,
                          int64_t vocab, int64_t ignore_index, float* d_row_loss, void* stream) {
   // the kGrad=false kernels only read the logits
-  return ce_rows_launch<false>(const_cast<uint16_t*>(d_logits), ld, d_labels, rows, vocab, ignore_index,
+  return ce_rows_launch<false>(const_cast<uint16_t*>(d_logits), ld, d_labels, rows, rows, vocab, vocab, ignore_index,
                                d_row_loss, stream, "tm_ce_rows_loss_bf16");
 }
 

@@ -1,7 +1,8 @@
 // tm_ce_gemm.hip -- gfx950 bf16 MFMA GEMMs of the fused linear + cross-entropy, per chunk of rows
 // (torchure/loss/fused_linear_ce.py:38,52,57: bf16 matmuls, fp32 accumulation, bf16 results):
-//   logits_ring_kernel   logits = h W^T         (rows x V, K = D), persistent, for dim a multiple
-//                        of 128 (>= 256) and vocab a multiple of 8; logits_gemm_kernel otherwise
+//   logits_ring_kernel   logits = h W^T         (rows x V, K = D), persistent, for dim at least
+//                        192 and logits rows a multiple of 8 elements apart; logits_gemm_kernel
+//                        otherwise
 //   grad_h_gemm_kernel   grad_h = grad_logits W (rows x D, K = V), split over K, reading W as it
 //                        is stored (V x D), with
 //   grad_h_reduce_kernel summing the fp32 partials of each element over the splits in a fixed
@@ -244,8 +245,8 @@ __device__ __forceinline__ void nt_mainloop(const uint16_t* __restrict__ A, cons
 }
 
 __global__ __launch_bounds__(256) void logits_gemm_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
-                                                          uint16_t* __restrict__ C, int M, int N, int K, int tiles_m,
-                                                          int tiles_n, int gm, int gn) {
+                                                          uint16_t* __restrict__ C, int M, int N, int64_t ldc, int K,
+                                                          int tiles_m, int tiles_n, int gm, int gn) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int T = tiles_m * tiles_n;
   const int t8 = (T + 7) / 8;
@@ -284,14 +285,14 @@ __global__ __launch_bounds__(256) void logits_gemm_kernel(const uint16_t* __rest
       }
   __builtin_amdgcn_s_waitcnt(0);  // this wave reads back only its own rows
   const int mb = m0 + wm * 128, nb = n0 + wn * 128;
-  const bool vec = (N & 7) == 0;
+  const bool vec = (ldc & 7) == 0;
 #pragma unroll 4
   for (int it = 0; it < 32; ++it) {
     const int mr = it * 4 + (lane >> 4), ch = lane & 15;
     const int m = mb + mr, n = nb + ch * 8;
     if (m >= M) continue;
     const u32x4 v = *(const u32x4*)(tile + mr * kLgPitch + ch * 16);
-    uint16_t* dst = C + static_cast<int64_t>(m) * N + n;
+    uint16_t* dst = C + m * ldc + n;
     if (vec && n + 8 <= N) {
       __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dst));  // streamed out: keep L2 for operands
     } else {
@@ -304,8 +305,9 @@ __global__ __launch_bounds__(256) void logits_gemm_kernel(const uint16_t* __rest
 // ------------------------------------------------ logits, persistent: one workgroup per CU
 //
 // The same product, tiles, fragments and summation order as logits_gemm_kernel (bit-identical
-// results), for the shapes the Qwen heads have (dim a multiple of 128 and at least 256, vocab a
-// multiple of 8, operands under 4 GiB). With K = dim short (16 slices at dim 1024), a tile's
+// results), for dim a multiple of 64 and at least 192, rows of the logits a multiple of 8 elements
+// apart, operands under 4 GiB (1024 x 768 x 32,001 with rows padded to 32,064: 47 us, against 100
+// on logits_gemm_kernel with rows 32,001 apart). With K = dim short (16 slices at dim 1024), a tile's
 // fill (its first two stages' loads) and its epilogue (its accumulators converted to bf16 and
 // written) were a large share of a tile's time; here both overlap the neighbouring tiles' MFMAs:
 //   - workgroup c of XCD x (blockIdx = 8 c + x) runs tile positions x t8 + c, + W, + 2W, ...
@@ -342,8 +344,8 @@ struct RgBool {
 };
 
 __global__ __launch_bounds__(512) void logits_ring_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
-                                                          uint16_t* __restrict__ C, int M, int N, int K, int tiles_m,
-                                                          int tiles_n, int gm, int gn, int wpx) {
+                                                          uint16_t* __restrict__ C, int M, int N, int ldc, int K,
+                                                          int tiles_m, int tiles_n, int gm, int gn, int wpx) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int T = tiles_m * tiles_n;
   const int t8 = (T + 7) / 8;
@@ -354,7 +356,8 @@ __global__ __launch_bounds__(512) void logits_ring_kernel(const uint16_t* __rest
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave >> 2, wn = wave & 3;
-  const int n_it = K / kSliceK;  // even, >= 4
+  const int n_it = K / kSliceK;  // >= 3
+  int par = 0;                   // the stage that holds the current tile's slice 0
 
   // Waves 0-3 load the A rows of the tile, waves 4-7 the B rows; load j of wave w fills rows
   // 64 (w % 4) + 8 j + lane / 8 of its operand, the lane's chunk (lane % 8) ^ (lane / 16) ^ (4 (j % 2)).
@@ -396,7 +399,7 @@ __global__ __launch_bounds__(512) void logits_ring_kernel(const uint16_t* __rest
     const int r = k * 8 + (lane >> 3);
     ra[k] = ebo + r * 128 + (((lane & 7) ^ ((r >> 1) & 7)) << 4);
   }
-  uint32_t sl = static_cast<uint32_t>(((lane >> 3) * N + (lane & 7) * 8) * 2);  // byte offset of the lane's store
+  uint32_t sl = static_cast<uint32_t>(((lane >> 3) * ldc + (lane & 7) * 8) * 2);  // byte offset of the lane's store
 
 #define TM_RD(dst, base, imm) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(base), "i"(imm))
 #define TM_WAIT6(f) \
@@ -430,11 +433,11 @@ __global__ __launch_bounds__(512) void logits_ring_kernel(const uint16_t* __rest
     for (int it = 0; it < 4; ++it) asm volatile("ds_read_b128 %0, %1" : "=v"(v[it]) : "v"(ra[it]));
     asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
     const int rows_left = M - (pm0 + wm * 128 + jj * 32), cols_left = N - (pn0 + wn * 64);
-    char* qb = reinterpret_cast<char*>(C) + (static_cast<int64_t>(pm0 + wm * 128 + jj * 32) * N + pn0 + wn * 64) * 2;
+    char* qb = reinterpret_cast<char*>(C) + (static_cast<int64_t>(pm0 + wm * 128 + jj * 32) * ldc + pn0 + wn * 64) * 2;
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
       if (it * 8 + (lane >> 3) < rows_left && (lane & 7) * 8 < cols_left)
-        __builtin_nontemporal_store(v[it], reinterpret_cast<u32x4*>(qb + (sl + static_cast<uint32_t>(it * 8 * N * 2))));
+        __builtin_nontemporal_store(v[it], reinterpret_cast<u32x4*>(qb + (sl + static_cast<uint32_t>(it * 8 * ldc * 2))));
     }
   };
 
@@ -469,7 +472,7 @@ __global__ __launch_bounds__(512) void logits_ring_kernel(const uint16_t* __rest
     auto stage = [&](int i, auto step) {
       constexpr bool kNext2 = decltype(step)::kNext2V, kPre = decltype(step)::kPreV;
       constexpr bool kFirst = decltype(step)::kFirstV, kEpi = decltype(step)::kEpiV;
-      const int s = i & 1;
+      const int s = (i + par) & 1;
       const uint32_t soff_s = s * kLgStage, noff = (s ^ 1) * kLgStage;
       if (kPre) {
         set_src(m0n, n0n);
@@ -529,6 +532,7 @@ __global__ __launch_bounds__(512) void logits_ring_kernel(const uint16_t* __rest
     for (int i = 1; i < n_it - 2; ++i) stage(i, RgFlags<true, false, false, false>{});
     stage(n_it - 2, RgFlags<true, true, false, false>{});
     stage(n_it - 1, RgFlags<true, false, false, false>{});
+    par = (par + n_it) & 1;  // an odd number of slices leaves the next tile's slice 0 in the other stage
     pm0 = m0;
     pn0 = n0;
   };
@@ -551,11 +555,12 @@ __global__ __launch_bounds__(512) void logits_ring_kernel(const uint16_t* __rest
 #undef TM_WAIT6
 }
 
-// The ring kernel's preconditions: K slices in an even number >= 4, whole 8-column store groups,
+// The ring kernel's preconditions: at least 3 K slices (a tile's first stage must not be the one
+// that already loads the next tile), whole 8-column store groups in a logits row of ld elements,
 // 32-bit operand offsets and store offsets.
-bool logits_ring_fits(int64_t rows, int64_t vocab, int64_t dim) {
-  return dim % 128 == 0 && dim >= 256 && vocab % 8 == 0 && rows * dim * 2 < (int64_t(1) << 32) &&
-         vocab * dim * 2 < (int64_t(1) << 32) && 32 * vocab * 2 < (int64_t(1) << 32);
+bool logits_ring_fits(int64_t rows, int64_t vocab, int64_t dim, int64_t ld) {
+  return dim % kSliceK == 0 && dim >= 3 * kSliceK && ld % 8 == 0 && rows * dim * 2 < (int64_t(1) << 32) &&
+         vocab * dim * 2 < (int64_t(1) << 32) && 32 * ld * 2 < (int64_t(1) << 31);
 }
 
 // ------------------------------------------------- grad_h = grad_logits @ W, K split over workgroups
@@ -575,19 +580,25 @@ bool logits_ring_fits(int64_t rows, int64_t vocab, int64_t dim) {
 // reads and 8 MFMAs per K16 step; 8 loads a stage a wave: waves 0-3 G, waves 4-7 W). Measured on
 // MI355X: as fast as, or up to 6% faster than, the same schedule on W^T (the bits are the same),
 // which also needed the transpose (0.13 ms at dim 1024, 0.34 at 2560).
+//
+// kRagged: rows or dim off a multiple of 256, or a vocabulary off a multiple of 64. Loads past the
+// last row, column group or weight row take the last one; G's rows are `ld` elements apart with
+// zeros from vocab to the next multiple of 64, so the weight row loaded again in the last K slice
+// meets zeros; the stores of rows and columns past the edge are left out.
 
+template <bool kRagged>
 __global__ __launch_bounds__(512) void grad_h_gemm_kernel(const uint16_t* __restrict__ G, const uint16_t* __restrict__ W,
-                                                          float* __restrict__ partials, int rows, int dim, int64_t K,
-                                                          int tiles, int splits, int iters_per_split) {
+                                                          float* __restrict__ partials, int rows, int dim, int64_t ld,
+                                                          int vocab, int tiles, int splits, int iters_per_split) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int pairs = tiles * splits;
   const int p8 = (pairs + 7) / 8;
   const int p = (blockIdx.x % 8) * p8 + blockIdx.x / 8;
   if (p >= pairs) return;
   const int s = p / tiles, tile = p - s * tiles;
-  const int tiles_n = dim / kLgTile;
+  const int tiles_n = kRagged ? (dim + kLgTile - 1) / kLgTile : dim / kLgTile;
   const int m0 = (tile / tiles_n) * kLgTile, n0 = (tile % tiles_n) * kLgTile;
-  const int total = static_cast<int>(K / kSliceK);
+  const int total = (vocab + kSliceK - 1) / kSliceK;
   const int it0 = s * iters_per_split;
   const int n_it = max(0, min(iters_per_split, total - it0));
   const int lane = threadIdx.x & 63;
@@ -605,16 +616,23 @@ __global__ __launch_bounds__(512) void grad_h_gemm_kernel(const uint16_t* __rest
     if (wave < 4) {
       const int r = (wave % 4) * 64 + 8 * j + lane / 8;
       const int c = (lane % 8) ^ ((r >> 1) & 7);
-      src[j] = G + static_cast<int64_t>(min(m0 + r, rows - 1)) * K + k0 + c * 8;
+      src[j] = G + static_cast<int64_t>(min(m0 + r, rows - 1)) * ld + k0 + c * 8;
     } else {
       const int kr = (wave % 4) * 16 + 2 * j + lane / 32;
       const int c = (lane % 32) ^ (4 * (kr & 3));
-      src[j] = W + (k0 + kr) * dim + n0 + 8 * c;
+      src[j] = W + (k0 + kr) * dim + (kRagged ? min(n0 + 8 * c, dim - 8) : n0 + 8 * c);
     }
   }
   const int64_t step = wave < 4 ? kSliceK : static_cast<int64_t>(kSliceK) * dim;  // elements per stage
+  // the slice (if it is this split's) with weight rows past the vocabulary
+  const int it_last = kRagged && vocab % kSliceK != 0 ? total - 1 - it0 : -1;
   auto load = [&](int it, int stage, int j) {
-    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(src[j] + it * step),
+    const uint16_t* from = src[j] + it * step;
+    if (kRagged && it == it_last && wave >= 4) {
+      const int64_t past = k0 + it * kSliceK + (wave % 4) * 16 + 2 * j + lane / 32 - (vocab - 1);
+      if (past > 0) from -= past * dim;
+    }
+    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)from,
                                      (void __attribute__((address_space(3)))*)(smem + stage * kLgStage + (wave * 8 + j) * 1024),
                                      16, 0, 0);
   };
@@ -719,7 +737,7 @@ __global__ __launch_bounds__(512) void grad_h_gemm_kernel(const uint16_t* __rest
         const int m = m0 + wm * 128 + jj * 32 + (lane & 31);
         const int n = n0 + wn * 64 + ii * 32 + 8 * q + 4 * (lane >> 5);
         const f32x4 v = {acc[ii][jj][4 * q], acc[ii][jj][4 * q + 1], acc[ii][jj][4 * q + 2], acc[ii][jj][4 * q + 3]};
-        *(f32x4*)(P + static_cast<int64_t>(m) * dim + n) = v;
+        if (!kRagged || (m < rows && n < dim)) *(f32x4*)(P + static_cast<int64_t>(m) * dim + n) = v;
       }
 }
 
@@ -736,13 +754,16 @@ __global__ __launch_bounds__(512) void grad_h_gemm_kernel(const uint16_t* __rest
 // rows 0-3 of column i; two such reads (rows +0 and +4) make a fragment. The slot swizzle puts
 // the 4 rows of a read, and the 32 columns two 16-lane groups read together, on 16 different
 // 16-byte bank groups. Columns past vocab or dim load a clamped (valid) column and are not stored.
+// G's rows are `ldg` elements apart. K rows are contracted, a multiple of 64; kRagged: H has only
+// k_rows of them, and G's rows past those are zero (a load of a later H row takes the last one).
 
 constexpr int kGwOp = 64 * 512;       // one operand's stage: 64 rows x 256 bf16
 constexpr int kGwStage = 2 * kGwOp;   // 64 KB
 
+template <bool kRagged>
 __global__ __launch_bounds__(256) void grad_w_gemm_kernel(const uint16_t* __restrict__ G, const uint16_t* __restrict__ H,
-                                                          uint16_t* __restrict__ C, int V, int D, int K, int tiles_v,
-                                                          int tiles_d, int gm, int gn) {
+                                                          uint16_t* __restrict__ C, int V, int ldg, int D, int K,
+                                                          int k_rows, int tiles_v, int tiles_d, int gm, int gn) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int T = tiles_v * tiles_d;
   const int t8 = (T + 7) / 8;
@@ -765,14 +786,19 @@ __global__ __launch_bounds__(256) void grad_w_gemm_kernel(const uint16_t* __rest
     const int q = wave * 16 + j;
     const int kr = 2 * (q % 32) + lane / 32;
     const int c = (lane % 32) ^ (4 * (kr & 3));
-    src[j] = q < 32 ? G + static_cast<int64_t>(kr) * V + min(v0 + 8 * c, V - 8)
+    src[j] = q < 32 ? G + static_cast<int64_t>(kr) * ldg + min(v0 + 8 * c, ldg - 8)
                     : H + static_cast<int64_t>(kr) * D + min(d0 + 8 * c, D - 8);
   }
-  const int64_t step_g = static_cast<int64_t>(kSliceK) * V, step_h = static_cast<int64_t>(kSliceK) * D;
+  const int64_t step_g = static_cast<int64_t>(kSliceK) * ldg, step_h = static_cast<int64_t>(kSliceK) * D;
   auto load = [&](int it, int stage, int j) {
     const int q = wave * 16 + j;
+    const uint16_t* from = src[j] + it * (q < 32 ? step_g : step_h);
+    if (kRagged && q >= 32 && (it + 1) * kSliceK > k_rows) {
+      const int64_t past = it * kSliceK + 2 * (q % 32) + lane / 32 - (k_rows - 1);
+      if (past > 0) from -= past * D;
+    }
     __builtin_amdgcn_global_load_lds(
-        (const void __attribute__((address_space(1)))*)(src[j] + it * (q < 32 ? step_g : step_h)),
+        (const void __attribute__((address_space(1)))*)from,
         (void __attribute__((address_space(3)))*)(smem + stage * kGwStage + q * 1024), 16, 0, 0);
   };
   // Fragment of 32-column block b at K16 step kk: lane l (s = l % 16) reads row
@@ -898,12 +924,15 @@ __global__ __launch_bounds__(256) void grad_w_gemm_kernel(const uint16_t* __rest
 // 8 MFMAs per K16 step; measured on MI355X: 4-10% faster than one wave a SIMD, the same bits);
 // the finished tile's accumulators are converted and staged block by block during the next tile's
 // first K16 step (32 vocab rows x the wave's 64 dim columns at a time through the wave's 4 KB past
-// the stages) and written as 128-byte row pieces of grad_W. For rows (K) a multiple of 128 and at
-// least 256, vocab and dim multiples of 8, operands under 4 GiB; grad_w_gemm_kernel otherwise.
+// the stages) and written as 128-byte row pieces of grad_W. For rows (K, with their padding) a
+// multiple of 128 and at least 256, dim a multiple of 8, operands under 4 GiB; grad_w_gemm_kernel
+// otherwise.
 
+template <bool kRagged>
 __global__ __launch_bounds__(512) void grad_w_ring_kernel(const uint16_t* __restrict__ G, const uint16_t* __restrict__ H,
-                                                          uint16_t* __restrict__ C, int V, int D, int K, int tiles_v,
-                                                          int tiles_d, int gm, int gn, int wpx) {
+                                                          uint16_t* __restrict__ C, int V, int ldg, int D, int K,
+                                                          int k_rows, int tiles_v, int tiles_d, int gm, int gn,
+                                                          int wpx) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int T = tiles_v * tiles_d;
   const int t8 = (T + 7) / 8;
@@ -920,10 +949,11 @@ __global__ __launch_bounds__(512) void grad_w_ring_kernel(const uint16_t* __rest
   // 16 (wave % 4) + 2 j + lane / 32, slot lane % 32 taking chunk (lane % 32) ^ (4 (row & 3)) =
   // (lane % 32) ^ (4 (lane / 32)) ^ (8 (j % 2)).
   const char* opnd = reinterpret_cast<const char*>(wave < 4 ? G : H);
-  const int ld = wave < 4 ? V : D;
+  const int ld = wave < 4 ? ldg : D;
   const int lim8 = ld - 8;
   const uint32_t step = static_cast<uint32_t>(kSliceK) * static_cast<uint32_t>(ld) * 2u;  // bytes per stage
   uint32_t soff[8];
+  uint32_t cap[2] = {0xFFFFFFFFu, 0xFFFFFFFFu};  // kRagged: last H row's offsets, even and odd j
   int lkr = lane >> 5;
   int lc = (lane & 31) ^ (4 * (lane >> 5));
   auto set_src = [&](int v0, int d0) {
@@ -934,11 +964,15 @@ __global__ __launch_bounds__(512) void grad_w_ring_kernel(const uint16_t* __rest
     for (int j = 0; j < 8; ++j) {
       const int kr = r0 + 2 * j + lkr;
       const int c = lc ^ (8 * (j & 1));
-      soff[j] = (static_cast<uint32_t>(kr) * static_cast<uint32_t>(ld) + static_cast<uint32_t>(min(col0 + 8 * c, lim8))) * 2u;
+      const uint32_t col = static_cast<uint32_t>(min(col0 + 8 * c, lim8));
+      soff[j] = (static_cast<uint32_t>(kr) * static_cast<uint32_t>(ld) + col) * 2u;
+      if (kRagged && j < 2 && wave >= 4) cap[j] = (static_cast<uint32_t>(k_rows - 1) * static_cast<uint32_t>(ld) + col) * 2u;
     }
   };
   auto load = [&](int it, int stage, int j) {
-    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(opnd + (soff[j] + static_cast<uint32_t>(it) * step)),
+    uint32_t off = soff[j] + static_cast<uint32_t>(it) * step;
+    if (kRagged) off = min(off, cap[j & 1]);
+    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(opnd + off),
                                      (void __attribute__((address_space(3)))*)(smem + stage * kGwStage + (wave * 8 + j) * 1024),
                                      16, 0, 0);
   };
@@ -1137,9 +1171,10 @@ __global__ __launch_bounds__(512) void grad_w_ring_kernel(const uint16_t* __rest
 }
 
 
-bool grad_w_ring_fits(int64_t rows, int64_t vocab, int64_t dim) {
-  return rows % 128 == 0 && rows >= 256 && vocab % 8 == 0 && dim % 8 == 0 && rows * vocab * 2 < (int64_t(1) << 32) &&
-         rows * dim * 2 < (int64_t(1) << 32) && 32 * dim * 2 < (int64_t(1) << 32);
+// k: the contracted rows (grad_logits' rows with their padding), ld: its row stride.
+bool grad_w_ring_fits(int64_t k, int64_t ld, int64_t dim) {
+  return k % 128 == 0 && k >= 256 && ld % 8 == 0 && dim % 8 == 0 && k * ld * 2 < (int64_t(1) << 32) &&
+         k * dim * 2 < (int64_t(1) << 32) && 32 * dim * 2 < (int64_t(1) << 32);
 }
 
 // Tile groups per XCD round (gm row tiles x gn weight panels, gm gn = 32), chosen from a sweep of
@@ -1168,8 +1203,8 @@ void logits_groups(int64_t tiles_m, int64_t dim, int& gm, int& gn) {
 // 5 TB/s. For the Qwen3-0.6B head (dim 1024) the model picks S = 16 for a 1024-row chunk
 // (16 tiles, 256 workgroups), 4 for 4096 rows and 2 for 8192 rows (128 tiles).
 int64_t splits_for(int64_t rows, int64_t vocab, int64_t dim) {
-  const int64_t tiles = (rows / kTile) * (dim / kTile);
-  const int64_t iters = vocab / kSliceK;
+  const int64_t tiles = ((rows + kTile - 1) / kTile) * ((dim + kTile - 1) / kTile);
+  const int64_t iters = (vocab + kSliceK - 1) / kSliceK;
   int64_t best = 1;
   double best_us = 0.0;
   for (int64_t s = 1; s <= 256; ++s) {
@@ -1191,11 +1226,11 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 // launch there. The device's CU count (for the ring kernels' workgroups per XCD) is read then.
 constexpr int kMaxDevices = 64;
 std::mutex g_lds_mu;
-bool g_lds_set[5][kMaxDevices] = {};
+bool g_lds_set[8][kMaxDevices] = {};
 int g_cus[kMaxDevices] = {};
 
 // which: 0 grad_h_gemm_kernel, 1 logits_gemm_kernel, 2 grad_w_gemm_kernel, 3 logits_ring_kernel,
-// 4 grad_w_ring_kernel.
+// 4 grad_w_ring_kernel, 5-7 the ragged forms of 0, 2 and 4.
 // `cus`, when given, receives the device's CU count.
 hipError_t allow_lds(hipStream_t stream, int which, int* cus = nullptr) {
   int dev = -1;
@@ -1210,10 +1245,12 @@ hipError_t allow_lds(hipStream_t stream, int which, int* cus = nullptr) {
   int cur = -1;
   e = hipGetDevice(&cur);
   if (e == hipSuccess && cur != dev) e = hipSetDevice(dev);
-  const void* fn[5] = {reinterpret_cast<const void*>(grad_h_gemm_kernel), reinterpret_cast<const void*>(logits_gemm_kernel),
-                       reinterpret_cast<const void*>(grad_w_gemm_kernel), reinterpret_cast<const void*>(logits_ring_kernel),
-                       reinterpret_cast<const void*>(grad_w_ring_kernel)};
-  const int bytes[5] = {2 * kLgStage, kLgLds, kLgLds, kRgLds, kRgLds};
+  const void* fn[8] = {
+      reinterpret_cast<const void*>(grad_h_gemm_kernel<false>), reinterpret_cast<const void*>(logits_gemm_kernel),
+      reinterpret_cast<const void*>(grad_w_gemm_kernel<false>), reinterpret_cast<const void*>(logits_ring_kernel),
+      reinterpret_cast<const void*>(grad_w_ring_kernel<false>), reinterpret_cast<const void*>(grad_h_gemm_kernel<true>),
+      reinterpret_cast<const void*>(grad_w_gemm_kernel<true>),  reinterpret_cast<const void*>(grad_w_ring_kernel<true>)};
+  const int bytes[8] = {2 * kLgStage, kLgLds, kLgLds, kRgLds, kRgLds, 2 * kLgStage, kLgLds, kRgLds};
   if (e == hipSuccess) e = hipFuncSetAttribute(fn[which], hipFuncAttributeMaxDynamicSharedMemorySize, bytes[which]);
   if (e == hipSuccess && g_cus[dev] == 0) e = hipDeviceGetAttribute(&g_cus[dev], hipDeviceAttributeMultiprocessorCount, dev);
   if (cur >= 0 && cur != dev) {
@@ -1232,8 +1269,8 @@ hipError_t allow_lds(hipStream_t stream, int which, int* cus = nullptr) {
 extern "C" {
 
 size_t tm_ce_grad_h_workspace_bytes(int64_t rows, int64_t vocab, int64_t dim) {
-  if (rows <= 0 || dim <= 0 || vocab <= 0 || rows % kTile || dim % kTile || vocab % kSliceK) return 0;
-  return static_cast<size_t>(splits_for(rows, vocab, dim)) * rows * dim * sizeof(float);
+  if (rows % kTile || dim % kTile || vocab % kSliceK) return 0;
+  return tm_ce_grad_h_ld_workspace_bytes(rows, vocab, dim);
 }
 
 int tm_ce_grad_h_bf16(uint16_t* d_grad_h, const uint16_t* d_grad_logits, const uint16_t* d_w, int64_t rows,
@@ -1242,28 +1279,50 @@ int tm_ce_grad_h_bf16(uint16_t* d_grad_h, const uint16_t* d_grad_logits, const u
     return gemm_fail(TM_EINVAL,
                      "tm_ce_grad_h_bf16: rows %lld and dim %lld must be positive multiples of %d, vocab %lld "
                      "of %d", (long long)rows, (long long)dim, kTile, (long long)vocab, kSliceK);
-  if (rows > (1 << 20) || dim > (1 << 16))
-    return gemm_fail(TM_EINVAL, "tm_ce_grad_h_bf16: rows %lld or dim %lld too large", (long long)rows,
-                     (long long)dim);
+  return tm_ce_grad_h_ld_bf16(d_grad_h, d_grad_logits, vocab, d_w, rows, vocab, dim, d_ws, ws_bytes, stream);
+}
+
+size_t tm_ce_grad_h_ld_workspace_bytes(int64_t rows, int64_t vocab, int64_t dim) {
+  if (rows <= 0 || dim <= 0 || vocab <= 0 || dim % 8) return 0;
+  return static_cast<size_t>(splits_for(rows, vocab, dim)) * rows * dim * sizeof(float);
+}
+
+int tm_ce_grad_h_ld_bf16(uint16_t* d_grad_h, const uint16_t* d_grad_logits, int64_t ld, const uint16_t* d_w,
+                         int64_t rows, int64_t vocab, int64_t dim, void* d_ws, size_t ws_bytes, void* stream) {
+  if (rows <= 0 || dim <= 0 || vocab <= 0 || dim % 8 || ld % 8 || ld < (vocab + kSliceK - 1) / kSliceK * kSliceK)
+    return gemm_fail(TM_EINVAL,
+                     "tm_ce_grad_h_bf16: rows %lld and vocab %lld must be positive, dim %lld a positive multiple of 8, "
+                     "grad_logits rows %lld elements apart a multiple of 8 and hold whole groups of %d", (long long)rows,
+                     (long long)vocab, (long long)dim, (long long)ld, kSliceK);
+  if (rows > (1 << 20) || dim > (1 << 16) || vocab > 0x7FFFFF00)
+    return gemm_fail(TM_EINVAL, "tm_ce_grad_h_bf16: rows %lld, dim %lld or vocab %lld too large", (long long)rows,
+                     (long long)dim, (long long)vocab);
   if (!d_grad_h || !d_grad_logits || !d_w || !d_ws)
     return gemm_fail(TM_EINVAL, "tm_ce_grad_h_bf16: null pointer");
   if (!aligned16(d_grad_h) || !aligned16(d_grad_logits) || !aligned16(d_w) || !aligned16(d_ws))
     return gemm_fail(TM_EINVAL, "tm_ce_grad_h_bf16: pointers must be 16-byte aligned");
-  if (ws_bytes < tm_ce_grad_h_workspace_bytes(rows, vocab, dim))
-    return gemm_fail(TM_EINVAL, "tm_ce_grad_h_bf16: workspace of %zu bytes, %zu needed", ws_bytes,
-                     tm_ce_grad_h_workspace_bytes(rows, vocab, dim));
+  const size_t need = tm_ce_grad_h_ld_workspace_bytes(rows, vocab, dim);
+  if (ws_bytes < need)
+    return gemm_fail(TM_EINVAL, "tm_ce_grad_h_bf16: workspace of %zu bytes, %zu needed", ws_bytes, need);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t splits = splits_for(rows, vocab, dim);
-  const int64_t tiles = (rows / kTile) * (dim / kTile);
-  const int64_t total_iters = vocab / kSliceK;
+  const int64_t tiles = ((rows + kTile - 1) / kTile) * ((dim + kTile - 1) / kTile);
+  const int64_t total_iters = (vocab + kSliceK - 1) / kSliceK;
   const int64_t per = (total_iters + splits - 1) / splits;
-  const hipError_t lds = allow_lds(s, 0);
+  const bool ragged = rows % kTile != 0 || dim % kTile != 0 || vocab % kSliceK != 0;
+  const hipError_t lds = allow_lds(s, ragged ? 5 : 0);
   if (lds != hipSuccess)
     return gemm_fail(TM_ELAUNCH, "tm_ce_grad_h_bf16: LDS attribute: %s", hipGetErrorString(lds));
   float* partials = static_cast<float*>(d_ws);
-  hipLaunchKernelGGL(grad_h_gemm_kernel, dim3(static_cast<uint32_t>((tiles * splits + 7) / 8 * 8)), dim3(512),
-                     2 * kLgStage, s, d_grad_logits, d_w, partials, static_cast<int>(rows), static_cast<int>(dim),
-                     vocab, static_cast<int>(tiles), static_cast<int>(splits), static_cast<int>(per));
+  const dim3 grid(static_cast<uint32_t>((tiles * splits + 7) / 8 * 8));
+  if (ragged)
+    hipLaunchKernelGGL(grad_h_gemm_kernel<true>, grid, dim3(512), 2 * kLgStage, s, d_grad_logits, d_w, partials,
+                       static_cast<int>(rows), static_cast<int>(dim), ld, static_cast<int>(vocab),
+                       static_cast<int>(tiles), static_cast<int>(splits), static_cast<int>(per));
+  else
+    hipLaunchKernelGGL(grad_h_gemm_kernel<false>, grid, dim3(512), 2 * kLgStage, s, d_grad_logits, d_w, partials,
+                       static_cast<int>(rows), static_cast<int>(dim), ld, static_cast<int>(vocab),
+                       static_cast<int>(tiles), static_cast<int>(splits), static_cast<int>(per));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return gemm_fail(TM_ELAUNCH, "grad_h_gemm_kernel: launch failed: %s", hipGetErrorString(e));
   const int64_t n = rows * dim;
@@ -1276,9 +1335,17 @@ int tm_ce_grad_h_bf16(uint16_t* d_grad_h, const uint16_t* d_grad_logits, const u
 
 int tm_ce_logits_bf16(uint16_t* d_logits, const uint16_t* d_hidden, const uint16_t* d_weight, int64_t rows,
                       int64_t vocab, int64_t dim, void* stream) {
+  return tm_ce_logits_ld_bf16(d_logits, vocab, d_hidden, d_weight, rows, vocab, dim, stream);
+}
+
+int tm_ce_logits_ld_bf16(uint16_t* d_logits, int64_t ld, const uint16_t* d_hidden, const uint16_t* d_weight,
+                         int64_t rows, int64_t vocab, int64_t dim, void* stream) {
   if (rows <= 0 || vocab <= 0 || dim <= 0 || dim % kSliceK)
     return gemm_fail(TM_EINVAL, "tm_ce_logits_bf16: rows %lld and vocab %lld must be positive, dim %lld a positive "
                      "multiple of %d", (long long)rows, (long long)vocab, (long long)dim, kSliceK);
+  if (ld < vocab || ld > 0x7FFFFFFF)
+    return gemm_fail(TM_EINVAL, "tm_ce_logits_bf16: logits rows %lld elements apart, vocab %lld", (long long)ld,
+                     (long long)vocab);
   const int64_t tiles_m = (rows + kLgTile - 1) / kLgTile, tiles_n = (vocab + kLgTile - 1) / kLgTile;
   if (rows > 0x7FFFFFFF || vocab > 0x7FFFFFFF || dim > 0x7FFFFFFF || tiles_m * tiles_n > 0x7FFFFFF0)
     return gemm_fail(TM_EINVAL, "tm_ce_logits_bf16: %lld x %lld x %lld is too large", (long long)rows,
@@ -1289,15 +1356,15 @@ int tm_ce_logits_bf16(uint16_t* d_logits, const uint16_t* d_hidden, const uint16
   hipStream_t s = static_cast<hipStream_t>(stream);
   int gm, gn;
   logits_groups(tiles_m, dim, gm, gn);
-  if (logits_ring_fits(rows, vocab, dim)) {
+  if (logits_ring_fits(rows, vocab, dim, ld)) {
     int cus = 0;
     const hipError_t lds = allow_lds(s, 3, &cus);
     if (lds != hipSuccess)
       return gemm_fail(TM_ELAUNCH, "tm_ce_logits_bf16: LDS attribute: %s", hipGetErrorString(lds));
     const int wpx = cus >= 16 ? cus / 8 : 1;  // one workgroup per CU of each XCD
     hipLaunchKernelGGL(logits_ring_kernel, dim3(static_cast<uint32_t>(8 * wpx)), dim3(512), kRgLds, s, d_hidden,
-                       d_weight, d_logits, static_cast<int>(rows), static_cast<int>(vocab), static_cast<int>(dim),
-                       static_cast<int>(tiles_m), static_cast<int>(tiles_n), gm, gn, wpx);
+                       d_weight, d_logits, static_cast<int>(rows), static_cast<int>(vocab), static_cast<int>(ld),
+                       static_cast<int>(dim), static_cast<int>(tiles_m), static_cast<int>(tiles_n), gm, gn, wpx);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return gemm_fail(TM_ELAUNCH, "logits_ring_kernel: launch failed: %s", hipGetErrorString(e));
     return TM_OK;
@@ -1307,7 +1374,7 @@ int tm_ce_logits_bf16(uint16_t* d_logits, const uint16_t* d_hidden, const uint16
     return gemm_fail(TM_ELAUNCH, "tm_ce_logits_bf16: LDS attribute: %s", hipGetErrorString(lds));
   const int64_t grid = (tiles_m * tiles_n + 7) / 8 * 8;
   hipLaunchKernelGGL(logits_gemm_kernel, dim3(static_cast<uint32_t>(grid)), dim3(256), kLgLds, s, d_hidden, d_weight,
-                     d_logits, static_cast<int>(rows), static_cast<int>(vocab), static_cast<int>(dim),
+                     d_logits, static_cast<int>(rows), static_cast<int>(vocab), ld, static_cast<int>(dim),
                      static_cast<int>(tiles_m), static_cast<int>(tiles_n), gm, gn);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return gemm_fail(TM_ELAUNCH, "logits_gemm_kernel: launch failed: %s", hipGetErrorString(e));
@@ -1319,8 +1386,19 @@ int tm_ce_grad_w_bf16(uint16_t* d_grad_w, const uint16_t* d_grad_logits, const u
   if (rows <= 0 || vocab <= 0 || dim <= 0 || rows % kSliceK || vocab % 8 || dim % 8)
     return gemm_fail(TM_EINVAL, "tm_ce_grad_w_bf16: rows %lld must be a positive multiple of %d, vocab %lld and dim "
                      "%lld positive multiples of 8", (long long)rows, kSliceK, (long long)vocab, (long long)dim);
+  return tm_ce_grad_w_ld_bf16(d_grad_w, d_grad_logits, vocab, rows, d_hidden, rows, vocab, dim, stream);
+}
+
+int tm_ce_grad_w_ld_bf16(uint16_t* d_grad_w, const uint16_t* d_grad_logits, int64_t ld, int64_t pad_rows,
+                         const uint16_t* d_hidden, int64_t rows, int64_t vocab, int64_t dim, void* stream) {
+  if (rows <= 0 || vocab <= 0 || dim <= 0 || dim % 8 || ld % 8 || ld < vocab || pad_rows % kSliceK || pad_rows < rows ||
+      pad_rows - rows >= 2 * kTile)
+    return gemm_fail(TM_EINVAL, "tm_ce_grad_w_bf16: rows %lld and vocab %lld must be positive, dim %lld a positive "
+                     "multiple of 8, grad_logits rows (%lld with padding, a multiple of %d) %lld elements apart, a "
+                     "multiple of 8", (long long)rows, (long long)vocab, (long long)dim, (long long)pad_rows, kSliceK,
+                     (long long)ld);
   const int64_t tiles_v = (vocab + kLgTile - 1) / kLgTile, tiles_d = (dim + kLgTile - 1) / kLgTile;
-  if (rows > 0x7FFFFFFF || vocab > 0x7FFFFFFF || dim > 0x7FFFFFFF || tiles_v * tiles_d > 0x7FFFFFF0)
+  if (pad_rows > 0x7FFFFFFF || ld > 0x7FFFFFFF || dim > 0x7FFFFFFF || tiles_v * tiles_d > 0x7FFFFFF0)
     return gemm_fail(TM_EINVAL, "tm_ce_grad_w_bf16: %lld x %lld x %lld is too large", (long long)rows,
                      (long long)vocab, (long long)dim);
   if (!d_grad_w || !d_grad_logits || !d_hidden) return gemm_fail(TM_EINVAL, "tm_ce_grad_w_bf16: null pointer");
@@ -1328,28 +1406,34 @@ int tm_ce_grad_w_bf16(uint16_t* d_grad_w, const uint16_t* d_grad_logits, const u
     return gemm_fail(TM_EINVAL, "tm_ce_grad_w_bf16: pointers must be 16-byte aligned");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int gn = static_cast<int>(tiles_d < 4 ? tiles_d : 4), gm = 32 / gn;  // a round of 32: 8 x 4
-  if (grad_w_ring_fits(rows, vocab, dim)) {
-    int cus = 0;
-    const hipError_t lds = allow_lds(s, 4, &cus);
-    if (lds != hipSuccess)
-      return gemm_fail(TM_ELAUNCH, "tm_ce_grad_w_bf16: LDS attribute: %s", hipGetErrorString(lds));
-    const int wpx = cus >= 16 ? cus / 8 : 1;
-    hipLaunchKernelGGL(grad_w_ring_kernel, dim3(static_cast<uint32_t>(8 * wpx)), dim3(512), kRgLds, s, d_grad_logits,
-                       d_hidden, d_grad_w, static_cast<int>(vocab), static_cast<int>(dim), static_cast<int>(rows),
-                       static_cast<int>(tiles_v), static_cast<int>(tiles_d), gm, gn, wpx);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return gemm_fail(TM_ELAUNCH, "grad_w_ring_kernel: launch failed: %s", hipGetErrorString(e));
-    return TM_OK;
-  }
-  const hipError_t lds = allow_lds(s, 2);
+  const bool ragged = rows != pad_rows, ring = grad_w_ring_fits(pad_rows, ld, dim);
+  int cus = 0;
+  const hipError_t lds = allow_lds(s, ring ? (ragged ? 7 : 4) : (ragged ? 6 : 2), &cus);
   if (lds != hipSuccess)
     return gemm_fail(TM_ELAUNCH, "tm_ce_grad_w_bf16: LDS attribute: %s", hipGetErrorString(lds));
-  const int64_t grid = (tiles_v * tiles_d + 7) / 8 * 8;
-  hipLaunchKernelGGL(grad_w_gemm_kernel, dim3(static_cast<uint32_t>(grid)), dim3(256), kLgLds, s, d_grad_logits,
-                     d_hidden, d_grad_w, static_cast<int>(vocab), static_cast<int>(dim), static_cast<int>(rows),
-                     static_cast<int>(tiles_v), static_cast<int>(tiles_d), gm, gn);
+  const int V = static_cast<int>(vocab), L = static_cast<int>(ld), D = static_cast<int>(dim),
+            K = static_cast<int>(pad_rows), R = static_cast<int>(rows), tv = static_cast<int>(tiles_v),
+            td = static_cast<int>(tiles_d);
+  if (ring) {
+    const int wpx = cus >= 16 ? cus / 8 : 1;
+    const dim3 grid(static_cast<uint32_t>(8 * wpx));
+    if (ragged)
+      hipLaunchKernelGGL(grad_w_ring_kernel<true>, grid, dim3(512), kRgLds, s, d_grad_logits, d_hidden, d_grad_w, V, L, D,
+                         K, R, tv, td, gm, gn, wpx);
+    else
+      hipLaunchKernelGGL(grad_w_ring_kernel<false>, grid, dim3(512), kRgLds, s, d_grad_logits, d_hidden, d_grad_w, V, L,
+                         D, K, R, tv, td, gm, gn, wpx);
+  } else {
+    const dim3 grid(static_cast<uint32_t>((tiles_v * tiles_d + 7) / 8 * 8));
+    if (ragged)
+      hipLaunchKernelGGL(grad_w_gemm_kernel<true>, grid, dim3(256), kLgLds, s, d_grad_logits, d_hidden, d_grad_w, V, L, D,
+                         K, R, tv, td, gm, gn);
+    else
+      hipLaunchKernelGGL(grad_w_gemm_kernel<false>, grid, dim3(256), kLgLds, s, d_grad_logits, d_hidden, d_grad_w, V, L,
+                         D, K, R, tv, td, gm, gn);
+  }
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return gemm_fail(TM_ELAUNCH, "grad_w_gemm_kernel: launch failed: %s", hipGetErrorString(e));
+  if (e != hipSuccess) return gemm_fail(TM_ELAUNCH, "grad_w kernel: launch failed: %s", hipGetErrorString(e));
   return TM_OK;
 }
 

@@ -7,18 +7,20 @@ semantics, :22-24), computes grad_hidden and grad_weight during the forward pass
 (:42-58) and scales them in place by grad_out / n_valid in backward (:94-127).
 
 Per chunk of rows:
-  logits = h @ W^T                  bf16 GEMM: tm_ce_logits_bf16, this build's MFMA GEMM, for dim a
+  logits = h @ W^T                  bf16 GEMM: tm_ce_logits_ld_bf16, this build's MFMA GEMM, for dim a
                                     multiple of 64 (torch.matmul on other shapes)
-  tm_ce_rows_bf16                   one fused kernel: logsumexp, per-row loss and
+  tm_ce_rows_padded_bf16            one fused kernel: logsumexp, per-row loss and
                                     grad_logits = bf16(softmax - onehot), in place
-  grad_h = grad_logits @ W          bf16 GEMM: tm_ce_grad_h_bf16, a split-K MFMA GEMM with a
-                                    fixed-order reduction, on chunks with at most
-                                    SPLITK_GRAD_H_MAX_TILES output tiles of 256 x 256, or any
-                                    number when D is not a power of two (rows and D multiples of
-                                    256, V of 64); hipBLASLt on other shapes
-  grad_W += grad_logits^T @ h       bf16 GEMM: tm_ce_grad_w_bf16, this build's MFMA GEMM, for rows a
-                                    multiple of 64 (torch.matmul on other shapes), then
-                                    tm_ce_grad_w_fold into fp32
+  grad_h = grad_logits @ W          bf16 GEMM: tm_ce_grad_h_ld_bf16, a split-K MFMA GEMM with a
+                                    fixed-order reduction, where grad_h_gemm_fits; hipBLASLt on
+                                    other shapes
+  grad_W += grad_logits^T @ h       bf16 GEMM: tm_ce_grad_w_ld_bf16, this build's MFMA GEMM, for dim
+                                    a multiple of 64 (and rows too where the logits are unpadded;
+                                    torch.matmul otherwise), then tm_ce_grad_w_fold into fp32
+The chunk's logits are padded to whole MFMA steps (PaddedLogits): rows a multiple of 64 elements
+apart and their number a multiple of 128, the padding zero once they are gradients. An odd
+vocabulary then keeps its rows 16-byte aligned, and any number of tokens is a whole number of
+K slices for grad_W.
 then tm_ce_loss sums the per-row losses in a fixed order (deterministic).
 
 The last chunk's bf16 grad_W is not added in forward: it waits for backward, where
@@ -208,24 +210,73 @@ def _logits(h: torch.Tensor, w: torch.Tensor, lib, stream) -> torch.Tensor:
     return out
 
 
+def padded_rows(rows: int) -> int:
+    """Rows of a chunk's padded logits: whole 64-row K slices of the grad_W GEMM, and from 129
+    rows an even number of them, at least 4 (its persistent kernel's form)."""
+    return -(-rows // 64) * 64 if rows <= 128 else max(256, -(-rows // 128) * 128)
+
+
+def padded_vocab(vocab: int) -> int:
+    """Elements from one padded logits row to the next: whole 64-column K slices of the grad_h
+    GEMM; every row then starts on a 16-byte boundary (on a cache line), for any vocabulary."""
+    return -(-vocab // 64) * 64
+
+
+class PaddedLogits:
+    """A chunk's logits in a buffer padded for the MFMA kernels (``padded_rows`` x
+    ``padded_vocab``), for hidden states and a weight ``logits_gemm_fits`` accepts. ``rows_()``
+    turns them into grad_logits and zeroes the padding; ``view`` is their rows x vocab part.
+    The loss alone (``grad=False``) needs no rows of padding."""
+
+    def __init__(self, h: torch.Tensor, w: torch.Tensor, lib, stream, grad: bool = True):
+        (self.rows, self.dim), self.vocab = h.shape, w.shape[0]
+        self.lib, self.stream, self.h = lib, stream, h
+        self.pad_rows = padded_rows(self.rows) if grad else self.rows
+        self.buf = torch.empty((self.pad_rows, padded_vocab(self.vocab)), dtype=torch.bfloat16, device=h.device)
+        self.ld = self.buf.shape[1]
+        _native.check(lib.tm_ce_logits_ld_bf16(self.buf.data_ptr(), self.ld, h.data_ptr(), w.data_ptr(), self.rows,
+                                               self.vocab, self.dim, stream), "tm_ce_logits_ld_bf16")
+
+    @property
+    def view(self) -> torch.Tensor:
+        return self.buf[: self.rows, : self.vocab]
+
+    def rows_(self, labels: torch.Tensor, ignore_index: int, row_loss: torch.Tensor) -> None:
+        _native.check(self.lib.tm_ce_rows_padded_bf16(self.buf.data_ptr(), self.ld, labels.data_ptr(), self.rows,
+                                                      self.pad_rows, self.vocab, ignore_index, row_loss.data_ptr(),
+                                                      self.stream), "tm_ce_rows_padded_bf16")
+
+    def grad_w(self) -> torch.Tensor:
+        """gw = grad_logits.t() @ h (fused_linear_ce.py:57): bf16 GEMM, bf16 result (V x D)."""
+        out = torch.empty((self.vocab, self.dim), dtype=torch.bfloat16, device=self.buf.device)
+        _native.check(self.lib.tm_ce_grad_w_ld_bf16(out.data_ptr(), self.buf.data_ptr(), self.ld, self.pad_rows,
+                                                    self.h.data_ptr(), self.rows, self.vocab, self.dim, self.stream),
+                      "tm_ce_grad_w_ld_bf16")
+        return out
+
+
 def grad_w_gemm_fits(g: torch.Tensor, h: torch.Tensor) -> bool:
-    """Chunks whose grad_W runs on this build's GEMM (tm_ce_grad_w_bf16): bf16 operands, both
-    contiguous and 16-byte aligned, rows a multiple of 64, vocab and dim multiples of 8. Other
-    shapes take torch.matmul."""
+    """Unpadded chunks whose grad_W runs on this build's GEMM: bf16 operands, both contiguous and
+    16-byte aligned, vocab and dim multiples of 8. Other shapes take torch.matmul."""
     return (g.dtype == torch.bfloat16 and h.dtype == torch.bfloat16 and g.dim() == 2 and h.dim() == 2
-            and g.shape[0] == h.shape[0] and g.shape[0] > 0 and g.shape[0] % 64 == 0 and g.shape[1] % 8 == 0
+            and g.shape[0] == h.shape[0] and g.shape[0] > 0 and g.shape[1] % 8 == 0
             and h.shape[1] % 8 == 0 and g.shape[1] > 0 and h.shape[1] > 0 and g.is_contiguous() and h.is_contiguous()
             and g.data_ptr() % 16 == 0 and h.data_ptr() % 16 == 0)
 
 
 def _grad_w(g: torch.Tensor, h: torch.Tensor, lib, stream) -> torch.Tensor:
-    """A chunk's gw = grad_logits.t() @ h (fused_linear_ce.py:57): bf16 GEMM, bf16 result (V x D)."""
-    if not grad_w_gemm_fits(g, h):
-        return torch.matmul(g.t(), h)
+    """A chunk's gw = grad_logits.t() @ h (fused_linear_ce.py:57) from unpadded grad_logits: bf16
+    GEMM, bf16 result (V x D). Rows off a multiple of 64 are copied into a zero-padded buffer."""
     rows, vocab = g.shape
+    if not grad_w_gemm_fits(g, h) or (rows % 64 and h.shape[1] % 64):
+        return torch.matmul(g.t(), h)
+    pad = rows if rows % 64 == 0 else padded_rows(rows)
+    if pad != rows:
+        g, short = torch.zeros((pad, vocab), dtype=torch.bfloat16, device=g.device), g
+        g[:rows].copy_(short)
     out = torch.empty((vocab, h.shape[1]), dtype=torch.bfloat16, device=g.device)
-    _native.check(lib.tm_ce_grad_w_bf16(out.data_ptr(), g.data_ptr(), h.data_ptr(), rows, vocab, h.shape[1], stream),
-                  "tm_ce_grad_w_bf16")
+    _native.check(lib.tm_ce_grad_w_ld_bf16(out.data_ptr(), g.data_ptr(), vocab, pad, h.data_ptr(), rows, vocab,
+                                           h.shape[1], stream), "tm_ce_grad_w_ld_bf16")
     return out
 
 
@@ -254,6 +305,29 @@ def splitk_grad_h_fits(rows: int, dim: int, vocab: int) -> bool:
     return (rows // 256) * (dim // 256) <= SPLITK_GRAD_H_MAX_TILES or (dim & (dim - 1)) != 0
 
 
+def grad_h_gemm_fits(rows: int, dim: int, vocab: int) -> bool:
+    """Padded chunks whose grad_h runs on the split-K GEMM: those ``splitk_grad_h_fits`` accepts,
+    and ragged ones (rows or dim off a multiple of 256, a vocabulary off a multiple of 64) under
+    the same rule for many tiles of a power-of-two width, from a vocabulary of
+    RAGGED_GRAD_H_MIN_VOCAB up: with a shorter K the partial tiles and their reduction cost more
+    than the split gives. us per call on MI355X, split-K / hipBLASLt on the same padded logits:
+
+        rows x dim x vocab     552 x 256 x 4096     27.6 /  18.5     1024 x 768 x 32001     63 / 181
+                               468 x 320 x 4376     29.3 /  20.9      452 x 768 x 32001     48 / 131
+                              7129 x 1216 x 1984    64.1 /  47.5     1905 x 1024 x 151936  538 / 703
+                              1024 x 320 x 7296     29.2 /  31.4     3000 x 2560 x 100000 1289 / 2061
+                              2046 x 2112 x 7296    77.5 /  74.4     6001 x 1024 x 151936 1616 / 1517
+    """
+    if splitk_grad_h_fits(rows, dim, vocab):
+        return True
+    if not (rows > 0 and dim > 0 and dim % 8 == 0 and dim <= 65536 and rows <= 1 << 20
+            and vocab >= RAGGED_GRAD_H_MIN_VOCAB and (rows % 256 or dim % 256 or vocab % 64)):
+        return False
+    return -(-rows // 256) * -(-dim // 256) <= SPLITK_GRAD_H_MAX_TILES or (dim & (dim - 1)) != 0
+
+
+RAGGED_GRAD_H_MIN_VOCAB = 7168
+
 FOLD_CHUNKS = 8  # chunks per grad_W fold (tm_ce_grad_w_fold takes at most 8)
 FOLD_BYTES = 4 << 30  # bf16 chunk grad_W held before a fold, at most
 
@@ -271,29 +345,32 @@ def _fold(lib, grad_weight, chunks, accumulated, g, n_valid, stream) -> None:
 
 class GradHidden:
     """grad_h = grad_logits @ W (fused_linear_ce.py:52, stored at :79) for the chunks of one
-    call: the split-K MFMA GEMM on the chunks ``splitk_grad_h_fits`` accepts, reading W as it is
-    stored, with one fp32 partials workspace shared by the chunks (stream-ordered), and
-    torch.matmul (hipBLASLt) on the others. ``w`` is the contiguous bf16 weight (V x D)."""
+    call: the split-K MFMA GEMM on the chunks it fits, reading W as it is stored, with one fp32
+    partials workspace shared by the chunks (stream-ordered), and torch.matmul (hipBLASLt) on the
+    others. ``w`` is the contiguous bf16 weight (V x D). ``padded``: the chunks' grad_logits are
+    views of PaddedLogits buffers (columns from the vocabulary to the next multiple of 64 zero),
+    and ``grad_h_gemm_fits`` decides; else they are contiguous, and ``splitk_grad_h_fits`` does."""
 
-    def __init__(self, w: torch.Tensor, chunk_rows, lib, stream):
+    def __init__(self, w: torch.Tensor, chunk_rows, lib, stream, padded: bool = False):
         self.w, self.lib, self.stream = w, lib, stream
         self.vocab, self.dim = w.shape
-        fits = [r for r in set(chunk_rows) if splitk_grad_h_fits(r, self.dim, self.vocab)]
+        self._fits = grad_h_gemm_fits if padded else splitk_grad_h_fits
+        fits = [r for r in set(chunk_rows) if self._fits(r, self.dim, self.vocab)]
         self.ws = None
         if fits:
-            nbytes = max(lib.tm_ce_grad_h_workspace_bytes(r, self.vocab, self.dim) for r in fits)
+            nbytes = max(lib.tm_ce_grad_h_ld_workspace_bytes(r, self.vocab, self.dim) for r in fits)
             self.ws = torch.empty(nbytes, dtype=torch.uint8, device=w.device)
 
     def __call__(self, grad_logits: torch.Tensor, out: torch.Tensor) -> None:
         rows = grad_logits.shape[0]
-        if self.ws is None or not splitk_grad_h_fits(rows, self.dim, self.vocab):
+        if self.ws is None or not self._fits(rows, self.dim, self.vocab):
             torch.matmul(grad_logits, self.w, out=out)
             return
-        if not (grad_logits.is_contiguous() and out.is_contiguous() and out.dtype == torch.bfloat16):
+        if not (grad_logits.stride(1) == 1 and out.is_contiguous() and out.dtype == torch.bfloat16):
             raise RuntimeError("fused_linear_cross_entropy: grad_h GEMM operands must be contiguous bf16")
-        _native.check(self.lib.tm_ce_grad_h_bf16(out.data_ptr(), grad_logits.data_ptr(), self.w.data_ptr(), rows,
-                                                 self.vocab, self.dim, self.ws.data_ptr(), self.ws.numel(),
-                                                 self.stream), "tm_ce_grad_h_bf16")
+        _native.check(self.lib.tm_ce_grad_h_ld_bf16(out.data_ptr(), grad_logits.data_ptr(), grad_logits.stride(0),
+                                                    self.w.data_ptr(), rows, self.vocab, self.dim, self.ws.data_ptr(),
+                                                    self.ws.numel(), self.stream), "tm_ce_grad_h_ld_bf16")
 
 
 def _bf16_weight(weight: torch.Tensor) -> torch.Tensor:
@@ -326,9 +403,14 @@ def _loss_only(hidden, weight, labels, ignore_index, chunk_size):
     row_loss = torch.empty(n, dtype=torch.float32, device=hidden.device)
     for s in range(0, n, chunk):
         e = min(s + chunk, n)
-        logits = _logits(hb[s:e], w, lib, stream) if dt == torch.bfloat16 else _bf16(torch.matmul(hb[s:e], w.t()), dt)
-        _native.check(rows_loss(logits.data_ptr(), v, labels[s:e].data_ptr(), e - s, v, int(ignore_index),
-                                row_loss[s:].data_ptr(), stream), "tm_ce_rows_loss")
+        if dt == torch.float32:
+            logits = _bf16(torch.matmul(hb[s:e], w.t()), dt)
+        elif logits_gemm_fits(hb[s:e], w):
+            logits = PaddedLogits(hb[s:e], w, lib, stream, grad=False).buf
+        else:
+            logits = _logits(hb[s:e], w, lib, stream)
+        _native.check(rows_loss(logits.data_ptr(), logits.shape[1], labels[s:e].data_ptr(), e - s, v,
+                                int(ignore_index), row_loss[s:].data_ptr(), stream), "tm_ce_rows_loss")
         del logits
     return _mean_loss(row_loss, labels, n, ignore_index, lib, stream)[0]
 
@@ -385,18 +467,26 @@ class _FusedLinearCE(torch.autograd.Function):
         pending, last_gw = [], None
         accumulated = False
         row_loss = torch.empty(n, dtype=torch.float32, device=hidden.device)
-        grad_h_of = GradHidden(w, [min(chunk, n - s) for s in range(0, n, chunk)], lib, stream) if want_h else None
+        padded = n > 0 and logits_gemm_fits(hb, w)  # every chunk then starts on a 16-byte boundary
+        grad_h_of = None
+        if want_h:
+            grad_h_of = GradHidden(w, [min(chunk, n - s) for s in range(0, n, chunk)], lib, stream, padded)
         for s in range(0, n, chunk):
             e = min(s + chunk, n)
             h = hb[s:e]
-            logits = _logits(h, w, lib, stream)  # (C, V) bf16
-            _native.check(lib.tm_ce_rows_bf16(logits.data_ptr(), v, labels[s:e].data_ptr(), e - s, v,
-                                              int(ignore_index), row_loss[s:].data_ptr(), stream),
-                          "tm_ce_rows_bf16")
+            if padded:
+                block = PaddedLogits(h, w, lib, stream)  # (C, V) bf16
+                block.rows_(labels[s:e], int(ignore_index), row_loss[s:])
+                logits = block.view
+            else:
+                logits = _logits(h, w, lib, stream)
+                _native.check(lib.tm_ce_rows_bf16(logits.data_ptr(), v, labels[s:e].data_ptr(), e - s, v,
+                                                  int(ignore_index), row_loss[s:].data_ptr(), stream),
+                              "tm_ce_rows_bf16")
             if want_h:
                 grad_h_of(logits, grad_hidden[s:e])
             if want_w:
-                gw = _grad_w(logits, h, lib, stream)  # (V, D) bf16
+                gw = block.grad_w() if padded else _grad_w(logits, h, lib, stream)  # (V, D) bf16
                 if e == n:
                     last_gw = gw
                 else:
@@ -408,7 +498,7 @@ class _FusedLinearCE(torch.autograd.Function):
                         _fold(lib, grad_weight, pending, accumulated, None, None, stream)
                         accumulated = True
                         pending = []
-            del logits
+            block = logits = None
         del grad_h_of
         loss, ctx.n_valid = _mean_loss(row_loss, labels, n, ignore_index, lib, stream)
         ctx.grad_hidden = grad_hidden
