@@ -387,6 +387,31 @@ int tm_ce_grad_w_bf16(uint16_t* d_grad_w, const uint16_t* d_grad_logits, const u
                       int64_t vocab, int64_t dim, void* stream);
 
 /*
+ * tm_ce_loss with its results in two places: d_out2 = (loss sum, n_valid), d_loss = the mean.
+ */
+int tm_ce_mean_loss(const float* d_row_loss, const int64_t* d_labels, int64_t rows, int64_t ignore_index,
+                    float* d_out2, float* d_loss, void* stream);
+
+/*
+ * d_dst0 = bf16(d_src0) over n0 elements and d_dst1 = bf16(d_src1) over n1 (either may be empty),
+ * RNE, NaN -> 0x7FC0 (tm_cast_bf16's rounding), in one launch: autocast's casts of the hidden
+ * states and the weight (fused_linear_ce.py:38,65 under autocast).
+ */
+int tm_ce_cast2(uint16_t* d_dst0, const float* d_src0, int64_t n0, uint16_t* d_dst1, const float* d_src1, int64_t n1,
+                void* stream);
+
+/*
+ * The whole of backward (fused_linear_ce.py:107-126) in one launch: d_grad_w over nw elements as
+ * tm_ce_grad_w_fold with a scale (n_chunks may be 0: a plain d_grad_w *= g / n_valid when
+ * accumulate is set), and grad_h over nh elements: d_grad_h_out (bf16, may be d_grad_h) =
+ * bf16(d_grad_h * bf16(g / n_valid)), or, with wide set, d_grad_h_out (fp32) =
+ * float(d_grad_h) * (g / n_valid). Either part may be empty.
+ */
+int tm_ce_finish(float* d_grad_w, const uint16_t* const* h_chunks, int n_chunks, int64_t nw, int accumulate,
+                 const uint16_t* d_grad_h, void* d_grad_h_out, int64_t nh, int wide, const float* d_grad_out,
+                 const float* d_n_valid, void* stream);
+
+/*
  * The chunk's kernels on padded logits, so that any row count and vocabulary runs on the same
  * MFMA kernels: a chunk's logits are pad_rows x ld, ld a multiple of 8 (of 64 for grad_h, or at
  * least the vocabulary's next multiple of 64), of which rows x vocab are used.

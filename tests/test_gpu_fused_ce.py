@@ -232,6 +232,74 @@ def test_fused_linear_ce_all_ignored_and_double_backward():
         loss.backward()
 
 
+@pytest.mark.parametrize("nw,k,accumulate,nh,wide,off_w,off_h", [
+    (0, 0, 0, 1, 0, 0, 0), (1, 1, 0, 0, 0, 0, 0),
+    (255, 1, 0, 511, 1, 0, 0), (257, 8, 1, 513, 0, 0, 0),      # around a slice of each part
+    (1000, 2, 1, 1027, 1, 1, 1), (1000, 3, 0, 1030, 0, 1, 3),  # nothing aligned
+    (515, 0, 1, 4096, 0, 0, 2),                                # no chunks: a plain scale; 4-byte grad_h
+    (70000, 5, 1, 33000, 1, 0, 0),
+])
+def test_ce_finish_bit_exact(nw, k, accumulate, nh, wide, off_w, off_h):
+    """tm_ce_finish: grad_W's chunks added in order and scaled, grad_h scaled (bf16 by the bf16
+    scale, or widened and scaled in fp32), each the same bits as the separate operations in torch,
+    and nothing else written."""
+    from torchure_amd import _native
+
+    lib, st = _native.lib(), _native.stream_handle(DEV)
+    g = torch.Generator(device=DEV).manual_seed(nw + nh)
+
+    def fenced(n, off, dtype):
+        buf = torch.randn(n + 64, device=DEV, generator=g).to(dtype)
+        return buf, buf.clone(), buf[off: off + n]
+
+    wbuf, wkeep, w = fenced(nw, off_w, torch.float32)
+    chunks = [fenced(nw, off_w, torch.bfloat16)[2] for _ in range(k)]
+    _, _, src = fenced(nh, off_h, torch.bfloat16)
+    if nh:
+        src[0] = -0.0
+    hbuf, hkeep, dst = fenced(nh, off_h, torch.float32 if wide else torch.bfloat16)
+    out, n_valid = torch.tensor(0.37, device=DEV), torch.tensor(123.0, device=DEV)
+    scale = out / n_valid
+    want = w.clone() if accumulate else torch.zeros_like(w)
+    for c in chunks:
+        want += c.float()
+    want = want * scale
+    want_h = src.float() * scale if wide else src * scale.to(torch.bfloat16)
+    import ctypes
+    ptrs = (ctypes.c_void_p * k)(*[c.data_ptr() for c in chunks])
+    _native.check(lib.tm_ce_finish(w.data_ptr(), ptrs, k, nw, accumulate, src.data_ptr(), dst.data_ptr(), nh, wide,
+                                   out.data_ptr(), n_valid.data_ptr(), st), "tm_ce_finish")
+    bits = torch.int32 if wide else torch.int16
+    assert torch.equal(w.view(torch.int32), want.view(torch.int32))
+    assert torch.equal(dst.view(bits), want_h.view(bits))
+    wkeep[off_w: off_w + nw] = w
+    hkeep[off_h: off_h + nh] = dst
+    assert torch.equal(wbuf, wkeep) and torch.equal(hbuf, hkeep)
+
+
+@pytest.mark.parametrize("n0,n1,off", [(0, 1, 0), (511, 0, 0), (513, 1025, 0), (4099, 300, 1), (1 << 20, 777, 0)])
+def test_ce_cast2_equals_the_device_cast(n0, n1, off):
+    """Two arrays cast in one launch: torch's device cast bit for bit, special values included, at
+    slice edges and unaligned starts, and nothing past either array written."""
+    from torchure_amd import _native
+
+    g = torch.Generator(device=DEV).manual_seed(n0 + n1)
+    parts = []
+    for n in (n0, n1):
+        src = torch.randn(n + 8, device=DEV, generator=g)
+        special = torch.tensor([float("nan"), float("inf"), -float("inf"), -0.0, 1e-40, 3.4e38, 1.00390625, 1.01171875], device=DEV)
+        src[: min(8, n + 8)] = special
+        dst = torch.full((n + 8,), 5.0, dtype=torch.bfloat16, device=DEV)
+        parts.append((src[off: off + n], dst[off: off + n], dst))
+    (s0, d0, b0), (s1, d1, b1) = parts
+    _native.check(_native.lib().tm_ce_cast2(d0.data_ptr(), s0.data_ptr(), n0, d1.data_ptr(), s1.data_ptr(), n1,
+                                            _native.stream_handle(DEV)), "tm_ce_cast2")
+    for src, dst, buf in parts:
+        want = torch.full_like(buf, 5.0)
+        want[off: off + src.numel()] = src.to(torch.bfloat16)
+        assert torch.equal(buf.view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("accumulate,scaled,n,offset", [
     (0, 0, 4096, 0), (1, 0, 4096, 0), (0, 1, 4096, 0), (1, 1, 4096, 0),
     (1, 1, 1003, 0), (1, 1, 2050, 1), (0, 1, 777, 3)])

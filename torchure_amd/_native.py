@@ -101,6 +101,9 @@ _SIGNATURES = {
     "tm_ce_rows_f32": (ctypes.c_int, [_vp, _i64, _vp, _i64, _i64, _i64, _vp, _vp]),
     "tm_ce_rows_loss_f32": (ctypes.c_int, [_vp, _i64, _vp, _i64, _i64, _i64, _vp, _vp]),
     "tm_ce_loss": (ctypes.c_int, [_vp, _vp, _i64, _i64, _vp, _vp]),
+    "tm_ce_mean_loss": (ctypes.c_int, [_vp, _vp, _i64, _i64, _vp, _vp, _vp]),
+    "tm_ce_cast2": (ctypes.c_int, [_vp, _vp, _i64, _vp, _vp, _i64, _vp]),
+    "tm_ce_finish": (ctypes.c_int, [_vp, _vp, ctypes.c_int, _i64, ctypes.c_int, _vp, _vp, _i64, ctypes.c_int, _vp, _vp, _vp]),
     "tm_ce_scale_grads": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _vp]),
     "tm_ce_grad_w": (ctypes.c_int, [_vp, _vp, _i64, ctypes.c_int, _vp, _vp, _vp]),
     "tm_ce_grad_w2": (ctypes.c_int, [_vp, _vp, _vp, _i64, ctypes.c_int, _vp, _vp, _vp]),

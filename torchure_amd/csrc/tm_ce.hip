@@ -17,8 +17,9 @@
 //                         the bf16 rounding is the hardware RNE convert.
 //   ce_loss_kernel        one workgroup: fixed-order sum of the per-row losses and of
 //                         the valid-row count -> loss_sum, n_valid, mean loss.
-//   ce_scale_kernel       backward: grad_h (bf16) *= bf16(g / n_valid),
-//                         grad_W (fp32) *= g / n_valid.
+//   ce_grads_kernel       the chunks' bf16 grad_W added into the fp32 grad_W, and backward's
+//                         scaling: grad_W *= g / n_valid, grad_h (bf16) *= bf16(g / n_valid) or
+//                         its fp32 widening times g / n_valid, in one launch.
 
 #include <hip/hip_runtime.h>
 
@@ -523,18 +524,32 @@ __global__ __launch_bounds__(256) void ce_rows_f32_kernel(float* __restrict__ lo
   for (int64_t i = vend + threadIdx.x; i < vocab; i += 256) row[i] = g_of(row[i], i);
 }
 
-// Fixed-order sums over rows: loss_sum, n_valid (count of label != ignore), mean.
-__global__ __launch_bounds__(256) void ce_loss_kernel(const float* __restrict__ row_loss,
-                                                      const int64_t* __restrict__ labels,
-                                                      int64_t rows, int64_t ignore_index,
-                                                      float* __restrict__ out3) {
-  __shared__ double sl[4];
-  __shared__ long long sn[4];
+// Fixed-order sums over rows: loss_sum, n_valid (count of label != ignore), mean. One workgroup,
+// whose time is the latency of its loads: 1024 threads with 4 rows of each in flight (8192 rows:
+// 10 us, against 16 with 256 threads and one row at a time).
+constexpr int kLossThreads = 1024, kLossUnroll = 4;
+__global__ __launch_bounds__(kLossThreads) void ce_loss_kernel(const float* __restrict__ row_loss,
+                                                               const int64_t* __restrict__ labels, int64_t rows,
+                                                               int64_t ignore_index, float* __restrict__ out2,
+                                                               float* __restrict__ mean) {
+  __shared__ double sl[kLossThreads / 64];
+  __shared__ long long sn[kLossThreads / 64];
   double acc = 0.0;
   long long cnt = 0;
-  for (int64_t i = threadIdx.x; i < rows; i += 256) {
-    acc += static_cast<double>(row_loss[i]);
-    cnt += labels[i] != ignore_index;
+  for (int64_t i0 = threadIdx.x; i0 < rows; i0 += kLossThreads * kLossUnroll) {
+    float x[kLossUnroll];
+    int64_t l[kLossUnroll];
+#pragma unroll
+    for (int u = 0; u < kLossUnroll; ++u) {
+      const int64_t i = i0 + u * kLossThreads;
+      x[u] = i < rows ? row_loss[i] : 0.0f;
+      l[u] = i < rows ? labels[i] : ignore_index;
+    }
+#pragma unroll
+    for (int u = 0; u < kLossUnroll; ++u) {
+      acc += static_cast<double>(x[u]);
+      cnt += l[u] != ignore_index;
+    }
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -547,30 +562,18 @@ __global__ __launch_bounds__(256) void ce_loss_kernel(const float* __restrict__ 
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    const double total = sl[0] + sl[1] + sl[2] + sl[3];
-    long long n = sn[0] + sn[1] + sn[2] + sn[3];
+    double total = 0.0;
+    long long n = 0;
+    for (int w = 0; w < kLossThreads / 64; ++w) {
+      total += sl[w];
+      n += sn[w];
+    }
     const float loss_sum = static_cast<float>(total);
     const float n_valid = static_cast<float>(n < 1 ? 1 : n);  // clamp_min(1)
-    out3[0] = loss_sum;
-    out3[1] = n_valid;
-    out3[2] = loss_sum / n_valid;
+    out2[0] = loss_sum;
+    out2[1] = n_valid;
+    *mean = loss_sum / n_valid;
   }
-}
-
-// Backward scaling, fused_linear_ce.py:117-126: grad_h (bf16) *= bf16(g / n_valid)
-// (the scale is cast to the grad's dtype, then a bf16 multiply), grad_W *= g / n_valid.
-__global__ __launch_bounds__(256) void ce_scale_kernel(uint16_t* __restrict__ gh, int64_t nh,
-                                                       float* __restrict__ gw, int64_t nw,
-                                                       const float* __restrict__ grad_out,
-                                                       const float* __restrict__ n_valid) {
-  const float scale = *grad_out / *n_valid;
-  const float scale_b = __uint_as_float(rne16(scale) << 16);
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < nh; i += stride)
-    gh[i] = static_cast<uint16_t>(rne16(__uint_as_float(static_cast<uint32_t>(gh[i]) << 16) * scale_b));
-  if (gw)
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < nw; i += stride)
-      gw[i] = gw[i] * scale;
 }
 
 // grad_W hand-over (fused_linear_ce.py:80-81 for each chunk in order, and :126 with kScale):
@@ -599,17 +602,72 @@ __device__ __forceinline__ void st_nt(T* p, T v) {
   __builtin_nontemporal_store(v, (CE_GLOBAL T*)p);
 }
 
+// grad_h's part of backward, over the slices after grad_W's in the same launch (one launch less,
+// and vectors where the scaling went 2 bytes at a time: 15 us for 8192 x 1024). 512 elements a
+// wave, two groups of 4 a lane, both loaded before either is stored (8192 x 1024: under 6 us).
+// fused_linear_ce.py:117-126: bf16 grad_h *= bf16(g / n_valid), the scale cast to the grad's
+// dtype, then a bf16 multiply. fp32 hidden states (:68,80,120; kWide): the reference's fp32
+// buffer holds the widened bf16 GEMM result (-0 kept) and is scaled in fp32.
+struct GradH {
+  const uint16_t* src;
+  void* dst;  // src itself (bf16), or fp32 when wide
+  int64_t n;
+  bool wide;
+};
+constexpr int kGradHSlice = 512;
+
+__device__ __forceinline__ void grad_h_slice(const GradH& gh, int64_t start, float scale) {
+  const float scale_b = __uint_as_float(rne16(scale) << 16);
+  const bool vec = (reinterpret_cast<uint64_t>(gh.src) & 7u) == 0 &&
+                   (reinterpret_cast<uint64_t>(gh.dst) & (gh.wide ? 15u : 7u)) == 0;
+  const int64_t end = start + kGradHSlice < gh.n ? start + kGradHSlice : gh.n;
+  int64_t done = start;
+  if (vec) {
+    done = start + ((end - start) & ~int64_t(3));
+    const int64_t e0 = start + static_cast<int64_t>(threadIdx.x) * 4, e1 = e0 + 256;
+    u32x2 w[2] = {};
+    if (e0 < done) w[0] = ld_nt(reinterpret_cast<const u32x2*>(gh.src + e0));
+    if (e1 < done) w[1] = ld_nt(reinterpret_cast<const u32x2*>(gh.src + e1));
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int64_t e = u == 0 ? e0 : e1;
+      if (e >= done) continue;
+      const f32x4 x = {lo16(w[u].x), hi16(w[u].x), lo16(w[u].y), hi16(w[u].y)};
+      if (gh.wide) {
+        st_nt(reinterpret_cast<f32x4*>(static_cast<float*>(gh.dst) + e),
+              f32x4{x.x * scale, x.y * scale, x.z * scale, x.w * scale});
+      } else {
+        u32x2 o;
+        o.x = rne16(x.x * scale_b) | (rne16(x.y * scale_b) << 16);
+        o.y = rne16(x.z * scale_b) | (rne16(x.w * scale_b) << 16);
+        st_nt(reinterpret_cast<u32x2*>(static_cast<uint16_t*>(gh.dst) + e), o);
+      }
+    }
+  }
+  for (int64_t i = done + threadIdx.x; i < end; i += 64) {
+    const float x = __uint_as_float(static_cast<uint32_t>(gh.src[i]) << 16);
+    if (gh.wide) static_cast<float*>(gh.dst)[i] = x * scale;
+    else static_cast<uint16_t*>(gh.dst)[i] = static_cast<uint16_t>(rne16(x * scale_b));
+  }
+}
+
+// Slices [0, fold_slices) are grad_W's; the later ones grad_h's (kScale only).
 template <bool kAccumulate, bool kScale>
-__global__ __launch_bounds__(64) void ce_grad_w_fold_kernel(float* __restrict__ acc, FoldChunks ch, int n,
-                                                            int64_t nw, int64_t first_slice,
-                                                            const float* __restrict__ grad_out,
-                                                            const float* __restrict__ n_valid) {
+__global__ __launch_bounds__(64) void ce_grads_kernel(float* __restrict__ acc, FoldChunks ch, int n, int64_t nw,
+                                                      int64_t fold_slices, int64_t first_slice, GradH gh,
+                                                      const float* __restrict__ grad_out,
+                                                      const float* __restrict__ n_valid) {
   const float scale = kScale ? *grad_out / *n_valid : 1.0f;
+  const int64_t slice = first_slice + blockIdx.x;
+  if (kScale && slice >= fold_slices) {
+    grad_h_slice(gh, (slice - fold_slices) * kGradHSlice, scale);
+    return;
+  }
   uint64_t misaligned = reinterpret_cast<uint64_t>(acc) & 15u;
 #pragma unroll
   for (int c = 0; c < kMaxFold; ++c)
     if (c < n) misaligned |= reinterpret_cast<uint64_t>(ch.p[c]) & 7u;
-  const int64_t e = (first_slice + blockIdx.x) * 256 + static_cast<int64_t>(threadIdx.x) * 4;
+  const int64_t e = slice * 256 + static_cast<int64_t>(threadIdx.x) * 4;
   if (misaligned == 0 && e + 4 <= nw) {
     u32x2 w[kMaxFold];
 #pragma unroll
@@ -640,30 +698,41 @@ __global__ __launch_bounds__(64) void ce_grad_w_fold_kernel(float* __restrict__ 
   }
 }
 
-// Backward of fp32 hidden states, fused_linear_ce.py:68,80,120: the reference keeps grad_hidden
-// in the hidden states' dtype, so under autocast its fp32 buffer holds the widened bf16 GEMM
-// result (`grad_hidden[s:e] = gh`, -0 kept) and is scaled in fp32 (`mul_(scale)`):
-// dst = float(src) * (g / n_valid).
-__global__ __launch_bounds__(256) void ce_widen_scale_kernel(float* __restrict__ dst,
-                                                             const uint16_t* __restrict__ src, int64_t n,
-                                                             const float* __restrict__ grad_out,
-                                                             const float* __restrict__ n_valid) {
-  const float scale = *grad_out / *n_valid;
-  const bool vec = ((reinterpret_cast<uint64_t>(dst) | reinterpret_cast<uint64_t>(src)) & 15u) == 0;
-  const int64_t vend = vec ? (n & ~int64_t(7)) : 0;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * 256 * 8;
-  for (int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 8; i < vend; i += stride) {
-    const u32x4 w = *reinterpret_cast<const u32x4*>(src + i);
-    f32x4 a = {lo16(w.x), hi16(w.x), lo16(w.y), hi16(w.y)};
-    f32x4 b = {lo16(w.z), hi16(w.z), lo16(w.w), hi16(w.w)};
-    a.x = a.x * scale; a.y = a.y * scale; a.z = a.z * scale; a.w = a.w * scale;
-    b.x = b.x * scale; b.y = b.y * scale; b.z = b.z * scale; b.w = b.w * scale;
-    *reinterpret_cast<f32x4*>(dst + i) = a;
-    *reinterpret_cast<f32x4*>(dst + i + 4) = b;
+// bf16 = RNE(fp32), NaN -> 0x7FC0, over two arrays in one launch: the hidden states and the weight
+// that autocast casts for the products. 512 elements a wave, two groups of 4 a lane, both loaded
+// before either is stored. Bound: HBM, 6 bytes an element; 138 us for 151,936 x 1024 (6.7 TB/s,
+// against 148 for the library's cast, which also took a launch for each array).
+struct CastPart {
+  uint16_t* dst;
+  const float* src;
+  int64_t n;
+};
+constexpr int kCastSlice = 512;
+
+__global__ __launch_bounds__(64) void ce_cast_kernel(CastPart a, CastPart b, int64_t slices_a, int64_t first_slice) {
+  int64_t slice = first_slice + blockIdx.x;
+  const CastPart p = slice < slices_a ? a : b;
+  if (slice >= slices_a) slice -= slices_a;
+  const int64_t start = slice * kCastSlice;
+  const int64_t end = start + kCastSlice < p.n ? start + kCastSlice : p.n;
+  int64_t done = start;
+  if (((reinterpret_cast<uint64_t>(p.src) & 15u) | (reinterpret_cast<uint64_t>(p.dst) & 7u)) == 0) {
+    done = start + ((end - start) & ~int64_t(3));
+    const int64_t e0 = start + static_cast<int64_t>(threadIdx.x) * 4, e1 = e0 + 256;
+    f32x4 x[2] = {};
+    if (e0 < done) x[0] = ld_nt(reinterpret_cast<const f32x4*>(p.src + e0));
+    if (e1 < done) x[1] = ld_nt(reinterpret_cast<const f32x4*>(p.src + e1));
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int64_t e = u == 0 ? e0 : e1;
+      if (e >= done) continue;
+      u32x2 o;
+      o.x = rne16(x[u].x) | (rne16(x[u].y) << 16);
+      o.y = rne16(x[u].z) | (rne16(x[u].w) << 16);
+      *reinterpret_cast<u32x2*>(p.dst + e) = o;  // read next by the GEMMs
+    }
   }
-  for (int64_t i = vend + static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < n;
-       i += static_cast<int64_t>(gridDim.x) * 256)
-    dst[i] = __uint_as_float(static_cast<uint32_t>(src[i]) << 16) * scale;
+  for (int64_t i = done + threadIdx.x; i < end; i += 64) p.dst[i] = static_cast<uint16_t>(rne16(p.src[i]));
 }
 
 int ce_check_launch(const char* what) {
@@ -771,30 +840,31 @@ int ce_rows_f32_launch(float* d_logits, int64_t ld, const int64_t* d_labels, int
   return TM_OK;
 }
 
-// One ce_grad_w_fold_kernel pass over nw elements: one 64-thread workgroup per 256-element
-// slice, over as many launches as the 2^32 work-item limit of a launch requires.
-int fold_launch(float* d_grad_w, const FoldChunks& ch, int n_chunks, int64_t nw, int accumulate,
-                const float* d_grad_out, const float* d_n_valid, void* stream) {
+// One ce_grads_kernel pass: grad_W's nw elements (one 64-thread workgroup per 256-element slice),
+// then grad_h's (512-element slices, only with a scale), over as many launches as the 2^32
+// work-item limit of a launch requires.
+int grads_launch(float* d_grad_w, const FoldChunks& ch, int n_chunks, int64_t nw, int accumulate, const GradH& gh,
+                 const float* d_grad_out, const float* d_n_valid, void* stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool scale = d_grad_out != nullptr;
-  const int64_t slices = (nw + 255) / 256;
+  const int64_t fold = (nw + 255) / 256, slices = fold + (gh.n + kGradHSlice - 1) / kGradHSlice;
   constexpr int64_t kMaxSlicesPerLaunch = int64_t(1) << 25;  // 2^31 work-items
   for (int64_t first = 0; first < slices; first += kMaxSlicesPerLaunch) {
     const int64_t count = slices - first < kMaxSlicesPerLaunch ? slices - first : kMaxSlicesPerLaunch;
     const dim3 grid(static_cast<uint32_t>(count)), block(64);
     if (accumulate && scale)
-      hipLaunchKernelGGL((ce_grad_w_fold_kernel<true, true>), grid, block, 0, s, d_grad_w, ch, n_chunks, nw,
-                         first, d_grad_out, d_n_valid);
+      hipLaunchKernelGGL((ce_grads_kernel<true, true>), grid, block, 0, s, d_grad_w, ch, n_chunks, nw, fold, first, gh,
+                         d_grad_out, d_n_valid);
     else if (accumulate)
-      hipLaunchKernelGGL((ce_grad_w_fold_kernel<true, false>), grid, block, 0, s, d_grad_w, ch, n_chunks, nw,
-                         first, d_grad_out, d_n_valid);
+      hipLaunchKernelGGL((ce_grads_kernel<true, false>), grid, block, 0, s, d_grad_w, ch, n_chunks, nw, fold, first, gh,
+                         d_grad_out, d_n_valid);
     else if (scale)
-      hipLaunchKernelGGL((ce_grad_w_fold_kernel<false, true>), grid, block, 0, s, d_grad_w, ch, n_chunks, nw,
-                         first, d_grad_out, d_n_valid);
+      hipLaunchKernelGGL((ce_grads_kernel<false, true>), grid, block, 0, s, d_grad_w, ch, n_chunks, nw, fold, first, gh,
+                         d_grad_out, d_n_valid);
     else
-      hipLaunchKernelGGL((ce_grad_w_fold_kernel<false, false>), grid, block, 0, s, d_grad_w, ch, n_chunks, nw,
-                         first, d_grad_out, d_n_valid);
-    const int rc = ce_check_launch("ce_grad_w_fold_kernel");
+      hipLaunchKernelGGL((ce_grads_kernel<false, false>), grid, block, 0, s, d_grad_w, ch, n_chunks, nw, fold, first,
+                         gh, d_grad_out, d_n_valid);
+    const int rc = ce_check_launch("ce_grads_kernel");
     if (rc != TM_OK) return rc;
   }
   return TM_OK;
@@ -811,23 +881,15 @@ int ce_grad_w_launch(float* d_grad_w, const uint16_t* d_chunk, const uint16_t* d
   FoldChunks ch = {};
   ch.p[0] = d_chunk;
   if (kTwo) ch.p[1] = d_chunk2;
-  return fold_launch(d_grad_w, ch, kTwo ? 2 : 1, nw, accumulate, d_grad_out, d_n_valid, stream);
+  return grads_launch(d_grad_w, ch, kTwo ? 2 : 1, nw, accumulate, GradH{}, d_grad_out, d_n_valid, stream);
 }
 
-int ce_grad_w_fold_launch(float* d_grad_w, const uint16_t* const* h_chunks, int n_chunks, int64_t nw,
-                          int accumulate, const float* d_grad_out, const float* d_n_valid, void* stream) {
-  const char* who = "tm_ce_grad_w_fold";
-  if (nw < 0 || n_chunks < 1 || n_chunks > kMaxFold)
-    return ce_fail(TM_EINVAL, "%s: %d chunks (1 to %d) of %lld elements", who, n_chunks, kMaxFold, (long long)nw);
-  if (!h_chunks || !d_grad_w || (d_grad_out != nullptr) != (d_n_valid != nullptr))
-    return ce_fail(TM_EINVAL, "%s: null pointer", who);
-  FoldChunks ch = {};
+int fold_chunks(const uint16_t* const* h_chunks, int n_chunks, FoldChunks& ch, const char* who) {
   for (int c = 0; c < n_chunks; ++c) {
-    if (!h_chunks[c]) return ce_fail(TM_EINVAL, "%s: null chunk %d", who, c);
+    if (!h_chunks || !h_chunks[c]) return ce_fail(TM_EINVAL, "%s: null chunk %d", who, c);
     ch.p[c] = h_chunks[c];
   }
-  if (nw == 0) return TM_OK;
-  return fold_launch(d_grad_w, ch, n_chunks, nw, accumulate, d_grad_out, d_n_valid, stream);
+  return TM_OK;
 }
 
 }  // namespace
@@ -870,12 +932,33 @@ int tm_ce_rows_loss_f32(const float* d_logits, int64_t ld, const int64_t* d_labe
 
 int tm_ce_loss(const float* d_row_loss, const int64_t* d_labels, int64_t rows, int64_t ignore_index,
                float* d_out3, void* stream) {
+  return tm_ce_mean_loss(d_row_loss, d_labels, rows, ignore_index, d_out3, d_out3 ? d_out3 + 2 : nullptr, stream);
+}
+
+int tm_ce_mean_loss(const float* d_row_loss, const int64_t* d_labels, int64_t rows, int64_t ignore_index,
+                    float* d_out2, float* d_loss, void* stream) {
   if (rows < 0) return ce_fail(TM_EINVAL, "tm_ce_loss: negative rows");
-  if (!d_out3 || (rows > 0 && (!d_row_loss || !d_labels)))
+  if (!d_out2 || !d_loss || (rows > 0 && (!d_row_loss || !d_labels)))
     return ce_fail(TM_EINVAL, "tm_ce_loss: null pointer");
-  hipLaunchKernelGGL(ce_loss_kernel, dim3(1), dim3(256), 0, static_cast<hipStream_t>(stream),
-                     d_row_loss, d_labels, rows, ignore_index, d_out3);
+  hipLaunchKernelGGL(ce_loss_kernel, dim3(1), dim3(kLossThreads), 0, static_cast<hipStream_t>(stream),
+                     d_row_loss, d_labels, rows, ignore_index, d_out2, d_loss);
   return ce_check_launch("ce_loss_kernel");
+}
+
+int tm_ce_finish(float* d_grad_w, const uint16_t* const* h_chunks, int n_chunks, int64_t nw, int accumulate,
+                 const uint16_t* d_grad_h, void* d_grad_h_out, int64_t nh, int wide, const float* d_grad_out,
+                 const float* d_n_valid, void* stream) {
+  const char* who = "tm_ce_finish";
+  if (nh < 0 || nw < 0 || n_chunks < 0 || n_chunks > kMaxFold)
+    return ce_fail(TM_EINVAL, "%s: %d chunks (0 to %d) of %lld elements, grad_h of %lld", who, n_chunks, kMaxFold,
+                   (long long)nw, (long long)nh);
+  if ((nh > 0 && (!d_grad_h || !d_grad_h_out)) || (nw > 0 && !d_grad_w) || !d_grad_out || !d_n_valid)
+    return ce_fail(TM_EINVAL, "%s: null pointer", who);
+  FoldChunks ch = {};
+  if (nw > 0)
+    if (int rc = fold_chunks(h_chunks, n_chunks, ch, who)) return rc;
+  return grads_launch(d_grad_w, ch, nw > 0 ? n_chunks : 0, nw, accumulate, GradH{d_grad_h, d_grad_h_out, nh, wide != 0},
+                      d_grad_out, d_n_valid, stream);
 }
 
 int tm_ce_scale_grads(uint16_t* d_grad_h, int64_t nh, float* d_grad_w, int64_t nw,
@@ -883,14 +966,24 @@ int tm_ce_scale_grads(uint16_t* d_grad_h, int64_t nh, float* d_grad_w, int64_t n
   if (nh < 0 || nw < 0) return ce_fail(TM_EINVAL, "tm_ce_scale_grads: negative size");
   if ((nh > 0 && !d_grad_h) || (nw > 0 && !d_grad_w) || !d_grad_out || !d_n_valid)
     return ce_fail(TM_EINVAL, "tm_ce_scale_grads: null pointer");
-  int64_t n = nh > nw ? nh : nw;
-  int64_t blocks = (n + 256 * 8 - 1) / (256 * 8);
-  if (blocks < 1) blocks = 1;
-  if (blocks > 65536) blocks = 65536;
-  hipLaunchKernelGGL(ce_scale_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), d_grad_h, nh, nw > 0 ? d_grad_w : nullptr, nw,
-                     d_grad_out, d_n_valid);
-  return ce_check_launch("ce_scale_kernel");
+  return tm_ce_finish(d_grad_w, nullptr, 0, nw, 1, d_grad_h, d_grad_h, nh, 0, d_grad_out, d_n_valid, stream);
+}
+
+int tm_ce_cast2(uint16_t* d_dst0, const float* d_src0, int64_t n0, uint16_t* d_dst1, const float* d_src1, int64_t n1,
+                void* stream) {
+  if (n0 < 0 || n1 < 0) return ce_fail(TM_EINVAL, "tm_ce_cast2: negative size");
+  if ((n0 > 0 && (!d_dst0 || !d_src0)) || (n1 > 0 && (!d_dst1 || !d_src1)))
+    return ce_fail(TM_EINVAL, "tm_ce_cast2: null pointer");
+  const int64_t s0 = (n0 + kCastSlice - 1) / kCastSlice, slices = s0 + (n1 + kCastSlice - 1) / kCastSlice;
+  constexpr int64_t kMaxSlicesPerLaunch = int64_t(1) << 25;  // 2^31 work-items
+  for (int64_t first = 0; first < slices; first += kMaxSlicesPerLaunch) {
+    const int64_t count = slices - first < kMaxSlicesPerLaunch ? slices - first : kMaxSlicesPerLaunch;
+    hipLaunchKernelGGL(ce_cast_kernel, dim3(static_cast<uint32_t>(count)), dim3(64), 0,
+                       static_cast<hipStream_t>(stream), CastPart{d_dst0, d_src0, n0}, CastPart{d_dst1, d_src1, n1}, s0,
+                       first);
+    if (int rc = ce_check_launch("ce_cast_kernel")) return rc;
+  }
+  return TM_OK;
 }
 
 int tm_ce_grad_w(float* d_grad_w, const uint16_t* d_chunk, int64_t nw, int accumulate,
@@ -907,7 +1000,15 @@ int tm_ce_grad_w2(float* d_grad_w, const uint16_t* d_chunk, const uint16_t* d_ch
 
 int tm_ce_grad_w_fold(float* d_grad_w, const uint16_t* const* h_chunks, int n_chunks, int64_t nw, int accumulate,
                       const float* d_grad_out, const float* d_n_valid, void* stream) {
-  return ce_grad_w_fold_launch(d_grad_w, h_chunks, n_chunks, nw, accumulate, d_grad_out, d_n_valid, stream);
+  const char* who = "tm_ce_grad_w_fold";
+  if (nw < 0 || n_chunks < 1 || n_chunks > kMaxFold)
+    return ce_fail(TM_EINVAL, "%s: %d chunks (1 to %d) of %lld elements", who, n_chunks, kMaxFold, (long long)nw);
+  if (!h_chunks || !d_grad_w || (d_grad_out != nullptr) != (d_n_valid != nullptr))
+    return ce_fail(TM_EINVAL, "%s: null pointer", who);
+  FoldChunks ch = {};
+  if (int rc = fold_chunks(h_chunks, n_chunks, ch, who)) return rc;
+  if (nw == 0) return TM_OK;
+  return grads_launch(d_grad_w, ch, n_chunks, nw, accumulate, GradH{}, d_grad_out, d_n_valid, stream);
 }
 
 int tm_ce_widen_scale(float* d_dst, const uint16_t* d_src, int64_t n, const float* d_grad_out,
@@ -915,11 +1016,7 @@ int tm_ce_widen_scale(float* d_dst, const uint16_t* d_src, int64_t n, const floa
   if (n < 0) return ce_fail(TM_EINVAL, "tm_ce_widen_scale: negative size");
   if (n == 0) return TM_OK;
   if (!d_dst || !d_src || !d_grad_out || !d_n_valid) return ce_fail(TM_EINVAL, "tm_ce_widen_scale: null pointer");
-  int64_t blocks = (n + 256 * 8 - 1) / (256 * 8);
-  if (blocks > 65536) blocks = 65536;
-  hipLaunchKernelGGL(ce_widen_scale_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), d_dst, d_src, n, d_grad_out, d_n_valid);
-  return ce_check_launch("ce_widen_scale_kernel");
+  return tm_ce_finish(nullptr, nullptr, 0, 0, 0, d_src, d_dst, n, 1, d_grad_out, d_n_valid, stream);
 }
 
 }  // extern "C"

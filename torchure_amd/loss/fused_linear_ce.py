@@ -24,7 +24,7 @@ K slices for grad_W.
 then tm_ce_loss sums the per-row losses in a fixed order (deterministic).
 
 The last chunk's bf16 grad_W is not added in forward: it waits for backward, where
-tm_ce_grad_w adds it and applies grad_out / n_valid in the same pass. With a single
+tm_ce_finish adds it and applies grad_out / n_valid in the same pass. With a single
 chunk (the usual case at 4 GiB of logits) the fp32 grad_W is then written once,
 straight from the bf16 GEMM output (6 B per element), instead of a zero fill, an
 accumulate and a scaling pass (22 B per element). With several chunks, the chunks'
@@ -44,7 +44,7 @@ Hidden states are bf16 or fp32. fp32 inside bf16 CUDA autocast is the trainer's 
 (objectives/autoregressive.py:38-44): it passes the final norm's fp32 output, for which the
 reference's buffers take fp32 (:65,68) and autocast runs the products on bf16 casts. Here
 hidden is cast to bf16 once (RNE, as autocast does), grad_hidden stays a bf16 GEMM output
-until backward, and tm_ce_widen_scale writes the fp32 gradient float(gh) * grad_out / n_valid
+until backward, and tm_ce_finish writes the fp32 gradient float(gh) * grad_out / n_valid
 (the reference's fp32 copy and mul_, :80,120). fp32 hidden states outside autocast take the
 reference's fp32 path: fp32 GEMMs on weight.to(fp32), tm_ce_rows_f32 on fp32 logits, and the
 reference's fp32 `+=` and `mul_` for grad_W.
@@ -185,10 +185,11 @@ def _bf16(logits: torch.Tensor, dtype=torch.bfloat16) -> torch.Tensor:
 
 def _mean_loss(row_loss, labels, n, ignore_index, lib, stream):
     """(mean loss as a 0-d tensor, n_valid as a 1-element view) from the per-row losses."""
-    out3 = torch.empty(3, dtype=torch.float32, device=row_loss.device)
-    _native.check(lib.tm_ce_loss(row_loss.data_ptr(), labels.data_ptr(), n, int(ignore_index),
-                                 out3.data_ptr(), stream), "tm_ce_loss")
-    return out3[2].clone(), out3[1:2]
+    out2 = torch.empty(2, dtype=torch.float32, device=row_loss.device)
+    loss = torch.empty((), dtype=torch.float32, device=row_loss.device)
+    _native.check(lib.tm_ce_mean_loss(row_loss.data_ptr(), labels.data_ptr(), n, int(ignore_index),
+                                      out2.data_ptr(), loss.data_ptr(), stream), "tm_ce_mean_loss")
+    return loss, out2[1:2]
 
 
 def logits_gemm_fits(h: torch.Tensor, w: torch.Tensor) -> bool:
@@ -332,15 +333,13 @@ FOLD_CHUNKS = 8  # chunks per grad_W fold (tm_ce_grad_w_fold takes at most 8)
 FOLD_BYTES = 4 << 30  # bf16 chunk grad_W held before a fold, at most
 
 
-def _fold(lib, grad_weight, chunks, accumulated, g, n_valid, stream) -> None:
-    """grad_weight = ((grad_weight or +0) + float(c0) + float(c1) + ...) [* g / n_valid], the
-    reference's `grad_weight += gw` per chunk in order (fused_linear_ce.py:80-81) and, with g,
-    its backward `mul_` (:126), in one pass over the fp32 buffer."""
+def _fold(lib, grad_weight, chunks, accumulated, stream) -> None:
+    """grad_weight = ((grad_weight or +0) + float(c0) + float(c1) + ...), the reference's
+    `grad_weight += gw` per chunk in order (fused_linear_ce.py:80-81), in one pass over the fp32
+    buffer."""
     ptrs = (ctypes.c_void_p * len(chunks))(*[c.data_ptr() for c in chunks])
     _native.check(lib.tm_ce_grad_w_fold(grad_weight.data_ptr(), ptrs, len(chunks), chunks[0].numel(),
-                                        int(accumulated), g.data_ptr() if g is not None else None,
-                                        n_valid.data_ptr() if n_valid is not None else None, stream),
-                  "tm_ce_grad_w_fold")
+                                        int(accumulated), None, None, stream), "tm_ce_grad_w_fold")
 
 
 class GradHidden:
@@ -373,19 +372,53 @@ class GradHidden:
                                                     self.ws.numel(), self.stream), "tm_ce_grad_h_ld_bf16")
 
 
-def _bf16_weight(weight: torch.Tensor) -> torch.Tensor:
-    """The contiguous bf16 weight the products run on: ``weight.to(bf16)`` (RNE, as autocast
-    casts), or, for an fp32 master whose bf16 working copy is current (attached with
-    torchure_amd.attach_bf16_working_params and rewritten by each AdamW step), that copy, which
-    holds the same bits, so the cast's read of 4 and write of 2 bytes per element is skipped.
-    A copy that does not start on a 16-byte boundary (the optimizer accepts copies at any
-    offset) is not taken: this op's kernels read the weight in 16-byte vectors, and the cast
-    gives a fresh, aligned buffer with the same bits."""
+def _copy_at_hand(weight: torch.Tensor):
+    """The current bf16 working copy of an fp32 master (attached with
+    torchure_amd.attach_bf16_working_params and rewritten by each AdamW step), which holds the
+    bits of ``weight.to(bf16)``, or None. A copy that does not start on a 16-byte boundary (the
+    optimizer accepts copies at any offset) is not taken: this op's kernels read the weight in
+    16-byte vectors, and the cast gives a fresh, aligned buffer with the same bits."""
     if weight.dtype == torch.float32:
         w = current_copy(weight)
         if w is not None and w.data_ptr() % 16 == 0:
             return w.detach()
-    return weight.to(torch.bfloat16).contiguous()
+    return None
+
+
+def _bf16_weight(weight: torch.Tensor) -> torch.Tensor:
+    """The contiguous bf16 weight the products run on: ``weight.to(bf16)`` (RNE, as autocast
+    casts), or its current working copy, which skips the cast's read of 4 and write of 2 bytes
+    per element."""
+    w = _copy_at_hand(weight)
+    return weight.to(torch.bfloat16).contiguous() if w is None else w
+
+
+def _castable(t: torch.Tensor) -> bool:
+    """fp32 values that tm_ce_cast2 may read from memory as they are; anything else (other
+    strides, a tensor subclass with a cast of its own, a lazy negation) takes ``Tensor.to``."""
+    return (t.dtype == torch.float32 and type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_contiguous()
+            and not t.is_neg())
+
+
+def _bf16_operands(hidden, weight, mode, lib, stream):
+    """(hidden, weight) in bf16 as the products read them: autocast's casts (RNE) where they are
+    fp32, both in one launch, unless a current working copy of the weight is at hand."""
+    hb, w = hidden, _copy_at_hand(weight)
+    parts = []
+    if mode == "autocast":
+        hb = torch.empty_like(hidden, dtype=torch.bfloat16) if _castable(hidden) else hidden.to(torch.bfloat16)
+        if _castable(hidden):
+            parts.append((hb, hidden))
+    if w is None:
+        if _castable(weight):
+            w = torch.empty_like(weight, dtype=torch.bfloat16)
+            parts.append((w, weight))
+        else:
+            w = weight.to(torch.bfloat16).contiguous()
+    if parts:
+        args = [x for dst, src in parts for x in (dst.data_ptr(), src.data_ptr(), src.numel())]
+        _native.check(lib.tm_ce_cast2(*(args + [None, None, 0])[:6], stream), "tm_ce_cast2")
+    return hb, w
 
 
 def _loss_only(hidden, weight, labels, ignore_index, chunk_size):
@@ -397,8 +430,10 @@ def _loss_only(hidden, weight, labels, ignore_index, chunk_size):
     lib = _native.lib()
     stream = _native.stream_handle(hidden.device)
     dt = torch.float32 if mode == "fp32" else torch.bfloat16
-    hb = hidden.to(torch.bfloat16) if mode == "autocast" else hidden  # autocast's cast (RNE)
-    w = weight.to(dt).contiguous() if mode == "fp32" else _bf16_weight(weight)
+    if mode == "fp32":
+        hb, w = hidden, weight.to(dt).contiguous()
+    else:
+        hb, w = _bf16_operands(hidden, weight, mode, lib, stream)
     rows_loss = lib.tm_ce_rows_loss_f32 if mode == "fp32" else lib.tm_ce_rows_loss_bf16
     row_loss = torch.empty(n, dtype=torch.float32, device=hidden.device)
     for s in range(0, n, chunk):
@@ -456,8 +491,7 @@ class _FusedLinearCE(torch.autograd.Function):
         fp32 = mode == "autocast"
         lib = _native.lib()
         stream = _native.stream_handle(hidden.device)
-        hb = hidden.to(torch.bfloat16) if fp32 else hidden  # autocast's cast (RNE)
-        w = _bf16_weight(weight)  # cast once, not per chunk (or the current working copy)
+        hb, w = _bf16_operands(hidden, weight, mode, lib, stream)  # cast once, not per chunk
         want_h, want_w = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         # bf16 GEMM output either way; for fp32 hidden it is widened and scaled in backward
         grad_hidden = torch.empty(hidden.shape, dtype=torch.bfloat16, device=hidden.device) if want_h else None
@@ -495,7 +529,7 @@ class _FusedLinearCE(torch.autograd.Function):
                     if len(pending) == FOLD_CHUNKS or len(pending) * pending[0].numel() * 2 >= FOLD_BYTES:
                         if grad_weight is None:
                             grad_weight = torch.empty(weight.shape, dtype=torch.float32, device=weight.device)
-                        _fold(lib, grad_weight, pending, accumulated, None, None, stream)
+                        _fold(lib, grad_weight, pending, accumulated, stream)
                         accumulated = True
                         pending = []
             block = logits = None
@@ -533,34 +567,29 @@ class _FusedLinearCE(torch.autograd.Function):
         lib = _native.lib()
         stream = _native.stream_handle(n_valid.device)
         g = grad_out.detach().to(torch.float32).contiguous()
-        scale_w = None  # an fp32 grad_W that still needs the plain scaling pass
+        # the chunks still pending, then the last (at most FOLD_CHUNKS), added into grad_W with the
+        # scaling, and grad_h scaled, in one launch
+        chunks, accumulated = [], ctx.accumulated
         if ctx.want_w:
             shape, device = ctx.weight_meta
             if last_gw is not None:
+                chunks = pending + [last_gw]
                 if grad_weight is None:
                     grad_weight = torch.empty(shape, dtype=torch.float32, device=device)
-                # the chunks still pending, then the last, with the scaling (at most FOLD_CHUNKS)
-                _fold(lib, grad_weight, pending + [last_gw], ctx.accumulated, g, n_valid, stream)
-                del last_gw, pending
             else:  # no rows at all: the reference scales its zero-filled buffer
-                grad_weight = scale_w = torch.zeros(shape, dtype=torch.float32, device=device)
-        if ctx.fp32_hidden and grad_hidden is not None:
+                grad_weight, accumulated = torch.zeros(shape, dtype=torch.float32, device=device), True
+        short, wide = grad_hidden, ctx.fp32_hidden
+        if wide and grad_hidden is not None:
             # fp32 hidden: the gradient is fp32 = float(bf16 GEMM result) * scale
-            wide = torch.empty(grad_hidden.shape, dtype=torch.float32, device=grad_hidden.device)
-            _native.check(lib.tm_ce_widen_scale(wide.data_ptr(), grad_hidden.data_ptr(), grad_hidden.numel(),
-                                                g.data_ptr(), n_valid.data_ptr(), stream), "tm_ce_widen_scale")
-            grad_hidden, wide = wide, grad_hidden
-            del wide
-            scale_h = None
-        else:
-            scale_h = grad_hidden
-        rc = lib.tm_ce_scale_grads(
-            scale_h.data_ptr() if scale_h is not None else None,
-            scale_h.numel() if scale_h is not None else 0,
-            scale_w.data_ptr() if scale_w is not None else None,
-            scale_w.numel() if scale_w is not None else 0,
-            g.data_ptr(), n_valid.data_ptr(), stream)
-        _native.check(rc, "tm_ce_scale_grads")
+            grad_hidden = torch.empty(short.shape, dtype=torch.float32, device=short.device)
+        rc = lib.tm_ce_finish(
+            grad_weight.data_ptr() if grad_weight is not None else None,
+            (ctypes.c_void_p * len(chunks))(*[c.data_ptr() for c in chunks]), len(chunks),
+            grad_weight.numel() if grad_weight is not None else 0, int(accumulated),
+            short.data_ptr() if short is not None else None,
+            grad_hidden.data_ptr() if grad_hidden is not None else None,
+            short.numel() if short is not None else 0, int(wide), g.data_ptr(), n_valid.data_ptr(), stream)
+        _native.check(rc, "tm_ce_finish")
         return grad_hidden, grad_weight, None, None, None
 
 
