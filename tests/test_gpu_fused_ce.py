@@ -1063,3 +1063,71 @@ def test_two_calls_on_two_streams_equal_sequential():
     for a, b in zip(seq, out):
         for x, y in zip(a, b):
             assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("mode", ["bf16", "autocast"])
+@pytest.mark.parametrize("n,chunk", [(640, 256), (256, 256), (2304, 256)])
+def test_native_chunk_loop_equals_the_unpadded_loop(mode, n, chunk):
+    """The native loop on padded logits and the Python loop on unpadded ones, on shapes that need
+    no padding (every kernel then runs on the same operands): the same bits of loss, counts,
+    gradients and hand-over (1, 3 and 9 chunks: one fold), with and without each gradient."""
+    from torchure_amd.loss import fused_linear_ce as fce
+
+    g = torch.Generator(device=DEV).manual_seed(n)
+    d, v = 256, 4096
+    hidden = torch.randn(n, d, device=DEV, generator=g)
+    hidden = hidden if mode == "autocast" else hidden.to(torch.bfloat16)
+    weight = torch.randn(v, d, device=DEV, generator=g) * 0.05
+    labels = torch.randint(0, v, (n,), device=DEV, generator=g)
+    labels[::9] = -100
+    bits = {torch.float32: torch.int32, torch.bfloat16: torch.int16}
+    for want_h, want_w in ((True, True), (True, False), (False, True)):
+        a = fce._run_chunks(hidden, weight, labels, -100, chunk, mode, True, want_h, want_w)
+        b = fce._chunks_unpadded(hidden, weight, labels, -100, n, v, chunk, mode, want_h, want_w)
+        assert a[5] == b[5] and len(a[4]) == len(b[4])
+        for x, y in zip([*a[:4], *a[4]], [*b[:4], *b[4]]):
+            assert (x is None) == (y is None)
+            assert x is None or torch.equal(x.view(bits[x.dtype]), y.view(bits[y.dtype]))
+    loss = fce._run_chunks(hidden, weight, labels, -100, chunk, mode, False, False, False)[0]
+    assert torch.equal(loss.view(torch.int32), a[0].view(torch.int32))
+
+
+def test_operands_the_native_loop_does_not_read_as_they_are():
+    """Weights that are strided, of another dtype or off 16 bytes, and hidden states off 16 bytes:
+    the op gives the gradients of the plain call on the same values (the same bits where the
+    products run on the same kernels), and a failed native call raises NativeError."""
+    from torchure_amd import _native
+    from torchure_amd.loss import fused_linear_cross_entropy
+
+    g = torch.Generator(device=DEV).manual_seed(5)
+    n, d, v = 384, 128, 1024
+    hidden = torch.randn(n, d, device=DEV, generator=g).to(torch.bfloat16)
+    weight = (torch.randn(v, d, device=DEV, generator=g) * 0.05).to(torch.bfloat16)
+    labels = torch.randint(0, v, (n,), device=DEV, generator=g)
+
+    def run(h, w):
+        h, w = h.detach().requires_grad_(True), w.detach().requires_grad_(True)
+        loss = fused_linear_cross_entropy(h, w, labels, -100, 128)
+        loss.backward()
+        return loss.detach(), h.grad, w.grad.to(torch.bfloat16)  # a bf16 weight's gradient is rounded
+
+    def off16(t):
+        buf = torch.empty(t.numel() + 8, dtype=t.dtype, device=DEV)
+        out = buf[1: 1 + t.numel()].view(t.shape)
+        out.copy_(t)
+        return out
+
+    plain = run(hidden, weight)
+    strided = torch.empty(d, v, dtype=torch.bfloat16, device=DEV).t()
+    strided.copy_(weight)
+    for h, w, same in ((hidden, weight.float(), True), (hidden, strided, True), (hidden, weight.double(), True),
+                       (off16(hidden), weight, False), (hidden, off16(weight), False)):
+        for x, y in zip(run(h, w), plain):
+            if same:
+                assert torch.equal(x.view(torch.int32 if x.dtype == torch.float32 else torch.int16),
+                                   y.view(torch.int32 if y.dtype == torch.float32 else torch.int16))
+            else:  # library products: the last bit of some bf16 results
+                torch.testing.assert_close(x.float(), y.float(), rtol=2.0 ** -7, atol=2.0 ** -16)
+    with pytest.raises(_native.NativeError, match="tm_ce_logits_ld_bf16"):
+        _native.ce_host().ce_forward(hidden, weight, False, False, labels, -100, 128, (128, 128), 64, (False, False),
+                                     True, True, True, 8, 1 << 30, _native.stream_handle(DEV))

@@ -629,3 +629,139 @@ def test_pooled_state_layout(tmp_path):
     torch.save(state, tmp_path / "pooled.pt")
     torch.save({i: {k: t.clone() for k, t in st.items()} for i, st in state.items()}, tmp_path / "separate.pt")
     assert os.path.getsize(tmp_path / "pooled.pt") <= os.path.getsize(tmp_path / "separate.pt")
+
+
+def _host():
+    from torchure_amd import _native
+
+    return _native.host()
+
+
+def _collect_by_hand(params):
+    gs, holders, marks = [], [], []
+    for p in params:
+        w = getattr(p, "_tm_working", None)
+        g = p.grad if p.grad is not None else (w.grad if w is not None else None)
+        if g is None:
+            continue
+        gs.append(g)
+        holders.append(p)
+        mark = getattr(p, "_tm_owner", None)
+        if not any(m is mark for m in marks):
+            marks.append(mark)
+    return gs, holders, marks
+
+
+def test_host_collect_walks_grads_params_and_owners():
+    """collect on every kind of param (own grad, working copy's grad, both, neither; owned by one
+    optimizer, another, none): the objects and order of the Python walk."""
+    h = _host()
+    ps = [torch.nn.Parameter(torch.zeros(i + 1)) for i in range(7)]
+    a, b = object(), object()
+    for p, own in zip(ps, (a, a, b, None, a, b, a)):
+        if own is not None:
+            p._tm_owner = own
+    for i in (0, 2, 3):
+        ps[i].grad = torch.ones(i + 1)
+    for i in (1, 2, 5, 6):
+        ps[i]._tm_working = torch.zeros(i + 1, dtype=torch.bfloat16, requires_grad=True)
+    for i in (1, 2, 5):
+        ps[i]._tm_working.grad = torch.ones(i + 1, dtype=torch.bfloat16)
+    ps[4]._tm_working = None
+    got, want = h.collect(ps), _collect_by_hand(ps)
+    for x, y in zip(got, want):
+        assert len(x) == len(y) and all(i is j for i, j in zip(x, y))
+    assert h.collect([]) == ([], [], [])
+    with pytest.raises(TypeError):
+        h.collect([1])
+
+
+def test_host_stamp_sees_every_change():
+    """A Stamp matches the same tensors at the same versions only, and holds nothing alive."""
+    import weakref
+
+    h = _host()
+    ts = [torch.zeros(3) for _ in range(3)]
+    stamp = h.Stamp(ts)
+    assert stamp.matches(list(ts))
+    assert not stamp.matches(ts[:2]) and not stamp.matches(ts[::-1])
+    assert not stamp.matches(ts[:2] + [ts[2].clone()])
+    ts[1].add_(1)
+    assert not stamp.matches(ts)
+    assert h.Stamp(ts).matches(ts) and h.Stamp([]).matches([])
+    gone = weakref.ref(ts[2])
+    stamp = h.Stamp(ts)
+    keep = ts[:2]
+    del ts
+    assert gone() is None and not stamp.matches(keep + [torch.zeros(3)])
+
+
+def test_host_plan_match_refuses_every_deviation():
+    """plan_match gives the grads and their pointers for an unchanged plan, and None after each
+    single change the step's full path must see."""
+    h = _host()
+
+    def build():
+        ps = [torch.nn.Parameter(torch.zeros(4)) for _ in range(3)]
+        ws = [None, torch.zeros(4, dtype=torch.bfloat16, requires_grad=True), None]
+        ps[1]._tm_working = ws[1]
+        ps[0].grad, ws[1].grad = torch.ones(4), torch.ones(4, dtype=torch.bfloat16)
+        used = ps[:2]
+        states = [{"step": torch.zeros(()), "exp_avg": torch.zeros(4), "exp_avg_sq": torch.zeros(4)} for _ in used]
+        smap = {p: st for p, st in zip(used, states)}
+        statics = [t for p, st in zip(used, states) for t in (p, st["exp_avg"], st["exp_avg_sq"], st["step"])] + [None]
+        h.stamp([ps[1]], [ws[1]])
+        d = dict(ps=ps, ws=ws, src=b"\x01\x02\x00", statics=statics, ptrs=h.ptrs(statics), smap=smap,
+                 keys=list(smap), values=list(smap.values()), states=states, ms=[s["exp_avg"] for s in states],
+                 vs=[s["exp_avg_sq"] for s in states], ss=[s["step"] for s in states], wp=[ps[1]], ww=[ws[1]])
+        return d
+
+    def match(d):
+        return h.plan_match(d["ps"], d["ws"], d["src"], d["statics"], d["ptrs"], d["smap"], d["keys"], d["values"],
+                            d["states"], d["ms"], d["vs"], d["ss"], d["wp"], d["ww"])
+
+    d = build()
+    grads, ptrs = match(d)
+    assert grads[0] is d["ps"][0].grad and grads[1] is d["ws"][1].grad
+    assert ptrs.tolist() == [g.data_ptr() for g in grads]
+
+    def changed(change):
+        d = build()
+        change(d)
+        return match(d) is None
+
+    def set_(obj, name, value):
+        setattr(obj, name, value)
+
+    assert changed(lambda d: set_(d["ps"][2], "grad", torch.ones(4)))          # one more grad
+    assert changed(lambda d: set_(d["ps"][1], "grad", torch.ones(4)))          # another source
+    assert changed(lambda d: set_(d["ps"][0], "grad", None))
+    assert changed(lambda d: set_(d["ps"][0], "_tm_working", d["ws"][1]))      # a copy attached
+    assert changed(lambda d: set_(d["ps"][1], "_tm_working", d["ws"][1].detach()))
+    assert changed(lambda d: set_(d["ps"][0], "data", torch.zeros(4)))         # storage swapped
+    assert changed(lambda d: d["states"][0].update(exp_avg=torch.zeros(4)))
+    assert changed(lambda d: d["states"][1].pop("step"))
+    assert changed(lambda d: d["smap"].update({d["ps"][0]: dict(d["states"][0])}))
+    assert changed(lambda d: d["smap"].pop(d["ps"][0]))
+    assert changed(lambda d: d["smap"].update({d["ps"][2]: {}}))
+    assert changed(lambda d: d["ps"][1].detach().add_(1))                      # its copy is stale
+
+    def strided(d):
+        d["ps"][0].grad = torch.ones(4, 2)[:, 0]
+
+    assert changed(strided)
+
+
+def test_host_clip_match():
+    """0 for other grads, 1 for the record's, 2 for the record's after an in-place change."""
+    h = _host()
+    gs = [torch.ones(2) for _ in range(3)]
+    rec, perm = [gs[2], gs[0], gs[1]], [1, 2, 0]
+    total = h.version_sum(rec)
+    assert h.clip_match(rec, perm, gs, total) == 1
+    assert h.clip_match(rec, perm, gs[:2], total) == 0
+    assert h.clip_match(rec, [0, 1, 2], gs, total) == 0
+    assert h.clip_match(rec, [1, 2, 7], gs, total) == 0
+    assert h.clip_match(rec, perm, [gs[0].clone(), gs[1], gs[2]], total) == 0
+    gs[1].mul_(2)
+    assert h.clip_match(rec, perm, gs, total) == 2

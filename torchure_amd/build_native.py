@@ -4,8 +4,8 @@
   position-independent shared object, and the packed-fp32 target feature switched off
   (``-Xclang -target-feature -Xclang -packed-fp32-ops``) so that no v_pk_{add,mul,fma}_f32
   instructions are emitted.
-- _tm_host.<ext>.so: host-side list primitives (CPU only) as a Python extension, with g++
-  against torch's headers and libraries.
+- _tm_host.<ext>.so: host-side list primitives and the fused CE call's host loop (CPU code) as a
+  Python extension, with g++ against torch's headers and libraries.
 
 Both are compiled in parallel.
 """
@@ -47,7 +47,7 @@ def command(output: str = OUTPUT, extra: list[str] | None = None) -> list[str]:
     ]
 
 
-HOST_SOURCE = os.path.join(_HERE, "csrc", "tm_host.cpp")
+HOST_SOURCES = [os.path.join(_HERE, "csrc", f) for f in ("tm_host.cpp", "tm_ce_host.cpp")]
 
 
 def host_output() -> str:
@@ -68,7 +68,7 @@ def host_command(output: str) -> list[str]:
         f"-D_GLIBCXX_USE_CXX11_ABI={abi}", "-DTORCH_EXTENSION_NAME=_tm_host", "-DTORCH_API_INCLUDE_EXTENSION_H",
         f"-I{tdir}/include", f"-I{tdir}/include/torch/csrc/api/include",
         f"-I{sysconfig.get_paths()['include']}",
-        HOST_SOURCE,
+        *HOST_SOURCES,
         f"-L{tdir}/lib", "-lc10", "-ltorch", "-ltorch_cpu", "-ltorch_python", f"-Wl,-rpath,{tdir}/lib",
         "-o", output,
     ]

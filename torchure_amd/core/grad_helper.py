@@ -45,10 +45,7 @@ def grads_of(params) -> tuple[list[torch.Tensor], list[torch.nn.Parameter]]:
     A master parameter without its own ``.grad`` contributes the bf16 grad of
     its attached working copy (torchure_amd.optimizer.working), if any.
     """
-    ps = params if isinstance(params, list) else list(params)
-    gs, _ = _native.host().grads(ps, [getattr(p, "_tm_working", None) for p in ps])
-    holders = [p for p, g in zip(ps, gs) if g is not None]
-    grads = [g for g in gs if g is not None]
+    grads, holders, _ = _native.host().collect(params if isinstance(params, list) else list(params))
     return grads, holders
 
 
@@ -65,21 +62,23 @@ class NormLaunch:
                  chunk_elems: int = tables.DEFAULT_CHUNK_ELEMS):
         who = "clip_grad_norm"
         device = grads[0].device
-        for g in grads:
-            if g.device != device:
-                raise RuntimeError(f"{who}: all grads must be on one device ({g.device} vs {device})")
-        rows = tables.grad_table(grads, who)
+        rows, numels, fine, one_device = _native.host().grad_rows(grads)
+        if not one_device:
+            other = next(g.device for g in grads if g.device != device)
+            raise RuntimeError(f"{who}: all grads must be on one device ({other} vs {device})")
+        if not fine:
+            tables.grad_table(grads, who)  # raises with the reason
         self.device = device
         self.n = len(grads)
         self.chunk_elems = chunk_elems
-        self.chunks, self.n_chunks = tables.CHUNKS.get(rows["numel"], chunk_elems, device)
+        self.chunks, self.n_chunks = tables.CHUNKS.get(numels, chunk_elems, device)
         self.d_rows = _NORM_UPLOAD(rows, device)
         self.ws = torch.empty(_native.workspace_bytes(len(grads)), dtype=torch.uint8, device=device)
         self.norm = torch.empty((), dtype=torch.float32, device=device)
         self.clip = max_norm is not None
         self.max_norm = float(max_norm) if self.clip else 0.0
         self.coef = torch.empty((), dtype=torch.float32, device=device) if self.clip else None
-        self.home = torch.cuda.current_stream(device)
+        self.home = _native.stream_handle(device)
 
     def __call__(self) -> None:
         tables.follow_home_stream(self.home, self.device,
@@ -171,14 +170,14 @@ def clip_grad_norm(params, mesh, max_norm, shard_dims=()) -> torch.Tensor:
     """
     if shard_dims:
         _check_shard_dims(mesh, shard_dims)
-    grads, holders = grads_of(params)
+    grads, holders, marks = _native.host().collect(params if isinstance(params, list) else list(params))
     if not grads:
         assert grads, "clip_grad_norm got no grads; backward didn't run, or all params are frozen"
 
     # A clip pending from an earlier call must land before these grads are measured.
-    from torchure_amd.optimizer.adamw import materialize_pending_for, owners_of
+    from torchure_amd.optimizer.adamw import materialize_pending_for
 
-    owners = owners_of(holders)
+    owners = {mark() if mark is not None else None for mark in marks}  # the AdamW objects, or None
     materialize_pending_for(holders, owners)
 
     from torchure_amd.optimizer.working import cached_norm

@@ -53,9 +53,10 @@ class TableUploader:
     """
 
     def __init__(self, slots: int = 4):
-        self._slots: list = [None] * slots  # (pinned uint8 tensor, event or None)
+        # (pinned uint8 tensor, the part of it last used, that part's numpy view, event, its device)
+        self._slots: list = [None] * slots
         self._next = 0
-        self._last = None  # (bytes, device tensor, stream handle)
+        self._last = None  # (bytes, device tensor, device, raw stream handle)
         self._lock = threading.Lock()
 
     def __call__(self, arr: np.ndarray, device: torch.device) -> torch.Tensor:
@@ -63,28 +64,30 @@ class TableUploader:
             return self._upload(arr, device)
 
     def _upload(self, arr: np.ndarray, device: torch.device) -> torch.Tensor:
-        raw = np.ascontiguousarray(arr).view(np.uint8).reshape(-1)
-        stream = torch.cuda.current_stream(device)
+        held = arr.tobytes()
+        handle = _native.stream_handle(device)
         last = self._last
-        if (last is not None and last[1].device == device and last[2] == stream.cuda_stream
-                and last[0].size == raw.size and np.array_equal(last[0], raw)):
+        if last is not None and last[3] == handle and last[2] == device and last[0] == held:
             return last[1]
         i = self._next
         self._next = (i + 1) % len(self._slots)
         slot = self._slots[i]
-        if slot is not None and slot[1] is not None:
-            slot[1].synchronize()
-        if slot is None or slot[0].numel() < raw.size:
-            buf = torch.empty(max(raw.size, 4096) * 2, dtype=torch.uint8, pin_memory=True)
-        else:
-            buf = slot[0]
-        buf.numpy()[: raw.size] = raw
-        dev = torch.empty(max(raw.size, 8), dtype=torch.uint8, device=device)
-        dev[: raw.size].copy_(buf[: raw.size], non_blocking=True)
-        ev = torch.cuda.Event()
-        ev.record(stream)
-        self._slots[i] = (buf, ev)
-        self._last = (raw.copy(), dev, stream.cuda_stream)
+        if slot is not None:
+            slot[3].synchronize()
+        size = max(len(held), 1)
+        if slot is None or slot[1].numel() != size or slot[4] != device:
+            # a training run keeps its size and device: sliced once, one event (an event belongs to
+            # the device it was first recorded on)
+            fits = slot is not None and slot[0].numel() >= size
+            buf = slot[0] if fits else torch.empty(max(size, 4096) * 2, dtype=torch.uint8, pin_memory=True)
+            part = buf[:size]
+            slot = self._slots[i] = (buf, part, part.numpy(), torch.cuda.Event(), device)
+        _, part, view, ev, _ = slot
+        view[: len(held)] = np.frombuffer(held, dtype=np.uint8)
+        dev = torch.empty(size, dtype=torch.uint8, device=device)
+        dev.copy_(part, non_blocking=True)
+        ev.record(torch.cuda.current_stream(device))
+        self._last = (held, dev, device, handle)
         return dev
 
 
@@ -92,14 +95,14 @@ def make_ready(table: torch.Tensor, device: torch.device) -> torch.Tensor:
     """Makes a cached device table safe to read on the device's current stream.
 
     A cached table was uploaded asynchronously on the stream current at the time
-    (``_tm_home``), and its upload is marked by ``_tm_ready``, an event recorded there
-    after the copy. On any other stream, the current stream first waits for that
+    (``_tm_home``, its raw handle), and its upload is marked by ``_tm_ready``, an event recorded
+    there after the copy. On any other stream, the current stream first waits for that
     event, so a launch there never reads a table whose copy has not run yet, and
     record_stream keeps the caching allocator from reusing its block before that
     stream's work has run, should the table be evicted and freed."""
-    cur = torch.cuda.current_stream(device)
     home = getattr(table, "_tm_home", None)
-    if home is not None and cur != home:
+    if home is not None and _native.stream_handle(device) != home:
+        cur = torch.cuda.current_stream(device)
         cur.wait_event(table._tm_ready)
         table.record_stream(cur)
     return table
@@ -128,7 +131,7 @@ class ChunkTableCache:
         home = torch.cuda.current_stream(device)
         ready = torch.cuda.Event()
         ready.record(home)
-        dev._tm_home = home
+        dev._tm_home = home.cuda_stream
         dev._tm_ready = ready
         val = (dev, len(table))
         self._d[key] = val
@@ -140,15 +143,16 @@ class ChunkTableCache:
 CHUNKS = ChunkTableCache()
 
 
-def follow_home_stream(home, device: torch.device, tensors) -> None:
-    """Before a launch that was planned on stream ``home`` runs on the device's current stream:
-    if the two differ, the current stream waits for ``home`` (the tables were uploaded there,
+def follow_home_stream(home: int, device: torch.device, tensors) -> None:
+    """Before a launch that was planned on the stream with raw handle ``home`` runs on the
+    device's current stream: if the two differ, the current stream waits for ``home`` (the tables were uploaded there,
     asynchronously) and each tensor is marked as used on the current stream, so the caching
     allocator does not hand its block to other work before this stream is done with it."""
-    cur = torch.cuda.current_stream(device)
-    if cur == home:
+    if _native.stream_handle(device) == home:
         return
-    cur.wait_stream(home)
+    cur = torch.cuda.current_stream(device)
+    # handle 0 is the default stream; ExternalStream(0) would make a new one
+    cur.wait_stream(torch.cuda.ExternalStream(home, device=device) if home else torch.cuda.default_stream(device))
     for t in tensors:
         if t is not None:
             t.record_stream(cur)
@@ -185,14 +189,8 @@ def grad_table(grads: list[torch.Tensor], who: str) -> np.ndarray:
     """tm_tensor_t rows for a grad-only call (norm / scale)."""
     if not grads:
         return np.zeros(0, _native.TENSOR_DTYPE)
-    ptr, numel, code = _native.host().grad_fields(grads)
-    if not (code != 255).all():
-        return _grad_table_checked(grads, who)  # raises with the reason
-    rows = np.zeros(len(grads), dtype=_native.TENSOR_DTYPE)
-    rows["grad"] = ptr
-    rows["numel"] = numel
-    rows["flags"] = code  # 0 = TM_GRAD_BF16, 1 = TM_GRAD_F32
-    return rows
+    rows, _, fine, _ = _native.host().grad_rows(grads)
+    return rows.view(_native.TENSOR_DTYPE) if fine else _grad_table_checked(grads, who)  # raises with the reason
 
 
 def _grad_table_checked(grads: list[torch.Tensor], who: str) -> np.ndarray:

@@ -13,13 +13,26 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/variable.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <stdexcept>
+#include <string>
 #include <utility>
+#include <vector>
 
 namespace py = pybind11;
 
 namespace {
+
+// The attribute `name` of o, or nullptr when it has none or it is None (new reference otherwise).
+// A missing attribute is looked up without raising: on a list of params without working copies
+// the AttributeErrors took most of the walk (150 ns each).
+PyObject* attr_or_null(PyObject* o, PyObject* name) {
+  PyObject* a = nullptr;
+  if (_PyObject_LookupAttr(o, name, &a) < 0) throw py::error_already_set();
+  if (a == Py_None) Py_CLEAR(a);
+  return a;
+}
 
 // nullptr for None; throws for anything that is not a tensor.
 inline const at::Tensor* tensor_or_null(PyObject* o) {
@@ -139,27 +152,50 @@ py::tuple grad_fields(const py::list& ts) {
 // True if, for every i, state_map[params[i]] is states[i] and that dict's "exp_avg",
 // "exp_avg_sq" and "step" entries are ms[i], vs[i] and ss[i] (object identity). A missing
 // entry is a mismatch: the lookup does not run a defaultdict's factory.
-bool states_same(const py::dict& state_map, const py::list& params, const py::list& states,
-                 const py::list& ms, const py::list& vs, const py::list& ss) {
-  const Py_ssize_t n = PyList_GET_SIZE(params.ptr());
-  for (const py::list* l : {&states, &ms, &vs, &ss})
+PyObject* dict_item(PyObject* d, PyObject* k) {  // borrowed, or nullptr if absent
+  PyObject* r = PyDict_GetItemWithError(d, k);
+  if (!r && PyErr_Occurred()) throw py::error_already_set();
+  return r;
+}
+
+// The entries' part of it: states[i] is a dict whose "exp_avg", "exp_avg_sq" and "step" are these.
+bool entries_same(const py::list& states, const py::list& ms, const py::list& vs, const py::list& ss) {
+  const Py_ssize_t n = PyList_GET_SIZE(states.ptr());
+  for (const py::list* l : {&ms, &vs, &ss})
     if (PyList_GET_SIZE(l->ptr()) != n) return false;
   static PyObject* k_m = PyUnicode_InternFromString("exp_avg");
   static PyObject* k_v = PyUnicode_InternFromString("exp_avg_sq");
   static PyObject* k_s = PyUnicode_InternFromString("step");
-  auto item = [](PyObject* d, PyObject* k) -> PyObject* {  // borrowed, or nullptr if absent
-    PyObject* r = PyDict_GetItemWithError(d, k);
-    if (!r && PyErr_Occurred()) throw py::error_already_set();
-    return r;
-  };
   for (Py_ssize_t i = 0; i < n; ++i) {
-    PyObject* st = item(state_map.ptr(), list_item(params, i));
-    if (!st || st != list_item(states, i) || !PyDict_Check(st)) return false;
-    if (item(st, k_m) != list_item(ms, i) || item(st, k_v) != list_item(vs, i) ||
-        item(st, k_s) != list_item(ss, i))
+    PyObject* st = list_item(states, i);
+    if (!PyDict_Check(st) || dict_item(st, k_m) != list_item(ms, i) || dict_item(st, k_v) != list_item(vs, i) ||
+        dict_item(st, k_s) != list_item(ss, i))
       return false;
   }
   return true;
+}
+
+bool states_same(const py::dict& state_map, const py::list& params, const py::list& states,
+                 const py::list& ms, const py::list& vs, const py::list& ss) {
+  const Py_ssize_t n = PyList_GET_SIZE(params.ptr());
+  if (PyList_GET_SIZE(states.ptr()) != n) return false;
+  for (Py_ssize_t i = 0; i < n; ++i)
+    if (dict_item(state_map.ptr(), list_item(params, i)) != list_item(states, i)) return false;
+  return entries_same(states, ms, vs, ss);
+}
+
+// True if d holds exactly these key and value objects in this order. Compared in the dict's own
+// order, so no key is hashed (a tensor's hash is a Python call, 0.2 us).
+bool items_same(const py::dict& d, const py::list& keys, const py::list& values) {
+  const Py_ssize_t n = PyList_GET_SIZE(keys.ptr());
+  if (PyDict_Size(d.ptr()) != n || PyList_GET_SIZE(values.ptr()) != n) return false;
+  PyObject *k, *v;
+  Py_ssize_t pos = 0, i = 0;
+  while (PyDict_Next(d.ptr(), &pos, &k, &v)) {
+    if (i >= n || k != list_item(keys, i) || v != list_item(values, i)) return false;
+    ++i;
+  }
+  return i == n;
 }
 
 // True if getattr(objs[i], name, None) is expected[i] for every i.
@@ -167,15 +203,9 @@ bool attrs_same(const py::list& objs, const py::str& name, const py::list& expec
   const Py_ssize_t n = PyList_GET_SIZE(objs.ptr());
   if (PyList_GET_SIZE(expected.ptr()) != n) return false;
   for (Py_ssize_t i = 0; i < n; ++i) {
-    PyObject* a = PyObject_GetAttr(list_item(objs, i), name.ptr());  // new reference
-    if (!a) {
-      if (!PyErr_ExceptionMatches(PyExc_AttributeError)) throw py::error_already_set();
-      PyErr_Clear();
-      Py_INCREF(Py_None);
-      a = Py_None;
-    }
-    const bool same_obj = a == list_item(expected, i);
-    Py_DECREF(a);
+    PyObject* a = attr_or_null(list_item(objs, i), name.ptr());
+    const bool same_obj = (a ? a : Py_None) == list_item(expected, i);
+    Py_XDECREF(a);
     if (!same_obj) return false;
   }
   return true;
@@ -234,10 +264,271 @@ bool stamped(const py::list& params, const py::list& works) {
   return true;
 }
 
+PyObject* working_name() {
+  static PyObject* name = PyUnicode_InternFromString("_tm_working");
+  return name;
+}
+
+// For a clip over params: (grads, the params that carry them, their distinct `_tm_owner` marks).
+// A master without a grad of its own contributes the grad of its working copy, if any.
+py::tuple collect(const py::list& params) {
+  static PyObject* k_owner = PyUnicode_InternFromString("_tm_owner");
+  const Py_ssize_t n = PyList_GET_SIZE(params.ptr());
+  py::list grads, holders, owners;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject* po = list_item(params, i);
+    const at::Tensor* p = tensor_or_null(po);
+    if (!p) continue;
+    py::object g;
+    if (p->grad().defined()) {
+      g = py::reinterpret_steal<py::object>(THPVariable_Wrap(p->grad()));
+    } else {
+      py::object wo = py::reinterpret_steal<py::object>(attr_or_null(po, working_name()));
+      const at::Tensor* w = wo.ptr() ? tensor_or_null(wo.ptr()) : nullptr;
+      if (!w || !w->grad().defined()) continue;
+      g = py::reinterpret_steal<py::object>(THPVariable_Wrap(w->grad()));
+    }
+    grads.append(g);
+    holders.append(py::reinterpret_borrow<py::object>(po));
+    py::object own = py::reinterpret_steal<py::object>(attr_or_null(po, k_owner));
+    if (!own.ptr()) own = py::none();
+    bool known = false;
+    for (const auto& o : owners) known = known || o.ptr() == own.ptr();
+    if (!known) owners.append(own);
+  }
+  return py::make_tuple(grads, holders, owners);
+}
+
+// tm_tensor_t (include/torchure_amd.h) as the host writes it.
+struct TensorRow {
+  uint64_t master, exp_avg, exp_avg_sq, grad, param_bf16, step;
+  int64_t numel;
+  int32_t group;
+  uint32_t flags;
+};
+static_assert(sizeof(TensorRow) == 64, "tm_tensor_t is 64 bytes");
+
+// dtype code of a dense contiguous GPU grad (0 bfloat16, 1 float32), 255 for anything else.
+inline uint8_t grad_code(const at::Tensor* t) {
+  if (!t || !t->defined() || t->layout() != at::kStrided || !t->is_cuda() || !t->is_contiguous()) return 255;
+  const auto st = t->scalar_type();
+  return st == at::kBFloat16 ? 0 : (st == at::kFloat ? 1 : 255);
+}
+
+// The tensor table of a grad-only call: (bytes of n tm_tensor_t with grad, numel and flags set,
+// numels, all usable, all on one device).
+py::tuple grad_rows(const py::list& grads) {
+  const Py_ssize_t n = PyList_GET_SIZE(grads.ptr());
+  py::array_t<uint8_t> rows(static_cast<py::ssize_t>(n * sizeof(TensorRow)));
+  py::array_t<int64_t> numels(n);
+  TensorRow* r = reinterpret_cast<TensorRow*>(rows.mutable_data());
+  int64_t* pn = numels.mutable_data();
+  bool fine = true, one = true;
+  c10::Device first(c10::kCPU);
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    const at::Tensor* t = tensor_or_null(list_item(grads, i));
+    const uint8_t code = grad_code(t);
+    r[i] = TensorRow{};
+    pn[i] = 0;
+    if (!t || !t->defined()) {
+      fine = false;
+      continue;
+    }
+    if (i == 0) first = t->device();
+    one = one && t->device() == first;
+    fine = fine && code != 255;
+    if (code == 255) continue;
+    r[i].grad = reinterpret_cast<uint64_t>(t->data_ptr());
+    r[i].numel = pn[i] = t->numel();
+    r[i].flags = code;  // 0 = TM_GRAD_BF16, 1 = TM_GRAD_F32
+  }
+  return py::make_tuple(rows, numels, fine, one);
+}
+
+// The checks of the steady-state step in one walk: every param's working copy and grad source are
+// the plan's, the grads dense and contiguous, the static tensors' pointers and the state dicts
+// unchanged, and the working copies current. Returns (grads, their pointers), or None.
+py::object plan_match(const py::list& all_params, const py::list& all_works, const py::bytes& src,
+                      const py::list& statics, const py::array_t<uint64_t>& static_ptrs, const py::dict& state_map,
+                      const py::list& state_keys, const py::list& state_values, const py::list& states,
+                      const py::list& ms, const py::list& vs, const py::list& ss, const py::list& wparams,
+                      const py::list& wworks) {
+  const Py_ssize_t n = PyList_GET_SIZE(all_params.ptr());
+  const char* want = PyBytes_AS_STRING(src.ptr());
+  if (PyBytes_GET_SIZE(src.ptr()) != n || !attrs_same(all_params, py::reinterpret_borrow<py::str>(working_name()), all_works))
+    return py::none();
+  py::list out;
+  std::vector<uint64_t> at_ptr;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    const at::Tensor* p = tensor_or_null(list_item(all_params, i));
+    const at::Tensor* w = tensor_or_null(list_item(all_works, i));
+    const at::Tensor* g = nullptr;
+    char from = 0;
+    if (p && p->grad().defined()) {
+      g = &p->grad();
+      from = 1;
+    } else if (w && w->grad().defined()) {
+      g = &w->grad();
+      from = 2;
+    }
+    if (from != want[i]) return py::none();
+    if (!g) continue;
+    if (g->layout() != at::kStrided || !g->is_contiguous()) return py::none();
+    at_ptr.push_back(reinterpret_cast<uint64_t>(g->data_ptr()));
+    out.append(py::reinterpret_steal<py::object>(THPVariable_Wrap(*g)));
+  }
+  const Py_ssize_t k = PyList_GET_SIZE(statics.ptr());
+  if (static_ptrs.size() != k) return py::none();
+  const uint64_t* sp = static_ptrs.data();
+  for (Py_ssize_t i = 0; i < k; ++i) {
+    const at::Tensor* t = tensor_or_null(list_item(statics, i));
+    if (((t && t->defined()) ? reinterpret_cast<uint64_t>(t->data_ptr()) : 0u) != sp[i]) return py::none();
+  }
+  if (!items_same(state_map, state_keys, state_values) || !entries_same(states, ms, vs, ss)) return py::none();
+  if (PyList_GET_SIZE(wparams.ptr()) && !stamped(wparams, wworks)) return py::none();
+  py::array_t<uint64_t> ptrs_out(static_cast<py::ssize_t>(at_ptr.size()));
+  std::copy(at_ptr.begin(), at_ptr.end(), ptrs_out.mutable_data());
+  return py::make_tuple(out, ptrs_out);
+}
+
+// The params a clip measured and their grads against the plan's: every grad of the record, taken
+// in the plan's order (perm), is the grad at hand, and none changed in place since.
+// 0: other grads, 1: the same, 2: the same but modified.
+int clip_match(const py::list& rec_grads, const std::vector<int64_t>& perm, const py::list& grads, int64_t total) {
+  const Py_ssize_t n = PyList_GET_SIZE(grads.ptr());
+  if (static_cast<Py_ssize_t>(perm.size()) != n) return 0;
+  int64_t sum = 0;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    if (perm[i] < 0 || perm[i] >= PyList_GET_SIZE(rec_grads.ptr())) return 0;
+    if (list_item(rec_grads, perm[i]) != list_item(grads, i)) return 0;
+    sum += static_cast<int64_t>(tensor_or_null(list_item(grads, i))->_version());
+  }
+  return sum == total ? 1 : 2;
+}
+
+// tm_accum_t (include/torchure_amd.h) as the host writes it.
+struct AccumRow {
+  uint64_t acc, micro;
+  int64_t numel, flags;
+};
+static_assert(sizeof(AccumRow) == 32, "tm_accum_t is 32 bytes");
+
+// One micro-step of accumulation over params: checks every param, its accumulator (p.grad) and
+// its working copy's grad, then, only if all are usable, gives first micro-steps their
+// accumulator (unfilled: the kernel assigns it). Returns (accumulators, those with a micro grad,
+// rows, numels, the working copies' grads, device index), or None when the caller's checks should
+// report why not (or there is nothing to do).
+py::object accumulate_scan(const py::list& params, bool last, int64_t assign_flag) {
+  const Py_ssize_t n = PyList_GET_SIZE(params.ptr());
+  struct Item {
+    const at::Tensor *p, *w;
+  };
+  std::vector<Item> todo;
+  std::vector<py::object> keep;  // the working copies, alive while their pointers are used
+  c10::Device first(c10::kCPU);
+  auto dense = [](const at::Tensor& t) { return t.layout() == at::kStrided && t.is_cuda() && t.is_contiguous(); };
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject* po = list_item(params, i);
+    const at::Tensor* p = tensor_or_null(po);
+    if (!p) return py::none();
+    py::object wo = py::reinterpret_steal<py::object>(attr_or_null(po, working_name()));
+    const at::Tensor* w = wo.ptr() ? tensor_or_null(wo.ptr()) : nullptr;
+    if (w && !w->grad().defined()) w = nullptr;
+    const at::Tensor& g = p->grad();
+    if (!w && (!last || !g.defined())) continue;
+    if (!dense(*p) || (g.defined() ? g : *p).scalar_type() != at::kFloat || (g.defined() && !dense(g))) return py::none();
+    if (w) {
+      const at::Tensor& m = w->grad();
+      if (!dense(m) || m.scalar_type() != at::kBFloat16 || m.numel() != p->numel() || m.device() != p->device())
+        return py::none();
+    }
+    if (todo.empty()) first = p->device();
+    if (p->device() != first) return py::none();
+    todo.push_back({p, w});
+    keep.push_back(wo);
+  }
+  if (todo.empty()) return py::none();
+  const py::ssize_t k = static_cast<py::ssize_t>(todo.size());
+  py::array_t<uint8_t> rows(k * static_cast<py::ssize_t>(sizeof(AccumRow)));
+  py::array_t<int64_t> numels(k);
+  AccumRow* r = reinterpret_cast<AccumRow*>(rows.mutable_data());
+  py::list accs(k), changed, micros;
+  for (py::ssize_t i = 0; i < k; ++i) {
+    const at::Tensor* p = todo[i].p;
+    const at::Tensor* w = todo[i].w;
+    const bool fresh = !p->grad().defined();
+    if (fresh) {
+      at::NoGradGuard no_grad;
+      p->mutable_grad() = at::empty(p->sizes(), p->options().requires_grad(false));
+    }
+    const at::Tensor& g = p->grad();
+    r[i] = AccumRow{reinterpret_cast<uint64_t>(g.data_ptr()), w ? reinterpret_cast<uint64_t>(w->grad().data_ptr()) : 0u,
+                    g.numel(), fresh ? assign_flag : 0};
+    numels.mutable_data()[i] = g.numel();
+    PyObject* acc = THPVariable_Wrap(g);
+    if (w) {
+      changed.append(py::reinterpret_borrow<py::object>(acc));
+      micros.append(py::reinterpret_steal<py::object>(THPVariable_Wrap(w->grad())));
+    }
+    PyList_SET_ITEM(accs.ptr(), i, acc);  // steals the reference
+  }
+  return py::make_tuple(accs, changed, rows, numels, micros, static_cast<int>(first.index()));
+}
+
+// Drops the grad of every param's working copy.
+void clear_work_grads(const py::list& params) {
+  const Py_ssize_t n = PyList_GET_SIZE(params.ptr());
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    py::object wo = py::reinterpret_steal<py::object>(attr_or_null(list_item(params, i), working_name()));
+    if (!wo.ptr()) continue;
+    const at::Tensor* w = tensor_or_null(wo.ptr());
+    if (w && w->grad().defined()) w->mutable_grad().reset();
+  }
+}
+
+// Which tensors, at which versions: matches() tells whether a list holds exactly these tensors,
+// unmodified since. Holds them weakly.
+struct Stamp {
+  std::vector<std::pair<c10::weak_intrusive_ptr<c10::TensorImpl>, int64_t>> seen;
+  explicit Stamp(const py::list& ts) {
+    const Py_ssize_t n = PyList_GET_SIZE(ts.ptr());
+    seen.reserve(static_cast<size_t>(n));
+    for (Py_ssize_t i = 0; i < n; ++i) {
+      const at::Tensor* t = tensor_or_null(list_item(ts, i));
+      if (!t) throw py::value_error("torchure_amd._tm_host.Stamp: expected tensors");
+      seen.emplace_back(t->getIntrusivePtr(), static_cast<int64_t>(t->_version()));
+    }
+  }
+  bool matches(const py::list& ts) const {
+    const Py_ssize_t n = PyList_GET_SIZE(ts.ptr());
+    if (static_cast<size_t>(n) != seen.size()) return false;
+    for (Py_ssize_t i = 0; i < n; ++i) {
+      const at::Tensor* t = tensor_or_null(list_item(ts, i));
+      // a tensor that died and another at its address: the weak reference has expired
+      if (!t || seen[i].first.expired() || seen[i].first._unsafe_get_target() != t->unsafeGetTensorImpl() ||
+          static_cast<int64_t>(t->_version()) != seen[i].second)
+        return false;
+    }
+    return true;
+  }
+};
+
 }  // namespace
+
+void tm_ce_host_bind(py::module_& m);  // tm_ce_host.cpp
 
 PYBIND11_MODULE(_tm_host, m) {
   m.doc() = "torchure_amd host-side list primitives (CPU only)";
+  tm_ce_host_bind(m);
+  m.def("collect", &collect, "(grads, their params, distinct owner marks) of a list of params");
+  m.def("grad_rows", &grad_rows, "tensor table of a grad-only call");
+  m.def("plan_match", &plan_match, "the steady-state step's checks: (grads, pointers) or None");
+  m.def("clip_match", &clip_match, "whether a clip's grads are the step's grads, unmodified");
+  m.def("accumulate_scan", &accumulate_scan, "checks and table of one accumulation micro-step, or None");
+  m.def("clear_work_grads", &clear_work_grads, "drop the grads of the params' working copies");
+  py::class_<Stamp>(m, "Stamp", "tensors and their versions, held weakly")
+      .def(py::init<const py::list&>())
+      .def("matches", &Stamp::matches);
   m.def("grads", &grads, "effective grad per master (p.grad or its working copy's grad)");
   m.def("ptrs", &ptrs, "data_ptr of each tensor (0 for None)");
   m.def("versions", &versions, "autograd version of each tensor (-1 for None)");

@@ -17,8 +17,8 @@ Per chunk of rows:
   grad_W += grad_logits^T @ h       bf16 GEMM: tm_ce_grad_w_ld_bf16, this build's MFMA GEMM, for dim
                                     a multiple of 64 (and rows too where the logits are unpadded;
                                     torch.matmul otherwise), then tm_ce_grad_w_fold into fp32
-The chunk's logits are padded to whole MFMA steps (PaddedLogits): rows a multiple of 64 elements
-apart and their number a multiple of 128, the padding zero once they are gradients. An odd
+The chunk's logits are padded to whole MFMA steps: rows a multiple of 64 elements (padded_vocab)
+apart and their number a multiple of 64 or 128 (padded_rows), the padding zero once they are gradients. An odd
 vocabulary then keeps its rows 16-byte aligned, and any number of tokens is a whole number of
 K slices for grad_W.
 then tm_ce_loss sums the per-row losses in a fixed order (deterministic).
@@ -184,12 +184,12 @@ def _bf16(logits: torch.Tensor, dtype=torch.bfloat16) -> torch.Tensor:
 
 
 def _mean_loss(row_loss, labels, n, ignore_index, lib, stream):
-    """(mean loss as a 0-d tensor, n_valid as a 1-element view) from the per-row losses."""
+    """(mean loss as a 0-d tensor, the loss sum and n_valid as one tensor) from the per-row losses."""
     out2 = torch.empty(2, dtype=torch.float32, device=row_loss.device)
     loss = torch.empty((), dtype=torch.float32, device=row_loss.device)
     _native.check(lib.tm_ce_mean_loss(row_loss.data_ptr(), labels.data_ptr(), n, int(ignore_index),
                                       out2.data_ptr(), loss.data_ptr(), stream), "tm_ce_mean_loss")
-    return loss, out2[1:2]
+    return loss, out2
 
 
 def logits_gemm_fits(h: torch.Tensor, w: torch.Tensor) -> bool:
@@ -221,39 +221,6 @@ def padded_vocab(vocab: int) -> int:
     """Elements from one padded logits row to the next: whole 64-column K slices of the grad_h
     GEMM; every row then starts on a 16-byte boundary (on a cache line), for any vocabulary."""
     return -(-vocab // 64) * 64
-
-
-class PaddedLogits:
-    """A chunk's logits in a buffer padded for the MFMA kernels (``padded_rows`` x
-    ``padded_vocab``), for hidden states and a weight ``logits_gemm_fits`` accepts. ``rows_()``
-    turns them into grad_logits and zeroes the padding; ``view`` is their rows x vocab part.
-    The loss alone (``grad=False``) needs no rows of padding."""
-
-    def __init__(self, h: torch.Tensor, w: torch.Tensor, lib, stream, grad: bool = True):
-        (self.rows, self.dim), self.vocab = h.shape, w.shape[0]
-        self.lib, self.stream, self.h = lib, stream, h
-        self.pad_rows = padded_rows(self.rows) if grad else self.rows
-        self.buf = torch.empty((self.pad_rows, padded_vocab(self.vocab)), dtype=torch.bfloat16, device=h.device)
-        self.ld = self.buf.shape[1]
-        _native.check(lib.tm_ce_logits_ld_bf16(self.buf.data_ptr(), self.ld, h.data_ptr(), w.data_ptr(), self.rows,
-                                               self.vocab, self.dim, stream), "tm_ce_logits_ld_bf16")
-
-    @property
-    def view(self) -> torch.Tensor:
-        return self.buf[: self.rows, : self.vocab]
-
-    def rows_(self, labels: torch.Tensor, ignore_index: int, row_loss: torch.Tensor) -> None:
-        _native.check(self.lib.tm_ce_rows_padded_bf16(self.buf.data_ptr(), self.ld, labels.data_ptr(), self.rows,
-                                                      self.pad_rows, self.vocab, ignore_index, row_loss.data_ptr(),
-                                                      self.stream), "tm_ce_rows_padded_bf16")
-
-    def grad_w(self) -> torch.Tensor:
-        """gw = grad_logits.t() @ h (fused_linear_ce.py:57): bf16 GEMM, bf16 result (V x D)."""
-        out = torch.empty((self.vocab, self.dim), dtype=torch.bfloat16, device=self.buf.device)
-        _native.check(self.lib.tm_ce_grad_w_ld_bf16(out.data_ptr(), self.buf.data_ptr(), self.ld, self.pad_rows,
-                                                    self.h.data_ptr(), self.rows, self.vocab, self.dim, self.stream),
-                      "tm_ce_grad_w_ld_bf16")
-        return out
 
 
 def grad_w_gemm_fits(g: torch.Tensor, h: torch.Tensor) -> bool:
@@ -344,32 +311,30 @@ def _fold(lib, grad_weight, chunks, accumulated, stream) -> None:
 
 class GradHidden:
     """grad_h = grad_logits @ W (fused_linear_ce.py:52, stored at :79) for the chunks of one
-    call: the split-K MFMA GEMM on the chunks it fits, reading W as it is stored, with one fp32
-    partials workspace shared by the chunks (stream-ordered), and torch.matmul (hipBLASLt) on the
-    others. ``w`` is the contiguous bf16 weight (V x D). ``padded``: the chunks' grad_logits are
-    views of PaddedLogits buffers (columns from the vocabulary to the next multiple of 64 zero),
-    and ``grad_h_gemm_fits`` decides; else they are contiguous, and ``splitk_grad_h_fits`` does."""
+    call on unpadded logits: the split-K MFMA GEMM on the chunks ``splitk_grad_h_fits`` accepts,
+    reading W as it is stored, with one fp32 partials workspace shared by the chunks
+    (stream-ordered), and torch.matmul (hipBLASLt) on the others. ``w`` is the contiguous bf16
+    weight (V x D)."""
 
-    def __init__(self, w: torch.Tensor, chunk_rows, lib, stream, padded: bool = False):
+    def __init__(self, w: torch.Tensor, chunk_rows, lib, stream):
         self.w, self.lib, self.stream = w, lib, stream
         self.vocab, self.dim = w.shape
-        self._fits = grad_h_gemm_fits if padded else splitk_grad_h_fits
-        fits = [r for r in set(chunk_rows) if self._fits(r, self.dim, self.vocab)]
+        fits = [r for r in set(chunk_rows) if splitk_grad_h_fits(r, self.dim, self.vocab)]
         self.ws = None
         if fits:
-            nbytes = max(lib.tm_ce_grad_h_ld_workspace_bytes(r, self.vocab, self.dim) for r in fits)
+            nbytes = max(lib.tm_ce_grad_h_workspace_bytes(r, self.vocab, self.dim) for r in fits)
             self.ws = torch.empty(nbytes, dtype=torch.uint8, device=w.device)
 
     def __call__(self, grad_logits: torch.Tensor, out: torch.Tensor) -> None:
         rows = grad_logits.shape[0]
-        if self.ws is None or not self._fits(rows, self.dim, self.vocab):
+        if self.ws is None or not splitk_grad_h_fits(rows, self.dim, self.vocab):
             torch.matmul(grad_logits, self.w, out=out)
             return
-        if not (grad_logits.stride(1) == 1 and out.is_contiguous() and out.dtype == torch.bfloat16):
+        if not (grad_logits.is_contiguous() and out.is_contiguous() and out.dtype == torch.bfloat16):
             raise RuntimeError("fused_linear_cross_entropy: grad_h GEMM operands must be contiguous bf16")
-        _native.check(self.lib.tm_ce_grad_h_ld_bf16(out.data_ptr(), grad_logits.data_ptr(), grad_logits.stride(0),
-                                                    self.w.data_ptr(), rows, self.vocab, self.dim, self.ws.data_ptr(),
-                                                    self.ws.numel(), self.stream), "tm_ce_grad_h_ld_bf16")
+        _native.check(self.lib.tm_ce_grad_h_bf16(out.data_ptr(), grad_logits.data_ptr(), self.w.data_ptr(), rows,
+                                                 self.vocab, self.dim, self.ws.data_ptr(), self.ws.numel(),
+                                                 self.stream), "tm_ce_grad_h_bf16")
 
 
 def _copy_at_hand(weight: torch.Tensor):
@@ -400,25 +365,34 @@ def _castable(t: torch.Tensor) -> bool:
             and not t.is_neg())
 
 
-def _bf16_operands(hidden, weight, mode, lib, stream):
-    """(hidden, weight) in bf16 as the products read them: autocast's casts (RNE) where they are
-    fp32, both in one launch, unless a current working copy of the weight is at hand."""
-    hb, w = hidden, _copy_at_hand(weight)
-    parts = []
-    if mode == "autocast":
-        hb = torch.empty_like(hidden, dtype=torch.bfloat16) if _castable(hidden) else hidden.to(torch.bfloat16)
-        if _castable(hidden):
-            parts.append((hb, hidden))
+def _run_chunks(hidden, weight, labels, ignore_index, chunk, mode, grad, want_h, want_w):
+    """The chunk loop on padded logits (``_tm_host.ce_forward``), for operands that the MFMA
+    kernels take (dim a multiple of 64, bf16 ones 16-byte aligned), or None on others. Returns
+    (loss, (loss sum, n_valid), grad_hidden, grad_weight, grad_W chunks still to be added,
+    accumulated). autocast's casts, or the weight's, are made there in one launch."""
+    (n, d), v = hidden.shape, weight.shape[0]
+    if n == 0 or d == 0 or v == 0 or d % 64:
+        return None
+    h, cast_h = hidden, mode == "autocast"
+    if cast_h and not _castable(h):
+        h, cast_h = h.to(torch.bfloat16), False
+    w, cast_w = _copy_at_hand(weight), False
     if w is None:
-        if _castable(weight):
-            w = torch.empty_like(weight, dtype=torch.bfloat16)
-            parts.append((w, weight))
-        else:
-            w = weight.to(torch.bfloat16).contiguous()
-    if parts:
-        args = [x for dst, src in parts for x in (dst.data_ptr(), src.data_ptr(), src.numel())]
-        _native.check(lib.tm_ce_cast2(*(args + [None, None, 0])[:6], stream), "tm_ce_cast2")
-    return hb, w
+        cast_w = _castable(weight)
+        w = weight if cast_w else weight.to(torch.bfloat16).contiguous()
+    if not (cast_h or h.data_ptr() % 16 == 0) or not (cast_w or w.data_ptr() % 16 == 0):
+        return None
+    chunk = min(chunk, n)
+    last = n - (n - 1) // chunk * chunk
+    return _native.ce_host().ce_forward(
+        h, w, cast_h, cast_w, labels, int(ignore_index), chunk, (padded_rows(chunk), padded_rows(last)),
+        padded_vocab(v), (grad_h_gemm_fits(chunk, d, v), grad_h_gemm_fits(last, d, v)), grad, want_h, want_w,
+        FOLD_CHUNKS, FOLD_BYTES, _native.stream_handle(hidden.device))
+
+
+def _bf16_operands(hidden, weight, mode):
+    """(hidden, weight) in bf16 as the products read them (autocast's casts, RNE)."""
+    return hidden.to(torch.bfloat16) if mode == "autocast" else hidden, _bf16_weight(weight)
 
 
 def _loss_only(hidden, weight, labels, ignore_index, chunk_size):
@@ -427,25 +401,24 @@ def _loss_only(hidden, weight, labels, ignore_index, chunk_size):
     bits, without the two gradient GEMMs or the gradient write. The reference's forward
     computes and drops the gradients in this case (fused_linear_ce.py:63-93)."""
     n, v, chunk, mode = _checked(hidden, weight, labels, chunk_size)
+    if mode != "fp32":
+        done = _run_chunks(hidden, weight, labels, ignore_index, chunk, mode, False, False, False)
+        if done is not None:
+            return done[0]
     lib = _native.lib()
     stream = _native.stream_handle(hidden.device)
     dt = torch.float32 if mode == "fp32" else torch.bfloat16
     if mode == "fp32":
         hb, w = hidden, weight.to(dt).contiguous()
     else:
-        hb, w = _bf16_operands(hidden, weight, mode, lib, stream)
+        hb, w = _bf16_operands(hidden, weight, mode)
     rows_loss = lib.tm_ce_rows_loss_f32 if mode == "fp32" else lib.tm_ce_rows_loss_bf16
     row_loss = torch.empty(n, dtype=torch.float32, device=hidden.device)
     for s in range(0, n, chunk):
         e = min(s + chunk, n)
-        if dt == torch.float32:
-            logits = _bf16(torch.matmul(hb[s:e], w.t()), dt)
-        elif logits_gemm_fits(hb[s:e], w):
-            logits = PaddedLogits(hb[s:e], w, lib, stream, grad=False).buf
-        else:
-            logits = _logits(hb[s:e], w, lib, stream)
-        _native.check(rows_loss(logits.data_ptr(), logits.shape[1], labels[s:e].data_ptr(), e - s, v,
-                                int(ignore_index), row_loss[s:].data_ptr(), stream), "tm_ce_rows_loss")
+        logits = _logits(hb[s:e], w, lib, stream) if dt == torch.bfloat16 else _bf16(torch.matmul(hb[s:e], w.t()), dt)
+        _native.check(rows_loss(logits.data_ptr(), v, labels[s:e].data_ptr(), e - s, v, int(ignore_index),
+                                row_loss[s:].data_ptr(), stream), "tm_ce_rows_loss")
         del logits
     return _mean_loss(row_loss, labels, n, ignore_index, lib, stream)[0]
 
@@ -475,11 +448,46 @@ def _fp32_forward(ctx, hidden, weight, labels, ignore_index, n, v, chunk):
         if want_w:
             grad_weight += torch.matmul(logits.t(), h)
         del logits
-    loss, ctx.n_valid = _mean_loss(row_loss, labels, n, ignore_index, lib, stream)
-    ctx.grad_hidden = grad_hidden
-    ctx.grad_weight = grad_weight
+    loss, out2 = _mean_loss(row_loss, labels, n, ignore_index, lib, stream)
+    ctx.stash = (out2, grad_hidden, grad_weight, [], False)
     ctx.fp32_path = True
     return loss
+
+
+def _chunks_unpadded(hidden, weight, labels, ignore_index, n, v, chunk, mode, want_h, want_w):
+    """The chunk loop for what ``_run_chunks`` does not take (a dim off 64, unaligned or strided
+    operands, no rows): logits rows vocab elements apart, library products where this build's
+    GEMMs do not fit. Returns what ``_run_chunks`` does."""
+    lib = _native.lib()
+    stream = _native.stream_handle(hidden.device)
+    hb, w = _bf16_operands(hidden, weight, mode)  # cast once, not per chunk
+    # bf16 GEMM output either way; for fp32 hidden it is widened and scaled in backward
+    grad_hidden = torch.empty(hidden.shape, dtype=torch.bfloat16, device=hidden.device) if want_h else None
+    # Chunks' bf16 grad_W wait in `pending` and are folded into the fp32 grad_W several at a
+    # time (one pass per fold); the last chunk, and those still pending, wait for backward.
+    grad_weight, pending, accumulated = None, [], False
+    row_loss = torch.empty(n, dtype=torch.float32, device=hidden.device)
+    grad_h_of = GradHidden(w, [min(chunk, n - s) for s in range(0, n, chunk)], lib, stream) if want_h else None
+    for s in range(0, n, chunk):
+        e = min(s + chunk, n)
+        h = hb[s:e]
+        logits = _logits(h, w, lib, stream)  # (C, V) bf16
+        _native.check(lib.tm_ce_rows_bf16(logits.data_ptr(), v, labels[s:e].data_ptr(), e - s, v,
+                                          int(ignore_index), row_loss[s:].data_ptr(), stream),
+                      "tm_ce_rows_bf16")
+        if want_h:
+            grad_h_of(logits, grad_hidden[s:e])
+        if want_w:
+            pending.append(_grad_w(logits, h, lib, stream))  # (V, D) bf16
+            if e < n and (len(pending) == FOLD_CHUNKS or len(pending) * pending[0].numel() * 2 >= FOLD_BYTES):
+                if grad_weight is None:
+                    grad_weight = torch.empty(weight.shape, dtype=torch.float32, device=weight.device)
+                _fold(lib, grad_weight, pending, accumulated, stream)
+                accumulated = True
+                pending = []
+        del logits
+    loss, out2 = _mean_loss(row_loss, labels, n, ignore_index, lib, stream)
+    return loss, out2, grad_hidden, grad_weight, pending, accumulated
 
 
 class _FusedLinearCE(torch.autograd.Function):
@@ -488,108 +496,42 @@ class _FusedLinearCE(torch.autograd.Function):
         n, v, chunk, mode = _checked(hidden, weight, labels, chunk_size)
         if mode == "fp32":
             return _fp32_forward(ctx, hidden, weight, labels, ignore_index, n, v, chunk)
-        fp32 = mode == "autocast"
-        lib = _native.lib()
-        stream = _native.stream_handle(hidden.device)
-        hb, w = _bf16_operands(hidden, weight, mode, lib, stream)  # cast once, not per chunk
-        want_h, want_w = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-        # bf16 GEMM output either way; for fp32 hidden it is widened and scaled in backward
-        grad_hidden = torch.empty(hidden.shape, dtype=torch.bfloat16, device=hidden.device) if want_h else None
-        # Chunks' bf16 grad_W wait in `pending` and are folded into the fp32 grad_W several at a
-        # time (one pass per fold); the last chunk, and those still pending, wait for backward.
-        grad_weight = None
-        pending, last_gw = [], None
-        accumulated = False
-        row_loss = torch.empty(n, dtype=torch.float32, device=hidden.device)
-        padded = n > 0 and logits_gemm_fits(hb, w)  # every chunk then starts on a 16-byte boundary
-        grad_h_of = None
-        if want_h:
-            grad_h_of = GradHidden(w, [min(chunk, n - s) for s in range(0, n, chunk)], lib, stream, padded)
-        for s in range(0, n, chunk):
-            e = min(s + chunk, n)
-            h = hb[s:e]
-            if padded:
-                block = PaddedLogits(h, w, lib, stream)  # (C, V) bf16
-                block.rows_(labels[s:e], int(ignore_index), row_loss[s:])
-                logits = block.view
-            else:
-                logits = _logits(h, w, lib, stream)
-                _native.check(lib.tm_ce_rows_bf16(logits.data_ptr(), v, labels[s:e].data_ptr(), e - s, v,
-                                                  int(ignore_index), row_loss[s:].data_ptr(), stream),
-                              "tm_ce_rows_bf16")
-            if want_h:
-                grad_h_of(logits, grad_hidden[s:e])
-            if want_w:
-                gw = block.grad_w() if padded else _grad_w(logits, h, lib, stream)  # (V, D) bf16
-                if e == n:
-                    last_gw = gw
-                else:
-                    pending.append(gw)
-                    del gw
-                    if len(pending) == FOLD_CHUNKS or len(pending) * pending[0].numel() * 2 >= FOLD_BYTES:
-                        if grad_weight is None:
-                            grad_weight = torch.empty(weight.shape, dtype=torch.float32, device=weight.device)
-                        _fold(lib, grad_weight, pending, accumulated, stream)
-                        accumulated = True
-                        pending = []
-            block = logits = None
-        del grad_h_of
-        loss, ctx.n_valid = _mean_loss(row_loss, labels, n, ignore_index, lib, stream)
-        ctx.grad_hidden = grad_hidden
-        ctx.fp32_hidden = fp32
         ctx.fp32_path = False
-        ctx.want_w = want_w
-        ctx.grad_weight = grad_weight
-        ctx.pending_gw = pending
-        ctx.last_gw = last_gw
-        ctx.accumulated = accumulated
+        ctx.wide = mode == "autocast"  # fp32 hidden states: grad_h is widened in backward
+        ctx.want_w = ctx.needs_input_grad[1]
         ctx.weight_meta = (weight.shape, weight.device)
-        return loss
+        done = _run_chunks(hidden, weight, labels, ignore_index, chunk, mode, True, ctx.needs_input_grad[0],
+                           ctx.needs_input_grad[1])
+        if done is None:
+            done = _chunks_unpadded(hidden, weight, labels, ignore_index, n, v, chunk, mode, *ctx.needs_input_grad[:2])
+        # what backward needs, consumed by it
+        ctx.stash = done[1:]
+        return done[0]
 
     @staticmethod
     def backward(ctx, grad_out):
-        if ctx.n_valid is None:
+        if ctx.stash is None:
             raise RuntimeError(
                 "fused_linear_cross_entropy: backward called twice. the stashed grads are "
                 "consumed in place on the first call, so retain_graph does not work through this op")
-        grad_hidden, grad_weight, n_valid = ctx.grad_hidden, ctx.grad_weight, ctx.n_valid
+        out2, grad_hidden, grad_weight, chunks, accumulated = ctx.stash
+        ctx.stash = None
         if ctx.fp32_path:
-            ctx.grad_hidden = ctx.grad_weight = ctx.n_valid = None
             # fused_linear_ce.py:107-126: scale = grad_out / n_valid, both buffers scaled in place
-            scale = grad_out.detach().to(torch.float32) / n_valid[0]
+            scale = grad_out.detach().to(torch.float32) / out2[1]
             if grad_hidden is not None:
                 grad_hidden.mul_(scale)
             if grad_weight is not None:
                 grad_weight.mul_(scale)
             return grad_hidden, grad_weight, None, None, None
-        last_gw, pending = ctx.last_gw, ctx.pending_gw
-        ctx.grad_hidden = ctx.grad_weight = ctx.n_valid = ctx.last_gw = ctx.pending_gw = None
-        lib = _native.lib()
-        stream = _native.stream_handle(n_valid.device)
-        g = grad_out.detach().to(torch.float32).contiguous()
-        # the chunks still pending, then the last (at most FOLD_CHUNKS), added into grad_W with the
-        # scaling, and grad_h scaled, in one launch
-        chunks, accumulated = [], ctx.accumulated
-        if ctx.want_w:
+        if ctx.want_w and not chunks:  # no rows at all: the reference scales its zero-filled buffer
             shape, device = ctx.weight_meta
-            if last_gw is not None:
-                chunks = pending + [last_gw]
-                if grad_weight is None:
-                    grad_weight = torch.empty(shape, dtype=torch.float32, device=device)
-            else:  # no rows at all: the reference scales its zero-filled buffer
-                grad_weight, accumulated = torch.zeros(shape, dtype=torch.float32, device=device), True
-        short, wide = grad_hidden, ctx.fp32_hidden
-        if wide and grad_hidden is not None:
-            # fp32 hidden: the gradient is fp32 = float(bf16 GEMM result) * scale
-            grad_hidden = torch.empty(short.shape, dtype=torch.float32, device=short.device)
-        rc = lib.tm_ce_finish(
-            grad_weight.data_ptr() if grad_weight is not None else None,
-            (ctypes.c_void_p * len(chunks))(*[c.data_ptr() for c in chunks]), len(chunks),
-            grad_weight.numel() if grad_weight is not None else 0, int(accumulated),
-            short.data_ptr() if short is not None else None,
-            grad_hidden.data_ptr() if grad_hidden is not None else None,
-            short.numel() if short is not None else 0, int(wide), g.data_ptr(), n_valid.data_ptr(), stream)
-        _native.check(rc, "tm_ce_finish")
+            grad_weight, accumulated = torch.zeros(shape, dtype=torch.float32, device=device), True
+        # the chunks still waiting (at most FOLD_CHUNKS) added into grad_W with the scaling, and
+        # grad_h scaled (fp32 hidden: float(bf16 GEMM result) * scale), in one launch
+        grad_hidden, grad_weight = _native.ce_host().ce_backward(
+            grad_out, out2, grad_hidden, ctx.wide, grad_weight, chunks, accumulated,
+            _native.stream_handle(out2.device))
         return grad_hidden, grad_weight, None, None, None
 
 

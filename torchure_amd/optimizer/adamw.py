@@ -198,8 +198,7 @@ class AdamW(torch.optim.Optimizer):
         autograd version: the reference scales at clip time, so a grad modified in
         place before the step cannot be reproduced by scaling later (the step raises),
         while a grad replaced by a new tensor simply steps unscaled, as it would there."""
-        grads = list(grads)
-        self._pending = (coef, _ClipRecord(list(params), grads, _native.host().versions(grads)))
+        self._pending = (coef, _ClipRecord(params, grads, _native.host().versions(grads)))
 
     @staticmethod
     def _modified_error() -> RuntimeError:
@@ -368,19 +367,13 @@ class AdamW(torch.optim.Optimizer):
                 return None
             b1, b2 = group["betas"]
             hyper.append((float(lr), float(b1), float(b2), float(group["weight_decay"]), float(group["eps"])))
-        if not host.attrs_same(plan.all_params, "_tm_working", plan.all_works):
+        found = host.plan_match(plan.all_params, plan.all_works, plan.src, plan.statics, plan.static_ptrs, self.state,
+                                plan.state_keys, plan.state_values, plan.states, plan.ms, plan.vs, plan.ss,
+                                plan.wparams, plan.wworks)
+        if found is None:
             return None
-        gs, src = host.grads(plan.all_params, plan.all_works)
-        if src != plan.src:
-            return None
-        gl = [g for g in gs if g is not None]
-        if not host.dense_contiguous(gl) or not np.array_equal(host.ptrs(plan.statics), plan.static_ptrs):
-            return None
-        if not host.states_same(self.state, plan.params, plan.states, plan.ms, plan.vs, plan.ss):
-            return None
-        if plan.wparams and not host.stamped(plan.wparams, plan.wworks):
-            return None
-        flags = plan.flags
+        gl, grad_ptrs = found
+        rows = plan.rows
         if coef is not None and clip_ids:
             if not isinstance(clip_ids, _ClipRecord) or len(clip_ids.grads) != len(gl):
                 return None
@@ -390,18 +383,16 @@ class AdamW(torch.optim.Optimizer):
                 if None in perm:
                     return None
                 plan.clip_holders, plan.clip_perm = rec.holders, perm
-            rg = rec.grads
-            if not host.same([rg[k] for k in plan.clip_perm], gl):
+            match = host.clip_match(rec.grads, plan.clip_perm, gl, rec.total)
+            if match == 0:
                 return None
-            if host.version_sum(gl) != rec.total:
+            if match == 2:  # versions only grow: an in-place change since the clip shows here
                 raise self._modified_error()
-            flags = flags | _native.TM_FLAG_CLIP
+            rows = plan.clip_rows
         device = plan.device
         if coef is not None and coef.device != device:
             return None
-        rows = plan.rows.copy()
-        rows["grad"] = host.ptrs(gl)
-        rows["flags"] = flags
+        rows["grad"] = grad_ptrs  # the plan's own table: uploaded from a copy of its bytes
         tables.make_ready(plan.chunks, device)
         return [StepLaunch(device, self._uploader(rows, device), plan.n, plan.chunks, plan.n_chunks,
                            self.chunk_elems, _native.hyper_array(hyper), len(hyper), coef,
@@ -540,13 +531,13 @@ class AdamW(torch.optim.Optimizer):
         self._pending = None
         super().zero_grad(set_to_none=set_to_none)
         for group in self.param_groups:
+            if set_to_none:
+                _native.host().clear_work_grads(list(group["params"]))
+                continue
             for p in group["params"]:
                 w = getattr(p, "_tm_working", None)
                 if w is not None and w.grad is not None:
-                    if set_to_none:
-                        w.grad = None
-                    else:
-                        w.grad.zero_()
+                    w.grad.zero_()
 
 
 class _ParamEntry:
@@ -578,7 +569,7 @@ class _ClipRecord:
 
     def __init__(self, holders: list, grads: list, versions):
         self.holders, self.grads, self.versions = holders, grads, versions
-        self.total = int(np.asarray(versions, dtype=np.int64).sum())
+        self.total = int(versions.sum())
         self._index = None
 
     @property
@@ -595,7 +586,7 @@ class _Plan:
     """The table of the last full step and what it was built from, for the fast path."""
 
     __slots__ = ("groups", "all_params", "all_works", "src", "params", "statics", "static_ptrs",
-                 "states", "ms", "vs", "ss", "wparams", "wworks", "rows", "flags", "n", "device",
+                 "states", "state_keys", "state_values", "ms", "vs", "ss", "wparams", "wworks", "rows", "clip_rows", "n", "device",
                  "chunks", "n_chunks", "chunk_elems", "written", "clip_holders", "clip_perm")
 
     def __init__(self, opt: "AdamW", order: list, launch: "StepLaunch"):
@@ -610,6 +601,7 @@ class _Plan:
         self.statics = [t for e in ents for t in (e.param, e.m, e.v, e.step, e.work)]
         self.static_ptrs = host.ptrs(self.statics)
         self.states = [opt.state[p] for p in self.params]
+        self.state_keys, self.state_values = list(opt.state.keys()), list(opt.state.values())
         self.ms = [e.m for e in ents]
         self.vs = [e.v for e in ents]
         self.ss = [e.step for e in ents]
@@ -619,7 +611,9 @@ class _Plan:
         self.chunks, self.n_chunks, self.chunk_elems = launch.chunks, launch.n_chunks, launch.chunk_elems
         self.written = launch.written
         self.rows = np.frombuffer(launch.host_rows, dtype=_native.TENSOR_DTYPE).copy()
-        self.flags = self.rows["flags"] & ~np.uint32(_native.TM_FLAG_CLIP)
+        self.rows["flags"] &= ~np.uint32(_native.TM_FLAG_CLIP)
+        self.clip_rows = self.rows.copy()  # the same table with every grad clipped
+        self.clip_rows["flags"] |= np.uint32(_native.TM_FLAG_CLIP)
         self.clip_holders = None
         self.clip_perm = None
 
@@ -650,7 +644,7 @@ class StepLaunch:
         self.n_groups = n_groups
         self.coef = coef
         self.ws = torch.empty(_native.workspace_bytes(n), dtype=torch.uint8, device=device)
-        self.home = torch.cuda.current_stream(device)  # where the table was uploaded
+        self.home = _native.stream_handle(device)  # where the table was uploaded
 
     def __call__(self) -> None:
         tables.follow_home_stream(self.home, self.device, (self.d_rows, self.chunks, self.ws))

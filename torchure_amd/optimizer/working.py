@@ -13,8 +13,6 @@ copy is a separate autograd leaf aliasing its slice.
 
 from __future__ import annotations
 
-import weakref
-
 import numpy as np
 import torch
 
@@ -131,16 +129,12 @@ def accumulate_grad_(acc: torch.Tensor, micro: torch.Tensor) -> None:
     torch.autograd.graph.increment_version(acc)
 
 
-# device -> (norm tensor, [(weakref(grad), grad._version), ...]) of the last fused
+# device -> (norm tensor, stamp of the grads and their versions) of the last fused
 # accumulate+norm call; clip_grad_norm reuses it when it sees exactly those grads,
 # unmodified (torch bumps _version on every in-place op; this package's own kernels
 # that write grads call increment_version or drop the entry).
 _NORM_CACHE: dict = {}
 _ACC_UPLOAD = tables.TableUploader()
-
-
-def _stamp(grads):
-    return [(weakref.ref(g), g._version) for g in grads]
 
 
 def cached_norm(grads: list[torch.Tensor]):
@@ -151,12 +145,7 @@ def cached_norm(grads: list[torch.Tensor]):
     if hit is None:
         return None
     norm, stamp = hit
-    if len(stamp) != len(grads):
-        return None
-    for (ref, ver), g in zip(stamp, grads):
-        if ref() is not g or g._version != ver:
-            return None
-    return norm
+    return norm if stamp.matches(grads) else None
 
 
 def drop_cached_norm(device=None) -> None:
@@ -182,8 +171,39 @@ def accumulate_grads_(params, *, last: bool = False,
     A following ``clip_grad_norm`` over the same params reuses it instead of reading
     every grad again; the value is bit-identical to what it would compute.
     """
-    who = "accumulate_grads_"
     params = list(params)
+    scan = _native.host().accumulate_scan(params, last, _native.TM_ACCUM_ASSIGN)
+    if scan is None:
+        scan = _accumulate_checked(params, last)
+        if scan is None:
+            return None
+    accs, changed, rows, numels, micros, index = scan
+    device = torch.device("cuda", index)
+    drop_cached_norm(device)
+    chunk_elems = tables.check_chunk_elems(chunk_elems)
+    chunks, n_chunks = tables.CHUNKS.get(numels, chunk_elems, device)
+    d_rows = _ACC_UPLOAD(rows, device)
+    norm = torch.empty((), dtype=torch.float32, device=device) if last else None
+    ws, ws_bytes = None, 0
+    if last:  # one fp64 partial per 256-element slice, reduced in a fixed order
+        ws_bytes = int(_native.lib().tm_accum_norm_workspace_bytes(n_chunks, chunk_elems))
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
+    rc = _native.lib().tm_grad_accumulate_list(
+        d_rows.data_ptr(), len(accs), chunks.data_ptr(), n_chunks, chunk_elems, int(last),
+        ws.data_ptr() if last else None, ws_bytes, norm.data_ptr() if last else None,
+        _native.stream_handle(device))
+    _native.check(rc, "tm_grad_accumulate_list")
+    _native.host().bump(changed)
+    _native.host().clear_work_grads(params)
+    if last:
+        _NORM_CACHE[device] = (norm, _native.host().Stamp(accs))
+    return norm
+
+
+def _accumulate_checked(params, last):
+    """The checks of one accumulation micro-step, one by one, with the reason for a refusal; returns
+    what ``_tm_host.accumulate_scan`` does, or None when there is nothing to accumulate."""
+    who = "accumulate_grads_"
     todo = []  # (param, its fp32 accumulator or None on a first micro-step, bf16 micro grad or None)
     for p in params:
         w = getattr(p, "_tm_working", None)
@@ -219,32 +239,10 @@ def accumulate_grads_(params, *, last: bool = False,
         accs.append(g)
         micros.append(mg)
         assign.append(fresh)
-    drop_cached_norm(device)
     rows = np.zeros(len(accs), dtype=_native.ACCUM_DTYPE)
     rows["acc"] = np.asarray([a.data_ptr() for a in accs], dtype=np.uint64)
     rows["micro"] = np.asarray([m.data_ptr() if m is not None else 0 for m in micros], dtype=np.uint64)
     rows["numel"] = np.asarray([a.numel() for a in accs], dtype=np.int64)
     rows["flags"] = np.asarray(assign, dtype=np.int64) * _native.TM_ACCUM_ASSIGN
-    chunk_elems = tables.check_chunk_elems(chunk_elems)
-    chunks, n_chunks = tables.CHUNKS.get(rows["numel"], chunk_elems, device)
-    d_rows = _ACC_UPLOAD(rows, device)
-    norm = torch.empty((), dtype=torch.float32, device=device) if last else None
-    ws = None
-    if last:  # one fp64 partial per 256-element slice, reduced in a fixed order
-        ws = torch.empty(int(_native.lib().tm_accum_norm_workspace_bytes(n_chunks, chunk_elems)),
-                         dtype=torch.uint8, device=device)
-    rc = _native.lib().tm_grad_accumulate_list(
-        d_rows.data_ptr(), len(accs), chunks.data_ptr(), n_chunks, chunk_elems, int(last),
-        ws.data_ptr() if last else None, ws.numel() if last else 0, norm.data_ptr() if last else None,
-        _native.stream_handle(device))
-    _native.check(rc, "tm_grad_accumulate_list")
-    for a, m in zip(accs, micros):
-        if m is not None:
-            torch.autograd.graph.increment_version(a)
-    for p in params:
-        w = getattr(p, "_tm_working", None)
-        if w is not None and w.grad is not None:
-            w.grad = None
-    if last:
-        _NORM_CACHE[device] = (norm, _stamp(accs))
-    return norm
+    changed = [a for a, m in zip(accs, micros) if m is not None]
+    return accs, changed, rows, rows["numel"], [m for m in micros if m is not None], device.index
