@@ -425,7 +425,10 @@ int tm_ce_finish(float* d_grad_w, const uint16_t* const* h_chunks, int n_chunks,
  *                            tm_ce_grad_h_ld_workspace_bytes(rows, vocab, dim) bytes.
  *   tm_ce_grad_w_ld_bf16     tm_ce_grad_w_bf16 for any rows and vocab: rows rows .. pad_rows - 1
  *                            of d_grad_logits must be 0 (pad_rows a multiple of 64, less than 512
- *                            past rows); d_hidden has `rows` rows.
+ *                            past rows); d_hidden has `rows` rows. Outputs of few tiles are split
+ *                            over the rows when d_ws is given (not NULL), with
+ *                            tm_ce_grad_w_ld_workspace_bytes(pad_rows, vocab, dim) bytes: fp32
+ *                            partial sums added in split order, then rounded once.
  * A padding zero times any finite value adds nothing; where the last weight or hidden row holds
  * an infinity or a NaN, its own products already make the same outputs NaN.
  */
@@ -436,8 +439,10 @@ int tm_ce_rows_padded_bf16(uint16_t* d_logits, int64_t ld, const int64_t* d_labe
 size_t tm_ce_grad_h_ld_workspace_bytes(int64_t rows, int64_t vocab, int64_t dim);
 int tm_ce_grad_h_ld_bf16(uint16_t* d_grad_h, const uint16_t* d_grad_logits, int64_t ld, const uint16_t* d_w,
                          int64_t rows, int64_t vocab, int64_t dim, void* d_ws, size_t ws_bytes, void* stream);
+size_t tm_ce_grad_w_ld_workspace_bytes(int64_t pad_rows, int64_t vocab, int64_t dim);
 int tm_ce_grad_w_ld_bf16(uint16_t* d_grad_w, const uint16_t* d_grad_logits, int64_t ld, int64_t pad_rows,
-                         const uint16_t* d_hidden, int64_t rows, int64_t vocab, int64_t dim, void* stream);
+                         const uint16_t* d_hidden, int64_t rows, int64_t vocab, int64_t dim, void* d_ws,
+                         size_t ws_bytes, void* stream);
 
 #ifdef __cplusplus
 }

@@ -460,6 +460,12 @@ def test_grad_w_ring_kernel_equals_one_tile_kernel(rows, vocab, dim):
     (1000, 32001, 768),
     (513, 640, 1216),      # 19 K slices
     (384, 4160, 192),      # aligned rows and vocabulary, odd slices
+    (520, 66001, 320),     # enough 256 x 256 tiles for the persistent kernels: 5 K slices, ragged rows
+    (390, 40003, 1216),    # the same with 19 slices, 4 row slices of padding, a width off both tiles
+    (7000, 1003, 264),     # grad_W of few tiles over 110 slices: split sums; dim off 64 in no tile
+    (4099, 300, 1032),     # grad_h on unsplit 128-wide tiles
+    (2048, 1003, 2056),    # and on unsplit 256-wide ones
+    (8192, 20001, 200),    # grad_W in splits of 256-wide tiles
 ])
 def test_padded_chunk_kernels_on_ragged_shapes(rows, vocab, dim):
     """The chunk's kernels on padded logits: the logits equal to tm_ce_logits_bf16 bit for bit, the
@@ -486,13 +492,19 @@ def test_padded_chunk_kernels_on_ragged_shapes(rows, vocab, dim):
         return bool((buf[:64] == -12345).all()) and bool((buf[-64:] == -12345).all())
 
     h, w = fenced(rows, dim, 1.0), fenced(vocab, dim, 0.05)
+    if dim % 64:  # the logits take whole slices of 64: the rest of the width is zeros there
+        whole = -(-dim // 64) * 64
+        hl, wl = (torch.zeros(t.shape[0], whole, dtype=t.dtype, device=DEV) for t in (h, w))
+        hl[:, :dim], wl[:, :dim] = h, w
+    else:
+        hl, wl = h, w
     pad, ld = padded_rows(rows), padded_vocab(vocab)
     assert pad % 64 == 0 and ld % 64 == 0 and rows <= pad < rows + 256 and vocab <= ld < vocab + 64
     buf, logits = guarded(pad, ld)
     logits.fill_(float("nan"))
-    native.check(lib.tm_ce_logits_ld_bf16(logits.data_ptr(), ld, h.data_ptr(), w.data_ptr(), rows, vocab, dim, stream),
-                 "logits")
-    plain, _ = _logits(h, w)
+    native.check(lib.tm_ce_logits_ld_bf16(logits.data_ptr(), ld, hl.data_ptr(), wl.data_ptr(), rows, vocab, hl.shape[1],
+                                          stream), "logits")
+    plain, _ = _logits(hl, wl)
     assert torch.equal(logits[:rows, :vocab].view(torch.int16), plain.view(torch.int16))
     assert bool(logits[rows:].isnan().all())
     labels = torch.randint(0, vocab, (rows,), device=DEV, generator=g)
@@ -521,17 +533,25 @@ def test_padded_chunk_kernels_on_ragged_shapes(rows, vocab, dim):
                                           ws.data_ptr(), nbytes, stream), "grad_h")
     check(gh, a @ wd, a.abs() @ wd.abs())
     assert intact(buf)
-    buf, gw = guarded(vocab, dim)
-    native.check(lib.tm_ce_grad_w_ld_bf16(gw.data_ptr(), logits.data_ptr(), ld, pad, h.data_ptr(), rows, vocab, dim,
-                                          stream), "grad_w")
-    check(gw, a.t().contiguous() @ hd, a.abs().t().contiguous() @ hd.abs())
-    assert intact(buf)
+    want, absum = a.t().contiguous() @ hd, a.abs().t().contiguous() @ hd.abs()
+    nbytes = lib.tm_ce_grad_w_ld_workspace_bytes(pad, vocab, dim)
+    for nb in {nbytes, 0}:  # with its workspace (splits, if it wants any) and without one
+        ws = torch.full((max(nb, 16),), 0x7F, dtype=torch.uint8, device=DEV)
+        buf, gw = guarded(vocab, dim)
+        native.check(lib.tm_ce_grad_w_ld_bf16(gw.data_ptr(), logits.data_ptr(), ld, pad, h.data_ptr(), rows, vocab, dim,
+                                              ws.data_ptr() if nb else None, nb, stream), "grad_w")
+        check(gw, want, absum)
+        assert intact(buf)
+        again = torch.empty_like(gw)
+        native.check(lib.tm_ce_grad_w_ld_bf16(again.data_ptr(), logits.data_ptr(), ld, pad, h.data_ptr(), rows, vocab,
+                                              dim, ws.data_ptr() if nb else None, nb, stream), "grad_w")
+        assert torch.equal(gw.view(torch.int16), again.view(torch.int16))
 
 
 def test_padded_chunk_kernels_argument_checks():
     """Strides, paddings and sizes that the padded kernels do not take are refused before a launch."""
     native, lib, stream = _lib()
-    t = torch.empty(1 << 16, dtype=torch.bfloat16, device=DEV)
+    t = torch.empty(1 << 24, dtype=torch.bfloat16, device=DEV)
     p = t.data_ptr()
     assert lib.tm_ce_logits_ld_bf16(p, 63, p, p, 8, 64, 64, stream) < 0       # rows shorter than vocab
     for ld, rows, pad in ((100, 8, 8), (64, 8, 7), (64, 0, 8)):
@@ -539,10 +559,13 @@ def test_padded_chunk_kernels_argument_checks():
     assert lib.tm_ce_rows_padded_bf16(p + 2, 64, p, 8, 8, 60, -100, p, stream) < 0
     for ld, rows, vocab, dim in ((64, 8, 65, 64), (100, 8, 100, 64), (64, 8, 64, 60), (64, 0, 64, 64)):
         assert lib.tm_ce_grad_h_ld_bf16(p, p, ld, p, rows, vocab, dim, p, 1 << 30, stream) < 0
-    assert lib.tm_ce_grad_h_ld_bf16(p, p, 64, p, 8, 64, 64, p, 16, stream) < 0  # workspace too small
+    assert lib.tm_ce_grad_h_ld_workspace_bytes(8, 8192, 64) > 16  # split sums: the workspace is checked
+    assert lib.tm_ce_grad_h_ld_bf16(p, p, 8192, p, 8, 8192, 64, p, 16, stream) < 0
     for ld, pad, rows, vocab, dim in ((64, 100, 100, 64, 64), (64, 64, 65, 64, 64), (64, 1024, 64, 64, 64),
                                       (60, 64, 64, 60, 64), (64, 64, 64, 65, 64), (64, 64, 64, 64, 60)):
-        assert lib.tm_ce_grad_w_ld_bf16(p, p, ld, pad, p, rows, vocab, dim, stream) < 0
+        assert lib.tm_ce_grad_w_ld_bf16(p, p, ld, pad, p, rows, vocab, dim, None, 0, stream) < 0
+    assert lib.tm_ce_grad_w_ld_workspace_bytes(8192, 2048, 256) > 16  # split sums: the workspace is checked
+    assert lib.tm_ce_grad_w_ld_bf16(p, p, 2048, 8192, p, 8192, 2048, 256, p, 16, stream) < 0
 
 
 def test_grad_w_gemm_argument_checks():

@@ -117,7 +117,8 @@ _SIGNATURES = {
     "tm_ce_rows_padded_bf16": (ctypes.c_int, [_vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _vp]),
     "tm_ce_grad_h_ld_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i64]),
     "tm_ce_grad_h_ld_bf16": (ctypes.c_int, [_vp, _vp, _i64, _vp, _i64, _i64, _i64, _vp, ctypes.c_size_t, _vp]),
-    "tm_ce_grad_w_ld_bf16": (ctypes.c_int, [_vp, _vp, _i64, _i64, _vp, _i64, _i64, _i64, _vp]),
+    "tm_ce_grad_w_ld_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i64]),
+    "tm_ce_grad_w_ld_bf16": (ctypes.c_int, [_vp, _vp, _i64, _i64, _vp, _i64, _i64, _i64, _vp, ctypes.c_size_t, _vp]),
 }
 
 EXPORTED = tuple(_SIGNATURES)

@@ -5,7 +5,7 @@
 //                        otherwise
 //   grad_h_gemm_kernel   grad_h = grad_logits W (rows x D, K = V), split over K, reading W as it
 //                        is stored (V x D), with
-//   grad_h_reduce_kernel summing the fp32 partials of each element over the splits in a fixed
+//   splits_reduce_kernel summing the fp32 partials of each element over the splits in a fixed
 //                        order (split 0 first) and rounding once to bf16 (RNE), so the result
 //                        does not depend on scheduling
 //   grad_w_ring_kernel   grad_W = grad_logits^T h (V x D, K = rows), persistent, for rows a
@@ -66,18 +66,26 @@ __device__ __forceinline__ uint32_t rne_bf16(float f) {
   return (f != f) ? 0x7FC0u : r;
 }
 
-// out[i] = bf16(((P[0][i] + P[1][i]) + P[2][i]) + ...), four elements per thread.
-__global__ __launch_bounds__(256) void grad_h_reduce_kernel(const float* __restrict__ partials,
+// out[i] = bf16(((P[0][i] + P[1][i]) + P[2][i]) + ...), four elements per thread, eight splits'
+// loads in flight (one at a time, a small output's 32 splits took 11 us of latency).
+__global__ __launch_bounds__(256) void splits_reduce_kernel(const float* __restrict__ partials,
                                                             uint16_t* __restrict__ out, int64_t n, int splits) {
   const int64_t e = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
   if (e >= n) return;
   f32x4 sum = *(const f32x4*)(partials + e);
-  for (int s = 1; s < splits; ++s) {
-    const f32x4 p = *(const f32x4*)(partials + static_cast<int64_t>(s) * n + e);
-    sum.x = sum.x + p.x;
-    sum.y = sum.y + p.y;
-    sum.z = sum.z + p.z;
-    sum.w = sum.w + p.w;
+  for (int s0 = 1; s0 < splits; s0 += 8) {
+    f32x4 p[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (s0 + u < splits) p[u] = *(const f32x4*)(partials + static_cast<int64_t>(s0 + u) * n + e);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (s0 + u >= splits) break;
+      sum.x = sum.x + p[u].x;
+      sum.y = sum.y + p[u].y;
+      sum.z = sum.z + p[u].z;
+      sum.w = sum.w + p[u].w;
+    }
   }
   u32x2 o;
   o.x = rne_bf16(sum.x) | (rne_bf16(sum.y) << 16);
@@ -569,7 +577,7 @@ bool logits_ring_fits(int64_t rows, int64_t vocab, int64_t dim, int64_t ld) {
 // W (V x dim), K = V. K is long and the output small (16 tiles for a 1024-row chunk at dim
 // 1024), so workgroup (split, tile) computes one 256 x 256 tile over one range of K slices and
 // writes its fp32 partial tile (straight from the accumulators, 16 bytes a lane: 4 consecutive
-// columns of one row; a split with no K slices writes zeros); grad_h_reduce_kernel adds the
+// columns of one row; a split with no K slices writes zeros); splits_reduce_kernel adds the
 // partials. Pair p = split x tiles + tile; workgroup w runs on XCD w % 8, which takes pairs
 // [x p8, (x+1) p8): the workgroups of an XCD share a split's K range of both operands in its L2.
 // A stage holds G's 256 rows x 64 K as 128-byte rows (the logits GEMM's layout and fragment
@@ -1177,6 +1185,237 @@ bool grad_w_ring_fits(int64_t k, int64_t ld, int64_t dim) {
          k * dim * 2 < (int64_t(1) << 32) && 32 * dim * 2 < (int64_t(1) << 32);
 }
 
+// ------------------------------------------------------- the three products on smaller tiles
+//
+// One kernel for shapes whose 256 x 256 tiles leave CUs idle (fewer tiles than CUs, a nearly empty
+// last round, a hidden size that wastes half a tile): C (M x N) = A B over K slices of 64, tiles
+// of 64 kMB x 128 kNB, 8 wave64 of (32 kMB) x (32 kNB), wave (wm, wn) = (w / 4, w % 4), with the
+// loads, LDS layouts, fragments and schedule of the 256 x 256 kernels:
+//   kAK: A is M x K (lda apart), else K x M; kBK: B is N x K, else K x N, of which only kb rows
+//   exist (a later row loads the last one against zeros of A).
+// Workgroup (split, tile) covers K slices [split * per, ..): with kPartial it writes its fp32 tile
+// to `out` + split * M * N for splits_reduce_kernel, else (one split) bf16, 16 bytes a lane after
+// v_permlane32_swap joins the two halves of a row's 8 columns.
+template <int kMB, int kNB, bool kAK, bool kBK, bool kPartial>
+__global__ __launch_bounds__(512) void gemm_tile_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
+                                                        void* __restrict__ out, int M, int N, int64_t lda, int64_t ldb,
+                                                        int64_t ldc, int slices, int kb, int tiles_m, int tiles_n,
+                                                        int gm, int gn, int per) {
+  constexpr int kTM = 64 * kMB, kTN = 128 * kNB, kLoads = (kTM + kTN) / 64, kInA = kTM / 8;
+  constexpr int kStage = (kTM + kTN) * 128;
+  constexpr int kRdA = kAK ? kMB : 2 * kMB, kRdB = kBK ? kNB : 2 * kNB, kRd = kRdA + kRdB, kMf = kMB * kNB;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  const int T = tiles_m * tiles_n, pairs = T * ((slices + per - 1) / per);
+  const int p8 = (pairs + 7) / 8;
+  const int p = (blockIdx.x % 8) * p8 + blockIdx.x / 8;
+  if (p >= pairs || static_cast<int>(blockIdx.x / 8) >= p8) return;
+  const int split = p / T;
+  int tm, tn;
+  lg_tile_of(p - split * T, tiles_m, tiles_n, gm, gn, tm, tn);
+  const int m0 = tm * kTM, n0 = tn * kTN;
+  const int it0 = split * per, n_it = min(per, slices - it0);
+  const int64_t k0 = static_cast<int64_t>(it0) * kSliceK;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+
+  // Load q = kLoads wave + j: 1 KB of A's stage (q < kInA), then of B's. K-contiguous: 8 rows of
+  // 128 bytes, chunk c of row r at slot c ^ ((r >> 1) & 7). K-major: whole rows of the tile's
+  // columns, chunk c of row k at slot c ^ (4 (k & 3)).
+  const uint16_t* src[kLoads];
+#pragma unroll
+  for (int j = 0; j < kLoads; ++j) {
+    const int q = wave * kLoads + j;
+    if (q < kInA) {
+      if constexpr (kAK) {
+        const int r = q * 8 + lane / 8;
+        src[j] = A + static_cast<int64_t>(min(m0 + r, M - 1)) * lda + k0 + ((lane % 8) ^ ((r >> 1) & 7)) * 8;
+      } else {
+        constexpr int kCpr = kTM / 8;
+        const int kr = q * (64 / kCpr) + lane / kCpr;
+        const int c = (lane % kCpr) ^ (4 * (kr & 3));
+        src[j] = A + (k0 + kr) * lda + min(static_cast<int64_t>(m0 + 8 * c), lda - 8);
+      }
+    } else {
+      const int qb = q - kInA;
+      if constexpr (kBK) {
+        const int r = qb * 8 + lane / 8;
+        src[j] = B + static_cast<int64_t>(min(n0 + r, N - 1)) * ldb + k0 + ((lane % 8) ^ ((r >> 1) & 7)) * 8;
+      } else {
+        constexpr int kCpr = kTN / 8;
+        const int kr = qb * (64 / kCpr) + lane / kCpr;
+        const int c = (lane % kCpr) ^ (4 * (kr & 3));
+        src[j] = B + (k0 + kr) * ldb + min(static_cast<int64_t>(n0 + 8 * c), ldb - 8);
+      }
+    }
+  }
+  const int64_t step_a = kAK ? kSliceK : kSliceK * lda, step_b = kBK ? kSliceK : kSliceK * ldb;
+  auto load = [&](int it, int stage, int j) {
+    const int q = wave * kLoads + j;
+    const uint16_t* from = src[j] + it * (q < kInA ? step_a : step_b);
+    if (!kBK && q >= kInA && k0 + static_cast<int64_t>(it + 1) * kSliceK > kb) {
+      constexpr int kCpr = kTN / 8;
+      const int64_t past = k0 + static_cast<int64_t>(it) * kSliceK + (q - kInA) * (64 / kCpr) + lane / kCpr - (kb - 1);
+      if (past > 0) from -= past * ldb;
+    }
+    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)from,
+                                     (void __attribute__((address_space(3)))*)(smem + stage * kStage + q * 1024), 16, 0, 0);
+  };
+  // Fragment addresses: K-contiguous, row lane % 32 of a block, chunk 2 kk + lane / 32; K-major,
+  // two transposing half-fragment reads (rows +0 and +4), as grad_w_gemm_kernel.
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem));
+  const int tx = (lane >> 5) ^ ((lane >> 1) & 7);
+  uint32_t vk[4];
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) vk[kk] = lds0 + (lane & 31) * 128 + (((2 * kk) ^ tx) * 16);
+  const int s16 = lane & 15, s4 = s16 >> 2;
+  const int lcf = ((lane >> 4) & 1) * 2 + ((s16 & 3) >> 1);
+  uint32_t ba[kMB], bb[kNB];
+#pragma unroll
+  for (int i = 0; i < kMB; ++i)
+    ba[i] = lds0 + (8 * (lane >> 5) + s4) * (kTM * 2) + (s16 & 1) * 8 + (4 * ((wm * kMB + i) ^ s4) + lcf) * 16;
+#pragma unroll
+  for (int i = 0; i < kNB; ++i)
+    bb[i] = lds0 + kInA * 1024 + (8 * (lane >> 5) + s4) * (kTN * 2) + (s16 & 1) * 8 +
+            (4 * ((wn * kNB + i) ^ s4) + lcf) * 16;
+  const uint32_t offA = wm * kMB * 32 * 128, offB = kInA * 1024 + wn * kNB * 32 * 128;
+
+#define TM_RD(dst, base, imm) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(base), "i"(imm))
+#define TM_TR(dst, base, imm) asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(dst) : "v"(base), "i"(imm))
+  bf16x8 a8[2][kAK ? kMB : 1], b8[2][kBK ? kNB : 1];
+  bf16x4 a4[2][kAK ? 1 : 2 * kMB], b4[2][kBK ? 1 : 2 * kNB];
+  // read g of a step (g < kRdA: A's) into set z
+  auto rd = [&](int z, uint32_t so, int kk, int g) {
+    if (g < kRdA) {
+      if constexpr (kAK) TM_RD(a8[z][g], vk[kk] + so + offA, g * 32 * 128);
+      else TM_TR(a4[z][g], ba[g >> 1] + so, kk * 16 * kTM * 2 + (g & 1) * 4 * kTM * 2);
+    } else {
+      const int h = g - kRdA;
+      if constexpr (kBK) TM_RD(b8[z][h], vk[kk] + so + offB, h * 32 * 128);
+      else TM_TR(b4[z][h], bb[h >> 1] + so, kk * 16 * kTN * 2 + (h & 1) * 4 * kTN * 2);
+    }
+  };
+  // waits for set z's reads; naming every fragment keeps the MFMAs that use them behind the wait
+  auto wait = [&](int z) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int g = 0; g < kRdA; ++g) {
+      if constexpr (kAK) asm volatile("" : "+v"(a8[z][g]));
+      else asm volatile("" : "+v"(a4[z][g]));
+    }
+#pragma unroll
+    for (int g = 0; g < kRdB; ++g) {
+      if constexpr (kBK) asm volatile("" : "+v"(b8[z][g]));
+      else asm volatile("" : "+v"(b4[z][g]));
+    }
+  };
+  auto afrag = [&](int z, int i) {
+    if constexpr (kAK) return a8[z][i];
+    else return __builtin_shufflevector(a4[z][2 * i], a4[z][2 * i + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+  auto bfrag = [&](int z, int i) {
+    if constexpr (kBK) return b8[z][i];
+    else return __builtin_shufflevector(b4[z][2 * i], b4[z][2 * i + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+
+  f32x16 acc[kNB][kMB];
+#pragma unroll
+  for (int i = 0; i < kNB; ++i)
+#pragma unroll
+    for (int j = 0; j < kMB; ++j) acc[i][j] = f32x16{};
+#pragma unroll
+  for (int j = 0; j < kLoads; ++j) load(0, 0, j);
+  if (n_it > 1) {
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) load(1, 1, j);
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(kLoads));
+  } else {
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+  }
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int g = 0; g < kRd; ++g) rd(0, 0, 0, g);
+  wait(0);
+  __builtin_amdgcn_sched_barrier(0);
+  auto stage = [&](int i, auto step_f) {
+    constexpr bool kNext = decltype(step_f)::kNextV, kNext2 = decltype(step_f)::kNext2V;
+    const int st = i & 1;
+    const uint32_t soff = st * kStage, noff = (st ^ 1) * kStage;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      const int z = kk & 1;
+      if (kk == 3 && kNext) {
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int f = 0; f < kMf; ++f) {  // one MFMA, its share of the next step's reads and of the loads
+#pragma unroll
+        for (int g = f * kRd / kMf; g < (f + 1) * kRd / kMf; ++g) {
+          if (kk < 3) rd(z ^ 1, soff, kk + 1, g);
+          else if (kNext) rd(z ^ 1, noff, 0, g);
+        }
+        if (kk == 3 && kNext2) {
+#pragma unroll
+          for (int j = f * kLoads / kMf; j < (f + 1) * kLoads / kMf; ++j) load(i + 2, st, j);
+        }
+        const int jj = f / kNB, ii = f % kNB;
+        acc[ii][jj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfrag(z, ii), afrag(z, jj), acc[ii][jj], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (kk < 3 || kNext) {
+        wait(z ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  int i = 0;
+  for (; i + 2 < n_it; ++i) stage(i, LgFlags<true, true>{});
+  if (i + 1 < n_it) stage(i++, LgFlags<true, false>{});
+  if (i < n_it) stage(i, LgFlags<false, false>{});
+#undef TM_RD
+#undef TM_TR
+
+  // D[n][m] of a block: register r of lane l holds n = 8 (r / 4) + 4 (l / 32) + r % 4, m = l % 32
+#pragma unroll
+  for (int jj = 0; jj < kMB; ++jj) {
+    const int m = m0 + (wm * kMB + jj) * 32 + (lane & 31);
+#pragma unroll
+    for (int ii = 0; ii < kNB; ++ii) {
+      const int nb = n0 + (wn * kNB + ii) * 32;
+      if constexpr (kPartial) {
+        float* P = static_cast<float*>(out) + static_cast<int64_t>(split) * M * N;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int n = nb + 8 * q + 4 * (lane >> 5);
+          const f32x4 v = {acc[ii][jj][4 * q], acc[ii][jj][4 * q + 1], acc[ii][jj][4 * q + 2], acc[ii][jj][4 * q + 3]};
+          if (m < M && n < N) *(f32x4*)(P + static_cast<int64_t>(m) * N + n) = v;
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; q += 2) {
+          uint32_t lo[2], hi[2];
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            lo[e] = pack_bf16x2(acc[ii][jj][4 * q + 2 * e], acc[ii][jj][4 * q + 2 * e + 1]);
+            hi[e] = pack_bf16x2(acc[ii][jj][4 * q + 4 + 2 * e], acc[ii][jj][4 * q + 5 + 2 * e]);
+            const auto s = __builtin_amdgcn_permlane32_swap(lo[e], hi[e], false, false);
+            lo[e] = s[0];
+            hi[e] = s[1];
+          }
+          // lanes below 32: columns 8 q .. 8 q + 7, lanes above: the next 8
+          const int n = nb + 8 * q + 8 * (lane >> 5);
+          const u32x4 v = {lo[0], lo[1], hi[0], hi[1]};
+          if (m < M && n < N)  // rows hold whole groups of 8 (ldc and the last group's end <= ldc)
+            *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(out) + m * ldc + n) = v;
+        }
+      }
+    }
+  }
+}
+
 // Tile groups per XCD round (gm row tiles x gn weight panels, gm gn = 32), chosen from a sweep of
 // the logits ring kernel on MI355X (V = 151,936; TFLOP/s of the best against the next best):
 //   dim <= 1024: 1 x 32 up to 4 row tiles (1063 against 855 for 4 x 8 at 1024 rows: the hidden
@@ -1196,27 +1435,72 @@ void logits_groups(int64_t tiles_m, int64_t dim, int& gm, int& gn) {
   gn = 32 / gm;
 }
 
-// Splits of the K range, chosen by a cost model of the launch. One workgroup (128 KB of LDS) fits
-// a CU, so tiles x S workgroups run in ceil(tiles x S / 256) rounds; a workgroup takes about
-// 1.7 us per 64-deep K slice (256 x 256 x 64 MFMA work at the main loop's pace) plus about 8 us
-// to store its 256 KB partial tile, and the reduction reads S x rows x dim fp32 partials at about
-// 5 TB/s. For the Qwen3-0.6B head (dim 1024) the model picks S = 16 for a 1024-row chunk
-// (16 tiles, 256 workgroups), 4 for 4096 rows and 2 for 8192 rows (128 tiles).
-int64_t splits_for(int64_t rows, int64_t vocab, int64_t dim) {
-  const int64_t tiles = ((rows + kTile - 1) / kTile) * ((dim + kTile - 1) / kTile);
-  const int64_t iters = (vocab + kSliceK - 1) / kSliceK;
-  int64_t best = 1;
-  double best_us = 0.0;
-  for (int64_t s = 1; s <= 256; ++s) {
-    const int64_t rounds = (tiles * s + 255) / 256;
-    const double us = static_cast<double>(rounds) * (1.7 * static_cast<double>((iters + s - 1) / s) + 8.0) +
-                      static_cast<double>(s) * static_cast<double>(rows * dim) * 4.0 / 5e6;
-    if (s == 1 || us < best_us) {
-      best = s;
-      best_us = us;
+// Which kernel, and how many splits of K: the least estimated time. The model is the launch's
+// rounds over the CUs, times K slices a workgroup, times the measured time of a slice, plus a
+// tile's epilogue, plus, with splits, the fp32 partials' way out and back and the reduction. Its
+// choice among the kernels was within 2% of the best one's time on average over 58 products from
+// 512 x 256 x 4096 to 2102 x 960 x 111,744 (at most 9% on any but one).
+// For the Qwen3-0.6B head (dim 1024) grad_h gets S = 16 for a 1024-row chunk (16 tiles, 256
+// workgroups), 4 for 4096 rows and 2 for 8192 rows (128 tiles).
+constexpr double kUsSlice256 = 1.42;       // a 64-deep K slice of a 256 x 256 tile, one workgroup a CU
+constexpr double kUsSlice128 = 0.62;       // of a 128 x 128 tile, one workgroup a CU: latency
+constexpr double kUsSlice128Pair = 0.95;   // the same with two a CU
+constexpr double kUsLaunch = 3.0, kUsEpilogue = 1.5, kUsReduce = 2.5, kBytesPerUs = 4.5e6;
+constexpr int64_t kMaxPartialBytes = int64_t(2) << 30;
+
+struct TilePlan {
+  bool wide;       // 256 x 256 tiles, else 128 x 128
+  int64_t splits;  // of K, every one with at least one slice
+  double us;
+};
+
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+double tile_us(bool wide, int64_t M, int64_t N, int64_t slices, int64_t splits) {
+  const int64_t edge = wide ? 256 : 128, per = ceil_div(slices, splits);
+  const int64_t wgs = ceil_div(M, edge) * ceil_div(N, edge) * splits;
+  double us = kUsLaunch;
+  if (wide) us += ceil_div(wgs, 256) * (per * kUsSlice256 + 2 * kUsEpilogue);
+  else if (wgs <= 256) us += per * kUsSlice128 + kUsEpilogue;
+  else us += ceil_div(wgs, 512) * (per * kUsSlice128Pair + kUsEpilogue);
+  if (splits > 1) us += kUsReduce + static_cast<double>(splits * M * N) * 8.0 / kBytesPerUs;
+  return us;
+}
+
+// The best of the two tile sizes over up to `most` splits. The small tiles have to be 5% ahead: a
+// workgroup's partials leave under the next round's products, which the model does not see, and
+// wide tiles gain more from that (1024 x 768 x 32,001: 66 us against 69, both estimated at 70).
+TilePlan best_tiles(int64_t M, int64_t N, int64_t slices, int64_t most, bool wide_unsplit) {
+  constexpr double kLead = 1.05;
+  TilePlan best = {false, 1, kLead * tile_us(false, M, N, slices, 1)};
+  for (int64_t s = 1; s <= most && s <= slices; ++s) {
+    if (ceil_div(slices, ceil_div(slices, s)) != s) continue;  // some split would be empty
+    if (s > 1 && s * M * N * 4 > kMaxPartialBytes) break;
+    for (const bool wide : {false, true}) {
+      if (wide && s == 1 && !wide_unsplit) continue;
+      const double us = tile_us(wide, M, N, slices, s) * (wide ? 1.0 : kLead);
+      if (us < best.us) best = {wide, s, us};
     }
   }
   return best;
+}
+
+TilePlan grad_h_plan(int64_t rows, int64_t vocab, int64_t dim) {
+  return best_tiles(rows, dim, ceil_div(vocab, kSliceK), 256, true);
+}
+
+// The persistent kernels' time: whole rounds of 256 x 256 tiles, the epilogue under the next
+// tile's products.
+double ring_us(int64_t M, int64_t N, int64_t slices) {
+  return kUsLaunch + 2.0 + ceil_div(ceil_div(M, kLgTile) * ceil_div(N, kLgTile), 256) * slices * kUsSlice256;
+}
+
+// grad_W on the tile kernel (splits > 0), or on the 256 x 256 kernels (0). Without a workspace
+// there are no splits.
+TilePlan grad_w_plan(int64_t pad_rows, int64_t vocab, int64_t dim, bool workspace) {
+  const int64_t slices = pad_rows / kSliceK;
+  const TilePlan p = best_tiles(vocab, dim, slices, workspace ? 256 : 1, false);
+  return p.us < ring_us(vocab, dim, slices) ? p : TilePlan{true, 0, 0.0};
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -1226,13 +1510,17 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 // launch there. The device's CU count (for the ring kernels' workgroups per XCD) is read then.
 constexpr int kMaxDevices = 64;
 std::mutex g_lds_mu;
-bool g_lds_set[8][kMaxDevices] = {};
+bool g_lds_set[15][kMaxDevices] = {};
 int g_cus[kMaxDevices] = {};
 
-// which: 0 grad_h_gemm_kernel, 1 logits_gemm_kernel, 2 grad_w_gemm_kernel, 3 logits_ring_kernel,
-// 4 grad_w_ring_kernel, 5-7 the ragged forms of 0, 2 and 4.
+enum Kernel {
+  kGradH, kLogits, kGradW, kLogitsRing, kGradWRing, kGradHRagged, kGradWRagged, kGradWRingRagged,
+  kTileLogits, kTileGradH, kTileGradHSplit, kTileGradHWide, kTileGradW, kTileGradWSplit, kTileGradWSplitWide,
+};
+constexpr int kTileLds128 = 2 * 256 * 128, kTileLds256 = 2 * 512 * 128;
+
 // `cus`, when given, receives the device's CU count.
-hipError_t allow_lds(hipStream_t stream, int which, int* cus = nullptr) {
+hipError_t allow_lds(hipStream_t stream, Kernel which, int* cus = nullptr) {
   int dev = -1;
   hipError_t e = stream ? hipStreamGetDevice(stream, &dev) : hipGetDevice(&dev);
   if (e != hipSuccess) return e;
@@ -1245,13 +1533,29 @@ hipError_t allow_lds(hipStream_t stream, int which, int* cus = nullptr) {
   int cur = -1;
   e = hipGetDevice(&cur);
   if (e == hipSuccess && cur != dev) e = hipSetDevice(dev);
-  const void* fn[8] = {
-      reinterpret_cast<const void*>(grad_h_gemm_kernel<false>), reinterpret_cast<const void*>(logits_gemm_kernel),
-      reinterpret_cast<const void*>(grad_w_gemm_kernel<false>), reinterpret_cast<const void*>(logits_ring_kernel),
-      reinterpret_cast<const void*>(grad_w_ring_kernel<false>), reinterpret_cast<const void*>(grad_h_gemm_kernel<true>),
-      reinterpret_cast<const void*>(grad_w_gemm_kernel<true>),  reinterpret_cast<const void*>(grad_w_ring_kernel<true>)};
-  const int bytes[8] = {2 * kLgStage, kLgLds, kLgLds, kRgLds, kRgLds, 2 * kLgStage, kLgLds, kRgLds};
-  if (e == hipSuccess) e = hipFuncSetAttribute(fn[which], hipFuncAttributeMaxDynamicSharedMemorySize, bytes[which]);
+  struct Entry {
+    const void* fn;
+    int bytes;
+  };
+  const Entry entries[15] = {
+      {reinterpret_cast<const void*>(grad_h_gemm_kernel<false>), 2 * kLgStage},
+      {reinterpret_cast<const void*>(logits_gemm_kernel), kLgLds},
+      {reinterpret_cast<const void*>(grad_w_gemm_kernel<false>), kLgLds},
+      {reinterpret_cast<const void*>(logits_ring_kernel), kRgLds},
+      {reinterpret_cast<const void*>(grad_w_ring_kernel<false>), kRgLds},
+      {reinterpret_cast<const void*>(grad_h_gemm_kernel<true>), 2 * kLgStage},
+      {reinterpret_cast<const void*>(grad_w_gemm_kernel<true>), kLgLds},
+      {reinterpret_cast<const void*>(grad_w_ring_kernel<true>), kRgLds},
+      {reinterpret_cast<const void*>(gemm_tile_kernel<2, 1, true, true, false>), kTileLds128},
+      {reinterpret_cast<const void*>(gemm_tile_kernel<2, 1, true, false, false>), kTileLds128},
+      {reinterpret_cast<const void*>(gemm_tile_kernel<2, 1, true, false, true>), kTileLds128},
+      {reinterpret_cast<const void*>(gemm_tile_kernel<4, 2, true, false, false>), kTileLds256},
+      {reinterpret_cast<const void*>(gemm_tile_kernel<2, 1, false, false, false>), kTileLds128},
+      {reinterpret_cast<const void*>(gemm_tile_kernel<2, 1, false, false, true>), kTileLds128},
+      {reinterpret_cast<const void*>(gemm_tile_kernel<4, 2, false, false, true>), kTileLds256},
+  };
+  if (e == hipSuccess)
+    e = hipFuncSetAttribute(entries[which].fn, hipFuncAttributeMaxDynamicSharedMemorySize, entries[which].bytes);
   if (e == hipSuccess && g_cus[dev] == 0) e = hipDeviceGetAttribute(&g_cus[dev], hipDeviceAttributeMultiprocessorCount, dev);
   if (cur >= 0 && cur != dev) {
     const hipError_t back = hipSetDevice(cur);
@@ -1264,82 +1568,35 @@ hipError_t allow_lds(hipStream_t stream, int which, int* cus = nullptr) {
   return e;
 }
 
-}  // namespace
-
-extern "C" {
-
-size_t tm_ce_grad_h_workspace_bytes(int64_t rows, int64_t vocab, int64_t dim) {
-  if (rows % kTile || dim % kTile || vocab % kSliceK) return 0;
-  return tm_ce_grad_h_ld_workspace_bytes(rows, vocab, dim);
-}
-
-int tm_ce_grad_h_bf16(uint16_t* d_grad_h, const uint16_t* d_grad_logits, const uint16_t* d_w, int64_t rows,
-                      int64_t vocab, int64_t dim, void* d_ws, size_t ws_bytes, void* stream) {
-  if (rows <= 0 || dim <= 0 || vocab <= 0 || rows % kTile || dim % kTile || vocab % kSliceK)
-    return gemm_fail(TM_EINVAL,
-                     "tm_ce_grad_h_bf16: rows %lld and dim %lld must be positive multiples of %d, vocab %lld "
-                     "of %d", (long long)rows, (long long)dim, kTile, (long long)vocab, kSliceK);
-  return tm_ce_grad_h_ld_bf16(d_grad_h, d_grad_logits, vocab, d_w, rows, vocab, dim, d_ws, ws_bytes, stream);
-}
-
-size_t tm_ce_grad_h_ld_workspace_bytes(int64_t rows, int64_t vocab, int64_t dim) {
-  if (rows <= 0 || dim <= 0 || vocab <= 0 || dim % 8) return 0;
-  return static_cast<size_t>(splits_for(rows, vocab, dim)) * rows * dim * sizeof(float);
-}
-
-int tm_ce_grad_h_ld_bf16(uint16_t* d_grad_h, const uint16_t* d_grad_logits, int64_t ld, const uint16_t* d_w,
-                         int64_t rows, int64_t vocab, int64_t dim, void* d_ws, size_t ws_bytes, void* stream) {
-  if (rows <= 0 || dim <= 0 || vocab <= 0 || dim % 8 || ld % 8 || ld < (vocab + kSliceK - 1) / kSliceK * kSliceK)
-    return gemm_fail(TM_EINVAL,
-                     "tm_ce_grad_h_bf16: rows %lld and vocab %lld must be positive, dim %lld a positive multiple of 8, "
-                     "grad_logits rows %lld elements apart a multiple of 8 and hold whole groups of %d", (long long)rows,
-                     (long long)vocab, (long long)dim, (long long)ld, kSliceK);
-  if (rows > (1 << 20) || dim > (1 << 16) || vocab > 0x7FFFFF00)
-    return gemm_fail(TM_EINVAL, "tm_ce_grad_h_bf16: rows %lld, dim %lld or vocab %lld too large", (long long)rows,
-                     (long long)dim, (long long)vocab);
-  if (!d_grad_h || !d_grad_logits || !d_w || !d_ws)
-    return gemm_fail(TM_EINVAL, "tm_ce_grad_h_bf16: null pointer");
-  if (!aligned16(d_grad_h) || !aligned16(d_grad_logits) || !aligned16(d_w) || !aligned16(d_ws))
-    return gemm_fail(TM_EINVAL, "tm_ce_grad_h_bf16: pointers must be 16-byte aligned");
-  const size_t need = tm_ce_grad_h_ld_workspace_bytes(rows, vocab, dim);
-  if (ws_bytes < need)
-    return gemm_fail(TM_EINVAL, "tm_ce_grad_h_bf16: workspace of %zu bytes, %zu needed", ws_bytes, need);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const int64_t splits = splits_for(rows, vocab, dim);
-  const int64_t tiles = ((rows + kTile - 1) / kTile) * ((dim + kTile - 1) / kTile);
-  const int64_t total_iters = (vocab + kSliceK - 1) / kSliceK;
-  const int64_t per = (total_iters + splits - 1) / splits;
-  const bool ragged = rows % kTile != 0 || dim % kTile != 0 || vocab % kSliceK != 0;
-  const hipError_t lds = allow_lds(s, ragged ? 5 : 0);
-  if (lds != hipSuccess)
-    return gemm_fail(TM_ELAUNCH, "tm_ce_grad_h_bf16: LDS attribute: %s", hipGetErrorString(lds));
-  float* partials = static_cast<float*>(d_ws);
-  const dim3 grid(static_cast<uint32_t>((tiles * splits + 7) / 8 * 8));
-  if (ragged)
-    hipLaunchKernelGGL(grad_h_gemm_kernel<true>, grid, dim3(512), 2 * kLgStage, s, d_grad_logits, d_w, partials,
-                       static_cast<int>(rows), static_cast<int>(dim), ld, static_cast<int>(vocab),
-                       static_cast<int>(tiles), static_cast<int>(splits), static_cast<int>(per));
-  else
-    hipLaunchKernelGGL(grad_h_gemm_kernel<false>, grid, dim3(512), 2 * kLgStage, s, d_grad_logits, d_w, partials,
-                       static_cast<int>(rows), static_cast<int>(dim), ld, static_cast<int>(vocab),
-                       static_cast<int>(tiles), static_cast<int>(splits), static_cast<int>(per));
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return gemm_fail(TM_ELAUNCH, "grad_h_gemm_kernel: launch failed: %s", hipGetErrorString(e));
-  const int64_t n = rows * dim;
-  hipLaunchKernelGGL(grad_h_reduce_kernel, dim3(static_cast<uint32_t>((n / 4 + 255) / 256)), dim3(256), 0, s,
-                     partials, d_grad_h, n, static_cast<int>(splits));
-  e = hipGetLastError();
-  if (e != hipSuccess) return gemm_fail(TM_ELAUNCH, "grad_h_reduce_kernel: launch failed: %s", hipGetErrorString(e));
+// One gemm_tile_kernel launch: M x N outputs of `slices` K slices in `splits` parts.
+template <int kMB, int kNB, bool kAK, bool kBK, bool kPartial>
+int tile_launch(Kernel which, const uint16_t* A, const uint16_t* B, void* out, int64_t M, int64_t N, int64_t lda,
+                int64_t ldb, int64_t ldc, int64_t slices, int64_t kb, int64_t gm, int64_t gn, int64_t splits,
+                hipStream_t s, const char* who) {
+  const hipError_t lds = allow_lds(s, which);
+  if (lds != hipSuccess) return gemm_fail(TM_ELAUNCH, "%s: LDS attribute: %s", who, hipGetErrorString(lds));
+  const int64_t tm = ceil_div(M, 64 * kMB), tn = ceil_div(N, 128 * kNB);
+  hipLaunchKernelGGL((gemm_tile_kernel<kMB, kNB, kAK, kBK, kPartial>),
+                     dim3(static_cast<uint32_t>((tm * tn * splits + 7) / 8 * 8)), dim3(512),
+                     (64 * kMB + 128 * kNB) * 256, s, A, B, out, static_cast<int>(M), static_cast<int>(N), lda, ldb, ldc,
+                     static_cast<int>(slices), static_cast<int>(kb), static_cast<int>(tm), static_cast<int>(tn),
+                     static_cast<int>(gm), static_cast<int>(gn), static_cast<int>(ceil_div(slices, splits)));
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return gemm_fail(TM_ELAUNCH, "%s: launch failed: %s", who, hipGetErrorString(e));
   return TM_OK;
 }
 
-int tm_ce_logits_bf16(uint16_t* d_logits, const uint16_t* d_hidden, const uint16_t* d_weight, int64_t rows,
-                      int64_t vocab, int64_t dim, void* stream) {
-  return tm_ce_logits_ld_bf16(d_logits, vocab, d_hidden, d_weight, rows, vocab, dim, stream);
+int reduce_launch(const float* partials, uint16_t* out, int64_t n, int64_t splits, hipStream_t s, const char* who) {
+  hipLaunchKernelGGL(splits_reduce_kernel, dim3(static_cast<uint32_t>((n / 4 + 255) / 256)), dim3(256), 0, s, partials,
+                     out, n, static_cast<int>(splits));
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return gemm_fail(TM_ELAUNCH, "%s: reduction failed: %s", who, hipGetErrorString(e));
+  return TM_OK;
 }
 
-int tm_ce_logits_ld_bf16(uint16_t* d_logits, int64_t ld, const uint16_t* d_hidden, const uint16_t* d_weight,
-                         int64_t rows, int64_t vocab, int64_t dim, void* stream) {
+// small_tiles: the tile kernel where the model finds it faster (the same bits).
+int logits_launch(uint16_t* d_logits, int64_t ld, const uint16_t* d_hidden, const uint16_t* d_weight, int64_t rows,
+                  int64_t vocab, int64_t dim, bool small_tiles, void* stream) {
   if (rows <= 0 || vocab <= 0 || dim <= 0 || dim % kSliceK)
     return gemm_fail(TM_EINVAL, "tm_ce_logits_bf16: rows %lld and vocab %lld must be positive, dim %lld a positive "
                      "multiple of %d", (long long)rows, (long long)vocab, (long long)dim, kSliceK);
@@ -1354,11 +1611,17 @@ int tm_ce_logits_ld_bf16(uint16_t* d_logits, int64_t ld, const uint16_t* d_hidde
   if (!aligned16(d_logits) || !aligned16(d_hidden) || !aligned16(d_weight))
     return gemm_fail(TM_EINVAL, "tm_ce_logits_bf16: pointers must be 16-byte aligned");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  const int64_t slices = dim / kSliceK;
+  if (small_tiles && ld % 8 == 0 && 1.05 * tile_us(false, rows, vocab, slices, 1) < ring_us(rows, vocab, slices)) {
+    const int64_t t128 = ceil_div(rows, 128), gm128 = t128 < 4 ? t128 : 4;
+    return tile_launch<2, 1, true, true, false>(kTileLogits, d_hidden, d_weight, d_logits, rows, vocab, dim, dim, ld,
+                                                slices, vocab, gm128, 32 / gm128, 1, s, "tm_ce_logits_bf16");
+  }
   int gm, gn;
   logits_groups(tiles_m, dim, gm, gn);
   if (logits_ring_fits(rows, vocab, dim, ld)) {
     int cus = 0;
-    const hipError_t lds = allow_lds(s, 3, &cus);
+    const hipError_t lds = allow_lds(s, kLogitsRing, &cus);
     if (lds != hipSuccess)
       return gemm_fail(TM_ELAUNCH, "tm_ce_logits_bf16: LDS attribute: %s", hipGetErrorString(lds));
     const int wpx = cus >= 16 ? cus / 8 : 1;  // one workgroup per CU of each XCD
@@ -1369,7 +1632,7 @@ int tm_ce_logits_ld_bf16(uint16_t* d_logits, int64_t ld, const uint16_t* d_hidde
     if (e != hipSuccess) return gemm_fail(TM_ELAUNCH, "logits_ring_kernel: launch failed: %s", hipGetErrorString(e));
     return TM_OK;
   }
-  const hipError_t lds = allow_lds(s, 1);
+  const hipError_t lds = allow_lds(s, kLogits);
   if (lds != hipSuccess)
     return gemm_fail(TM_ELAUNCH, "tm_ce_logits_bf16: LDS attribute: %s", hipGetErrorString(lds));
   const int64_t grid = (tiles_m * tiles_n + 7) / 8 * 8;
@@ -1381,16 +1644,11 @@ int tm_ce_logits_ld_bf16(uint16_t* d_logits, int64_t ld, const uint16_t* d_hidde
   return TM_OK;
 }
 
-int tm_ce_grad_w_bf16(uint16_t* d_grad_w, const uint16_t* d_grad_logits, const uint16_t* d_hidden, int64_t rows,
-                      int64_t vocab, int64_t dim, void* stream) {
-  if (rows <= 0 || vocab <= 0 || dim <= 0 || rows % kSliceK || vocab % 8 || dim % 8)
-    return gemm_fail(TM_EINVAL, "tm_ce_grad_w_bf16: rows %lld must be a positive multiple of %d, vocab %lld and dim "
-                     "%lld positive multiples of 8", (long long)rows, kSliceK, (long long)vocab, (long long)dim);
-  return tm_ce_grad_w_ld_bf16(d_grad_w, d_grad_logits, vocab, rows, d_hidden, rows, vocab, dim, stream);
-}
-
-int tm_ce_grad_w_ld_bf16(uint16_t* d_grad_w, const uint16_t* d_grad_logits, int64_t ld, int64_t pad_rows,
-                         const uint16_t* d_hidden, int64_t rows, int64_t vocab, int64_t dim, void* stream) {
+// tiles: the tile kernel where the model finds it faster, with splits of K (other bits) if the
+// workspace holds them.
+int grad_w_launch(uint16_t* d_grad_w, const uint16_t* d_grad_logits, int64_t ld, int64_t pad_rows,
+                  const uint16_t* d_hidden, int64_t rows, int64_t vocab, int64_t dim, void* d_ws, size_t ws_bytes,
+                  bool tiles, void* stream) {
   if (rows <= 0 || vocab <= 0 || dim <= 0 || dim % 8 || ld % 8 || ld < vocab || pad_rows % kSliceK || pad_rows < rows ||
       pad_rows - rows >= 2 * kTile)
     return gemm_fail(TM_EINVAL, "tm_ce_grad_w_bf16: rows %lld and vocab %lld must be positive, dim %lld a positive "
@@ -1405,10 +1663,33 @@ int tm_ce_grad_w_ld_bf16(uint16_t* d_grad_w, const uint16_t* d_grad_logits, int6
   if (!aligned16(d_grad_w) || !aligned16(d_grad_logits) || !aligned16(d_hidden))
     return gemm_fail(TM_EINVAL, "tm_ce_grad_w_bf16: pointers must be 16-byte aligned");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  TilePlan plan = {true, 0, 0.0};
+  if (tiles) {
+    plan = grad_w_plan(pad_rows, vocab, dim, d_ws != nullptr);
+    if (plan.splits > 1 && ws_bytes < static_cast<size_t>(plan.splits) * vocab * dim * sizeof(float))
+      return gemm_fail(TM_EINVAL, "tm_ce_grad_w_bf16: workspace of %zu bytes, %zu needed", ws_bytes,
+                       static_cast<size_t>(plan.splits) * vocab * dim * sizeof(float));
+    if (plan.splits > 1 && !aligned16(d_ws))
+      return gemm_fail(TM_EINVAL, "tm_ce_grad_w_bf16: pointers must be 16-byte aligned");
+  }
+  if (plan.splits > 0) {
+    const char* who = "tm_ce_grad_w_bf16";
+    const int64_t slices = pad_rows / kSliceK, tn = ceil_div(dim, plan.wide ? 256 : 128);
+    const int64_t pn = tn < 8 ? tn : 8, pm = 32 / pn;
+    if (plan.splits == 1)
+      return tile_launch<2, 1, false, false, false>(kTileGradW, d_grad_logits, d_hidden, d_grad_w, vocab, dim, ld, dim,
+                                                    dim, slices, rows, pm, pn, 1, s, who);
+    const int rc =
+        plan.wide ? tile_launch<4, 2, false, false, true>(kTileGradWSplitWide, d_grad_logits, d_hidden, d_ws, vocab, dim,
+                                                          ld, dim, dim, slices, rows, pm, pn, plan.splits, s, who)
+                  : tile_launch<2, 1, false, false, true>(kTileGradWSplit, d_grad_logits, d_hidden, d_ws, vocab, dim, ld,
+                                                          dim, dim, slices, rows, pm, pn, plan.splits, s, who);
+    return rc ? rc : reduce_launch(static_cast<const float*>(d_ws), d_grad_w, vocab * dim, plan.splits, s, who);
+  }
   const int gn = static_cast<int>(tiles_d < 4 ? tiles_d : 4), gm = 32 / gn;  // a round of 32: 8 x 4
   const bool ragged = rows != pad_rows, ring = grad_w_ring_fits(pad_rows, ld, dim);
   int cus = 0;
-  const hipError_t lds = allow_lds(s, ring ? (ragged ? 7 : 4) : (ragged ? 6 : 2), &cus);
+  const hipError_t lds = allow_lds(s, ring ? (ragged ? kGradWRingRagged : kGradWRing) : (ragged ? kGradWRagged : kGradW), &cus);
   if (lds != hipSuccess)
     return gemm_fail(TM_ELAUNCH, "tm_ce_grad_w_bf16: LDS attribute: %s", hipGetErrorString(lds));
   const int V = static_cast<int>(vocab), L = static_cast<int>(ld), D = static_cast<int>(dim),
@@ -1435,6 +1716,112 @@ int tm_ce_grad_w_ld_bf16(uint16_t* d_grad_w, const uint16_t* d_grad_logits, int6
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return gemm_fail(TM_ELAUNCH, "grad_w kernel: launch failed: %s", hipGetErrorString(e));
   return TM_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t tm_ce_grad_h_workspace_bytes(int64_t rows, int64_t vocab, int64_t dim) {
+  if (rows % kTile || dim % kTile || vocab % kSliceK) return 0;
+  return tm_ce_grad_h_ld_workspace_bytes(rows, vocab, dim);
+}
+
+int tm_ce_grad_h_bf16(uint16_t* d_grad_h, const uint16_t* d_grad_logits, const uint16_t* d_w, int64_t rows,
+                      int64_t vocab, int64_t dim, void* d_ws, size_t ws_bytes, void* stream) {
+  if (rows <= 0 || dim <= 0 || vocab <= 0 || rows % kTile || dim % kTile || vocab % kSliceK)
+    return gemm_fail(TM_EINVAL,
+                     "tm_ce_grad_h_bf16: rows %lld and dim %lld must be positive multiples of %d, vocab %lld "
+                     "of %d", (long long)rows, (long long)dim, kTile, (long long)vocab, kSliceK);
+  return tm_ce_grad_h_ld_bf16(d_grad_h, d_grad_logits, vocab, d_w, rows, vocab, dim, d_ws, ws_bytes, stream);
+}
+
+size_t tm_ce_grad_h_ld_workspace_bytes(int64_t rows, int64_t vocab, int64_t dim) {
+  if (rows <= 0 || dim <= 0 || vocab <= 0 || dim % 8) return 0;
+  const TilePlan plan = grad_h_plan(rows, vocab, dim);
+  return plan.splits > 1 ? static_cast<size_t>(plan.splits) * rows * dim * sizeof(float) : 16;
+}
+
+int tm_ce_grad_h_ld_bf16(uint16_t* d_grad_h, const uint16_t* d_grad_logits, int64_t ld, const uint16_t* d_w,
+                         int64_t rows, int64_t vocab, int64_t dim, void* d_ws, size_t ws_bytes, void* stream) {
+  if (rows <= 0 || dim <= 0 || vocab <= 0 || dim % 8 || ld % 8 || ld < (vocab + kSliceK - 1) / kSliceK * kSliceK)
+    return gemm_fail(TM_EINVAL,
+                     "tm_ce_grad_h_bf16: rows %lld and vocab %lld must be positive, dim %lld a positive multiple of 8, "
+                     "grad_logits rows %lld elements apart a multiple of 8 and hold whole groups of %d", (long long)rows,
+                     (long long)vocab, (long long)dim, (long long)ld, kSliceK);
+  if (rows > (1 << 20) || dim > (1 << 16) || vocab > 0x7FFFFF00)
+    return gemm_fail(TM_EINVAL, "tm_ce_grad_h_bf16: rows %lld, dim %lld or vocab %lld too large", (long long)rows,
+                     (long long)dim, (long long)vocab);
+  if (!d_grad_h || !d_grad_logits || !d_w || !d_ws)
+    return gemm_fail(TM_EINVAL, "tm_ce_grad_h_bf16: null pointer");
+  if (!aligned16(d_grad_h) || !aligned16(d_grad_logits) || !aligned16(d_w) || !aligned16(d_ws))
+    return gemm_fail(TM_EINVAL, "tm_ce_grad_h_bf16: pointers must be 16-byte aligned");
+  const size_t need = tm_ce_grad_h_ld_workspace_bytes(rows, vocab, dim);
+  if (ws_bytes < need)
+    return gemm_fail(TM_EINVAL, "tm_ce_grad_h_bf16: workspace of %zu bytes, %zu needed", ws_bytes, need);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const char* who = "tm_ce_grad_h_bf16";
+  const TilePlan plan = grad_h_plan(rows, vocab, dim);
+  const int64_t splits = plan.splits, slices = ceil_div(vocab, kSliceK);
+  float* partials = static_cast<float*>(d_ws);
+  if (!plan.wide || splits == 1) {
+    const int64_t gm = ceil_div(rows, plan.wide ? 256 : 128) < 8 ? ceil_div(rows, plan.wide ? 256 : 128) : 8;
+    if (splits == 1)
+      return plan.wide ? tile_launch<4, 2, true, false, false>(kTileGradHWide, d_grad_logits, d_w, d_grad_h, rows, dim,
+                                                               ld, dim, dim, slices, vocab, gm, 4, 1, s, who)
+                       : tile_launch<2, 1, true, false, false>(kTileGradH, d_grad_logits, d_w, d_grad_h, rows, dim, ld,
+                                                               dim, dim, slices, vocab, gm, 4, 1, s, who);
+    const int rc = tile_launch<2, 1, true, false, true>(kTileGradHSplit, d_grad_logits, d_w, partials, rows, dim, ld, dim,
+                                                        dim, slices, vocab, gm, 4, splits, s, who);
+    return rc ? rc : reduce_launch(partials, d_grad_h, rows * dim, splits, s, who);
+  }
+  const int64_t tiles = ceil_div(rows, kTile) * ceil_div(dim, kTile), per = ceil_div(slices, splits);
+  const bool ragged = rows % kTile != 0 || dim % kTile != 0 || vocab % kSliceK != 0;
+  const hipError_t lds = allow_lds(s, ragged ? kGradHRagged : kGradH);
+  if (lds != hipSuccess)
+    return gemm_fail(TM_ELAUNCH, "tm_ce_grad_h_bf16: LDS attribute: %s", hipGetErrorString(lds));
+  const dim3 grid(static_cast<uint32_t>((tiles * splits + 7) / 8 * 8));
+  if (ragged)
+    hipLaunchKernelGGL(grad_h_gemm_kernel<true>, grid, dim3(512), 2 * kLgStage, s, d_grad_logits, d_w, partials,
+                       static_cast<int>(rows), static_cast<int>(dim), ld, static_cast<int>(vocab),
+                       static_cast<int>(tiles), static_cast<int>(splits), static_cast<int>(per));
+  else
+    hipLaunchKernelGGL(grad_h_gemm_kernel<false>, grid, dim3(512), 2 * kLgStage, s, d_grad_logits, d_w, partials,
+                       static_cast<int>(rows), static_cast<int>(dim), ld, static_cast<int>(vocab),
+                       static_cast<int>(tiles), static_cast<int>(splits), static_cast<int>(per));
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return gemm_fail(TM_ELAUNCH, "grad_h_gemm_kernel: launch failed: %s", hipGetErrorString(e));
+  return reduce_launch(partials, d_grad_h, rows * dim, splits, s, who);
+}
+
+int tm_ce_logits_bf16(uint16_t* d_logits, const uint16_t* d_hidden, const uint16_t* d_weight, int64_t rows,
+                      int64_t vocab, int64_t dim, void* stream) {
+  return logits_launch(d_logits, vocab, d_hidden, d_weight, rows, vocab, dim, false, stream);
+}
+
+int tm_ce_logits_ld_bf16(uint16_t* d_logits, int64_t ld, const uint16_t* d_hidden, const uint16_t* d_weight,
+                         int64_t rows, int64_t vocab, int64_t dim, void* stream) {
+  return logits_launch(d_logits, ld, d_hidden, d_weight, rows, vocab, dim, true, stream);
+}
+
+int tm_ce_grad_w_bf16(uint16_t* d_grad_w, const uint16_t* d_grad_logits, const uint16_t* d_hidden, int64_t rows,
+                      int64_t vocab, int64_t dim, void* stream) {
+  if (rows <= 0 || vocab <= 0 || dim <= 0 || rows % kSliceK || vocab % 8 || dim % 8)
+    return gemm_fail(TM_EINVAL, "tm_ce_grad_w_bf16: rows %lld must be a positive multiple of %d, vocab %lld and dim "
+                     "%lld positive multiples of 8", (long long)rows, kSliceK, (long long)vocab, (long long)dim);
+  return grad_w_launch(d_grad_w, d_grad_logits, vocab, rows, d_hidden, rows, vocab, dim, nullptr, 0, false, stream);
+}
+
+size_t tm_ce_grad_w_ld_workspace_bytes(int64_t pad_rows, int64_t vocab, int64_t dim) {
+  if (pad_rows <= 0 || vocab <= 0 || dim <= 0 || pad_rows % kSliceK) return 0;
+  const TilePlan plan = grad_w_plan(pad_rows, vocab, dim, true);
+  return plan.splits > 1 ? static_cast<size_t>(plan.splits) * vocab * dim * sizeof(float) : 0;
+}
+
+int tm_ce_grad_w_ld_bf16(uint16_t* d_grad_w, const uint16_t* d_grad_logits, int64_t ld, int64_t pad_rows,
+                         const uint16_t* d_hidden, int64_t rows, int64_t vocab, int64_t dim, void* d_ws,
+                         size_t ws_bytes, void* stream) {
+  return grad_w_launch(d_grad_w, d_grad_logits, ld, pad_rows, d_hidden, rows, vocab, dim, d_ws, ws_bytes, true, stream);
 }
 
 }  // extern "C"

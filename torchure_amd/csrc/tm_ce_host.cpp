@@ -25,7 +25,7 @@ typedef int (*rows_t)(void*, i64, const void*, i64, i64, i64, i64, void*, void*)
 typedef int (*rows_loss_t)(const void*, i64, const void*, i64, i64, i64, void*, void*);
 typedef size_t (*gh_bytes_t)(i64, i64, i64);
 typedef int (*grad_h_t)(void*, const void*, i64, const void*, i64, i64, i64, void*, size_t, void*);
-typedef int (*grad_w_t)(void*, const void*, i64, i64, const void*, i64, i64, i64, void*);
+typedef int (*grad_w_t)(void*, const void*, i64, i64, const void*, i64, i64, i64, void*, size_t, void*);
 typedef int (*fold_t)(void*, const void* const*, int, i64, int, const void*, const void*, void*);
 typedef int (*mean_t)(const void*, const void*, i64, i64, void*, void*, void*);
 typedef int (*finish_t)(void*, const void* const*, int, i64, int, const void*, void*, i64, int, const void*, const void*,
@@ -37,7 +37,7 @@ struct Abi {
   logits_t logits;
   rows_t rows;
   rows_loss_t rows_loss;
-  gh_bytes_t grad_h_bytes;
+  gh_bytes_t grad_h_bytes, grad_w_bytes;
   grad_h_t grad_h;
   grad_w_t grad_w;
   fold_t fold;
@@ -57,6 +57,7 @@ void ce_bind(const py::dict& addresses, const py::object& native_error) {
   a->rows = reinterpret_cast<rows_t>(at("tm_ce_rows_padded_bf16"));
   a->rows_loss = reinterpret_cast<rows_loss_t>(at("tm_ce_rows_loss_bf16"));
   a->grad_h_bytes = reinterpret_cast<gh_bytes_t>(at("tm_ce_grad_h_ld_workspace_bytes"));
+  a->grad_w_bytes = reinterpret_cast<gh_bytes_t>(at("tm_ce_grad_w_ld_workspace_bytes"));
   a->grad_h = reinterpret_cast<grad_h_t>(at("tm_ce_grad_h_ld_bf16"));
   a->grad_w = reinterpret_cast<grad_w_t>(at("tm_ce_grad_w_ld_bf16"));
   a->fold = reinterpret_cast<fold_t>(at("tm_ce_grad_w_fold"));
@@ -107,13 +108,18 @@ py::tuple ce_forward(const at::Tensor& hidden, const at::Tensor& weight, bool ca
           "tm_ce_cast2");
   const i64 last = n - (n - 1) / chunk * chunk;  // rows of the last chunk
   at::Tensor row_loss = at::empty({n}, f32), grad_hidden, grad_weight, ws;
+  // one workspace for both gradients' split sums over the chunks (stream-ordered)
+  size_t bytes = 0;
   if (grad && want_h) {
     grad_hidden = at::empty({n, d}, bf16);
-    size_t bytes = 0;
     if (own_h.first && n > chunk) bytes = a.grad_h_bytes(chunk, v, d);
     if (own_h.second) bytes = std::max(bytes, a.grad_h_bytes(last, v, d));
-    if (bytes) ws = at::empty({static_cast<i64>(bytes)}, f32.dtype(at::kByte));
   }
+  if (grad && want_w) {
+    if (n > chunk) bytes = std::max(bytes, a.grad_w_bytes(pad.first, v, d));
+    bytes = std::max(bytes, a.grad_w_bytes(pad.second, v, d));
+  }
+  if (bytes) ws = at::empty({static_cast<i64>(bytes)}, f32.dtype(at::kByte));
   std::vector<at::Tensor> pending;
   bool accumulated = false;
   for (i64 s = 0; s < n; s += chunk) {
@@ -131,7 +137,7 @@ py::tuple ce_forward(const at::Tensor& hidden, const at::Tensor& weight, bool ca
     check(a.rows(ptr(logits), ld, lab, rows, pad_rows, v, ignore, losses, stream), "tm_ce_rows_padded_bf16");
     if (want_h) {
       if (is_last ? own_h.second : own_h.first) {
-        check(a.grad_h(ptr(grad_hidden) + s * d * 2, ptr(logits), ld, ptr(w), rows, v, d, ptr(ws), ws.numel(), stream),
+        check(a.grad_h(ptr(grad_hidden) + s * d * 2, ptr(logits), ld, ptr(w), rows, v, d, ptr(ws), bytes, stream),
               "tm_ce_grad_h_ld_bf16");
       } else {
         at::Tensor out = grad_hidden.narrow(0, s, rows);
@@ -140,7 +146,7 @@ py::tuple ce_forward(const at::Tensor& hidden, const at::Tensor& weight, bool ca
     }
     if (want_w) {
       at::Tensor gw = at::empty({v, d}, bf16);
-      check(a.grad_w(ptr(gw), ptr(logits), ld, pad_rows, hs, rows, v, d, stream), "tm_ce_grad_w_ld_bf16");
+      check(a.grad_w(ptr(gw), ptr(logits), ld, pad_rows, hs, rows, v, d, ptr(ws), bytes, stream), "tm_ce_grad_w_ld_bf16");
       pending.push_back(gw);
       const i64 held = static_cast<i64>(pending.size());
       if (!is_last && (held == fold_chunks || held * v * d * 2 >= fold_bytes)) {

@@ -243,8 +243,10 @@ def _grad_w(g: torch.Tensor, h: torch.Tensor, lib, stream) -> torch.Tensor:
         g, short = torch.zeros((pad, vocab), dtype=torch.bfloat16, device=g.device), g
         g[:rows].copy_(short)
     out = torch.empty((vocab, h.shape[1]), dtype=torch.bfloat16, device=g.device)
+    nbytes = lib.tm_ce_grad_w_ld_workspace_bytes(pad, vocab, h.shape[1])
+    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=g.device)
     _native.check(lib.tm_ce_grad_w_ld_bf16(out.data_ptr(), g.data_ptr(), vocab, pad, h.data_ptr(), rows, vocab,
-                                           h.shape[1], stream), "tm_ce_grad_w_ld_bf16")
+                                           h.shape[1], ws.data_ptr(), nbytes, stream), "tm_ce_grad_w_ld_bf16")
     return out
 
 
@@ -274,17 +276,17 @@ def splitk_grad_h_fits(rows: int, dim: int, vocab: int) -> bool:
 
 
 def grad_h_gemm_fits(rows: int, dim: int, vocab: int) -> bool:
-    """Padded chunks whose grad_h runs on the split-K GEMM: those ``splitk_grad_h_fits`` accepts,
+    """Padded chunks whose grad_h runs on this build's GEMM: those ``splitk_grad_h_fits`` accepts,
     and ragged ones (rows or dim off a multiple of 256, a vocabulary off a multiple of 64) under
     the same rule for many tiles of a power-of-two width, from a vocabulary of
-    RAGGED_GRAD_H_MIN_VOCAB up: with a shorter K the partial tiles and their reduction cost more
-    than the split gives. us per call on MI355X, split-K / hipBLASLt on the same padded logits:
+    RAGGED_GRAD_H_MIN_VOCAB up (below, K is short, both take under 50 us, and neither leads
+    throughout). us per call on MI355X, this build / hipBLASLt on the same padded logits:
 
-        rows x dim x vocab     552 x 256 x 4096     27.6 /  18.5     1024 x 768 x 32001     63 / 181
-                               468 x 320 x 4376     29.3 /  20.9      452 x 768 x 32001     48 / 131
-                              7129 x 1216 x 1984    64.1 /  47.5     1905 x 1024 x 151936  538 / 703
-                              1024 x 320 x 7296     29.2 /  31.4     3000 x 2560 x 100000 1289 / 2061
-                              2046 x 2112 x 7296    77.5 /  74.4     6001 x 1024 x 151936 1616 / 1517
+        rows x dim x vocab    7129 x 1216 x 1984     50 /  48     1024 x 768 x 32001      69 / 183
+                              1184 x 384 x 2535      16 /  19      452 x 768 x 32001      41 / 135
+                               552 x 256 x 4097      14 /  19     1905 x 1024 x 151936   562 / 721
+                              1024 x 320 x 7296      21 /  33     3000 x 2560 x 100000  1337 / 2076
+                              2046 x 2112 x 7296     79 /  83     6001 x 1024 x 151936  1656 / 1570
     """
     if splitk_grad_h_fits(rows, dim, vocab):
         return True
@@ -294,7 +296,7 @@ def grad_h_gemm_fits(rows: int, dim: int, vocab: int) -> bool:
     return -(-rows // 256) * -(-dim // 256) <= SPLITK_GRAD_H_MAX_TILES or (dim & (dim - 1)) != 0
 
 
-RAGGED_GRAD_H_MIN_VOCAB = 7168
+RAGGED_GRAD_H_MIN_VOCAB = 4097
 
 FOLD_CHUNKS = 8  # chunks per grad_W fold (tm_ce_grad_w_fold takes at most 8)
 FOLD_BYTES = 4 << 30  # bf16 chunk grad_W held before a fold, at most
