@@ -1440,8 +1440,6 @@ void logits_groups(int64_t tiles_m, int64_t dim, int& gm, int& gn) {
 // tile's epilogue, plus, with splits, the fp32 partials' way out and back and the reduction. Its
 // choice among the kernels was within 2% of the best one's time on average over 58 products from
 // 512 x 256 x 4096 to 2102 x 960 x 111,744 (at most 9% on any but one).
-// For the Qwen3-0.6B head (dim 1024) grad_h gets S = 16 for a 1024-row chunk (16 tiles, 256
-// workgroups), 4 for 4096 rows and 2 for 8192 rows (128 tiles).
 constexpr double kUsSlice256 = 1.42;       // a 64-deep K slice of a 256 x 256 tile, one workgroup a CU
 constexpr double kUsSlice128 = 0.62;       // of a 128 x 128 tile, one workgroup a CU: latency
 constexpr double kUsSlice128Pair = 0.95;   // the same with two a CU
@@ -1467,26 +1465,47 @@ double tile_us(bool wide, int64_t M, int64_t N, int64_t slices, int64_t splits) 
   return us;
 }
 
-// The best of the two tile sizes over up to `most` splits. The small tiles have to be 5% ahead: a
+// The small tiles' best number of splits, up to `most`. They have to be 5% ahead of the others: a
 // workgroup's partials leave under the next round's products, which the model does not see, and
 // wide tiles gain more from that (1024 x 768 x 32,001: 66 us against 69, both estimated at 70).
-TilePlan best_tiles(int64_t M, int64_t N, int64_t slices, int64_t most, bool wide_unsplit) {
-  constexpr double kLead = 1.05;
-  TilePlan best = {false, 1, kLead * tile_us(false, M, N, slices, 1)};
-  for (int64_t s = 1; s <= most && s <= slices; ++s) {
+constexpr double kLead = 1.05;
+
+TilePlan best_tiles(bool wide, int64_t M, int64_t N, int64_t slices, int64_t least, int64_t most) {
+  const double lead = wide ? 1.0 : kLead;
+  TilePlan best = {wide, 0, 0.0};
+  for (int64_t s = least; s <= most && s <= slices; ++s) {
     if (ceil_div(slices, ceil_div(slices, s)) != s) continue;  // some split would be empty
     if (s > 1 && s * M * N * 4 > kMaxPartialBytes) break;
-    for (const bool wide : {false, true}) {
-      if (wide && s == 1 && !wide_unsplit) continue;
-      const double us = tile_us(wide, M, N, slices, s) * (wide ? 1.0 : kLead);
-      if (us < best.us) best = {wide, s, us};
+    const double us = lead * tile_us(wide, M, N, slices, s);
+    if (best.splits == 0 || us < best.us) best = {wide, s, us};
+  }
+  return best;
+}
+
+// Splits of grad_h on 256 x 256 tiles: whole rounds of workgroups at 1.7 us a K slice and 8 us to
+// store a partial tile, and the reduction at about 5 TB/s. S = 16 for a 1024-row chunk of the
+// Qwen3-0.6B head (dim 1024: 16 tiles, 256 workgroups), 4 for 4096 rows and 2 for 8192 rows.
+int64_t wide_splits(int64_t rows, int64_t vocab, int64_t dim) {
+  const int64_t tiles = ceil_div(rows, kTile) * ceil_div(dim, kTile), iters = ceil_div(vocab, kSliceK);
+  int64_t best = 1;
+  double best_us = 0.0;
+  for (int64_t s = 1; s <= 256; ++s) {
+    const double us = static_cast<double>(ceil_div(tiles * s, 256)) * (1.7 * static_cast<double>(ceil_div(iters, s)) + 8.0) +
+                      static_cast<double>(s) * static_cast<double>(rows * dim) * 4.0 / 5e6;
+    if (s == 1 || us < best_us) {
+      best = s;
+      best_us = us;
     }
   }
   return best;
 }
 
 TilePlan grad_h_plan(int64_t rows, int64_t vocab, int64_t dim) {
-  return best_tiles(rows, dim, ceil_div(vocab, kSliceK), 256, true);
+  const int64_t slices = ceil_div(vocab, kSliceK);
+  TilePlan plan = {true, wide_splits(rows, vocab, dim), 0.0};
+  plan.us = tile_us(true, rows, dim, slices, plan.splits);
+  const TilePlan small = best_tiles(false, rows, dim, slices, 1, plan.splits);
+  return small.splits > 0 && small.us < plan.us ? small : plan;
 }
 
 // The persistent kernels' time: whole rounds of 256 x 256 tiles, the epilogue under the next
@@ -1499,7 +1518,9 @@ double ring_us(int64_t M, int64_t N, int64_t slices) {
 // there are no splits.
 TilePlan grad_w_plan(int64_t pad_rows, int64_t vocab, int64_t dim, bool workspace) {
   const int64_t slices = pad_rows / kSliceK;
-  const TilePlan p = best_tiles(vocab, dim, slices, workspace ? 256 : 1, false);
+  TilePlan p = best_tiles(false, vocab, dim, slices, 1, workspace ? 256 : 1);
+  const TilePlan wide = best_tiles(true, vocab, dim, slices, 2, workspace ? 256 : 1);
+  if (wide.splits > 0 && wide.us < p.us) p = wide;
   return p.us < ring_us(vocab, dim, slices) ? p : TilePlan{true, 0, 0.0};
 }
 
@@ -1612,7 +1633,7 @@ int logits_launch(uint16_t* d_logits, int64_t ld, const uint16_t* d_hidden, cons
     return gemm_fail(TM_EINVAL, "tm_ce_logits_bf16: pointers must be 16-byte aligned");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t slices = dim / kSliceK;
-  if (small_tiles && ld % 8 == 0 && 1.05 * tile_us(false, rows, vocab, slices, 1) < ring_us(rows, vocab, slices)) {
+  if (small_tiles && ld % 8 == 0 && kLead * tile_us(false, rows, vocab, slices, 1) < ring_us(rows, vocab, slices)) {
     const int64_t t128 = ceil_div(rows, 128), gm128 = t128 < 4 ? t128 : 4;
     return tile_launch<2, 1, true, true, false>(kTileLogits, d_hidden, d_weight, d_logits, rows, vocab, dim, dim, ld,
                                                 slices, vocab, gm128, 32 / gm128, 1, s, "tm_ce_logits_bf16");
@@ -1738,8 +1759,8 @@ int tm_ce_grad_h_bf16(uint16_t* d_grad_h, const uint16_t* d_grad_logits, const u
 
 size_t tm_ce_grad_h_ld_workspace_bytes(int64_t rows, int64_t vocab, int64_t dim) {
   if (rows <= 0 || dim <= 0 || vocab <= 0 || dim % 8) return 0;
-  const TilePlan plan = grad_h_plan(rows, vocab, dim);
-  return plan.splits > 1 ? static_cast<size_t>(plan.splits) * rows * dim * sizeof(float) : 16;
+  // enough for either tile size: the small tiles take no more splits than the wide ones would
+  return static_cast<size_t>(wide_splits(rows, vocab, dim)) * rows * dim * sizeof(float);
 }
 
 int tm_ce_grad_h_ld_bf16(uint16_t* d_grad_h, const uint16_t* d_grad_logits, int64_t ld, const uint16_t* d_w,
