@@ -404,8 +404,9 @@ int tm_ce_cast2(uint16_t* d_dst0, const float* d_src0, int64_t n0, uint16_t* d_d
  * The whole of backward (fused_linear_ce.py:107-126) in one launch: d_grad_w over nw elements as
  * tm_ce_grad_w_fold with a scale (n_chunks may be 0: a plain d_grad_w *= g / n_valid when
  * accumulate is set), and grad_h over nh elements: d_grad_h_out (bf16, may be d_grad_h) =
- * bf16(d_grad_h * bf16(g / n_valid)), or, with wide set, d_grad_h_out (fp32) =
- * float(d_grad_h) * (g / n_valid). Either part may be empty.
+ * bf16(d_grad_h * bf16(g / n_valid)), or, with wide = 1, d_grad_h_out (fp32) =
+ * float(d_grad_h) * (g / n_valid), or, with wide = 2, both are one fp32 buffer, scaled in place.
+ * Either part may be empty.
  */
 int tm_ce_finish(float* d_grad_w, const uint16_t* const* h_chunks, int n_chunks, int64_t nw, int accumulate,
                  const uint16_t* d_grad_h, void* d_grad_h_out, int64_t nh, int wide, const float* d_grad_out,

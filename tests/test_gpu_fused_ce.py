@@ -866,6 +866,88 @@ def test_ce_rows_f32_kernel_vs_fp64(vocab):
     assert bool((work[~valid] == 0).all())
 
 
+@pytest.mark.parametrize("vocab", [
+    1, 4, 1024, 1028, 2048, 2052, 4096, 4100, 8192, 8196, 12288, 12292, 20480,  # 1 to 20 vectors, four waves
+    20484, 24580, 40960, 40964, 49156, 81920,  # eight and sixteen waves
+    81924, 90001,                              # too long for registers
+    3001, 10241, 81922,                        # packed rows off 16 bytes
+])
+def test_ce_rows_f32_at_the_edges_of_the_row_shapes(vocab):
+    """tm_ce_rows_f32 on both sides of every change of its threads and vectors a row, rows packed
+    (off 16 bytes where the vocabulary is) and 32 elements apart: losses and gradients against
+    fp64, the loss-only pass bit for bit equal, -inf, NaN, +inf and the type's lowest value where
+    only some threads or batches see them, nothing written past the vocabulary. Bounds: a sum of
+    positive terms is off by at most one rounding of 2^-24 per addition on the longest chain: 3 a
+    vector, 7 rescales of 5 (with their exponentials) and 10 additions over the lanes, or vocab /
+    1024 online steps of 5; lse moves by that plus its own roundings and the difference's."""
+    from torchure_amd import _native
+
+    lib, st = _native.lib(), _native.stream_handle(DEV)
+    g = torch.Generator(device=DEV).manual_seed(vocab)
+    rows, low = 13, torch.finfo(torch.float32).min
+    x = torch.randn(rows, vocab, device=DEV, generator=g) * 3.0
+    x[1, : vocab // 2] = float("-inf")
+    x[2, : max(0, vocab - 2)] = low          # whole threads at the mask value
+    x[3] = 3.3e38
+    x[4] -= 300.0
+    x[5, vocab // 3] = float("nan")
+    x[6] = float("-inf")
+    x[6, vocab - 1] = float("nan")
+    x[7, vocab // 2] = float("inf")
+    labels = torch.randint(0, vocab, (rows,), device=DEV, generator=g)
+    labels[1:3] = vocab - 1
+    labels[7] = 0 if vocab > 1 else -100     # not the +inf entry
+    labels[8] = -100
+    xd = x.double()
+    lse = torch.logsumexp(xd, dim=1)
+    want = lse - xd.gather(1, labels.clamp_min(0)[:, None])[:, 0]
+    want[labels == -100] = 0.0
+    probs = torch.exp(xd - lse[:, None])
+    grads = probs.clone()
+    grads[torch.arange(rows), labels.clamp_min(0)] -= 1.0
+    grads[labels == -100] = 0.0
+    fine = [r for r in range(rows) if r not in (5, 6, 7)]
+    chain = max(20, vocab // 4096) * 3 + max(7, vocab // 16384) * 5 + 10 + vocab // 1024 * 5 * (vocab % 4 != 0)
+    tol = 2.0 ** -24 * (chain + 4 * lse.abs())
+    for ld in (vocab, -(-vocab // 32) * 32):
+        buf = torch.full((rows, ld), 7.0, device=DEV)
+        buf[:, :vocab] = x
+        loss_only, loss = torch.empty(rows, device=DEV), torch.empty(rows, device=DEV)
+        for fn, out in ((lib.tm_ce_rows_loss_f32, loss_only), (lib.tm_ce_rows_f32, loss)):
+            _native.check(fn(buf.data_ptr(), ld, labels.data_ptr(), rows, vocab, -100, out.data_ptr(), st), "rows")
+        assert torch.equal(loss_only.view(torch.int32), loss.view(torch.int32))
+        assert (buf[:, vocab:] == 7.0).all()
+        assert ((loss.double() - want).abs() <= tol)[fine].all(), (loss, want)
+        assert loss[5].isnan() and loss[6].isnan()
+        got = buf[:, :vocab].double()
+        dist = (xd - lse[:, None]).abs().clamp_max(200.0)  # further off the probability is 0 either way
+        off = (got - grads).abs() - (probs * (2.0 * tol[:, None] + 2.0 ** -22 * (1 + dist)) + 2.0 ** -23)
+        assert (off <= 0)[fine].all(), off[fine].max()
+        assert got[5].isnan().all() and got[6].isnan().all()
+        if vocab > 1:  # as torch.logsumexp: lse = +inf, no probability anywhere but at the +inf entry
+            assert loss[7] == float("inf")
+            rest = torch.arange(vocab, device=DEV) != vocab // 2
+            rest[0] = False
+            assert (got[7, rest] == 0).all() and got[7, vocab // 2].isnan()
+
+
+@pytest.mark.parametrize("n", [1, 63, 64 * 64, 64 * 64 + 1, 300_001])
+def test_finish_scales_fp32_grad_h_in_place(n):
+    """tm_ce_finish with an fp32 grad_h: both gradients times grad_out / n_valid, the bits of the
+    fp32 product, in one launch, for sizes on both sides of a workgroup's slice."""
+    from torchure_amd import _native
+
+    g = torch.Generator(device=DEV).manual_seed(n)
+    gh, gw = torch.randn(n + 1, device=DEV, generator=g), torch.randn(n + 5, device=DEV, generator=g)
+    gh[0], gw[0] = float("inf"), -0.0
+    keep = gh[n].clone()
+    go, out2 = torch.tensor(3.0, device=DEV), torch.tensor([5.0, 7.0], device=DEV)
+    want_h, want_w = gh[:n] * (go / out2[1]), gw * (go / out2[1])
+    _native.ce_host().ce_backward(go, out2, gh[:n], 2, gw, [], True, _native.stream_handle(DEV))
+    assert torch.equal(gh[:n].view(torch.int32), want_h.view(torch.int32)) and gh[n] == keep
+    assert torch.equal(gw.view(torch.int32), want_w.view(torch.int32))
+
+
 @pytest.mark.parametrize("chunk", [None, 300])
 def test_fp32_hidden_without_autocast(chunk):
     """fp32 hidden states outside autocast: the reference runs fp32 GEMMs on w =

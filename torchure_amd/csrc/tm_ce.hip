@@ -428,19 +428,7 @@ __global__ __launch_bounds__(kCeThreads, kGrad ? 4 : 8) void ce_rows_kernel(uint
   for (int64_t i = vocab + threadIdx.x; i < width; i += kCeThreads) row[i] = 0;
 }
 
-// (max, sum of exp(x - max)) with the full-precision expf, for fp32 outputs.
-__device__ __forceinline__ void ms_merge_f(float& m, float& s, float m2, float s2) {
-  if (m2 == -INFINITY) return;
-  if (m2 > m) {
-    s = s * expf(m - m2) + s2;
-    m = m2;
-  } else if (m2 == m) {
-    s = s + s2;
-  } else {
-    s = s + s2 * expf(m2 - m);
-  }
-}
-
+// x joined to (max, sum of exp(x - max)), with the full-precision expf, for fp32 outputs.
 __device__ __forceinline__ void ms_add_f(float& m, float& s, float x) {
   if (x == -INFINITY) return;
   if (x > m) {
@@ -451,36 +439,30 @@ __device__ __forceinline__ void ms_add_f(float& m, float& s, float x) {
   }
 }
 
-// Block-wide (max, sumexp) of 256-thread workgroups, fixed order, full-precision exp.
-__device__ __forceinline__ void block_ms_f(float& m, float& s) {
-  __shared__ float lm[4], ls[4];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const float m2 = __shfl_xor(m, off, 64);
-    const float s2 = __shfl_xor(s, off, 64);
-    ms_merge_f(m, s, m2, s2);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    lm[threadIdx.x >> 6] = m;
-    ls[threadIdx.x >> 6] = s;
-  }
-  __syncthreads();
-  m = lm[0];
-  s = ls[0];
-  for (int w = 1; w < 4; ++w) ms_merge_f(m, s, lm[w], ls[w]);
-  __syncthreads();
-}
+// What the sum's exponents are taken against: the maximum, 0 where that is infinite, as
+// torch.logsumexp does: a +inf logit makes lse +inf, not NaN.
+__device__ __forceinline__ float finite_ref(float top) { return fabsf(top) == INFINITY ? 0.0f : top; }
+
+// What a sum under the maximum m is multiplied by when the maximum becomes top (>= m).
+__device__ __forceinline__ float raised(float m, float top) { return m == top ? 1.0f : expf(m - top); }
 
 // fp32 logits: hidden states and weight in fp32 outside autocast, where the reference's
 // products are fp32 GEMMs (fused_linear_ce.py:38,52,57 with w = weight.to(hidden.dtype) at
-// :65) and its chunk math runs on fp32 logits (:39-51). One 256-thread workgroup per row and
-// two reads of it: an online (max, sum of exp) pass, lse = max + log(sum); then (kGrad) the
-// gradient in place, exp(x - lse) on valid rows (0 on ignored rows) minus 1 at the label,
-// with the reference's rounding steps: the fp32 difference x - lse, then a full-precision exp.
-template <bool kGrad>
-__global__ __launch_bounds__(256) void ce_rows_f32_kernel(float* __restrict__ logits, int64_t ld,
-                                                          const int64_t* __restrict__ labels, int64_t vocab,
-                                                          int64_t ignore_index, float* __restrict__ row_loss) {
+// :65) and its chunk math runs on fp32 logits (:39-51): lse = max + log(sum), then (kGrad) the
+// gradient in place, exp(x - lse) on valid rows (0 on ignored rows) minus 1 at the label, with
+// the reference's rounding steps: the fp32 difference x - lse, then a full-precision exp.
+// One workgroup of kCeThreads per row. kCols > 0: the row stays in registers, kCols vectors of 4
+// a thread, all loaded before the first is used and reduced by batches, so it is read once.
+// kCols = 0: longer rows, read by batches and again for the gradient, and rows off 16 bytes,
+// element by element. Bound: HBM, 8 bytes an element (4 for the loss alone). Against 256 threads
+// that read every row twice with an online (max, sum): 1024 x 20,008 52 -> 40 us (4.1 TB/s), the
+// loss alone 30 -> 19; 4096 x 4096 36 -> 27; 256 x 151,936 (too long) 230 -> 96; 1024 x 20,001
+// (off 16 bytes) 90 -> 59.
+template <int kCols, int kCeThreads, bool kGrad>
+__global__ __launch_bounds__(kCeThreads, 4) void ce_rows_f32_kernel(float* __restrict__ logits, int64_t ld,
+                                                                    const int64_t* __restrict__ labels,
+                                                                    int64_t vocab, int64_t ignore_index,
+                                                                    float* __restrict__ row_loss) {
   const int64_t r = blockIdx.x;
   float* row = logits + r * ld;
   const int64_t label = labels[r];
@@ -488,21 +470,65 @@ __global__ __launch_bounds__(256) void ce_rows_f32_kernel(float* __restrict__ lo
   const int64_t nvec = vocab >> 2;  // full 4-element vectors (16 B)
   const bool vec = ((reinterpret_cast<uint64_t>(row) & 15u) == 0);
   const int64_t vend = vec ? nvec * 4 : 0;
+  constexpr int kBatch = kCols > 0 && kCols < 4 ? kCols : 4;
+  f32x4 keep[kCols > 0 ? kCols : kBatch];
   float m = -INFINITY, s = 0.0f;
-  if (vec) {
-    float mm[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY}, ss[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int64_t v = threadIdx.x; v < nvec; v += 256) {
-      const f32x4 x = *reinterpret_cast<const f32x4*>(row + v * 4);
-      ms_add_f(mm[0], ss[0], x.x);
-      ms_add_f(mm[1], ss[1], x.y);
-      ms_add_f(mm[2], ss[2], x.z);
-      ms_add_f(mm[3], ss[3], x.w);
-    }
+  auto load = [&](int64_t v) {  // past the end: the last vector again, skipped in add
+    return *reinterpret_cast<const f32x4*>(row + (v < nvec ? v : nvec - 1) * 4);
+  };
+  auto add = [&](const f32x4* w, int64_t v0) {  // kBatch vectors, the first one v0
+    float top = m;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) ms_merge_f(m, s, mm[j], ss[j]);
+    for (int k = 0; k < kBatch; ++k) top = fmaxf(top, fmaxf(fmaxf(w[k].x, w[k].y), fmaxf(w[k].z, w[k].w)));
+    const float ref = finite_ref(top);
+    s = s * raised(m, top);
+    m = top;
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k)
+      if (v0 + k * kCeThreads < nvec)
+        s += (expf(w[k].x - ref) + expf(w[k].y - ref)) + (expf(w[k].z - ref) + expf(w[k].w - ref));
+  };
+  if (vec && nvec > 0) {
+    if constexpr (kCols > 0) {
+#pragma unroll
+      for (int k = 0; k < kCols; ++k) keep[k] = load(threadIdx.x + static_cast<int64_t>(k) * kCeThreads);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < kCols; k += kBatch) {
+        add(keep + k, threadIdx.x + static_cast<int64_t>(k) * kCeThreads);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      for (int64_t v = threadIdx.x; v < nvec; v += kBatch * kCeThreads) {
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) keep[k] = load(v + k * kCeThreads);
+        add(keep, v);
+      }
+    }
   }
-  for (int64_t i = vend + threadIdx.x; i < vocab; i += 256) ms_add_f(m, s, row[i]);
-  block_ms_f(m, s);
+  for (int64_t i = vend + threadIdx.x; i < vocab; i += kCeThreads) ms_add_f(m, s, row[i]);
+  // The workgroup's (max, sum) in a fixed order, in every thread: the maximum first, so that a
+  // thread's sum is rescaled once a level (4096 x 1024: 15.8 us merging pairs step by step, 11.4 so).
+  constexpr int kCeWaves = kCeThreads / 64;
+  auto join = [&](int lanes) {
+    float top = m;
+#pragma unroll
+    for (int off = lanes / 2; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off, 64));
+    s = s * raised(m, top);
+    m = top;
+#pragma unroll
+    for (int off = lanes / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  };
+  join(64);
+  __shared__ float lm[kCeWaves], ls[kCeWaves];
+  if ((threadIdx.x & 63) == 0) {
+    lm[threadIdx.x >> 6] = m;
+    ls[threadIdx.x >> 6] = s;
+  }
+  __syncthreads();
+  m = lm[threadIdx.x & (kCeWaves - 1)];
+  s = ls[threadIdx.x & (kCeWaves - 1)];
+  join(kCeWaves);
   const float lse = m + logf(s);
   const bool in_range = label >= 0 && label < vocab;
   const float target = (valid && in_range) ? row[label] : 0.0f;
@@ -514,14 +540,23 @@ __global__ __launch_bounds__(256) void ce_rows_f32_kernel(float* __restrict__ lo
     const float p = expf(x - lse);
     return idx == label ? p - 1.0f : p;
   };
+  auto put = [&](const f32x4 x, int64_t v) {
+    const int64_t b = v * 4;
+    const f32x4 g = {g_of(x.x, b), g_of(x.y, b + 1), g_of(x.z, b + 2), g_of(x.w, b + 3)};
+    *reinterpret_cast<f32x4*>(row + b) = g;  // read next by the products
+  };
   if (vec) {
-    for (int64_t v = threadIdx.x; v < nvec; v += 256) {
-      const f32x4 x = *reinterpret_cast<const f32x4*>(row + v * 4);
-      const int64_t b = v * 4;
-      *reinterpret_cast<f32x4*>(row + b) = f32x4{g_of(x.x, b), g_of(x.y, b + 1), g_of(x.z, b + 2), g_of(x.w, b + 3)};
+    if constexpr (kCols > 0) {
+#pragma unroll
+      for (int k = 0; k < kCols; ++k) {
+        const int64_t v = threadIdx.x + static_cast<int64_t>(k) * kCeThreads;
+        if (v < nvec) put(keep[k], v);
+      }
+    } else {
+      for (int64_t v = threadIdx.x; v < nvec; v += kCeThreads) put(*reinterpret_cast<const f32x4*>(row + v * 4), v);
     }
   }
-  for (int64_t i = vend + threadIdx.x; i < vocab; i += 256) row[i] = g_of(row[i], i);
+  for (int64_t i = vend + threadIdx.x; i < vocab; i += kCeThreads) row[i] = g_of(row[i], i);
 }
 
 // Fixed-order sums over rows: loss_sum, n_valid (count of label != ignore), mean. One workgroup,
@@ -606,13 +641,14 @@ __device__ __forceinline__ void st_nt(T* p, T v) {
 // and vectors where the scaling went 2 bytes at a time: 15 us for 8192 x 1024). 512 elements a
 // wave, two groups of 4 a lane, both loaded before either is stored (8192 x 1024: under 6 us).
 // fused_linear_ce.py:117-126: bf16 grad_h *= bf16(g / n_valid), the scale cast to the grad's
-// dtype, then a bf16 multiply. fp32 hidden states (:68,80,120; kWide): the reference's fp32
-// buffer holds the widened bf16 GEMM result (-0 kept) and is scaled in fp32.
+// dtype, then a bf16 multiply. fp32 hidden states under autocast (:68,80,120; wide): the
+// reference's fp32 buffer holds the widened bf16 GEMM result (-0 kept) and is scaled in fp32.
+// Without autocast (single): grad_h is fp32 and scaled in place.
 struct GradH {
   const uint16_t* src;
-  void* dst;  // src itself (bf16), or fp32 when wide
+  void* dst;  // src itself (bf16), or fp32 when wide or single
   int64_t n;
-  bool wide;
+  bool wide, single;
 };
 constexpr int kGradHSlice = 512;
 
@@ -622,6 +658,11 @@ __device__ __forceinline__ void grad_h_slice(const GradH& gh, int64_t start, flo
                    (reinterpret_cast<uint64_t>(gh.dst) & (gh.wide ? 15u : 7u)) == 0;
   const int64_t end = start + kGradHSlice < gh.n ? start + kGradHSlice : gh.n;
   int64_t done = start;
+  if (gh.single) {
+    float* g = static_cast<float*>(gh.dst);
+    for (int64_t i = start + threadIdx.x; i < end; i += 64) g[i] = g[i] * scale;
+    return;
+  }
   if (vec) {
     done = start + ((end - start) & ~int64_t(3));
     const int64_t e0 = start + static_cast<int64_t>(threadIdx.x) * 4, e1 = e0 + 256;
@@ -821,6 +862,13 @@ int ce_rows_launch(uint16_t* d_logits, int64_t ld, const int64_t* d_labels, int6
   return TM_OK;
 }
 
+template <int kCols, int kThreads, bool kGrad>
+void row_f32_launch(float* logits, int64_t ld, const int64_t* labels, int64_t vocab, int64_t ignore_index,
+                    float* row_loss, uint32_t rows, hipStream_t s) {
+  hipLaunchKernelGGL((ce_rows_f32_kernel<kCols, kThreads, kGrad>), dim3(rows), dim3(kThreads), 0, s, logits, ld, labels,
+                     vocab, ignore_index, row_loss);
+}
+
 template <bool kGrad>
 int ce_rows_f32_launch(float* d_logits, int64_t ld, const int64_t* d_labels, int64_t rows, int64_t vocab,
                        int64_t ignore_index, float* d_row_loss, void* stream, const char* who) {
@@ -830,11 +878,31 @@ int ce_rows_f32_launch(float* d_logits, int64_t ld, const int64_t* d_labels, int
   if (rows == 0) return TM_OK;
   if (!d_logits || !d_labels || !d_row_loss) return ce_fail(TM_EINVAL, "%s: null pointer", who);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int64_t max_rows = 0xFFFFFFFFll / 256;  // a launch holds fewer than 2^32 work-items
+  // As many threads as a row takes at 20 vectors each, from 256 on: an fp32 chunk's 1024 rows are
+  // too few for one wave a row (1024 x 5120: 16.8 us with 64 threads, 14.6 with 256).
+  const bool aligned = ld % 4 == 0 && (reinterpret_cast<uintptr_t>(d_logits) & 15u) == 0;
+  const int64_t nvec = vocab >> 2;
+  const int threads = aligned && nvec <= 256 * kRegCols ? 256 : aligned && nvec <= 512 * kRegCols ? 512 : 1024;
+  const int64_t need = (nvec + threads - 1) / threads;
+  const int64_t cols = !aligned || need > kRegCols ? 0 : threads > 256 ? (need <= 12 ? 12 : kRegCols)
+                   : need <= 2 ? (need > 0 ? need : 1) : need <= 12 ? (need + 3) / 4 * 4 : kRegCols;
+  const int64_t max_rows = 0xFFFFFFFFll / threads;  // a launch holds fewer than 2^32 work-items
   for (int64_t r0 = 0; r0 < rows; r0 += max_rows) {
     const uint32_t nr = static_cast<uint32_t>(rows - r0 < max_rows ? rows - r0 : max_rows);
-    hipLaunchKernelGGL((ce_rows_f32_kernel<kGrad>), dim3(nr), dim3(256), 0, s, d_logits + r0 * ld, ld,
-                       d_labels + r0, vocab, ignore_index, d_row_loss + r0);
+    float* lg = d_logits + r0 * ld;
+    const int64_t* lab = d_labels + r0;
+    float* loss = d_row_loss + r0;
+    if (cols == 0) row_f32_launch<0, 1024, kGrad>(lg, ld, lab, vocab, ignore_index, loss, nr, s);
+    else if (threads == 256 && cols == 1) row_f32_launch<1, 256, kGrad>(lg, ld, lab, vocab, ignore_index, loss, nr, s);
+    else if (threads == 256 && cols == 2) row_f32_launch<2, 256, kGrad>(lg, ld, lab, vocab, ignore_index, loss, nr, s);
+    else if (threads == 256 && cols == 8) row_f32_launch<8, 256, kGrad>(lg, ld, lab, vocab, ignore_index, loss, nr, s);
+    else if (threads == 256 && cols == 4) row_f32_launch<4, 256, kGrad>(lg, ld, lab, vocab, ignore_index, loss, nr, s);
+    else if (threads == 256 && cols == 12) row_f32_launch<12, 256, kGrad>(lg, ld, lab, vocab, ignore_index, loss, nr, s);
+    else if (threads == 256) row_f32_launch<kRegCols, 256, kGrad>(lg, ld, lab, vocab, ignore_index, loss, nr, s);
+    else if (threads == 512 && cols == 12) row_f32_launch<12, 512, kGrad>(lg, ld, lab, vocab, ignore_index, loss, nr, s);
+    else if (threads == 512) row_f32_launch<kRegCols, 512, kGrad>(lg, ld, lab, vocab, ignore_index, loss, nr, s);
+    else if (cols == 12) row_f32_launch<12, 1024, kGrad>(lg, ld, lab, vocab, ignore_index, loss, nr, s);
+    else row_f32_launch<kRegCols, 1024, kGrad>(lg, ld, lab, vocab, ignore_index, loss, nr, s);
     if (int rc = ce_check_launch(who)) return rc;
   }
   return TM_OK;
@@ -952,12 +1020,14 @@ int tm_ce_finish(float* d_grad_w, const uint16_t* const* h_chunks, int n_chunks,
   if (nh < 0 || nw < 0 || n_chunks < 0 || n_chunks > kMaxFold)
     return ce_fail(TM_EINVAL, "%s: %d chunks (0 to %d) of %lld elements, grad_h of %lld", who, n_chunks, kMaxFold,
                    (long long)nw, (long long)nh);
+  if (wide < 0 || wide > 2 || (wide == 2 && static_cast<const void*>(d_grad_h) != d_grad_h_out))
+    return ce_fail(TM_EINVAL, "%s: grad_h kind %d (2 is in place)", who, wide);
   if ((nh > 0 && (!d_grad_h || !d_grad_h_out)) || (nw > 0 && !d_grad_w) || !d_grad_out || !d_n_valid)
     return ce_fail(TM_EINVAL, "%s: null pointer", who);
   FoldChunks ch = {};
   if (nw > 0)
     if (int rc = fold_chunks(h_chunks, n_chunks, ch, who)) return rc;
-  return grads_launch(d_grad_w, ch, nw > 0 ? n_chunks : 0, nw, accumulate, GradH{d_grad_h, d_grad_h_out, nh, wide != 0},
+  return grads_launch(d_grad_w, ch, nw > 0 ? n_chunks : 0, nw, accumulate, GradH{d_grad_h, d_grad_h_out, nh, wide == 1, wide == 2},
                       d_grad_out, d_n_valid, stream);
 }
 

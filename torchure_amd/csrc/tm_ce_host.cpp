@@ -167,22 +167,22 @@ py::tuple ce_forward(const at::Tensor& hidden, const at::Tensor& weight, bool ca
 }
 
 // Backward: the waiting chunks added into grad_weight (made here if there is none and want_w) and
-// both gradients scaled by grad_out / n_valid. short_h: the bf16 grad_hidden, or None; wide: the
-// gradient is fp32. Returns (grad_hidden, grad_weight).
-py::tuple ce_backward(const at::Tensor& grad_out, const at::Tensor& out2, const c10::optional<at::Tensor>& short_h,
-                      bool wide, const c10::optional<at::Tensor>& grad_w, const std::vector<at::Tensor>& chunks,
+// both gradients scaled by grad_out / n_valid. held_h: grad_hidden, or None; kind: 0 bf16, 1 bf16
+// whose gradient is fp32, 2 fp32. Returns (grad_hidden, grad_weight).
+py::tuple ce_backward(const at::Tensor& grad_out, const at::Tensor& out2, const c10::optional<at::Tensor>& held_h,
+                      int kind, const c10::optional<at::Tensor>& grad_w, const std::vector<at::Tensor>& chunks,
                       bool accumulated, uintptr_t stream_handle) {
   HANDLE_TH_ERRORS
   const Abi& a = abi();
   at::Tensor g = grad_out.detach().to(at::kFloat).contiguous();
-  at::Tensor gw = grad_w ? *grad_w : at::Tensor(), gh = short_h ? *short_h : at::Tensor();
+  at::Tensor gw = grad_w ? *grad_w : at::Tensor(), gh = held_h ? *held_h : at::Tensor();
   const auto f32 = out2.options();
   if (!gw.defined() && !chunks.empty()) gw = at::empty(chunks[0].sizes(), f32);
-  if (wide && gh.defined()) gh = at::empty(gh.sizes(), f32);
+  if (kind == 1 && gh.defined()) gh = at::empty(gh.sizes(), f32);
   std::vector<const void*> p;
   for (const at::Tensor& t : chunks) p.push_back(ptr(t));
   check(a.finish(ptr(gw), p.data(), static_cast<int>(p.size()), gw.defined() ? gw.numel() : 0, accumulated,
-                 short_h ? ptr(*short_h) : nullptr, ptr(gh), gh.defined() ? gh.numel() : 0, wide, ptr(g),
+                 held_h ? ptr(*held_h) : nullptr, ptr(gh), gh.defined() ? gh.numel() : 0, kind, ptr(g),
                  out2.data_ptr<float>() + 1, reinterpret_cast<void*>(stream_handle)),
         "tm_ce_finish");
   return py::make_tuple(or_none(gh), or_none(gw));

@@ -46,8 +46,8 @@ reference's buffers take fp32 (:65,68) and autocast runs the products on bf16 ca
 hidden is cast to bf16 once (RNE, as autocast does), grad_hidden stays a bf16 GEMM output
 until backward, and tm_ce_finish writes the fp32 gradient float(gh) * grad_out / n_valid
 (the reference's fp32 copy and mul_, :80,120). fp32 hidden states outside autocast take the
-reference's fp32 path: fp32 GEMMs on weight.to(fp32), tm_ce_rows_f32 on fp32 logits, and the
-reference's fp32 `+=` and `mul_` for grad_W.
+reference's fp32 path: fp32 GEMMs on weight.to(fp32), tm_ce_rows_f32 on fp32 logits, grad_W
+summed in fp32 by the product, and tm_ce_finish for the scaling of both.
 
 Chunking: 1024 rows by default, the reference's default (:131). ``chunk_size=None`` or
 ``"auto"`` opts into MI355X sizing: chunks whose bf16 logits take up to 4 GiB, so that
@@ -175,11 +175,11 @@ def _checked(hidden, weight, labels, chunk_size):
     return n, v, chunk, mode
 
 
-def _bf16(logits: torch.Tensor, dtype=torch.bfloat16) -> torch.Tensor:
-    """The row kernels read bf16 bits (fp32 on the fp32 path): refuse anything else loudly."""
-    if logits.dtype != dtype or not logits.is_contiguous():
+def _bf16(logits: torch.Tensor) -> torch.Tensor:
+    """The row kernel reads bf16 bits: refuse anything else loudly."""
+    if logits.dtype != torch.bfloat16 or not logits.is_contiguous():
         raise RuntimeError(f"fused_linear_cross_entropy: the logits GEMM returned {logits.dtype} "
-                           f"(contiguous: {logits.is_contiguous()}), the row kernels need contiguous {dtype}")
+                           f"(contiguous: {logits.is_contiguous()}), the row kernels need contiguous bfloat16")
     return logits
 
 
@@ -403,57 +403,61 @@ def _loss_only(hidden, weight, labels, ignore_index, chunk_size):
     bits, without the two gradient GEMMs or the gradient write. The reference's forward
     computes and drops the gradients in this case (fused_linear_ce.py:63-93)."""
     n, v, chunk, mode = _checked(hidden, weight, labels, chunk_size)
-    if mode != "fp32":
-        done = _run_chunks(hidden, weight, labels, ignore_index, chunk, mode, False, False, False)
-        if done is not None:
-            return done[0]
+    if mode == "fp32":
+        return _fp32_chunks(hidden, weight, labels, ignore_index, n, v, chunk, False, False, False)[0]
+    done = _run_chunks(hidden, weight, labels, ignore_index, chunk, mode, False, False, False)
+    if done is not None:
+        return done[0]
     lib = _native.lib()
     stream = _native.stream_handle(hidden.device)
-    dt = torch.float32 if mode == "fp32" else torch.bfloat16
-    if mode == "fp32":
-        hb, w = hidden, weight.to(dt).contiguous()
-    else:
-        hb, w = _bf16_operands(hidden, weight, mode)
-    rows_loss = lib.tm_ce_rows_loss_f32 if mode == "fp32" else lib.tm_ce_rows_loss_bf16
+    hb, w = _bf16_operands(hidden, weight, mode)
     row_loss = torch.empty(n, dtype=torch.float32, device=hidden.device)
     for s in range(0, n, chunk):
         e = min(s + chunk, n)
-        logits = _logits(hb[s:e], w, lib, stream) if dt == torch.bfloat16 else _bf16(torch.matmul(hb[s:e], w.t()), dt)
-        _native.check(rows_loss(logits.data_ptr(), v, labels[s:e].data_ptr(), e - s, v, int(ignore_index),
-                                row_loss[s:].data_ptr(), stream), "tm_ce_rows_loss")
+        logits = _logits(hb[s:e], w, lib, stream)
+        _native.check(lib.tm_ce_rows_loss_bf16(logits.data_ptr(), v, labels[s:e].data_ptr(), e - s, v,
+                                               int(ignore_index), row_loss[s:].data_ptr(), stream),
+                      "tm_ce_rows_loss_bf16")
         del logits
     return _mean_loss(row_loss, labels, n, ignore_index, lib, stream)[0]
 
 
-def _fp32_forward(ctx, hidden, weight, labels, ignore_index, n, v, chunk):
+def _fp32_chunks(hidden, weight, labels, ignore_index, n, v, chunk, grad, want_h, want_w):
     """fp32 hidden states outside autocast. The reference then casts the weight to fp32 once
     (fused_linear_ce.py:65), its three products are fp32 GEMMs and its buffers are fp32
-    (:66-72). This path does the same: per chunk, fp32 logits from torch.matmul, tm_ce_rows_f32
-    in place (the chunk math of :39-51 on fp32 logits), grad_h = grad_logits @ w into the fp32
-    grad_hidden (:52,79), and grad_weight += grad_logits^T @ h into a zero-filled fp32 buffer
-    (:57,80-81), the reference's own fp32 `+=`. Backward scales both in place."""
+    (:66-72). This loop does the same: per chunk, fp32 logits from the library product, their
+    rows a multiple of 32 elements apart, tm_ce_rows_f32 in place (the chunk math of :39-51 on
+    fp32 logits), grad_h = grad_logits @ w into the fp32 grad_hidden (:52,79), and
+    grad_logits^T @ h into the fp32 grad_weight (:57,80-81): the first chunk's product is
+    written there, the later ones are added by the product (a zero fill and an fp32 `+=` would
+    pass over it three times more a chunk). Backward scales both in place. Returns what
+    ``_run_chunks`` does."""
     lib = _native.lib()
     stream = _native.stream_handle(hidden.device)
     w = weight.to(torch.float32).contiguous()
-    want_h, want_w = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
+    ld = -(-v // 32) * 32
     grad_hidden = torch.empty(hidden.shape, dtype=torch.float32, device=hidden.device) if want_h else None
-    grad_weight = torch.zeros(weight.shape, dtype=torch.float32, device=weight.device) if want_w else None
+    grad_weight = None
+    if want_w:
+        grad_weight = (torch.empty if n else torch.zeros)(weight.shape, dtype=torch.float32, device=weight.device)
     row_loss = torch.empty(n, dtype=torch.float32, device=hidden.device)
+    rows_of = lib.tm_ce_rows_f32 if grad else lib.tm_ce_rows_loss_f32
     for s in range(0, n, chunk):
         e = min(s + chunk, n)
         h = hidden[s:e]
-        logits = _bf16(torch.matmul(h, w.t()), torch.float32)  # (C, V) fp32
-        _native.check(lib.tm_ce_rows_f32(logits.data_ptr(), v, labels[s:e].data_ptr(), e - s, v,
-                                         int(ignore_index), row_loss[s:].data_ptr(), stream), "tm_ce_rows_f32")
+        logits = torch.empty((e - s, ld), dtype=torch.float32, device=hidden.device)[:, :v]
+        torch.mm(h, w.t(), out=logits)
+        _native.check(rows_of(logits.data_ptr(), ld, labels[s:e].data_ptr(), e - s, v, int(ignore_index),
+                              row_loss[s:].data_ptr(), stream), "tm_ce_rows_f32")
         if want_h:
-            torch.matmul(logits, w, out=grad_hidden[s:e])
-        if want_w:
-            grad_weight += torch.matmul(logits.t(), h)
+            torch.mm(logits, w, out=grad_hidden[s:e])
+        if want_w and s == 0:
+            torch.mm(logits.t(), h, out=grad_weight)
+        elif want_w:
+            grad_weight.addmm_(logits.t(), h)
         del logits
     loss, out2 = _mean_loss(row_loss, labels, n, ignore_index, lib, stream)
-    ctx.stash = (out2, grad_hidden, grad_weight, [], False)
-    ctx.fp32_path = True
-    return loss
+    return loss, out2, grad_hidden, grad_weight, [], True
 
 
 def _chunks_unpadded(hidden, weight, labels, ignore_index, n, v, chunk, mode, want_h, want_w):
@@ -496,16 +500,17 @@ class _FusedLinearCE(torch.autograd.Function):
     @staticmethod
     def forward(ctx, hidden, weight, labels, ignore_index, chunk_size):
         n, v, chunk, mode = _checked(hidden, weight, labels, chunk_size)
-        if mode == "fp32":
-            return _fp32_forward(ctx, hidden, weight, labels, ignore_index, n, v, chunk)
-        ctx.fp32_path = False
-        ctx.wide = mode == "autocast"  # fp32 hidden states: grad_h is widened in backward
-        ctx.want_w = ctx.needs_input_grad[1]
+        want_h, want_w = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
+        # grad_hidden as held for backward: bf16, bf16 that becomes fp32, or fp32
+        ctx.kind = {"bf16": 0, "autocast": 1, "fp32": 2}[mode]
+        ctx.want_w = want_w
         ctx.weight_meta = (weight.shape, weight.device)
-        done = _run_chunks(hidden, weight, labels, ignore_index, chunk, mode, True, ctx.needs_input_grad[0],
-                           ctx.needs_input_grad[1])
-        if done is None:
-            done = _chunks_unpadded(hidden, weight, labels, ignore_index, n, v, chunk, mode, *ctx.needs_input_grad[:2])
+        if mode == "fp32":
+            done = _fp32_chunks(hidden, weight, labels, ignore_index, n, v, chunk, True, want_h, want_w)
+        else:
+            done = _run_chunks(hidden, weight, labels, ignore_index, chunk, mode, True, want_h, want_w)
+            if done is None:
+                done = _chunks_unpadded(hidden, weight, labels, ignore_index, n, v, chunk, mode, want_h, want_w)
         # what backward needs, consumed by it
         ctx.stash = done[1:]
         return done[0]
@@ -518,21 +523,15 @@ class _FusedLinearCE(torch.autograd.Function):
                 "consumed in place on the first call, so retain_graph does not work through this op")
         out2, grad_hidden, grad_weight, chunks, accumulated = ctx.stash
         ctx.stash = None
-        if ctx.fp32_path:
-            # fused_linear_ce.py:107-126: scale = grad_out / n_valid, both buffers scaled in place
-            scale = grad_out.detach().to(torch.float32) / out2[1]
-            if grad_hidden is not None:
-                grad_hidden.mul_(scale)
-            if grad_weight is not None:
-                grad_weight.mul_(scale)
-            return grad_hidden, grad_weight, None, None, None
-        if ctx.want_w and not chunks:  # no rows at all: the reference scales its zero-filled buffer
+        if ctx.want_w and not chunks and grad_weight is None:
+            # no rows at all: the reference scales its zero-filled buffer
             shape, device = ctx.weight_meta
             grad_weight, accumulated = torch.zeros(shape, dtype=torch.float32, device=device), True
-        # the chunks still waiting (at most FOLD_CHUNKS) added into grad_W with the scaling, and
-        # grad_h scaled (fp32 hidden: float(bf16 GEMM result) * scale), in one launch
+        # fused_linear_ce.py:107-126: the chunks still waiting (at most FOLD_CHUNKS) added into grad_W
+        # with the scaling, and grad_h scaled (under autocast float(bf16 GEMM result) * scale), in one
+        # launch
         grad_hidden, grad_weight = _native.ce_host().ce_backward(
-            grad_out, out2, grad_hidden, ctx.wide, grad_weight, chunks, accumulated,
+            grad_out, out2, grad_hidden, ctx.kind, grad_weight, chunks, accumulated,
             _native.stream_handle(out2.device))
         return grad_hidden, grad_weight, None, None, None
 
