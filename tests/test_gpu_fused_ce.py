@@ -1211,5 +1211,62 @@ def test_operands_the_native_loop_does_not_read_as_they_are():
             else:  # library products: the last bit of some bf16 results
                 torch.testing.assert_close(x.float(), y.float(), rtol=2.0 ** -7, atol=2.0 ** -16)
     with pytest.raises(_native.NativeError, match="tm_ce_logits_ld_bf16"):
-        _native.ce_host().ce_forward(hidden, weight, False, False, labels, -100, 128, (128, 128), 64, (False, False),
+        _native.ce_host().ce_forward(hidden, weight, False, False, labels, -100, 128, 1, (128, 128), 64, (False, False),
                                      True, True, True, 8, 1 << 30, _native.stream_handle(DEV))
+
+
+def _same_bits(a, b):
+    for x, y in zip([*a[:4], *a[4]], [*b[:4], *b[4]]):
+        assert (x is None) == (y is None)
+        kind = None if x is None else torch.int32 if x.dtype == torch.float32 else torch.int16
+        assert x is None or torch.equal(x.view(kind), y.view(kind))
+
+
+@pytest.mark.parametrize("n,d,v,chunk", [
+    (2500, 192, 4001, 1024),  # one group, a ragged last chunk and vocabulary
+    (1300, 128, 1000, 128),   # 11 chunks (a fold among them), the last of 20 rows
+    (17000, 64, 300, 1024),   # more rows than a group takes: two groups
+    (900, 128, 1000, 200),    # chunks with padding of their own run one by one
+])
+def test_logits_of_several_chunks_together_keep_the_bits(monkeypatch, n, d, v, chunk):
+    """The logits and the row pass of several chunks as one launch each, against chunk by chunk."""
+    from torchure_amd.loss import fused_linear_ce as fce
+
+    g = torch.Generator(device=DEV).manual_seed(n)
+    hidden = torch.randn(n, d, device=DEV, generator=g)
+    weight = torch.randn(v, d, device=DEV, generator=g) * 0.05
+    labels = torch.randint(0, v, (n,), device=DEV, generator=g)
+    labels[::9] = -100
+
+    def run():
+        return [fce._run_chunks(hidden, weight, labels, -100, chunk, "autocast", grad, grad, grad) for grad in (True, False)]
+
+    together = run()
+    assert fce.group_chunks(n, chunk, v, True) == (1 if chunk == 200 else min(-(-n // chunk), 9 if n == 17000 else 99))
+    monkeypatch.setattr(fce, "GROUP_BYTES", 0)
+    for a, b in zip(together, run()):
+        _same_bits(a, b)
+
+
+def test_logits_of_several_chunks_run_one_by_one_where_memory_is_short():
+    """A call that fits with one chunk's logits still does: a group whose logits cannot be had is
+    run chunk by chunk, with the same bits. The limit is the process's own, set on the allocator."""
+    from torchure_amd.loss import fused_linear_ce as fce
+
+    n, d, v, chunk = 8192, 64, 16384, 1024  # 32 MiB of logits a chunk, 256 MiB together
+    hidden = torch.randn(n, d, device=DEV).to(torch.bfloat16)
+    weight = (torch.randn(v, d, device=DEV) * 0.05).to(torch.bfloat16)
+    labels = torch.randint(0, v, (n,), device=DEV)
+    assert fce.group_chunks(n, chunk, v, True) == 8
+    want = fce._run_chunks(hidden, weight, labels, -100, chunk, "bf16", True, True, True)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(DEV).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(DEV) + (200 << 20)) / total, DEV)
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(256 << 20, dtype=torch.uint8, device=DEV)
+        got = fce._run_chunks(hidden, weight, labels, -100, chunk, "bf16", True, True, True)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, DEV)
+    _same_bits(got, want)

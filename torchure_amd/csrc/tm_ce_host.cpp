@@ -87,12 +87,14 @@ py::object or_none(const at::Tensor& t) { return t.defined() ? py::cast(t) : py:
 
 // The chunks of one call. hidden (n x d) and weight (v x d) are contiguous, bf16 or (cast_h,
 // cast_w) fp32; the chunks have `chunk` rows, the last one the rest, and their logits
-// pad[0] x ld (the last one's pad[1] x ld). own_h[i]: grad_h on the split-K kernel, else the
+// pad[0] x ld (the last one's pad[1] x ld). The logits and their row pass run over `group` chunks
+// at a time, in one buffer (group > 1 only where a chunk has no padding rows of its own); where
+// memory for that is short, chunk by chunk. own_h[i]: grad_h on the split-K kernel, else the
 // library's product. grad = false: the loss alone.
 // Returns (loss, (loss sum, n_valid), grad_hidden, grad_weight, chunks' grad_W still to be added
 // (the last one at the end), whether grad_weight holds earlier chunks).
 py::tuple ce_forward(const at::Tensor& hidden, const at::Tensor& weight, bool cast_h, bool cast_w,
-                     const at::Tensor& labels, i64 ignore, i64 chunk, std::pair<i64, i64> pad, i64 ld,
+                     const at::Tensor& labels, i64 ignore, i64 chunk, i64 group, std::pair<i64, i64> pad, i64 ld,
                      std::pair<bool, bool> own_h, bool grad, bool want_h, bool want_w, i64 fold_chunks, i64 fold_bytes,
                      uintptr_t stream_handle) {
   HANDLE_TH_ERRORS
@@ -122,19 +124,35 @@ py::tuple ce_forward(const at::Tensor& hidden, const at::Tensor& weight, bool ca
   if (bytes) ws = at::empty({static_cast<i64>(bytes)}, f32.dtype(at::kByte));
   std::vector<at::Tensor> pending;
   bool accumulated = false;
+  at::Tensor held;  // the group's logits
+  i64 first = 0, until = 0;  // and its rows
   for (i64 s = 0; s < n; s += chunk) {
     const bool is_last = s + chunk >= n;
     const i64 rows = is_last ? last : chunk, pad_rows = grad ? (is_last ? pad.second : pad.first) : rows;
-    at::Tensor logits = at::empty({pad_rows, ld}, bf16);
     const char* hs = ptr(h) + s * d * 2;
-    const i64* lab = labels.data_ptr<i64>() + s;
-    float* losses = row_loss.data_ptr<float>() + s;
-    check(a.logits(ptr(logits), ld, hs, ptr(w), rows, v, d, stream), "tm_ce_logits_ld_bf16");
-    if (!grad) {
-      check(a.rows_loss(ptr(logits), ld, lab, rows, v, ignore, losses, stream), "tm_ce_rows_loss_bf16");
-      continue;
+    if (s >= until) {
+      held = at::Tensor();
+      first = s;
+      until = std::min(n, s + group * chunk);
+      const i64 over = until == n ? (grad ? pad.second - last : 0) : pad_rows - rows;
+      try {
+        held = at::empty({until - s + over, ld}, bf16);
+      } catch (const c10::OutOfMemoryError&) {
+        if (group == 1) throw;
+        group = 1;
+        until = std::min(n, s + chunk);
+        held = at::empty({pad_rows, ld}, bf16);
+      }
+      const i64* lab = labels.data_ptr<i64>() + s;
+      float* losses = row_loss.data_ptr<float>() + s;
+      check(a.logits(ptr(held), ld, hs, ptr(w), until - s, v, d, stream), "tm_ce_logits_ld_bf16");
+      if (grad)
+        check(a.rows(ptr(held), ld, lab, until - s, held.size(0), v, ignore, losses, stream), "tm_ce_rows_padded_bf16");
+      else
+        check(a.rows_loss(ptr(held), ld, lab, until - s, v, ignore, losses, stream), "tm_ce_rows_loss_bf16");
     }
-    check(a.rows(ptr(logits), ld, lab, rows, pad_rows, v, ignore, losses, stream), "tm_ce_rows_padded_bf16");
+    if (!grad) continue;
+    const at::Tensor logits = held.narrow(0, s - first, pad_rows);
     if (want_h) {
       if (is_last ? own_h.second : own_h.first) {
         check(a.grad_h(ptr(grad_hidden) + s * d * 2, ptr(logits), ld, ptr(w), rows, v, d, ptr(ws), bytes, stream),
@@ -148,12 +166,12 @@ py::tuple ce_forward(const at::Tensor& hidden, const at::Tensor& weight, bool ca
       at::Tensor gw = at::empty({v, d}, bf16);
       check(a.grad_w(ptr(gw), ptr(logits), ld, pad_rows, hs, rows, v, d, ptr(ws), bytes, stream), "tm_ce_grad_w_ld_bf16");
       pending.push_back(gw);
-      const i64 held = static_cast<i64>(pending.size());
-      if (!is_last && (held == fold_chunks || held * v * d * 2 >= fold_bytes)) {
+      const i64 waiting = static_cast<i64>(pending.size());
+      if (!is_last && (waiting == fold_chunks || waiting * v * d * 2 >= fold_bytes)) {
         if (!grad_weight.defined()) grad_weight = at::empty({v, d}, f32);
         std::vector<const void*> p;
         for (const at::Tensor& t : pending) p.push_back(ptr(t));
-        check(a.fold(ptr(grad_weight), p.data(), static_cast<int>(held), v * d, accumulated, nullptr, nullptr, stream),
+        check(a.fold(ptr(grad_weight), p.data(), static_cast<int>(waiting), v * d, accumulated, nullptr, nullptr, stream),
               "tm_ce_grad_w_fold");
         accumulated = true;
         pending.clear();

@@ -21,7 +21,7 @@ The chunk's logits are padded to whole MFMA steps: rows a multiple of 64 element
 apart and their number a multiple of 64 or 128 (padded_rows), the padding zero once they are gradients. An odd
 vocabulary then keeps its rows 16-byte aligned, and any number of tokens is a whole number of
 K slices for grad_W.
-then tm_ce_loss sums the per-row losses in a fixed order (deterministic).
+then tm_ce_mean_loss sums the per-row losses in a fixed order (deterministic).
 
 The last chunk's bf16 grad_W is not added in forward: it waits for backward, where
 tm_ce_finish adds it and applies grad_out / n_valid in the same pass. With a single
@@ -298,6 +298,26 @@ def grad_h_gemm_fits(rows: int, dim: int, vocab: int) -> bool:
 
 RAGGED_GRAD_H_MIN_VOCAB = 4097
 
+GROUP_BYTES = 1 << 30  # logits of the chunks whose logits and row pass run together, at most
+GROUP_ROWS = 16384  # and their rows
+
+
+def group_chunks(rows: int, chunk: int, vocab: int, grad: bool) -> int:
+    """Chunks whose logits GEMM and row pass run as one launch each. Both work row by row, so the
+    chunking fixes none of their bits (as it does grad_W's, which stay per chunk), and more rows
+    fill the last round of tiles better: a 1024-row chunk of the Qwen3-0.6B head has 9.3 rounds of
+    256 x 256 tiles and takes 10, three together 27.8 (8192 rows: 8709 -> 8374 us a call; 2500 x
+    768 x 32,001: 610 -> 578). Chunks with padding rows of their own (not a
+    multiple of 128) are not contiguous in K and run one by one. Bounded by GROUP_BYTES (0.4% of
+    the GPU's memory; a caller's larger chunk is taken as it is), and by rows, so that the hidden
+    states keep 32-bit offsets."""
+    most = min(GROUP_BYTES // (2 * chunk * padded_vocab(vocab)), GROUP_ROWS // chunk)
+    if rows <= chunk or most <= 1 or (grad and padded_rows(chunk) != chunk):
+        return 1
+    chunks = -(-rows // chunk)
+    return -(-chunks // -(-chunks // most))  # groups of about the same size
+
+
 FOLD_CHUNKS = 8  # chunks per grad_W fold (tm_ce_grad_w_fold takes at most 8)
 FOLD_BYTES = 4 << 30  # bf16 chunk grad_W held before a fold, at most
 
@@ -387,8 +407,8 @@ def _run_chunks(hidden, weight, labels, ignore_index, chunk, mode, grad, want_h,
     chunk = min(chunk, n)
     last = n - (n - 1) // chunk * chunk
     return _native.ce_host().ce_forward(
-        h, w, cast_h, cast_w, labels, int(ignore_index), chunk, (padded_rows(chunk), padded_rows(last)),
-        padded_vocab(v), (grad_h_gemm_fits(chunk, d, v), grad_h_gemm_fits(last, d, v)), grad, want_h, want_w,
+        h, w, cast_h, cast_w, labels, int(ignore_index), chunk, group_chunks(n, chunk, v, grad),
+        (padded_rows(chunk), padded_rows(last)), padded_vocab(v), (grad_h_gemm_fits(chunk, d, v), grad_h_gemm_fits(last, d, v)), grad, want_h, want_w,
         FOLD_CHUNKS, FOLD_BYTES, _native.stream_handle(hidden.device))
 
 
