@@ -20,7 +20,8 @@ Per chunk of rows:
 The chunk's logits are padded to whole MFMA steps: rows a multiple of 64 elements (padded_vocab)
 apart and their number a multiple of 64 or 128 (padded_rows), the padding zero once they are gradients. An odd
 vocabulary then keeps its rows 16-byte aligned, and any number of tokens is a whole number of
-K slices for grad_W.
+K slices for grad_W. The logits and the row kernel run over several chunks at a time
+(group_chunks), the gradients chunk by chunk;
 then tm_ce_mean_loss sums the per-row losses in a fixed order (deterministic).
 
 The last chunk's bf16 grad_W is not added in forward: it waits for backward, where
