@@ -149,16 +149,15 @@ py::tuple grad_fields(const py::list& ts) {
   return py::make_tuple(ptr, numel, code);
 }
 
-// True if, for every i, state_map[params[i]] is states[i] and that dict's "exp_avg",
-// "exp_avg_sq" and "step" entries are ms[i], vs[i] and ss[i] (object identity). A missing
-// entry is a mismatch: the lookup does not run a defaultdict's factory.
+// Lookup that does not run a defaultdict's factory: a missing entry is a mismatch below.
 PyObject* dict_item(PyObject* d, PyObject* k) {  // borrowed, or nullptr if absent
   PyObject* r = PyDict_GetItemWithError(d, k);
   if (!r && PyErr_Occurred()) throw py::error_already_set();
   return r;
 }
 
-// The entries' part of it: states[i] is a dict whose "exp_avg", "exp_avg_sq" and "step" are these.
+// True if every states[i] is a dict whose "exp_avg", "exp_avg_sq" and "step" entries are ms[i],
+// vs[i] and ss[i] (object identity).
 bool entries_same(const py::list& states, const py::list& ms, const py::list& vs, const py::list& ss) {
   const Py_ssize_t n = PyList_GET_SIZE(states.ptr());
   for (const py::list* l : {&ms, &vs, &ss})
@@ -175,6 +174,7 @@ bool entries_same(const py::list& states, const py::list& ms, const py::list& vs
   return true;
 }
 
+// The same, and state_map[params[i]] is states[i] for every i.
 bool states_same(const py::dict& state_map, const py::list& params, const py::list& states,
                  const py::list& ms, const py::list& vs, const py::list& ss) {
   const Py_ssize_t n = PyList_GET_SIZE(params.ptr());
@@ -355,7 +355,8 @@ py::object plan_match(const py::list& all_params, const py::list& all_works, con
                       const py::list& wworks) {
   const Py_ssize_t n = PyList_GET_SIZE(all_params.ptr());
   const char* want = PyBytes_AS_STRING(src.ptr());
-  if (PyBytes_GET_SIZE(src.ptr()) != n || !attrs_same(all_params, py::reinterpret_borrow<py::str>(working_name()), all_works))
+  if (PyBytes_GET_SIZE(src.ptr()) != n ||
+      !attrs_same(all_params, py::reinterpret_borrow<py::str>(working_name()), all_works))
     return py::none();
   py::list out;
   std::vector<uint64_t> at_ptr;
@@ -436,7 +437,8 @@ py::object accumulate_scan(const py::list& params, bool last, int64_t assign_fla
     if (w && !w->grad().defined()) w = nullptr;
     const at::Tensor& g = p->grad();
     if (!w && (!last || !g.defined())) continue;
-    if (!dense(*p) || (g.defined() ? g : *p).scalar_type() != at::kFloat || (g.defined() && !dense(g))) return py::none();
+    if (!dense(*p) || (g.defined() ? g : *p).scalar_type() != at::kFloat || (g.defined() && !dense(g)))
+      return py::none();
     if (w) {
       const at::Tensor& m = w->grad();
       if (!dense(m) || m.scalar_type() != at::kBFloat16 || m.numel() != p->numel() || m.device() != p->device())

@@ -409,7 +409,8 @@ def _run_chunks(hidden, weight, labels, ignore_index, chunk, mode, grad, want_h,
     last = n - (n - 1) // chunk * chunk
     return _native.ce_host().ce_forward(
         h, w, cast_h, cast_w, labels, int(ignore_index), chunk, group_chunks(n, chunk, v, grad),
-        (padded_rows(chunk), padded_rows(last)), padded_vocab(v), (grad_h_gemm_fits(chunk, d, v), grad_h_gemm_fits(last, d, v)), grad, want_h, want_w,
+        (padded_rows(chunk), padded_rows(last)), padded_vocab(v),
+        (grad_h_gemm_fits(chunk, d, v), grad_h_gemm_fits(last, d, v)), grad, want_h, want_w,
         FOLD_CHUNKS, FOLD_BYTES, _native.stream_handle(hidden.device))
 
 

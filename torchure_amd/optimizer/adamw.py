@@ -586,8 +586,8 @@ class _Plan:
     """The table of the last full step and what it was built from, for the fast path."""
 
     __slots__ = ("groups", "all_params", "all_works", "src", "params", "statics", "static_ptrs",
-                 "states", "state_keys", "state_values", "ms", "vs", "ss", "wparams", "wworks", "rows", "clip_rows", "n", "device",
-                 "chunks", "n_chunks", "chunk_elems", "written", "clip_holders", "clip_perm")
+                 "states", "state_keys", "state_values", "ms", "vs", "ss", "wparams", "wworks", "rows",
+                 "clip_rows", "n", "device", "chunks", "n_chunks", "chunk_elems", "written", "clip_holders", "clip_perm")
 
     def __init__(self, opt: "AdamW", order: list, launch: "StepLaunch"):
         host = _native.host()
