@@ -776,6 +776,28 @@ def test_cached_norm_invalidated_by_inplace_change():
     assert abs(n2 - want) <= 1e-6 * want and abs(n2 - n1) > 1e-3 * n1
 
 
+def test_accumulate_a_param_that_stands_in_the_list_twice():
+    """A repeated param takes each micro-step's grad once (the first assigns it), exactly, and
+    counts twice in the norm, as clip_grad_norm counts it over the same list."""
+    import torchure_amd as ta
+    from torchure_amd.optimizer.working import accumulate_grads_
+
+    g = torch.Generator(device=DEV).manual_seed(31)
+    p, q = (torch.nn.Parameter(torch.randn(n, device=DEV, generator=g)) for n in (70_001, 300))
+    ta.attach_bf16_working_params([p, q])
+    want = {}
+    for last in (False, False, True):
+        for t in (p, q):
+            t._tm_working.grad = torch.randn(t.shape, device=DEV, generator=g).to(torch.bfloat16)
+            want[t] = t._tm_working.grad.float() + want.get(t, 0.0)
+        norm = accumulate_grads_([p, q, p], last=last)
+        for t in (p, q):
+            assert torch.equal(t.grad, want[t]) and t._tm_working.grad is None
+    assert torch.equal(norm, ta.clip_grad_norm([p, q, p], None, None))
+    exact = (2 * want[p].double().square().sum() + want[q].double().square().sum()).sqrt()
+    assert abs(norm.double() - exact) <= 1e-6 * exact
+
+
 def test_accumulate_rejects_before_touching_any_grad():
     """A bad entry anywhere in the list raises before any p.grad is created or written,
     so the params ahead of it keep their grads (here: none, and one existing)."""

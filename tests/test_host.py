@@ -765,3 +765,40 @@ def test_host_clip_match():
     assert h.clip_match(rec, perm, [gs[0].clone(), gs[1], gs[2]], total) == 0
     gs[1].mul_(2)
     assert h.clip_match(rec, perm, gs, total) == 2
+
+
+def test_host_accumulate_scan_refuses_a_repeated_param():
+    """A param that stands twice in the list, its working copy carrying a grad: the scan hands out
+    no table (two rows of one launch would write one accumulator) and leaves p.grad as it was, with
+    and without an accumulator at hand; other lists give one row per param. The params are fake
+    tensors of a GPU device: no memory and no GPU behind them."""
+    import warnings
+
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from torchure_amd import _native
+
+    h = _host()
+    with FakeTensorMode(), warnings.catch_warnings():
+        warnings.simplefilter("ignore")  # the table holds the fake pointers
+
+        def param(n):
+            p = torch.nn.Parameter(torch.empty(n, device="cuda"))
+            p._tm_working = torch.empty(n, device="cuda", dtype=torch.bfloat16)
+            p._tm_working.grad = torch.empty(n, device="cuda", dtype=torch.bfloat16)
+            return p
+
+        def scan(params, last=False):
+            return h.accumulate_scan(params, last, _native.TM_ACCUM_ASSIGN)
+
+        p, q = param(8), param(16)
+        for params in ([p, p], [p, q, p], [q, q, p]):
+            assert scan(params) is None and scan(params, True) is None
+            assert p.grad is None and q.grad is None
+        accs, _, rows, numels, _, _ = scan([p, q])
+        assert numels.tolist() == [8, 16] and accs[0] is p.grad and accs[1] is q.grad
+        table = rows.view(_native.ACCUM_DTYPE)
+        assert table["flags"].tolist() == [_native.TM_ACCUM_ASSIGN] * 2
+        assert scan([p, q, p]) is None
+        q._tm_working.grad = None  # q is only measured, and may be measured twice
+        assert scan([q, p, q], True)[3].tolist() == [16, 8, 16]

@@ -418,7 +418,8 @@ static_assert(sizeof(AccumRow) == 32, "tm_accum_t is 32 bytes");
 // its working copy's grad, then, only if all are usable, gives first micro-steps their
 // accumulator (unfilled: the kernel assigns it). Returns (accumulators, those with a micro grad,
 // rows, numels, the working copies' grads, device index), or None when the caller's checks should
-// report why not (or there is nothing to do).
+// report why not (or there is nothing to do). None too where a param with a micro grad stands in
+// the list more than once: its rows would write one accumulator from several workgroups of a launch.
 py::object accumulate_scan(const py::list& params, bool last, int64_t assign_flag) {
   const Py_ssize_t n = PyList_GET_SIZE(params.ptr());
   struct Item {
@@ -426,6 +427,7 @@ py::object accumulate_scan(const py::list& params, bool last, int64_t assign_fla
   };
   std::vector<Item> todo;
   std::vector<py::object> keep;  // the working copies, alive while their pointers are used
+  std::vector<const void*> written;  // the params whose accumulator the launch writes
   c10::Device first(c10::kCPU);
   auto dense = [](const at::Tensor& t) { return t.layout() == at::kStrided && t.is_cuda() && t.is_contiguous(); };
   for (Py_ssize_t i = 0; i < n; ++i) {
@@ -448,8 +450,11 @@ py::object accumulate_scan(const py::list& params, bool last, int64_t assign_fla
     if (p->device() != first) return py::none();
     todo.push_back({p, w});
     keep.push_back(wo);
+    if (w) written.push_back(p->unsafeGetTensorImpl());
   }
   if (todo.empty()) return py::none();
+  std::sort(written.begin(), written.end());
+  if (std::adjacent_find(written.begin(), written.end()) != written.end()) return py::none();
   const py::ssize_t k = static_cast<py::ssize_t>(todo.size());
   py::array_t<uint8_t> rows(k * static_cast<py::ssize_t>(sizeof(AccumRow)));
   py::array_t<int64_t> numels(k);

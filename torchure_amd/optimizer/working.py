@@ -18,6 +18,7 @@ import torch
 
 from torchure_amd import _native
 from torchure_amd.core import tables
+from torchure_amd.core.grad_helper import grad_norm_launch
 
 _ALIGN_ELEMS = 8  # 16 bytes of bf16
 
@@ -170,10 +171,19 @@ def accumulate_grads_(params, *, last: bool = False,
     accumulated fp32 grads of all ``params`` (returned as a 0-d fp32 device tensor).
     A following ``clip_grad_norm`` over the same params reuses it instead of reading
     every grad again; the value is bit-identical to what it would compute.
+
+    A param that stands in the list several times takes its micro-step grad once, and counts
+    in the norm as often as it stands there, as ``clip_grad_norm`` counts it.
     """
     params = list(params)
     scan = _native.host().accumulate_scan(params, last, _native.TM_ACCUM_ASSIGN)
     if scan is None:
+        once = list(dict.fromkeys(params))
+        if len(once) != len(params):
+            norm = accumulate_grads_(once, last=last, chunk_elems=chunk_elems)
+            if norm is not None:
+                norm, _ = grad_norm_launch([p.grad for p in params if p.grad is not None], None, chunk_elems)
+            return norm
         scan = _accumulate_checked(params, last)
         if scan is None:
             return None
