@@ -1248,11 +1248,22 @@ def test_logits_of_several_chunks_together_keep_the_bits(monkeypatch, n, d, v, c
         _same_bits(a, b)
 
 
+def _release_memory():
+    """Gives the allocator's free memory back, the rest of segments that only hold a library's
+    workspace too, so that what a test then holds lies in memory of its own and a limit on what is
+    reserved is a limit on what is to be had."""
+    torch.cuda.synchronize()
+    torch._C._cuda_clearCublasWorkspaces()
+    torch.cuda.empty_cache()
+    assert torch.cuda.memory_reserved(DEV) - torch.cuda.memory_allocated(DEV) < 64 << 20
+
+
 def test_logits_of_several_chunks_run_one_by_one_where_memory_is_short():
     """A call that fits with one chunk's logits still does: a group whose logits cannot be had is
     run chunk by chunk, with the same bits. The limit is the process's own, set on the allocator."""
     from torchure_amd.loss import fused_linear_ce as fce
 
+    _release_memory()
     n, d, v, chunk = 8192, 64, 16384, 1024  # 32 MiB of logits a chunk, 256 MiB together
     hidden = torch.randn(n, d, device=DEV).to(torch.bfloat16)
     weight = (torch.randn(v, d, device=DEV) * 0.05).to(torch.bfloat16)
@@ -1270,3 +1281,60 @@ def test_logits_of_several_chunks_run_one_by_one_where_memory_is_short():
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0, DEV)
     _same_bits(got, want)
+
+
+def _with_memory_limit(extra, call):
+    """``call`` with ``extra`` bytes to be had beyond what is reserved now (the allocator's own limit
+    for this process, none of the GPU's)."""
+    _release_memory()
+    total = torch.cuda.get_device_properties(DEV).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(DEV) + extra) / total, DEV)
+        return call()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, DEV)
+
+
+@pytest.mark.parametrize("n,d,v,chunk,unpadded", [
+    (4096, 256, 65536, 1024, False),  # 128 MiB of logits a chunk, 512 together, 32 a grad_W
+    (16320, 512, 4128, 16320, True),  # one chunk of 128 MiB, and 56 for grad_W's split sums
+])
+def test_forward_goes_on_where_memory_is_short_for_what_follows_the_logits(monkeypatch, n, d, v, chunk, unpadded):
+    """A group's logits that can be had, and then no grad_W beside them: the call goes on with one
+    chunk's logits at a time, with the same bits. And with no room for a workspace either: on the
+    unpadded loop, whose grad_W is summed without splits (one ulp of bf16 off, and 2^-20 of the
+    absolute sum, which is under 2^6 / n here)."""
+    from torchure_amd import _native
+    from torchure_amd.loss import fused_linear_ce as fce
+
+    _release_memory()
+    hidden = torch.randn(n, d, device=DEV).to(torch.bfloat16)
+    weight = (torch.randn(v, d, device=DEV) * 0.05).to(torch.bfloat16).requires_grad_(True)
+    labels = torch.randint(0, v, (n,), device=DEV)
+    ws = _native.lib().tm_ce_grad_w_ld_workspace_bytes(fce.padded_rows(n), v, d)
+    if unpadded:
+        assert ws > 48 << 20
+        limit = 2 * fce.padded_rows(n) * fce.padded_vocab(v) + ws // 2 + (8 << 20)
+    else:
+        assert fce.group_chunks(n, chunk, v, True) == 4
+        limit = 560 << 20
+    runs, loop = [], fce._chunks_unpadded
+    monkeypatch.setattr(fce, "_chunks_unpadded", lambda *a: runs.append(1) or loop(*a))
+
+    def call():
+        return fce._FusedLinearCE.apply(hidden, weight, labels, -100, chunk)
+
+    def grads(loss):
+        loss.backward()
+        got, weight.grad = weight.grad.cpu(), None
+        return loss.detach().cpu(), got
+
+    want = grads(call())
+    assert not runs
+    got = grads(_with_memory_limit(limit, call))
+    assert len(runs) == unpadded
+    assert torch.equal(got[0].view(torch.int32), want[0].view(torch.int32))
+    if unpadded:
+        torch.testing.assert_close(got[1].float(), want[1].float(), rtol=2.0 ** -7, atol=2.0 ** -14 / n)
+    else:
+        assert torch.equal(got[1].view(torch.int16), want[1].view(torch.int16))

@@ -802,3 +802,33 @@ def test_host_accumulate_scan_refuses_a_repeated_param():
         assert scan([p, q, p]) is None
         q._tm_working.grad = None  # q is only measured, and may be measured twice
         assert scan([q, p, q], True)[3].tolist() == [16, 8, 16]
+
+
+def test_ce_forward_goes_on_with_less_memory(monkeypatch):
+    """Where the native chunk loop finds no memory it is called again with one chunk's logits at a
+    time, once, and then left to the unpadded loop; other errors pass through."""
+    from torchure_amd import _native
+    from torchure_amd.loss import fused_linear_ce as fce
+
+    class Host:
+        def __init__(self, fits, error=torch.OutOfMemoryError):
+            self.fits, self.error, self.groups = fits, error, []
+
+        def ce_forward(self, *args):
+            self.groups.append(args[7])
+            if args[7] > self.fits:
+                raise self.error("short")
+            return "done"
+
+    def run(host, n):
+        monkeypatch.setattr(_native, "ce_host", lambda: host)
+        h, w = torch.zeros(n, 64, dtype=torch.bfloat16), torch.zeros(1024, 64, dtype=torch.bfloat16)
+        return fce._run_chunks(h, w, torch.zeros(n, dtype=torch.int64), -100, 128, "bf16", True, True, True)
+
+    monkeypatch.setattr(_native, "stream_handle", lambda device: 0)
+    for n, fits, want, groups in ((512, 4, "done", [4]), (512, 1, "done", [4, 1]), (512, 0, None, [4, 1]),
+                                  (128, 1, "done", [1]), (128, 0, None, [1])):
+        host = Host(fits)
+        assert run(host, n) == want and host.groups == groups
+    with pytest.raises(_native.NativeError):
+        run(Host(1, _native.NativeError), 512)

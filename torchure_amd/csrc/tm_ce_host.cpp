@@ -88,9 +88,9 @@ py::object or_none(const at::Tensor& t) { return t.defined() ? py::cast(t) : py:
 // The chunks of one call. hidden (n x d) and weight (v x d) are contiguous, bf16 or (cast_h,
 // cast_w) fp32; the chunks have `chunk` rows, the last one the rest, and their logits
 // pad[0] x ld (the last one's pad[1] x ld). The logits and their row pass run over `group` chunks
-// at a time, in one buffer (group > 1 only where a chunk has no padding rows of its own); where
-// memory for that is short, chunk by chunk. own_h[i]: grad_h on the split-K kernel, else the
-// library's product. grad = false: the loss alone.
+// at a time, in one buffer (group > 1 only where a chunk has no padding rows of its own). own_h[i]:
+// grad_h on the split-K kernel, else the library's product. grad = false: the loss alone. An
+// allocation that fails leaves nothing held: the caller may call again with less to hold.
 // Returns (loss, (loss sum, n_valid), grad_hidden, grad_weight, chunks' grad_W still to be added
 // (the last one at the end), whether grad_weight holds earlier chunks).
 py::tuple ce_forward(const at::Tensor& hidden, const at::Tensor& weight, bool cast_h, bool cast_w,
@@ -135,14 +135,7 @@ py::tuple ce_forward(const at::Tensor& hidden, const at::Tensor& weight, bool ca
       first = s;
       until = std::min(n, s + group * chunk);
       const i64 over = until == n ? (grad ? pad.second - last : 0) : pad_rows - rows;
-      try {
-        held = at::empty({until - s + over, ld}, bf16);
-      } catch (const c10::OutOfMemoryError&) {
-        if (group == 1) throw;
-        group = 1;
-        until = std::min(n, s + chunk);
-        held = at::empty({pad_rows, ld}, bf16);
-      }
+      held = at::empty({until - s + over, ld}, bf16);
       const i64* lab = labels.data_ptr<i64>() + s;
       float* losses = row_loss.data_ptr<float>() + s;
       check(a.logits(ptr(held), ld, hs, ptr(w), until - s, v, d, stream), "tm_ce_logits_ld_bf16");

@@ -235,19 +235,27 @@ def grad_w_gemm_fits(g: torch.Tensor, h: torch.Tensor) -> bool:
 
 def _grad_w(g: torch.Tensor, h: torch.Tensor, lib, stream) -> torch.Tensor:
     """A chunk's gw = grad_logits.t() @ h (fused_linear_ce.py:57) from unpadded grad_logits: bf16
-    GEMM, bf16 result (V x D). Rows off a multiple of 64 are copied into a zero-padded buffer."""
+    GEMM, bf16 result (V x D). Rows off a multiple of 64 are copied into a zero-padded buffer. The
+    product does without the copy and the workspace for its split sums where memory for them is
+    short."""
     rows, vocab = g.shape
     if not grad_w_gemm_fits(g, h) or (rows % 64 and h.shape[1] % 64):
         return torch.matmul(g.t(), h)
-    pad = rows if rows % 64 == 0 else padded_rows(rows)
-    if pad != rows:
-        g, short = torch.zeros((pad, vocab), dtype=torch.bfloat16, device=g.device), g
-        g[:rows].copy_(short)
     out = torch.empty((vocab, h.shape[1]), dtype=torch.bfloat16, device=g.device)
+    pad = rows if rows % 64 == 0 else padded_rows(rows)
     nbytes = lib.tm_ce_grad_w_ld_workspace_bytes(pad, vocab, h.shape[1])
-    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=g.device)
-    _native.check(lib.tm_ce_grad_w_ld_bf16(out.data_ptr(), g.data_ptr(), vocab, pad, h.data_ptr(), rows, vocab,
-                                           h.shape[1], ws.data_ptr(), nbytes, stream), "tm_ce_grad_w_ld_bf16")
+    padded, ws = g, None
+    try:
+        if pad != rows:
+            padded = torch.zeros((pad, vocab), dtype=torch.bfloat16, device=g.device)
+            padded[:rows].copy_(g)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=g.device) if nbytes else None
+    except torch.OutOfMemoryError:
+        if pad != rows:
+            return torch.matmul(g.t(), h, out=out)
+    _native.check(lib.tm_ce_grad_w_ld_bf16(out.data_ptr(), padded.data_ptr(), vocab, pad, h.data_ptr(), rows, vocab,
+                                           h.shape[1], None if ws is None else ws.data_ptr(), 0 if ws is None else nbytes,
+                                           stream), "tm_ce_grad_w_ld_bf16")
     return out
 
 
@@ -392,7 +400,11 @@ def _run_chunks(hidden, weight, labels, ignore_index, chunk, mode, grad, want_h,
     """The chunk loop on padded logits (``_tm_host.ce_forward``), for operands that the MFMA
     kernels take (dim a multiple of 64, bf16 ones 16-byte aligned), or None on others. Returns
     (loss, (loss sum, n_valid), grad_hidden, grad_weight, grad_W chunks still to be added,
-    accumulated). autocast's casts, or the weight's, are made there in one launch."""
+    accumulated). autocast's casts, or the weight's, are made there in one launch.
+
+    Where memory is short, whichever allocation of the call it fails: once more with one chunk's
+    logits at a time (the same bits), then None, for the unpadded loop, which holds neither padding
+    nor a workspace for grad_W."""
     (n, d), v = hidden.shape, weight.shape[0]
     if n == 0 or d == 0 or v == 0 or d % 64:
         return None
@@ -407,11 +419,15 @@ def _run_chunks(hidden, weight, labels, ignore_index, chunk, mode, grad, want_h,
         return None
     chunk = min(chunk, n)
     last = n - (n - 1) // chunk * chunk
-    return _native.ce_host().ce_forward(
-        h, w, cast_h, cast_w, labels, int(ignore_index), chunk, group_chunks(n, chunk, v, grad),
-        (padded_rows(chunk), padded_rows(last)), padded_vocab(v),
-        (grad_h_gemm_fits(chunk, d, v), grad_h_gemm_fits(last, d, v)), grad, want_h, want_w,
-        FOLD_CHUNKS, FOLD_BYTES, _native.stream_handle(hidden.device))
+    group = group_chunks(n, chunk, v, grad)
+    for chunks_held in dict.fromkeys((group, 1)):
+        with contextlib.suppress(torch.OutOfMemoryError):
+            return _native.ce_host().ce_forward(
+                h, w, cast_h, cast_w, labels, int(ignore_index), chunk, chunks_held,
+                (padded_rows(chunk), padded_rows(last)), padded_vocab(v),
+                (grad_h_gemm_fits(chunk, d, v), grad_h_gemm_fits(last, d, v)), grad, want_h, want_w,
+                FOLD_CHUNKS, FOLD_BYTES, _native.stream_handle(hidden.device))
+    return None
 
 
 def _bf16_operands(hidden, weight, mode):
@@ -484,8 +500,8 @@ def _fp32_chunks(hidden, weight, labels, ignore_index, n, v, chunk, grad, want_h
 
 def _chunks_unpadded(hidden, weight, labels, ignore_index, n, v, chunk, mode, want_h, want_w):
     """The chunk loop for what ``_run_chunks`` does not take (a dim off 64, unaligned or strided
-    operands, no rows): logits rows vocab elements apart, library products where this build's
-    GEMMs do not fit. Returns what ``_run_chunks`` does."""
+    operands, no rows) or finds no memory for: logits rows vocab elements apart, library products
+    where this build's GEMMs do not fit. Returns what ``_run_chunks`` does."""
     lib = _native.lib()
     stream = _native.stream_handle(hidden.device)
     hb, w = _bf16_operands(hidden, weight, mode)  # cast once, not per chunk
