@@ -1338,3 +1338,32 @@ def test_forward_goes_on_where_memory_is_short_for_what_follows_the_logits(monke
         torch.testing.assert_close(got[1].float(), want[1].float(), rtol=2.0 ** -7, atol=2.0 ** -14 / n)
     else:
         assert torch.equal(got[1].view(torch.int16), want[1].view(torch.int16))
+
+
+def test_backward_goes_on_where_memory_is_short():
+    """No room for the fp32 grad_W and the fp32 grad_hidden beside the chunk that waits for backward:
+    grad_W is finished first and the chunk's memory serves grad_hidden, with the same bits."""
+    from torchure_amd.loss import fused_linear_cross_entropy
+
+    _release_memory()
+    n, d, v = 8192, 1024, 8192  # 32 MiB for each result, 16 for the chunk's grad_W
+    hidden = torch.randn(n, d, device=DEV, requires_grad=True)
+    weight = (torch.randn(v, d, device=DEV) * 0.05).requires_grad_(True)
+    labels = torch.randint(0, v, (n,), device=DEV)
+
+    def loss():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            return fused_linear_cross_entropy(hidden, weight, labels, -100, n)
+
+    def grads():
+        out = hidden.grad.cpu(), weight.grad.cpu()
+        hidden.grad = weight.grad = None
+        return out
+
+    loss().backward()
+    want = grads()
+    _release_memory()  # each of the call's buffers in memory of its own
+    short = loss()
+    _with_memory_limit(56 << 20, short.backward)
+    for a, b in zip(grads(), want):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))

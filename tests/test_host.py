@@ -832,3 +832,40 @@ def test_ce_forward_goes_on_with_less_memory(monkeypatch):
         assert run(host, n) == want and host.groups == groups
     with pytest.raises(_native.NativeError):
         run(Host(1, _native.NativeError), 512)
+
+
+def test_ce_backward_goes_on_with_less_memory(monkeypatch):
+    """Where both gradients' results cannot be had beside the waiting chunks, grad_W is finished
+    first and the chunks let go before grad_hidden's is asked for."""
+    import types
+    import weakref
+
+    from torchure_amd import _native
+    from torchure_amd.loss import fused_linear_ce as fce
+
+    class Host:
+        calls, chunks = [], []
+
+        def ce_backward(self, grad_out, out2, grad_hidden, kind, grad_weight, chunks, accumulated, stream):
+            alive = [c for c in self.chunks if c() is not None]
+            self.calls.append((grad_hidden, grad_weight, len(chunks), accumulated, len(alive)))
+            if grad_hidden is not None and alive:
+                raise torch.OutOfMemoryError("short")
+            return grad_hidden and "gh", "gw" if chunks or grad_weight else None
+
+    host = Host()
+    monkeypatch.setattr(_native, "ce_host", lambda: host)
+    monkeypatch.setattr(_native, "stream_handle", lambda device: 0)
+
+    def run(want_w, grad_weight, n_chunks, accumulated):
+        chunks = [torch.zeros(2) for _ in range(n_chunks)]
+        host.calls, host.chunks = [], [weakref.ref(c) for c in chunks]
+        ctx = types.SimpleNamespace(stash=(torch.zeros(2), "held", grad_weight, chunks, accumulated), kind=1,
+                                    want_w=want_w)
+        del chunks
+        return fce._FusedLinearCE.backward(ctx, torch.ones(()))
+
+    assert run(True, None, 2, False) == ("gh", "gw", None, None, None)
+    assert host.calls == [("held", None, 2, False, 2), (None, None, 2, False, 2), ("held", None, 0, True, 0)]
+    assert run(True, "acc", 0, True) == ("gh", "gw", None, None, None)
+    assert host.calls == [("held", "acc", 0, True, 0)]

@@ -567,10 +567,16 @@ class _FusedLinearCE(torch.autograd.Function):
             grad_weight, accumulated = torch.zeros(shape, dtype=torch.float32, device=device), True
         # fused_linear_ce.py:107-126: the chunks still waiting (at most FOLD_CHUNKS) added into grad_W
         # with the scaling, and grad_h scaled (under autocast float(bf16 GEMM result) * scale), in one
-        # launch
-        grad_hidden, grad_weight = _native.ce_host().ce_backward(
-            grad_out, out2, grad_hidden, ctx.kind, grad_weight, chunks, accumulated,
-            _native.stream_handle(out2.device))
+        # launch; where there is no memory for both results beside the chunks, one after the other
+        def finish(grad_hidden, grad_weight, chunks, accumulated):
+            return _native.ce_host().ce_backward(grad_out, out2, grad_hidden, ctx.kind, grad_weight, chunks,
+                                                 accumulated, _native.stream_handle(out2.device))
+
+        with contextlib.suppress(torch.OutOfMemoryError):
+            return *finish(grad_hidden, grad_weight, chunks, accumulated), None, None, None
+        grad_weight = finish(None, grad_weight, chunks, accumulated)[1]
+        del chunks
+        grad_hidden = finish(grad_hidden, None, [], True)[0]
         return grad_hidden, grad_weight, None, None, None
 
 
