@@ -420,13 +420,15 @@ def _run_chunks(hidden, weight, labels, ignore_index, chunk, mode, grad, want_h,
     chunk = min(chunk, n)
     last = n - (n - 1) // chunk * chunk
     group = group_chunks(n, chunk, v, grad)
-    for chunks_held in dict.fromkeys((group, 1)):
-        with contextlib.suppress(torch.OutOfMemoryError):
+    for held in (group, 1) if group > 1 else (1,):
+        try:
             return _native.ce_host().ce_forward(
-                h, w, cast_h, cast_w, labels, int(ignore_index), chunk, chunks_held,
+                h, w, cast_h, cast_w, labels, int(ignore_index), chunk, held,
                 (padded_rows(chunk), padded_rows(last)), padded_vocab(v),
                 (grad_h_gemm_fits(chunk, d, v), grad_h_gemm_fits(last, d, v)), grad, want_h, want_w,
                 FOLD_CHUNKS, FOLD_BYTES, _native.stream_handle(hidden.device))
+        except torch.OutOfMemoryError:
+            pass
     return None
 
 
@@ -568,15 +570,16 @@ class _FusedLinearCE(torch.autograd.Function):
         # fused_linear_ce.py:107-126: the chunks still waiting (at most FOLD_CHUNKS) added into grad_W
         # with the scaling, and grad_h scaled (under autocast float(bf16 GEMM result) * scale), in one
         # launch; where there is no memory for both results beside the chunks, one after the other
-        def finish(grad_hidden, grad_weight, chunks, accumulated):
-            return _native.ce_host().ce_backward(grad_out, out2, grad_hidden, ctx.kind, grad_weight, chunks,
-                                                 accumulated, _native.stream_handle(out2.device))
-
-        with contextlib.suppress(torch.OutOfMemoryError):
-            return *finish(grad_hidden, grad_weight, chunks, accumulated), None, None, None
-        grad_weight = finish(None, grad_weight, chunks, accumulated)[1]
+        finish, stream = _native.ce_host().ce_backward, _native.stream_handle(out2.device)
+        try:
+            grad_hidden, grad_weight = finish(grad_out, out2, grad_hidden, ctx.kind, grad_weight, chunks, accumulated,
+                                              stream)
+            return grad_hidden, grad_weight, None, None, None
+        except torch.OutOfMemoryError:
+            pass
+        grad_weight = finish(grad_out, out2, None, ctx.kind, grad_weight, chunks, accumulated, stream)[1]
         del chunks
-        grad_hidden = finish(grad_hidden, None, [], True)[0]
+        grad_hidden = finish(grad_out, out2, grad_hidden, ctx.kind, None, [], True, stream)[0]
         return grad_hidden, grad_weight, None, None, None
 
 
