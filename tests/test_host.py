@@ -869,3 +869,34 @@ def test_ce_backward_goes_on_with_less_memory(monkeypatch):
     assert host.calls == [("held", None, 2, False, 2), (None, None, 2, False, 2), ("held", None, 0, True, 0)]
     assert run(True, "acc", 0, True) == ("gh", "gw", None, None, None)
     assert host.calls == [("held", "acc", 0, True, 0)]
+
+
+def test_fused_ce_host_loop_runs_without_the_gil():
+    """Every C entry point of the fused CE's forward and backward is reached with the GIL released:
+    each is bound (in a process of its own) to CPython's PyGILState_Check, whose 1 for "held" is an
+    error status here and whose 0 is success, on CPU tensors that nothing then touches."""
+    import subprocess
+    import sys
+
+    code = """
+import ctypes
+import torch
+from torchure_amd import _native
+h, api = _native.host(), ctypes.pythonapi
+at = lambda f: ctypes.cast(f, ctypes.c_void_p).value
+entries = dict.fromkeys(_native.EXPORTED, at(api.PyGILState_Check)) | {"tm_last_error": at(api.Py_GetVersion)}
+h.ce_bind(entries, _native.NativeError)
+x, w, labels = torch.zeros(640, 64), torch.zeros(128, 64), torch.zeros(640, dtype=torch.int64)
+for grad in (True, False):
+    out = h.ce_forward(x, w, True, True, labels, -100, 256, 1, (256, 128), 128, (True, True), grad, grad, grad,
+                       2, 1 << 30, 0)
+    assert [t is None for t in out[:4]] == [False, False, not grad, not grad] and len(out[4]) == grad
+    assert out[5] == grad
+    if grad:
+        gh, gw = h.ce_backward(torch.ones(()), out[1], out[2], 1, out[3], out[4], out[5], 0)
+        assert gh.dtype == gw.dtype == torch.float32 and gh.shape == x.shape and gw.shape == w.shape
+print("ok")
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    done = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=300)
+    assert done.returncode == 0 and done.stdout.strip() == "ok", done.stderr

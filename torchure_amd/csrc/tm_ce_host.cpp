@@ -73,12 +73,27 @@ const Abi& abi() {
   return *g_abi;
 }
 
-// A non-zero status becomes torchure_amd._native.NativeError, as from the Python callers.
+struct EntryFailed : std::runtime_error {
+  using std::runtime_error::runtime_error;
+};
+
 void check(int rc, const char* what) {
-  if (rc == 0) return;
-  const std::string msg = std::string(what) + " failed (" + std::to_string(rc) + "): " + abi().last_error();
-  PyErr_SetString(abi().native_error.ptr(), msg.c_str());
-  throw py::error_already_set();
+  if (rc != 0)
+    throw EntryFailed(std::string(what) + " failed (" + std::to_string(rc) + "): " + abi().last_error());
+}
+
+// Runs body without the GIL: its allocations may wait for the device, and its launches for room in
+// the queue, while other Python threads go on. A failed entry point becomes
+// torchure_amd._native.NativeError, as from the Python callers.
+template <typename Body>
+auto without_gil(Body&& body) -> decltype(body()) {
+  try {
+    py::gil_scoped_release released;
+    return body();
+  } catch (const EntryFailed& e) {  // the GIL is held again
+    PyErr_SetString(abi().native_error.ptr(), e.what());
+    throw py::error_already_set();
+  }
 }
 
 char* ptr(const at::Tensor& t) { return t.defined() ? static_cast<char*>(t.data_ptr()) : nullptr; }
@@ -91,13 +106,17 @@ py::object or_none(const at::Tensor& t) { return t.defined() ? py::cast(t) : py:
 // at a time, in one buffer (group > 1 only where a chunk has no padding rows of its own). own_h[i]:
 // grad_h on the split-K kernel, else the library's product. grad = false: the loss alone. An
 // allocation that fails leaves nothing held: the caller may call again with less to hold.
-// Returns (loss, (loss sum, n_valid), grad_hidden, grad_weight, chunks' grad_W still to be added
-// (the last one at the end), whether grad_weight holds earlier chunks).
-py::tuple ce_forward(const at::Tensor& hidden, const at::Tensor& weight, bool cast_h, bool cast_w,
+struct Forward {
+  at::Tensor loss, out2;  // out2: loss sum, n_valid
+  at::Tensor grad_hidden, grad_weight;
+  std::vector<at::Tensor> pending;  // chunks' grad_W still to be added, the last one at the end
+  bool accumulated = false;         // whether grad_weight holds earlier chunks
+};
+
+Forward run_forward(const at::Tensor& hidden, const at::Tensor& weight, bool cast_h, bool cast_w,
                      const at::Tensor& labels, i64 ignore, i64 chunk, i64 group, std::pair<i64, i64> pad, i64 ld,
                      std::pair<bool, bool> own_h, bool grad, bool want_h, bool want_w, i64 fold_chunks, i64 fold_bytes,
                      uintptr_t stream_handle) {
-  HANDLE_TH_ERRORS
   const Abi& a = abi();
   void* stream = reinterpret_cast<void*>(stream_handle);
   const i64 n = hidden.size(0), d = hidden.size(1), v = weight.size(0);
@@ -109,7 +128,10 @@ py::tuple ce_forward(const at::Tensor& hidden, const at::Tensor& weight, bool ca
                   cast_w ? ptr(w) : nullptr, cast_w ? ptr(weight) : nullptr, cast_w ? v * d : 0, stream),
           "tm_ce_cast2");
   const i64 last = n - (n - 1) / chunk * chunk;  // rows of the last chunk
-  at::Tensor row_loss = at::empty({n}, f32), grad_hidden, grad_weight, ws;
+  at::Tensor row_loss = at::empty({n}, f32), ws;
+  Forward out;
+  at::Tensor &grad_hidden = out.grad_hidden, &grad_weight = out.grad_weight;
+  std::vector<at::Tensor>& pending = out.pending;
   // one workspace for both gradients' split sums over the chunks (stream-ordered)
   size_t bytes = 0;
   if (grad && want_h) {
@@ -122,8 +144,6 @@ py::tuple ce_forward(const at::Tensor& hidden, const at::Tensor& weight, bool ca
     bytes = std::max(bytes, a.grad_w_bytes(pad.second, v, d));
   }
   if (bytes) ws = at::empty({static_cast<i64>(bytes)}, f32.dtype(at::kByte));
-  std::vector<at::Tensor> pending;
-  bool accumulated = false;
   at::Tensor held;  // the group's logits
   i64 first = 0, until = 0;  // and its rows
   for (i64 s = 0; s < n; s += chunk) {
@@ -151,8 +171,8 @@ py::tuple ce_forward(const at::Tensor& hidden, const at::Tensor& weight, bool ca
         check(a.grad_h(ptr(grad_hidden) + s * d * 2, ptr(logits), ld, ptr(w), rows, v, d, ptr(ws), bytes, stream),
               "tm_ce_grad_h_ld_bf16");
       } else {
-        at::Tensor out = grad_hidden.narrow(0, s, rows);
-        at::mm_out(out, logits.narrow(0, 0, rows).narrow(1, 0, v), w);
+        at::Tensor gh = grad_hidden.narrow(0, s, rows);
+        at::mm_out(gh, logits.narrow(0, 0, rows).narrow(1, 0, v), w);
       }
     }
     if (want_w) {
@@ -164,16 +184,32 @@ py::tuple ce_forward(const at::Tensor& hidden, const at::Tensor& weight, bool ca
         if (!grad_weight.defined()) grad_weight = at::empty({v, d}, f32);
         std::vector<const void*> p;
         for (const at::Tensor& t : pending) p.push_back(ptr(t));
-        check(a.fold(ptr(grad_weight), p.data(), static_cast<int>(waiting), v * d, accumulated, nullptr, nullptr, stream),
+        check(a.fold(ptr(grad_weight), p.data(), static_cast<int>(waiting), v * d, out.accumulated, nullptr, nullptr,
+                     stream),
               "tm_ce_grad_w_fold");
-        accumulated = true;
+        out.accumulated = true;
         pending.clear();
       }
     }
   }
-  at::Tensor out2 = at::empty({2}, f32), loss = at::empty({}, f32);
-  check(a.mean_loss(ptr(row_loss), ptr(labels), n, ignore, ptr(out2), ptr(loss), stream), "tm_ce_mean_loss");
-  return py::make_tuple(loss, out2, or_none(grad_hidden), or_none(grad_weight), py::cast(pending), accumulated);
+  out.out2 = at::empty({2}, f32);
+  out.loss = at::empty({}, f32);
+  check(a.mean_loss(ptr(row_loss), ptr(labels), n, ignore, ptr(out.out2), ptr(out.loss), stream), "tm_ce_mean_loss");
+  return out;
+}
+
+// Returns (loss, out2, grad_hidden, grad_weight, pending, accumulated) of run_forward.
+py::tuple ce_forward(const at::Tensor& hidden, const at::Tensor& weight, bool cast_h, bool cast_w,
+                     const at::Tensor& labels, i64 ignore, i64 chunk, i64 group, std::pair<i64, i64> pad, i64 ld,
+                     std::pair<bool, bool> own_h, bool grad, bool want_h, bool want_w, i64 fold_chunks, i64 fold_bytes,
+                     uintptr_t stream_handle) {
+  HANDLE_TH_ERRORS
+  const Forward f = without_gil([&] {
+    return run_forward(hidden, weight, cast_h, cast_w, labels, ignore, chunk, group, pad, ld, own_h, grad, want_h,
+                       want_w, fold_chunks, fold_bytes, stream_handle);
+  });
+  return py::make_tuple(f.loss, f.out2, or_none(f.grad_hidden), or_none(f.grad_weight), py::cast(f.pending),
+                        f.accumulated);
   END_HANDLE_TH_ERRORS_PYBIND
 }
 
@@ -185,17 +221,19 @@ py::tuple ce_backward(const at::Tensor& grad_out, const at::Tensor& out2, const 
                       bool accumulated, uintptr_t stream_handle) {
   HANDLE_TH_ERRORS
   const Abi& a = abi();
-  at::Tensor g = grad_out.detach().to(at::kFloat).contiguous();
   at::Tensor gw = grad_w ? *grad_w : at::Tensor(), gh = held_h ? *held_h : at::Tensor();
-  const auto f32 = out2.options();
-  if (!gw.defined() && !chunks.empty()) gw = at::empty(chunks[0].sizes(), f32);
-  if (kind == 1 && gh.defined()) gh = at::empty(gh.sizes(), f32);
-  std::vector<const void*> p;
-  for (const at::Tensor& t : chunks) p.push_back(ptr(t));
-  check(a.finish(ptr(gw), p.data(), static_cast<int>(p.size()), gw.defined() ? gw.numel() : 0, accumulated,
-                 held_h ? ptr(*held_h) : nullptr, ptr(gh), gh.defined() ? gh.numel() : 0, kind, ptr(g),
-                 out2.data_ptr<float>() + 1, reinterpret_cast<void*>(stream_handle)),
-        "tm_ce_finish");
+  without_gil([&] {
+    at::Tensor g = grad_out.detach().to(at::kFloat).contiguous();
+    const auto f32 = out2.options();
+    if (!gw.defined() && !chunks.empty()) gw = at::empty(chunks[0].sizes(), f32);
+    if (kind == 1 && gh.defined()) gh = at::empty(gh.sizes(), f32);
+    std::vector<const void*> p;
+    for (const at::Tensor& t : chunks) p.push_back(ptr(t));
+    check(a.finish(ptr(gw), p.data(), static_cast<int>(p.size()), gw.defined() ? gw.numel() : 0, accumulated,
+                   held_h ? ptr(*held_h) : nullptr, ptr(gh), gh.defined() ? gh.numel() : 0, kind, ptr(g),
+                   out2.data_ptr<float>() + 1, reinterpret_cast<void*>(stream_handle)),
+          "tm_ce_finish");
+  });
   return py::make_tuple(or_none(gh), or_none(gw));
   END_HANDLE_TH_ERRORS_PYBIND
 }
