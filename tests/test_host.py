@@ -900,3 +900,28 @@ print("ok")
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     done = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=300)
     assert done.returncode == 0 and done.stdout.strip() == "ok", done.stderr
+
+
+def test_grad_h_choice_stays_within_what_the_kernels_take():
+    """No size whose grad_h is sent to this build's kernels is one that they refuse, on both sides of
+    their limits: with null pointers the entry points name those, not the sizes."""
+    from torchure_amd import _native
+    from torchure_amd.loss.fused_linear_ce import grad_h_gemm_fits, padded_vocab, splitk_grad_h_fits
+
+    lib = _native.lib()
+
+    def refused(name, *args):
+        assert getattr(lib, name)(*args) < 0
+        return b"null pointer" not in lib.tm_last_error()
+
+    seen = set()
+    for rows in (0, 1, 255, 256, 1 << 20, (1 << 20) + 1, (1 << 20) + 256, 1 << 21):
+        for dim in (0, 8, 60, 768, 1024, 65536 - 256, 65536, 65536 + 64, 65536 + 256):
+            for vocab in (0, 64, 1024, 4097, 5000, 151936, 0x7FFFFF00, 0x7FFFFF01, 0x7FFFFF40):
+                ragged = refused("tm_ce_grad_h_ld_bf16", None, None, padded_vocab(vocab), None, rows, vocab, dim,
+                                 None, 0, None)
+                whole = refused("tm_ce_grad_h_bf16", None, None, None, rows, vocab, dim, None, 0, None)
+                assert not (ragged and grad_h_gemm_fits(rows, dim, vocab)), (rows, dim, vocab)
+                assert not (whole and splitk_grad_h_fits(rows, dim, vocab)), (rows, dim, vocab)
+                seen.add((grad_h_gemm_fits(rows, dim, vocab), ragged))
+    assert seen == {(True, False), (False, False), (False, True)}

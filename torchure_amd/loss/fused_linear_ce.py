@@ -262,6 +262,11 @@ def _grad_w(g: torch.Tensor, h: torch.Tensor, lib, stream) -> torch.Tensor:
 SPLITK_GRAD_H_MAX_TILES = 64
 
 
+def _grad_h_takes(rows: int, dim: int, vocab: int) -> bool:
+    """Sizes that tm_ce_grad_h_ld_bf16 accepts."""
+    return 0 < rows <= 1 << 20 and 0 < dim <= 1 << 16 and dim % 8 == 0 and 0 < vocab <= 0x7FFFFF00
+
+
 def splitk_grad_h_fits(rows: int, dim: int, vocab: int) -> bool:
     """Chunks whose grad_h runs on the split-K MFMA GEMM (tm_ce_grad_h_bf16): the shapes it
     tiles (rows and dim multiples of 256, vocab of 64), except where the library GEMM measured
@@ -278,8 +283,7 @@ def splitk_grad_h_fits(rows: int, dim: int, vocab: int) -> bool:
         4096  1.07 / 1.88    2.11 / 2.03    4.16 / 3.88    8.35 / 7.76
         5120  1.43 / 1.89    3.11 / 3.48    5.70 / 7.07    11.34 / 13.41
     """
-    if not (rows > 0 and dim > 0 and rows % 256 == 0 and dim % 256 == 0 and dim <= 65536
-            and vocab > 0 and vocab % 64 == 0):
+    if not _grad_h_takes(rows, dim, vocab) or rows % 256 or dim % 256 or vocab % 64:
         return False
     return (rows // 256) * (dim // 256) <= SPLITK_GRAD_H_MAX_TILES or (dim & (dim - 1)) != 0
 
@@ -299,8 +303,8 @@ def grad_h_gemm_fits(rows: int, dim: int, vocab: int) -> bool:
     """
     if splitk_grad_h_fits(rows, dim, vocab):
         return True
-    if not (rows > 0 and dim > 0 and dim % 8 == 0 and dim <= 65536 and rows <= 1 << 20
-            and vocab >= RAGGED_GRAD_H_MIN_VOCAB and (rows % 256 or dim % 256 or vocab % 64)):
+    if not (_grad_h_takes(rows, dim, vocab) and vocab >= RAGGED_GRAD_H_MIN_VOCAB
+            and (rows % 256 or dim % 256 or vocab % 64)):
         return False
     return -(-rows // 256) * -(-dim // 256) <= SPLITK_GRAD_H_MAX_TILES or (dim & (dim - 1)) != 0
 
