@@ -1367,3 +1367,39 @@ def test_backward_goes_on_where_memory_is_short():
     _with_memory_limit(56 << 20, short.backward)
     for a, b in zip(grads(), want):
         assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
+@pytest.mark.parametrize("vocab,ld,cols", [
+    (20001, 20032, (0, 20000)),  # one thread's vector and its element past the last vector
+    (20002, 20032, (20000, 20001)),
+    (20001, 20001, (0, 1024)),   # rows off 16 bytes: one thread's first two elements
+    (20001, 20001, (7, 19999)),
+    (9, 32, (0, 8)),
+    (90001, 90016, (0, 90000)),  # too long for registers
+])
+def test_ce_rows_f32_with_several_infinite_logits(vocab, ld, cols):
+    """Two logits of +inf, wherever a thread meets them: lse and the loss are +inf as
+    torch.logsumexp's, the gradient 0 but at the two, where inf - inf leaves NaN. A row that is -inf
+    but for one element stays finite."""
+    from torchure_amd import _native
+
+    lib, st = _native.lib(), _native.stream_handle(DEV)
+    x = torch.randn(3, ld, device=DEV)
+    x[1] = x[2] = float("-inf")
+    x[0, list(cols)] = float("inf")
+    x[1, cols[1]] = 2.0
+    x[2, list(cols)] = float("inf")
+    labels = torch.tensor([vocab // 2, cols[1], vocab // 2], device=DEV)
+    loss, loss_only = torch.empty(3, device=DEV), torch.empty(3, device=DEV)
+    for fn, out in ((lib.tm_ce_rows_loss_f32, loss_only), (lib.tm_ce_rows_f32, loss)):
+        _native.check(fn(x.data_ptr(), ld, labels.data_ptr(), 3, vocab, -100, out.data_ptr(), st), "rows")
+    for out in (loss_only, loss):
+        assert out[0] == float("inf") and out[1] == 0.0 and out[2] == float("inf"), out
+    rest = torch.ones(vocab, dtype=torch.bool, device=DEV)
+    rest[list(cols)] = False
+    for r in (0, 2):
+        assert x[r, list(cols)].isnan().all()
+        want = torch.zeros(vocab, device=DEV)
+        want[vocab // 2] = -1.0
+        assert torch.equal(x[r, :vocab][rest], want[rest])
+    assert (x[1, :vocab] == 0).all()

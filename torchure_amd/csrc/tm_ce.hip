@@ -435,12 +435,13 @@ __device__ __forceinline__ void ms_add_f(float& m, float& s, float x) {
     s = s * expf(m - x) + 1.0f;
     m = x;
   } else {
-    s = s + expf(x - m);
+    s = s + (x == m ? 1.0f : expf(x - m));  // equal: exp(0), also where both are +inf
   }
 }
 
 // What the sum's exponents are taken against: the maximum, 0 where that is infinite, as
-// torch.logsumexp does: a +inf logit makes lse +inf, not NaN.
+// torch.logsumexp does: a +inf logit makes lse +inf, not NaN, however many there are (ms_add_f counts
+// them).
 __device__ __forceinline__ float finite_ref(float top) { return fabsf(top) == INFINITY ? 0.0f : top; }
 
 // What a sum under the maximum m is multiplied by when the maximum becomes top (>= m).
