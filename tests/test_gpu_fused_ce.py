@@ -140,19 +140,47 @@ def test_ce_rows_at_the_edges_of_the_row_shapes(vocab):
     assert got[5].isnan().all() and got[6].isnan().all()
 
 
-def test_ce_rows_beyond_one_launch_of_single_waves():
-    """More rows than one launch of 64-thread workgroups holds."""
+@pytest.mark.parametrize("grad", [False, True])
+def test_ce_rows_beyond_one_launch_of_single_waves(grad):
+    """More rows than one launch of 64-thread workgroups holds (2^32 work-items). Rows 8 elements
+    apart are 16-byte aligned, which a vocabulary this short runs with one wave a row (packed rows
+    of 2 would take 1024 threads each). Every row on both sides of the line is checked: the losses,
+    the gradients (p - 1 and p of two logits, RNE) and, with them, the cleared padding."""
     from torchure_amd import _native
 
-    rows, v = 0xFFFFFFFF // 64 + 77, 2
-    x = torch.zeros(rows, v, dtype=torch.bfloat16, device=DEV)
+    line = 0xFFFFFFFF // 64
+    rows, v, ld = line + 77, 2, 8
+    x = torch.zeros(rows, ld, dtype=torch.bfloat16, device=DEV)
     x[:, 1] = (torch.arange(rows, device=DEV) % 5).to(torch.bfloat16)
+    x[:, v:] = 7.0  # past the vocabulary: not part of the row
     labels = torch.zeros(rows, dtype=torch.int64, device=DEV)
-    loss = torch.empty(rows, device=DEV)
-    _native.check(_native.lib().tm_ce_rows_loss_bf16(x.data_ptr(), v, labels.data_ptr(), rows, v, -100,
-                                                     loss.data_ptr(), _native.stream_handle(DEV)), "rows")
-    want = torch.log1p(torch.exp(torch.arange(5, device=DEV).double()))[torch.arange(rows, device=DEV) % 5]
-    torch.testing.assert_close(loss.double(), want, rtol=1e-6, atol=1e-6)
+    labels[line - 1::3] = -100
+    loss = torch.full((rows,), -1.0, device=DEV)
+    lib, stream = _native.lib(), _native.stream_handle(DEV)
+    if grad:
+        _native.check(lib.tm_ce_rows_padded_bf16(x.data_ptr(), ld, labels.data_ptr(), rows, rows, v, -100,
+                                                 loss.data_ptr(), stream), "rows")
+    else:
+        _native.check(lib.tm_ce_rows_loss_bf16(x.data_ptr(), ld, labels.data_ptr(), rows, v, -100, loss.data_ptr(),
+                                               stream), "rows")
+    a = torch.arange(5, device=DEV).double()
+    kind, valid = torch.arange(rows, device=DEV) % 5, labels != -100
+    assert bool(valid[line - 2]) and not bool(valid[line - 1]) and bool(valid[line]) and not bool(valid[line + 2])
+    want = torch.where(valid, torch.log1p(torch.exp(a)).float()[kind], 0.0)
+    torch.testing.assert_close(loss, want, rtol=1e-6, atol=1e-6)
+    p = torch.sigmoid(a)
+    g = torch.zeros(5, ld, dtype=torch.float64, device=DEV)
+    g[:, 0], g[:, 1] = -p, p
+    g = g.to(torch.bfloat16).view(torch.int16)
+    for r in range(0, rows, 1 << 24):  # torch's own gather does not fill results of over 2^29 elements
+        got, ok = x[r:r + (1 << 24)], valid[r:r + (1 << 24)]
+        if not grad:
+            assert bool((got[:, v:] == 7.0).all())
+            continue
+        # one ulp of bf16: the kernel's p is fp32, and p - 1 cancels
+        off = (got.view(torch.int16) - g[kind[r:r + (1 << 24)]]).abs()[ok]
+        assert int(off.max()) <= 1 and int(off[:, v:].max()) == 0
+        assert not bool(got.view(torch.int16)[~ok].any())
 
 
 def test_ce_rows_beyond_one_launch():
