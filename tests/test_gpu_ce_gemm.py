@@ -225,6 +225,44 @@ def test_op_grad_h_choice_above_64_tiles(d, split):
     assert torch.equal(h1.grad.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("n,d,v,own", [
+    (7129, 1216, 4160, False),  # 140 tiles, a short vocabulary
+    (6145, 1088, 16448, True),  # 125 tiles, a long one
+    (2046, 1216, 4161, True),   # 40 tiles
+])
+def test_op_grad_h_choice_on_ragged_chunks(n, d, v, own):
+    """One ragged chunk: grad_h is this build's product, or torch.matmul's on the padded logits, times
+    the bf16 scale, bit for bit."""
+    from torchure_amd.loss import fused_linear_cross_entropy
+    from torchure_amd.loss.fused_linear_ce import padded_rows, padded_vocab
+
+    native, lib, stream = _lib()
+    g = torch.Generator(device=DEV).manual_seed(n)
+    hidden = torch.randn(n, d, device=DEV, generator=g).to(torch.bfloat16)
+    w = (torch.randn(v, d, device=DEV, generator=g) * 0.05).to(torch.bfloat16)
+    labels = torch.randint(0, v, (n,), device=DEV, generator=g)
+    labels[::17] = -100
+    h1 = hidden.clone().requires_grad_(True)
+    fused_linear_cross_entropy(h1, w, labels, -100, None).backward()
+    pad, ld = padded_rows(n), padded_vocab(v)
+    logits = torch.empty(pad, ld, dtype=torch.bfloat16, device=DEV)
+    loss = torch.empty(n, device=DEV)
+    native.check(lib.tm_ce_logits_ld_bf16(logits.data_ptr(), ld, hidden.data_ptr(), w.data_ptr(), n, v, d, stream),
+                 "logits")
+    native.check(lib.tm_ce_rows_padded_bf16(logits.data_ptr(), ld, labels.data_ptr(), n, pad, v, -100, loss.data_ptr(),
+                                            stream), "rows")
+    if own:
+        nbytes = lib.tm_ce_grad_h_ld_workspace_bytes(n, v, d)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+        want = torch.empty_like(hidden)
+        native.check(lib.tm_ce_grad_h_ld_bf16(want.data_ptr(), logits.data_ptr(), ld, w.data_ptr(), n, v, d,
+                                              ws.data_ptr(), nbytes, stream), "grad_h")
+    else:
+        want = torch.matmul(logits[:n, :v], w)
+    want.mul_((torch.tensor(1.0, device=DEV) / (labels != -100).sum()).to(torch.bfloat16))
+    assert torch.equal(h1.grad.view(torch.int16), want.view(torch.int16))
+
+
 def _logits(h, w, pad=64, sentinel=0x7BCD):
     """tm_ce_logits_bf16 into a view with `pad` guard elements on both sides (sentinel bits),
     returning (logits, guard intact)."""

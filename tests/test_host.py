@@ -925,3 +925,18 @@ def test_grad_h_choice_stays_within_what_the_kernels_take():
                 assert not (whole and splitk_grad_h_fits(rows, dim, vocab)), (rows, dim, vocab)
                 seen.add((grad_h_gemm_fits(rows, dim, vocab), ragged))
     assert seen == {(True, False), (False, False), (False, True)}
+
+
+def test_ragged_grad_h_choice_by_tiles_and_vocabulary():
+    """Both sides of each line of the ragged chunks' rule, and that it leaves the aligned ones alone."""
+    from torchure_amd.loss.fused_linear_ce import grad_h_gemm_fits, splitk_grad_h_fits
+
+    assert grad_h_gemm_fits(552, 256, 4097) and not grad_h_gemm_fits(552, 256, 4096)
+    # 96 tiles of 256 x 256 at a width that is no power of two, then 97 and more
+    assert grad_h_gemm_fits(6001, 832, 7296) and not grad_h_gemm_fits(97 * 256 - 1, 192, 7296)
+    assert not grad_h_gemm_fits(7129, 1216, 4097) and not grad_h_gemm_fits(7129, 1216, 16383)
+    assert grad_h_gemm_fits(7129, 1216, 16384) and grad_h_gemm_fits(8000, 2560, 151936)
+    # a power of two: 64 tiles, whatever the vocabulary
+    assert grad_h_gemm_fits(4000, 1024, 151936) and not grad_h_gemm_fits(4097, 1024, 151936)
+    for rows, dim, vocab in ((7168, 1280, 7296), (8192, 768, 4096), (512, 256, 4096)):
+        assert grad_h_gemm_fits(rows, dim, vocab) and splitk_grad_h_fits(rows, dim, vocab)

@@ -288,28 +288,43 @@ def splitk_grad_h_fits(rows: int, dim: int, vocab: int) -> bool:
     return (rows // 256) * (dim // 256) <= SPLITK_GRAD_H_MAX_TILES or (dim & (dim - 1)) != 0
 
 
+RAGGED_GRAD_H_MIN_VOCAB = 4097
+RAGGED_GRAD_H_MAX_TILES = 96
+RAGGED_GRAD_H_LONG_VOCAB = 16384
+
+
 def grad_h_gemm_fits(rows: int, dim: int, vocab: int) -> bool:
     """Padded chunks whose grad_h runs on this build's GEMM: those ``splitk_grad_h_fits`` accepts,
-    and ragged ones (rows or dim off a multiple of 256, a vocabulary off a multiple of 64) under
-    the same rule for many tiles of a power-of-two width, from a vocabulary of
-    RAGGED_GRAD_H_MIN_VOCAB up (below, K is short, both take under 50 us, and neither leads
-    throughout). us per call on MI355X, this build / hipBLASLt on the same padded logits:
+    and of the ragged ones (rows or dim off a multiple of 256, a vocabulary off a multiple of 64)
+    those of a vocabulary above 4096, of at most 64 tiles at a power-of-two width and 96 at others,
+    and at those other widths of any more tiles from a vocabulary of RAGGED_GRAD_H_LONG_VOCAB up.
+    us per call on MI355X, this build / hipBLASLt on the same padded logits:
 
-        rows x dim x vocab    7129 x 1216 x 1984     50 /  48     1024 x 768 x 32001      69 / 183
-                              1184 x 384 x 2535      16 /  19      452 x 768 x 32001      41 / 135
-                               552 x 256 x 4097      14 /  19     1905 x 1024 x 151936   562 / 721
-                              1024 x 320 x 7296      21 /  33     3000 x 2560 x 100000  1337 / 2076
-                              2046 x 2112 x 7296     79 /  83     6001 x 1024 x 151936  1656 / 1570
-    """
+        rows x dim (tiles)    vocab 1984     4097-5001      7296         12001         20032         32001
+        1184 x  384  (10)       15 /  20      18 /  25     22 /  33
+        2046 x 1216  (40)       24 /  28      39 /  53     56 /  59
+        4000 x 1024  (64)       26 /  26      56 /  55     75 /  67    103 / 113     159 / 211     248 / 335
+        4001 x 1216  (80)       33 /  36      65 /  77     82 /  97    120 / 160     193 / 251     299 / 406
+        6001 x  832  (96)       34 /  37      74 /  77     95 /  96    151 / 161     240 / 294     383 / 466
+        3000 x 2560 (120)       38 /  37      88 /  82    113 / 103    170 / 169     279 / 384     442 / 616
+        7129 x 1216 (140)       51 /  47     119 /  98    152 / 126    232 / 209     388 / 526     593 / 806
+        8000 x 2560 (320)      104 / 100     221 / 227    358 / 253    536 / 423     804 / 697    1219 / 1686
+
+    With few tiles the library leaves CUs idle. With many it fills the chip and this kernel's splits
+    only cost their partials, until K is long: past some 16,000 the library's kernels for these
+    widths fall behind by a quarter to a half. The lower line is not one of speed: a ragged chunk of
+    a vocabulary up to 4096 keeps the library's product and its bits, though this kernel would be
+    the faster there too (from level to 2x at up to 96 tiles)."""
     if splitk_grad_h_fits(rows, dim, vocab):
         return True
     if not (_grad_h_takes(rows, dim, vocab) and vocab >= RAGGED_GRAD_H_MIN_VOCAB
             and (rows % 256 or dim % 256 or vocab % 64)):
         return False
-    return -(-rows // 256) * -(-dim // 256) <= SPLITK_GRAD_H_MAX_TILES or (dim & (dim - 1)) != 0
+    tiles = -(-rows // 256) * -(-dim // 256)
+    if dim & (dim - 1) == 0:
+        return tiles <= SPLITK_GRAD_H_MAX_TILES
+    return tiles <= RAGGED_GRAD_H_MAX_TILES or vocab >= RAGGED_GRAD_H_LONG_VOCAB
 
-
-RAGGED_GRAD_H_MIN_VOCAB = 4097
 
 GROUP_BYTES = 1 << 30  # logits of the chunks whose logits and row pass run together, at most
 GROUP_ROWS = 16384  # and their rows
