@@ -457,7 +457,8 @@ def run_gpu_fp32acc(config: str, steps: int, warmup: int, chunk_elems, dev):
     """Config-3 style step: bf16 micro-grads accumulated into fp32 .grad; the last
     micro-step's accumulation also yields the global norm (fused), clip_grad_norm
     reuses it, and the step reads fp32 grads. Per iteration: last micro-step
-    accumulate+norm (10 B/param), then clip (no grad read) + step (32 B/param)."""
+    accumulate+norm (10 B/param), then clip (no grad read) + step (30 B/param: fp32 grad 4,
+    master and moments 24, bf16 copy 2)."""
     import torch
 
     import torchure_amd as ta
@@ -501,8 +502,8 @@ def run_gpu_fp32acc(config: str, steps: int, warmup: int, chunk_elems, dev):
         last_microstep_accumulate_norm_ms=round(acc_ms, 4),
         accumulate_GBps=round(10 * n_params / (acc_ms * 1e-3) / 1e9, 1),
         step_ms=round(step_ms, 4),
-        step_bytes_per_param=32,
-        step_GBps=round(32 * n_params / (step_ms * 1e-3) / 1e9, 1),
+        step_bytes_per_param=30,
+        step_GBps=round(30 * n_params / (step_ms * 1e-3) / 1e9, 1),
     )
     del params, work, opt, micro
     torch.cuda.empty_cache()

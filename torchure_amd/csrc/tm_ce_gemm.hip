@@ -10,14 +10,18 @@
 //                        does not depend on scheduling
 //   grad_w_ring_kernel   grad_W = grad_logits^T h (V x D, K = rows), persistent, for rows a
 //                        multiple of 128 (>= 256); grad_w_gemm_kernel otherwise
+//   gemm_tile_kernel     any of the three where those leave CUs idle: 128 x 128 tiles (256 x 256 for
+//                        some grad_h and grad_W), K split where that pays
+// A cost model (tile_us, wide_splits, ring_us) chooses.
 //
-// All three are 256 x 256 output tiles per workgroup on v_mfma_f32_32x32x16_bf16 with fp32
-// accumulation: the ring kernels and grad_h_gemm_kernel on 8 wave64, two a SIMD (each 128 x 64,
-// 128 accumulators), so that one wave's MFMAs run while the other waits; the one-tile kernels on
-// 4 wave64 (each 128 x 128, 256 accumulators in the AGPRs). Every element sees the same MFMA
-// sequence in the ring and one-tile kernels. Operands stream
-// global -> LDS with direct loads (global_load_lds, 16 bytes a lane) into two 64 KB stages of
-// 64-deep K slices. gfx950's LDS has 64 four-byte banks and serves a 16-byte-per-lane read 16
+// The others are 256 x 256 output tiles per workgroup. All are on v_mfma_f32_32x32x16_bf16 with fp32
+// accumulation: the ring kernels, grad_h_gemm_kernel and gemm_tile_kernel on 8 wave64, two a SIMD
+// (each 128 x 64 of a 256 x 256 tile, 128 accumulators), so that one wave's MFMAs run while the
+// other waits; the one-tile kernels on 4 wave64 (each 128 x 128, 256 accumulators in the AGPRs).
+// Every element sees the same MFMA sequence in the ring, the one-tile and the unsplit small-tile
+// kernels. Operands stream
+// global -> LDS with direct loads (global_load_lds, 16 bytes a lane) into two stages (64 KB for a
+// 256 x 256 tile) of 64-deep K slices. gfx950's LDS has 64 four-byte banks and serves a 16-byte-per-lane read 16
 // lanes at a time, so the 16 lanes reading 16 consecutive 128-byte rows must hit 16 different
 // 16-byte bank groups: a row's chunk c sits at slot c ^ ((row >> 1) & 7), which gives rows 2j and
 // 2j+1 (one even, one odd: the two halves of the banks) the slot pattern c ^ j. (The 32-bank
@@ -1437,9 +1441,10 @@ void logits_groups(int64_t tiles_m, int64_t dim, int& gm, int& gn) {
 
 // Which kernel, and how many splits of K: the least estimated time. The model is the launch's
 // rounds over the CUs, times K slices a workgroup, times the measured time of a slice, plus a
-// tile's epilogue, plus, with splits, the fp32 partials' way out and back and the reduction. Its
-// choice among the kernels was within 2% of the best one's time on average over 58 products from
-// 512 x 256 x 4096 to 2102 x 960 x 111,744 (at most 9% on any but one).
+// tile's epilogue, plus, with splits, the fp32 partials' way out and back and the reduction. Over 78
+// products (64-7129 rows, dim 256-2560, vocabulary 1000-152,000) its choice took 0.8% more time than
+// the best one on average, over 3% more in 5 of them, at most 16%. The rounds are those of a
+// whole MI355X's 256 CUs: on a partition with fewer the choice is as valid but may not be the fastest.
 constexpr double kUsSlice256 = 1.42;       // a 64-deep K slice of a 256 x 256 tile, one workgroup a CU
 constexpr double kUsSlice128 = 0.62;       // of a 128 x 128 tile, one workgroup a CU: latency
 constexpr double kUsSlice128Pair = 0.95;   // the same with two a CU

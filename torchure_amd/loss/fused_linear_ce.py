@@ -273,15 +273,15 @@ def splitk_grad_h_fits(rows: int, dim: int, vocab: int) -> bool:
     faster on MI355X: more than SPLITK_GRAD_H_MAX_TILES output tiles of 256 x 256 with dim a
     power of two. With few tiles and K = vocab a library GEMM leaves most of the 256 CUs idle and
     the split-K kernel spreads K over them; with many, the library's kernels fill the chip
-    themselves, and beat this kernel by 1.5-7% when dim is a power of two, but run 12-50% behind
+    themselves, and beat this kernel by 3-11% when dim is a power of two, but run 12-51% behind
     it at the other Qwen3 head widths (ms per call at V = 151,936, split-K / hipBLASLt):
 
         dim   rows 1024      2048           4096           8192
-        1024  0.30 / 0.78    0.65 / 1.08    1.07 / 1.51    2.11 / 2.08
-        2048  0.55 / 0.90    1.04 / 1.65    2.06 / 2.01    4.11 / 3.95
-        2560  0.69 / 1.03    1.35 / 1.90    2.82 / 3.52    5.42 / 7.40
-        4096  1.07 / 1.88    2.11 / 2.03    4.16 / 3.88    8.35 / 7.76
-        5120  1.43 / 1.89    3.11 / 3.48    5.70 / 7.07    11.34 / 13.41
+        1024  0.28 / 0.72    0.62 / 1.03    1.07 / 1.44    2.06 / 1.99
+        2048  0.51 / 0.89    1.00 / 1.61    2.00 / 1.93    4.13 / 3.69
+        2560  0.66 / 1.00    1.33 / 1.84    2.75 / 3.38    5.24 / 7.44
+        4096  1.03 / 1.82    2.05 / 1.91    4.11 / 3.66    8.13 / 7.40
+        5120  1.38 / 1.87    2.98 / 3.34    5.58 / 6.85    10.85 / 13.16
     """
     if not _grad_h_takes(rows, dim, vocab) or rows % 256 or dim % 256 or vocab % 64:
         return False
@@ -311,8 +311,8 @@ def grad_h_gemm_fits(rows: int, dim: int, vocab: int) -> bool:
         8000 x 2560 (320)      104 / 100     221 / 227    358 / 253    536 / 423     804 / 697    1219 / 1686
 
     With few tiles the library leaves CUs idle. With many it fills the chip and this kernel's splits
-    only cost their partials, until K is long: past some 16,000 the library's kernels for these
-    widths fall behind by a quarter to a half. The lower line is not one of speed: a ragged chunk of
+    only cost their partials, until K is long: past some 16,000 (20,000 at 320 tiles) the library's
+    kernels for these widths fall behind by a quarter to a half. The lower line is not one of speed: a ragged chunk of
     a vocabulary up to 4096 keeps the library's product and its bits, though this kernel would be
     the faster there too (from level to 2x at up to 96 tiles)."""
     if splitk_grad_h_fits(rows, dim, vocab):
