@@ -231,7 +231,7 @@ def test_op_grad_h_choice_above_64_tiles(d, split):
     (2046, 1216, 4161, True),   # 40 tiles
 ])
 def test_op_grad_h_choice_on_ragged_chunks(n, d, v, own):
-    """One ragged chunk: grad_h is this build's product, or torch.matmul's on the padded logits, times
+    """One ragged chunk: grad_h is this package's product, or torch.matmul's on the padded logits, times
     the bf16 scale, bit for bit."""
     from torchure_amd.loss import fused_linear_cross_entropy
     from torchure_amd.loss.fused_linear_ce import padded_rows, padded_vocab

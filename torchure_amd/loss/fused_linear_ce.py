@@ -7,14 +7,14 @@ semantics, :22-24), computes grad_hidden and grad_weight during the forward pass
 (:42-58) and scales them in place by grad_out / n_valid in backward (:94-127).
 
 Per chunk of rows:
-  logits = h @ W^T                  bf16 GEMM: tm_ce_logits_ld_bf16, this build's MFMA GEMM, for dim a
+  logits = h @ W^T                  bf16 GEMM: tm_ce_logits_ld_bf16, this package's MFMA GEMM, for dim a
                                     multiple of 64 (torch.matmul on other shapes)
   tm_ce_rows_padded_bf16            one fused kernel: logsumexp, per-row loss and
                                     grad_logits = bf16(softmax - onehot), in place
   grad_h = grad_logits @ W          bf16 GEMM: tm_ce_grad_h_ld_bf16, a split-K MFMA GEMM with a
                                     fixed-order reduction, where grad_h_gemm_fits; hipBLASLt on
                                     other shapes
-  grad_W += grad_logits^T @ h       bf16 GEMM: tm_ce_grad_w_ld_bf16, this build's MFMA GEMM, for dim
+  grad_W += grad_logits^T @ h       bf16 GEMM: tm_ce_grad_w_ld_bf16, this package's MFMA GEMM, for dim
                                     a multiple of 64 (and rows too where the logits are unpadded;
                                     torch.matmul otherwise), then tm_ce_grad_w_fold into fp32
 The chunk's logits are padded to whole MFMA steps: rows a multiple of 64 elements (padded_vocab)
@@ -194,7 +194,7 @@ def _mean_loss(row_loss, labels, n, ignore_index, lib, stream):
 
 
 def logits_gemm_fits(h: torch.Tensor, w: torch.Tensor) -> bool:
-    """Chunks whose logits run on this build's GEMM (tm_ce_logits_bf16): bf16 operands, both
+    """Chunks whose logits run on this package's GEMM (tm_ce_logits_bf16): bf16 operands, both
     contiguous and 16-byte aligned, dim a multiple of 64. Other shapes take torch.matmul."""
     return (h.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and h.dim() == 2 and w.dim() == 2
             and h.shape[1] == w.shape[1] and h.shape[1] % 64 == 0 and h.shape[0] > 0 and w.shape[0] > 0
@@ -225,7 +225,7 @@ def padded_vocab(vocab: int) -> int:
 
 
 def grad_w_gemm_fits(g: torch.Tensor, h: torch.Tensor) -> bool:
-    """Unpadded chunks whose grad_W runs on this build's GEMM: bf16 operands, both contiguous and
+    """Unpadded chunks whose grad_W runs on this package's GEMM: bf16 operands, both contiguous and
     16-byte aligned, vocab and dim multiples of 8. Other shapes take torch.matmul."""
     return (g.dtype == torch.bfloat16 and h.dtype == torch.bfloat16 and g.dim() == 2 and h.dim() == 2
             and g.shape[0] == h.shape[0] and g.shape[0] > 0 and g.shape[1] % 8 == 0
@@ -294,11 +294,11 @@ RAGGED_GRAD_H_LONG_VOCAB = 16384
 
 
 def grad_h_gemm_fits(rows: int, dim: int, vocab: int) -> bool:
-    """Padded chunks whose grad_h runs on this build's GEMM: those ``splitk_grad_h_fits`` accepts,
+    """Padded chunks whose grad_h runs on this package's GEMM: those ``splitk_grad_h_fits`` accepts,
     and of the ragged ones (rows or dim off a multiple of 256, a vocabulary off a multiple of 64)
     those of a vocabulary above 4096, of at most 64 tiles at a power-of-two width and 96 at others,
     and at those other widths of any more tiles from a vocabulary of RAGGED_GRAD_H_LONG_VOCAB up.
-    us per call on MI355X, this build / hipBLASLt on the same padded logits:
+    us per call on MI355X, this package / hipBLASLt on the same padded logits:
 
         rows x dim (tiles)    vocab 1984     4097-5001      7296         12001         20032         32001
         1184 x  384  (10)       15 /  20      18 /  25     22 /  33
@@ -522,7 +522,7 @@ def _fp32_chunks(hidden, weight, labels, ignore_index, n, v, chunk, grad, want_h
 def _chunks_unpadded(hidden, weight, labels, ignore_index, n, v, chunk, mode, want_h, want_w):
     """The chunk loop for what ``_run_chunks`` does not take (a dim off 64, unaligned or strided
     operands, no rows) or finds no memory for: logits rows vocab elements apart, library products
-    where this build's GEMMs do not fit. Returns what ``_run_chunks`` does."""
+    where this package's GEMMs do not fit. Returns what ``_run_chunks`` does."""
     lib = _native.lib()
     stream = _native.stream_handle(hidden.device)
     hb, w = _bf16_operands(hidden, weight, mode)  # cast once, not per chunk
